@@ -4,7 +4,8 @@
 // sort by probability, a pass that drops near-identical boxes of different classes, a greedy
 // pass inside every (image, class) group, each of them a sequential loop.  Here the number of
 // records stays on the device, so every launch is sized for the capacity and the workgroups past
-// the live count leave at once.  Steps:
+// the live count leave at once.  Lists of at most 512 records take one workgroup, lists of ordinary length go
+// image by image (both further down); the steps for the longest ones:
 //   1. LSD radix sort (8-bit digits) of (probability descending, emission order) -> global rank;
 //   2. two to four more stable passes on (image, class) -> groups contiguous, rank order inside;
 //   3. duplicate pass as a fixed point: a record is decided once every conflicting record of
@@ -16,6 +17,7 @@
 #include "pixienn_hip_test.h"
 
 #include <atomic>
+#include <type_traits>
 
 namespace pxh {
 namespace {
@@ -605,6 +607,450 @@ __global__ __launch_bounds__(kWide) void nms_small_kernel(const pxh_detection* r
     if (t == 0) *kept_count = static_cast<int>(total);
 }
 
+// ---------------------------------------------------------------- lists of ordinary length
+// Every decision of nms is taken inside one image, so the records are grouped by image first and
+// nothing is sorted: six launches in place of the sorting path's forty-five, whose cost at the few
+// thousand records of a validation batch is the launches and the latency of short dependent steps
+// (7126 records of 16 images in a list for 32768: 440 us in kernels, here 60).
+//   1. images are counted per tile of 1024 records, 2. the records' keys are laid out image by image,
+//      in any order inside one;
+//   3. a record's place in its image is the number of smaller keys there, counted directly: n^2 of the
+//      cheapest comparisons per image, all independent, where a radix sort is a chain of thirty launches;
+//   4. every pair of an image is looked at once, 64 x 64 pairs per wave: bit masks of the earlier
+//      records that conflict, one for each of the two passes (other class and overlap above 0.9, same
+//      class and overlap above the threshold);
+//   5. one workgroup per image settles both passes on the masks alone, the states as bit sets in LDS;
+//   6. a survivor's place in the whole list is the number of survivors before it in each image, found
+//      by bisection, one lane per image.
+// A mask has 64 words, of which as many that are not empty are stored as 10 MB hold for the whole list (all
+// of them up to 8738 records, eight for 65536), so that the longest list fits the library's first workspace.
+// Step 5 looks at the pairs of a further one again, and at those of a set bit in an image of more than 4096
+// records, where a bit stands for 2, 4, ... 16 neighbouring places.
+constexpr int kImageCapacity = 65536;                 // longest list: a state bit set is 8 KB of LDS
+constexpr int kImageBatch = kWide;                    // most images: one lane each
+constexpr int kMaskWords = 64;
+constexpr size_t kMaskBytes = 10u << 20;
+
+// words of a mask that are stored, each with the byte that says which one it is
+int mask_slots(int capacity)
+{
+    const size_t fit = kMaskBytes / (2 * 9 * static_cast<size_t>(capacity));
+    return fit < 8 ? 8 : fit > kMaskWords ? kMaskWords : static_cast<int>(fit);
+}
+constexpr int kBitSetWords = kImageCapacity / 64;
+
+// 64 places of one image
+struct PlaceBlock {
+    uint32_t image_begin, image_end, first, image;
+};
+
+struct ImageArgs {
+    const pxh_detection* records;
+    const int* count;
+    int capacity, batch, classes;
+    float threshold;
+    uint32_t* tile_images;    // [tile][image] records
+    uint32_t* image_begin;    // [batch + 1]
+    uint32_t* block_count;
+    PlaceBlock* blocks;
+    uint64_t* loose_key;      // image by image, unordered
+    uint32_t* loose_source;
+    uint64_t* key;            // image by image, in rank order; from here on by place
+    uint32_t* source;
+    float4* box;
+    uint32_t* cls;
+    uint32_t* group_index;    // earlier records of the same image and class
+    int mask_slots;
+    uint32_t* slots;          // stored words of a place's masks: [0] other classes, [1] same class << 8
+    uint8_t* ids[2];          // [slot][place]: which word it is
+    uint64_t* masks[2];       // [slot][place]
+    uint64_t* beyond[2];      // words that are not empty and not stored
+    uint64_t* kept_key;       // survivors, image by image, in rank order
+    uint32_t* kept_source;
+    uint32_t* kept_images;    // survivors per image
+};
+
+__device__ __forceinline__ uint32_t image_of(const pxh_detection& d, int batch)
+{
+    return static_cast<uint32_t>(min(max(d.batch, 0), batch - 1));
+}
+
+// log2 of the places that a mask bit stands for
+__device__ __forceinline__ int mask_grain(uint32_t places)
+{
+    int g = 0;
+    while ((static_cast<uint32_t>(kMaskWords * 64) << g) < places) ++g;
+    return g;
+}
+
+__global__ __launch_bounds__(kWide) void nms_count_images_kernel(ImageArgs a)
+{
+    __shared__ uint32_t bins[kImageBatch];
+    const uint32_t n = live_count(a.count, a.capacity);
+    if (blockIdx.x * kWide >= n) return;
+    const uint32_t t = threadIdx.x;
+    bins[t] = 0;
+    __syncthreads();
+    const uint32_t i = blockIdx.x * kWide + t;
+    if (i < n) atomicAdd(&bins[image_of(a.records[i], a.batch)], 1u);
+    __syncthreads();
+    if (t < static_cast<uint32_t>(a.batch)) a.tile_images[blockIdx.x * a.batch + t] = bins[t];
+}
+
+// Every workgroup works out where each image begins for itself; the first also writes it down, with the
+// blocks of 64 places of all images.
+__global__ __launch_bounds__(kWide) void nms_group_images_kernel(ImageArgs a)
+{
+    __shared__ uint32_t scan_lds[kWide / kWave + 1];
+    __shared__ uint32_t cursor[kImageBatch];
+    const uint32_t n = live_count(a.count, a.capacity);
+    const uint32_t t = threadIdx.x;
+    if (blockIdx.x * kWide >= n && blockIdx.x != 0) return;
+    const uint32_t tiles = (n + kWide - 1) / kWide;
+    uint32_t before = 0, all = 0;
+    if (t < static_cast<uint32_t>(a.batch)) {
+        for (uint32_t tile = 0; tile < tiles; ++tile) {
+            const uint32_t c = a.tile_images[tile * a.batch + t];
+            if (tile < blockIdx.x) before += c;
+            all += c;
+        }
+    }
+    uint32_t total;
+    const uint32_t begin = wide_exclusive_scan(all, scan_lds, total);
+    cursor[t] = begin + before;
+    __syncthreads();
+    if (blockIdx.x == 0) {
+        const uint32_t mine = (all + 63) / 64;
+        const uint32_t first_block = wide_exclusive_scan(mine, scan_lds, total);
+        if (t <= static_cast<uint32_t>(a.batch) && t < kWide) a.image_begin[t] = begin;
+        if (t == 0) {
+            *a.block_count = total;
+            a.image_begin[a.batch] = n;
+        }
+        for (uint32_t k = 0; k < mine; ++k) a.blocks[first_block + k] = PlaceBlock{ begin, begin + all, begin + 64 * k, t };
+    }
+    const uint32_t i = blockIdx.x * kWide + t;
+    if (i >= n) return;
+    const pxh_detection d = a.records[i];
+    const uint32_t at = atomicAdd(&cursor[image_of(d, a.batch)], 1u);
+    a.loose_key[at] = (static_cast<uint64_t>(descending_bits(d.prob)) << 32) | d.order;
+    a.loose_source[at] = i;
+}
+
+__device__ __forceinline__ uint64_t key_of_lane(uint64_t key, int lane)
+{
+    const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(key), lane);
+    const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(key >> 32), lane);
+    return (static_cast<uint64_t>(hi) << 32) | lo;
+}
+
+// One workgroup per 64 records, a lane per record in each of its 16 waves, the waves side by side over
+// the image's keys.  Records of equal key keep their input order.
+__global__ __launch_bounds__(kWide) void nms_place_kernel(ImageArgs a)
+{
+    __shared__ uint32_t smaller[kWave];
+    if (live_count(a.count, a.capacity) == 0 || blockIdx.x >= *a.block_count) return;
+    const PlaceBlock b = a.blocks[blockIdx.x];
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    const uint32_t wave = threadIdx.x / kWave;
+    if (threadIdx.x < kWave) smaller[threadIdx.x] = 0;
+    __syncthreads();
+    const bool live = b.first + lane < b.image_end;
+    const uint32_t p = live ? b.first + lane : b.first;
+    const uint64_t mine = a.loose_key[p];
+    const uint32_t source = a.loose_source[p];
+    uint32_t rank = 0;
+    for (uint32_t q0 = b.image_begin + wave * kWave; q0 < b.image_end; q0 += kWide) {
+        const uint32_t here = min(static_cast<uint32_t>(kWave), b.image_end - q0);
+        // lanes past the end carry the largest key: none is smaller than any record's
+        const uint64_t keys = lane < here ? a.loose_key[q0 + lane] : ~0ull;
+        bool equal = false;
+#pragma unroll 16
+        for (int j = 0; j < kWave; ++j) {
+            const uint64_t k = key_of_lane(keys, j);
+            rank += k < mine ? 1u : 0u;
+            equal |= k == mine;
+        }
+        if (__ballot(equal)) {
+            for (uint32_t j = 0; j < here; ++j)
+                if (key_of_lane(keys, static_cast<int>(j)) == mine && a.loose_source[q0 + j] < source) ++rank;
+        }
+    }
+    if (rank) atomicAdd(&smaller[lane], rank);
+    __syncthreads();
+    if (wave != 0 || !live) return;
+    const uint32_t place = b.image_begin + smaller[lane];
+    const pxh_detection d = a.records[source];
+    a.key[place] = mine;
+    a.source[place] = source;
+    a.box[place] = normalized_rect(d);
+    a.cls[place] = static_cast<uint32_t>(min(max(d.class_index, 0), a.classes - 1));
+}
+
+// One workgroup per 64 places, a lane per place, a wave per word of its masks: the earlier places that
+// the word stands for are loaded 64 at a time and handed round lane by lane.
+__global__ __launch_bounds__(kWide) void nms_conflicts_kernel(ImageArgs a)
+{
+    __shared__ uint64_t beyond[2][kWave];
+    __shared__ uint32_t slots[2][kWave];
+    __shared__ uint32_t index[kWave];
+    if (live_count(a.count, a.capacity) == 0 || blockIdx.x >= *a.block_count) return;
+    const PlaceBlock b = a.blocks[blockIdx.x];
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    const uint32_t wave = threadIdx.x / kWave;
+    if (threadIdx.x < kWave) {
+        for (int pass = 0; pass < 2; ++pass) {
+            beyond[pass][threadIdx.x] = 0;
+            slots[pass][threadIdx.x] = 0;
+        }
+        index[threadIdx.x] = 0;
+    }
+    __syncthreads();
+    const bool live = b.first + lane < b.image_end;
+    const uint32_t p = live ? b.first + lane : b.first;
+    const float4 box = a.box[p];
+    const uint32_t cls = a.cls[p];
+    const int grain = mask_grain(b.image_end - b.image_begin);
+    const uint32_t upto = min(b.first + kWave, b.image_end);
+    uint32_t same_before = 0;
+    for (uint32_t word = wave; ; word += kWide / kWave) {
+        const uint32_t q_first = b.image_begin + ((word * 64u) << grain);
+        if (word >= kMaskWords || q_first >= upto) break;
+        const uint32_t q_end = min(q_first + (64u << grain), upto);
+        uint64_t found[2] = { 0, 0 };
+        for (uint32_t q0 = q_first; q0 < q_end; q0 += kWave) {
+            const uint32_t mine = min(q0 + lane, q_end - 1);
+            const float4 their_box = a.box[mine];
+            const int their_class = static_cast<int>(a.cls[mine]);
+            const int here = static_cast<int>(min(static_cast<uint32_t>(kWave), q_end - q0));
+            for (int j = 0; j < here; ++j) {
+                const float4 other = make_float4(from_lane(their_box.x, j), from_lane(their_box.y, j),
+                                                 from_lane(their_box.z, j), from_lane(their_box.w, j));
+                const bool same = static_cast<uint32_t>(__builtin_amdgcn_readlane(their_class, j)) == cls;
+                if (q0 + j < p && live) {
+                    same_before += same ? 1u : 0u;
+                    if (overlaps_above(box, other, same ? a.threshold : kDuplicateOverlap)) {
+                        const uint64_t bit = 1ull << ((q0 - q_first + j) >> grain);
+                        if (same) found[1] |= bit;
+                        else found[0] |= bit;
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int pass = 0; pass < 2; ++pass) {
+            if (!found[pass]) continue;
+            const uint32_t slot = atomicAdd(&slots[pass][lane], 1u);
+            if (slot < static_cast<uint32_t>(a.mask_slots)) {
+                a.masks[pass][static_cast<size_t>(slot) * a.capacity + p] = found[pass];
+                a.ids[pass][static_cast<size_t>(slot) * a.capacity + p] = static_cast<uint8_t>(word);
+            } else {
+                atomicOr(reinterpret_cast<unsigned long long*>(&beyond[pass][lane]), 1ull << word);
+            }
+        }
+    }
+    if (same_before) atomicAdd(&index[lane], same_before);
+    __syncthreads();
+    if (wave != 0 || !live) return;
+    for (int pass = 0; pass < 2; ++pass) a.beyond[pass][p] = beyond[pass][lane];
+    const uint32_t most = a.mask_slots;
+    a.slots[p] = min(slots[0][lane], most) | min(slots[1][lane], most) << 8;
+    a.group_index[p] = index[lane];
+}
+
+__device__ __forceinline__ uint64_t load_bits(const uint64_t* set, uint32_t word)
+{
+    return __hip_atomic_load(set + word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+__device__ __forceinline__ void set_bit(uint64_t* set, uint32_t at)
+{
+    atomicOr(reinterpret_cast<unsigned long long*>(set + (at >> 6)), 1ull << (at & 63));
+}
+
+// What the records of lower rank say about place p (places are relative to the image here): 1 = a kept
+// one conflicts, 2 = none does but one that may is undecided, 0 = neither.  Every place below `open` is
+// decided; `from`: places below it have been looked at before.
+struct Standing {
+    int pass;
+    uint32_t image_begin, p, from, open;
+    int grain;
+    const uint64_t* kept;
+    const uint64_t* gone;
+};
+
+// The same for places [first, first + count) of one word of the bit sets, pair by pair.
+__device__ __forceinline__ int recheck(const ImageArgs& a, const Standing& s, uint32_t first, uint32_t count,
+                                       const float4& box, uint32_t cls)
+{
+    const uint32_t word = first >> 6;
+    // `kept` is read first: a bit that is set in between shows up as undecided, never as absent
+    const uint64_t kept = load_bits(s.kept, word);
+    uint64_t bits = first + 64 > s.open ? kept | ~load_bits(s.gone, word) : kept;
+    if (count < 64) bits &= ((1ull << count) - 1) << (first & 63);
+    if (word == s.p >> 6) bits &= (1ull << (s.p & 63)) - 1;
+    bool pending = false;
+    for (; bits; bits &= bits - 1) {
+        const int bit = __builtin_ctzll(bits);
+        const uint32_t q = s.image_begin + word * 64 + bit;
+        if ((a.cls[q] == cls) != (s.pass == 1)) continue;
+        if (!overlaps_above(box, a.box[q], s.pass == 0 ? kDuplicateOverlap : a.threshold)) continue;
+        if ((kept >> bit) & 1) return 1;
+        pending = true;
+    }
+    return pending ? 2 : 0;
+}
+
+__device__ __forceinline__ int conflict_state(const ImageArgs& a, const Standing& s)
+{
+    const uint32_t place = s.image_begin + s.p;
+    const int stored = (a.slots[place] >> (8 * s.pass)) & 0xFF;
+    if (stored == 0) return 0;                      // nothing is kept beyond the stored words either
+    uint64_t beyond = stored == a.mask_slots ? a.beyond[s.pass][place] : 0ull;
+    bool pending = false;
+    float4 box = make_float4(0, 0, 0, 0);
+    uint32_t cls = 0;
+    if (beyond || s.grain) {
+        box = a.box[place];
+        cls = a.cls[place];
+    }
+    for (int slot = 0; slot < stored; ++slot) {
+        const size_t at = static_cast<size_t>(slot) * a.capacity + place;
+        const uint32_t word = a.ids[s.pass][at];
+        if (((word + 1) * 64) << s.grain <= s.from) continue;
+        const uint64_t mask = a.masks[s.pass][at];
+        if (s.grain == 0) {
+            if (mask & load_bits(s.kept, word)) return 1;
+            pending = pending || (mask & ~load_bits(s.gone, word)) != 0;
+            continue;
+        }
+        for (uint64_t bits = mask; bits; bits &= bits - 1) {
+            const uint32_t first = (word * 64 + static_cast<uint32_t>(__builtin_ctzll(bits))) << s.grain;
+            const int state = recheck(a, s, first, 1u << s.grain, box, cls);
+            if (state == 1) return 1;
+            pending = pending || state == 2;
+        }
+    }
+    for (; beyond; beyond &= beyond - 1) {          // words that were not stored: all of their places
+        const uint32_t first = (static_cast<uint32_t>(__builtin_ctzll(beyond)) * 64) << s.grain;
+        const uint32_t end = min(first + (64u << s.grain), s.p);
+        for (uint32_t q = max(first, s.from & ~63u); q < end; q += 64) {
+            const int state = recheck(a, s, q, 64, box, cls);
+            if (state == 1) return 1;
+            pending = pending || state == 2;
+        }
+    }
+    return pending ? 2 : 0;
+}
+
+// One workgroup per image, a lane per place, 1024 places at a time in rank order, so that only conflicts
+// among those can be pending.  Rounds until each of them is decided: a round decides at least the
+// undecided place of lowest rank; the bound makes the exit unconditional.
+__global__ __launch_bounds__(kWide) void nms_settle_kernel(ImageArgs a)
+{
+    __shared__ uint64_t kept[kBitSetWords], gone[kBitSetWords];
+    __shared__ uint32_t word_first[kBitSetWords];
+    __shared__ uint32_t scan_lds[kWide / kWave + 1];
+    static_assert(kBitSetWords == kWide, "one word of a bit set per lane");
+    const uint32_t t = threadIdx.x;
+    if (live_count(a.count, a.capacity) == 0) return;
+    const uint32_t begin = a.image_begin[blockIdx.x];
+    const uint32_t places = a.image_begin[blockIdx.x + 1] - begin;
+    gone[t] = 0;
+    Standing s{};
+    s.image_begin = begin;
+    s.grain = mask_grain(places);
+    s.kept = kept;
+    s.gone = gone;
+    for (s.pass = 0; s.pass < 2; ++s.pass) {
+        // the second pass starts from what the first dropped: absent there
+        kept[t] = 0;
+        __syncthreads();
+        for (s.open = 0; s.open < places; s.open += kWide) {
+            s.p = s.open + t;
+            s.from = 0;
+            bool undecided = s.p < places;
+            if (undecided && s.pass == 1) {
+                if ((load_bits(gone, s.p >> 6) >> (s.p & 63)) & 1) {
+                    undecided = false;
+                } else if (a.group_index[begin + s.p] >= static_cast<uint32_t>(kGroupVisit)) {
+                    // places past the first 1024 of a group are never visited: they stay
+                    set_bit(kept, s.p);
+                    undecided = false;
+                }
+            }
+            for (uint32_t round = 0; round <= kWide; ++round) {
+                if (undecided) {
+                    const int state = conflict_state(a, s);
+                    if (state != 2) {
+                        set_bit(state == 1 ? gone : kept, s.p);
+                        undecided = false;
+                    }
+                    s.from = s.open;
+                }
+                if (__syncthreads_or(undecided) == 0) break;
+            }
+        }
+        __syncthreads();
+    }
+    const uint64_t mine = kept[t];
+    uint32_t total;
+    word_first[t] = wide_exclusive_scan(static_cast<uint32_t>(__popcll(mine)), scan_lds, total);
+    __syncthreads();
+    for (uint32_t p = t; p < places; p += kWide) {
+        const uint64_t word = kept[p >> 6];
+        if (!((word >> (p & 63)) & 1)) continue;
+        const uint32_t at = begin + word_first[p >> 6] + __popcll(word & ((1ull << (p & 63)) - 1));
+        a.kept_key[at] = a.key[begin + p];
+        a.kept_source[at] = a.source[begin + p];
+    }
+    if (t == 0) a.kept_images[blockIdx.x] = total;
+}
+
+// One wave per survivor, a lane per other image: how many of that image's survivors come before it.
+__global__ __launch_bounds__(kWide) void nms_merge_images_kernel(ImageArgs a, pxh_detection* kept, int* kept_count)
+{
+    const uint32_t n = live_count(a.count, a.capacity);
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    const uint32_t wave = threadIdx.x / kWave;
+    if (blockIdx.x == 0 && wave == 0) {
+        uint32_t sum = 0;
+        if (n)
+            for (uint32_t i = lane; i < static_cast<uint32_t>(a.batch); i += kWave) sum += a.kept_images[i];
+#pragma unroll
+        for (int off = kWave / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, kWave);
+        if (lane == 0) *kept_count = static_cast<int>(sum);
+    }
+    if (n == 0 || blockIdx.x >= *a.block_count) return;
+    const PlaceBlock b = a.blocks[blockIdx.x];
+    const uint32_t end = min(b.first + kWave, b.image_begin + a.kept_images[b.image]);
+    for (uint32_t at = b.first + wave; at < end; at += kWide / kWave) {
+        const uint64_t key = a.kept_key[at];
+        const uint32_t source = a.kept_source[at];
+        uint32_t before = 0;
+        for (uint32_t i = lane; i < static_cast<uint32_t>(a.batch); i += kWave) {
+            if (i == b.image) {
+                before += at - b.image_begin;
+                continue;
+            }
+            const uint32_t first = a.image_begin[i];
+            uint32_t lo = first, hi = first + a.kept_images[i];
+            while (lo < hi) {
+                const uint32_t mid = lo + (hi - lo) / 2;
+                const uint64_t k = a.kept_key[mid];
+                if (k < key || (k == key && a.kept_source[mid] < source)) lo = mid + 1;
+                else hi = mid;
+            }
+            before += lo - first;
+        }
+#pragma unroll
+        for (int off = kWave / 2; off > 0; off >>= 1) before += __shfl_xor(before, off, kWave);
+        constexpr uint32_t kRecordWords = sizeof(pxh_detection) / 4;
+        if (lane < kRecordWords)
+            reinterpret_cast<uint32_t*>(kept + before)[lane] = reinterpret_cast<const uint32_t*>(a.records + source)[lane];
+    }
+}
+
 size_t align256(size_t b) { return (b + 255) & ~static_cast<size_t>(255); }
 
 struct Workspace {
@@ -651,6 +1097,53 @@ Workspace carve(void* base, int capacity)
     return w;
 }
 
+// Which lists go by image.  Measured on both paths, us sorted -> by image: 600 records of 64 images 161 -> 34,
+// 7000 of 16 336 -> 78, 60000 of 32 1172 -> 388, 8000 of one image 1447 -> 674.  One workgroup settles an
+// image, so a list that may all lie in one and is longer than that stays with the sweeps of the sorting
+// path, which spread over the chip (30000 records of one image around 20 places: 8.0 ms, by image 16.9).
+// More than 2048 places per image of the batch make such a list possible by their number; fewer still allow
+// it, at that price, where nearly all records are of one image.
+bool by_image(int capacity, int batch)
+{
+    return batch <= kImageBatch && capacity <= kImageCapacity && (capacity <= 8192 || capacity / 2048 <= batch);
+}
+
+// The same for the launches by image; `args` gets every pointer.
+size_t carve_images(void* base, int capacity, int batch, ImageArgs& args)
+{
+    const size_t cap = static_cast<size_t>(capacity);
+    const size_t tiles = (cap + kWide - 1) / kWide, images = static_cast<size_t>(batch);
+    args.mask_slots = mask_slots(capacity);
+    char* p = static_cast<char*>(base);
+    size_t at = 0;
+    auto take = [&](auto*& out, size_t count) {
+        using T = std::remove_reference_t<decltype(*out)>;
+        out = p ? reinterpret_cast<T*>(p + at) : nullptr;
+        at += align256(count * sizeof(T));
+    };
+    take(args.tile_images, tiles * images);
+    take(args.image_begin, images + 1);
+    take(args.block_count, 1);
+    take(args.blocks, cap / 64 + images + 1);
+    take(args.loose_key, cap);
+    take(args.loose_source, cap);
+    take(args.key, cap);
+    take(args.source, cap);
+    take(args.box, cap);
+    take(args.cls, cap);
+    take(args.group_index, cap);
+    take(args.slots, cap);
+    for (int k = 0; k < 2; ++k) {
+        take(args.ids[k], cap * args.mask_slots);
+        take(args.beyond[k], cap);
+        take(args.masks[k], cap * args.mask_slots);
+    }
+    take(args.kept_key, cap);
+    take(args.kept_source, cap);
+    take(args.kept_images, images);
+    return at;
+}
+
 std::atomic<int> g_sweeps{ 6 };      // parallel sweeps of the duplicate pass before the per-image loop takes over
 
 }  // namespace
@@ -663,7 +1156,12 @@ extern "C" {
 size_t pxh_nms_workspace_bytes(int capacity)
 {
     if (capacity <= 0) return 0;
-    return carve(nullptr, capacity).bytes;
+    const size_t sorted = carve(nullptr, capacity).bytes;
+    if (capacity <= kSmall) return sorted;
+    // the most that any batch asks for; a longer list's bytes also serve every shorter one
+    ImageArgs args{};
+    const size_t by_image = carve_images(nullptr, capacity < kImageCapacity ? capacity : kImageCapacity, kImageBatch, args);
+    return by_image > sorted ? by_image : sorted;
 }
 
 int pxh_debug_nms_sweeps(int sweeps)
@@ -691,6 +1189,27 @@ int pxh_nms(const pxh_detection* records, const int* count, int capacity, int ba
         return check_launch("pxh_nms");
     }
     void* ws;
+    if (by_image(capacity, batch)) {
+        ImageArgs a{};
+        int rc = resolve_workspace(workspace, workspace_bytes, carve_images(nullptr, capacity, batch, a), &ws,
+                                   as_stream(stream));
+        if (rc) return rc;
+        carve_images(ws, capacity, batch, a);
+        a.records = records; a.count = count; a.capacity = capacity; a.batch = batch; a.classes = classes;
+        a.threshold = threshold;
+        hipStream_t s = as_stream(stream);
+        const dim3 wide(kWide), per_tile(grid_for(capacity, kWide));
+        // blocks of 64 places: every image but the last may leave one of them partly empty
+        const int images = batch < capacity ? batch : capacity;
+        const dim3 per_block(static_cast<unsigned>(capacity / 64 + images));
+        hipLaunchKernelGGL(nms_count_images_kernel, per_tile, wide, 0, s, a);
+        hipLaunchKernelGGL(nms_group_images_kernel, per_tile, wide, 0, s, a);
+        hipLaunchKernelGGL(nms_place_kernel, per_block, wide, 0, s, a);
+        hipLaunchKernelGGL(nms_conflicts_kernel, per_block, wide, 0, s, a);
+        hipLaunchKernelGGL(nms_settle_kernel, dim3(batch), wide, 0, s, a);
+        hipLaunchKernelGGL(nms_merge_images_kernel, per_block, wide, 0, s, a, kept, kept_count);
+        return check_launch("pxh_nms");
+    }
     int rc = resolve_workspace(workspace, workspace_bytes, carve(nullptr, capacity).bytes, &ws, as_stream(stream));
     if (rc) return rc;
     const Workspace w = carve(ws, capacity);

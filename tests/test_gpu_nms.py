@@ -183,3 +183,33 @@ def test_detections_of_two_heads_then_nms(ops, oracle):
     # the device's own records (pixel boxes may differ from the checker's by a truncation) are the input
     kept, kept_count = ops.nms(records, count, N, K, 0.45)
     same(ops.nms_to_host(kept, kept_count), oracle.nms(got_all, 0.45), "two heads")
+
+
+@pytest.mark.parametrize("n,used,batch,capacity", [
+    (513, 1, 1, 513), (1024, 16, 16, 1024), (1025, 1024, 1024, 1025),      # edges of the tiles, most images
+    (4096, 1, 1, 4097), (4097, 1, 1, 4097), (8192, 1, 1, 8192),            # one and two places per mask bit
+    (9000, 1, 16, 32768), (9000, 1, 32, 65536),                            # four, few mask words stored
+    (1025, 1025, 1025, 1025), (8193, 1, 1, 8193), (700, 3, 31, 65536), (6000, 2, 33, 65537),   # the sorting path
+], ids=lambda v: str(v))
+@pytest.mark.parametrize("classes,clusters,thr", [(1, 40, 0.5), (7, 3, 0.3)])
+def test_nms_by_image_and_by_sorting(ops, oracle, n, used, batch, capacity, classes, clusters, thr):
+    """Whole results at the limits of the two paths for lists above 512; spread-out clusters leave many
+    survivors, dense ones more conflicting words than a record stores, one class more than 1024 members."""
+    rec = random_detections(oracle, 100 + n + classes, n, used, classes, clusters)
+    rec["order"] = np.random.Generator(np.random.Philox(key=n)).permutation(n)
+    rec["prob"][::7] = rec["prob"][0]                             # ties keep the order
+    want = oracle.nms(rec[np.argsort(rec["order"])], thr)
+    same(run(ops, rec, batch, classes, thr, capacity), want, "%d of %d images" % (n, used))
+
+
+@pytest.mark.parametrize("capacity,batch", [(70000, 5), (2000, 1025)])
+def test_nms_sorting_path_chains(ops, oracle, capacity, batch):
+    """Dependency chains longer than the sorting path's sweeps (lists of more than 65536 or 1024 images)."""
+    parts = []
+    for b in range(5):
+        c = chain(oracle, 30 + b, 0.92, 3)
+        c["batch"] = b
+        parts.append(c)
+    rec = np.concatenate(parts)
+    rec["order"] = np.arange(len(rec))
+    same(run(ops, rec, batch, 3, 0.95, capacity), oracle.nms(rec, 0.95), "chains")
