@@ -2,6 +2,7 @@
 // Index and copy work is bit-exact against the CPU layers; accumulation follows their order.
 #include "stream.h"
 
+#include <algorithm>
 #include <cfloat>
 
 namespace pxh {
@@ -12,19 +13,13 @@ struct PoolGeom {
 };
 
 // ------------------------------------------------------------------ max-pool, any geometry
-// One output per lane.  Taps in row-major order; the first in-bounds tap is taken, later taps
-// only when strictly greater (include/MaxPoolLayer.h:106-127 of the reference).
-__global__ __launch_bounds__(kBlock) void maxpool_fwd_generic_kernel(const float* in, float* out, int* indexes,
-                                                                     uint32_t total, PoolGeom g, FastDiv by_ow,
-                                                                     FastDiv by_oh)
+// One window.  Taps in row-major order; the first in-bounds tap is taken, later taps only when strictly
+// greater (include/MaxPoolLayer.h:106-127 of the reference).
+__device__ __forceinline__ void scan_window(const float* in, const PoolGeom& g, uint32_t plane, uint32_t oy, uint32_t ox,
+                                            float& best, int& best_at)
 {
-    const uint32_t o = blockIdx.x * kBlock + threadIdx.x;
-    if (o >= total) return;
-    uint32_t rows, ox, plane, oy;
-    by_ow.divmod(o, rows, ox);
-    by_oh.divmod(rows, plane, oy);
-    float best = -FLT_MAX;
-    int best_at = -1;
+    best = -FLT_MAX;
+    best_at = -1;
     for (int ky = 0; ky < g.kernel; ++ky) {
         const int y = g.origin + static_cast<int>(oy) * g.stride + ky;
         if (y < 0 || y >= g.ih) continue;
@@ -39,8 +34,123 @@ __global__ __launch_bounds__(kBlock) void maxpool_fwd_generic_kernel(const float
             }
         }
     }
+}
+
+// One output per lane.
+__global__ __launch_bounds__(kBlock) void maxpool_fwd_generic_kernel(const float* in, float* out, int* indexes,
+                                                                     uint32_t total, PoolGeom g, FastDiv by_ow,
+                                                                     FastDiv by_oh)
+{
+    const uint32_t o = blockIdx.x * kBlock + threadIdx.x;
+    if (o >= total) return;
+    uint32_t rows, ox, plane, oy;
+    by_ow.divmod(o, rows, ox);
+    by_oh.divmod(rows, plane, oy);
+    float best;
+    int best_at;
+    scan_window(in, g, plane, oy, ox, best, best_at);
     out[o] = best;
     indexes[o] = best_at;
+}
+
+// ------------------------------------------------------------------ max-pool through LDS
+// Overlapping windows read every input k * k times; from the caches, at one lane per output, that is what
+// the kernel above costs (8192 planes of 19 x 19: k = 5 44 us, k = 13 191 us, for 36 MB of traffic).  Here a
+// workgroup takes a tile -- whole planes while they are small, else a strip of rows of one plane -- into LDS
+// and works separably: the first largest tap of every row segment, then the first largest of k segments,
+// 2k reads in place of k * k (17 and 24 us).  Row-major first-wins order survives the split: a segment keeps
+// its first largest tap, and a later segment only wins when strictly greater.  The tile is framed by -inf,
+// so that no tap has to be checked against the border; where that could decide (a window whose largest
+// value is -inf) or a NaN is in the tile (as the first tap it is taken, later it is not), the window is
+// scanned as above.
+struct PoolTile {
+    uint32_t planes;        // of the tensor
+    uint32_t per_tile;      // planes per tile; more than one only of whole planes
+    uint32_t strips;        // tiles per plane
+    uint32_t rows;          // output (forward) or input (backward) rows per strip
+};
+
+// K: the window, or 0 for any other
+template<int K>
+__global__ __launch_bounds__(kBlock) void maxpool_fwd_tile_kernel(const float* in, float* out, int* indexes,
+                                                                  PoolTile tile, PoolGeom g, FastDiv by_strips,
+                                                                  FastDiv by_iw, FastDiv by_ih, FastDiv by_ow,
+                                                                  FastDiv by_oh, uint32_t tile_cells, uint32_t segments)
+{
+    extern __shared__ float lds[];
+    float* cells = lds;                                        // [tile_cells]: framed rows
+    float* best_of = lds + tile_cells;                         // [segments]
+    uint8_t* tap_of = reinterpret_cast<uint8_t*>(best_of + segments);
+    const int k = K ? K : g.kernel;
+    uint32_t group, strip;
+    by_strips.divmod(blockIdx.x, group, strip);
+    const uint32_t p0 = group * tile.per_tile;
+    const uint32_t planes = min(tile.per_tile, tile.planes - p0);
+    const int oy0 = static_cast<int>(strip * tile.rows);
+    const int rows_out = min(static_cast<int>(tile.rows), g.oh - oy0);
+    // the frame: what the windows of the tile cover, from row y_frame and column g.origin on
+    const int y_frame = g.origin + oy0 * g.stride;
+    const uint32_t frame_h = (rows_out - 1) * g.stride + k, frame_w = (g.ow - 1) * g.stride + k;
+    int y_lo = 0, rows_in = g.ih;
+    if (tile.strips > 1) {
+        y_lo = min(max(0, y_frame), g.ih);
+        rows_in = max(0, min(g.ih, y_frame + static_cast<int>(frame_h)) - y_lo);
+    }
+    for (uint32_t i = threadIdx.x; i < planes * rows_in * frame_w; i += kBlock) cells[i] = -INFINITY;
+    for (uint32_t i = threadIdx.x; i < planes * frame_h * g.ow; i += kBlock) best_of[i] = -INFINITY;
+    __syncthreads();
+    const uint32_t in0 = (p0 * g.ih + y_lo) * g.iw;
+    bool nan = false;
+    for (uint32_t i = threadIdx.x; i < planes * rows_in * g.iw; i += kBlock) {
+        uint32_t row, x;
+        by_iw.divmod(i, row, x);
+        const float v = in[in0 + i];
+        nan |= v != v;
+        const uint32_t column = x - g.origin;
+        if (column < frame_w) cells[row * frame_w + column] = v;
+    }
+    const bool by_scan = __syncthreads_or(nan) != 0;
+    for (uint32_t j = threadIdx.x; j < planes * rows_in * g.ow; j += kBlock) {
+        uint32_t row, ox, plane = 0;
+        by_ow.divmod(j, row, ox);
+        const float* line = cells + row * frame_w + ox * g.stride;
+        if (tile.strips == 1) by_ih.divmod(row, plane, row);
+        const uint32_t frame_row = y_lo + row - y_frame;
+        if (frame_row >= frame_h) continue;
+        float best = line[0];
+        int tap = 0;
+#pragma unroll
+        for (int kx = 1; kx < k; ++kx) {
+            const float v = line[kx];
+            tap = v > best ? kx : tap;
+            best = v > best ? v : best;         // not fmaxf: of two zeros the first stays
+        }
+        const uint32_t seg = (plane * frame_h + frame_row) * g.ow + ox;
+        best_of[seg] = best;
+        tap_of[seg] = static_cast<uint8_t>(tap);
+    }
+    __syncthreads();
+    const uint32_t out0 = (p0 * g.oh + oy0) * g.ow;
+    for (uint32_t j = threadIdx.x; j < planes * rows_out * g.ow; j += kBlock) {
+        uint32_t row, ox, plane = 0;
+        by_ow.divmod(j, row, ox);
+        if (tile.strips == 1) by_oh.divmod(row, plane, row);
+        const uint32_t seg = (plane * frame_h + row * g.stride) * g.ow + ox;
+        float best = best_of[seg];
+        int tap = 0;
+#pragma unroll
+        for (int ky = 1; ky < k; ++ky) {
+            const float v = best_of[seg + ky * g.ow];
+            tap = v > best ? ky : tap;
+            best = v > best ? v : best;         // not fmaxf: of two zeros the first stays
+        }
+        const int x = g.origin + static_cast<int>(ox) * g.stride + tap_of[seg + tap * g.ow];
+        const int y = y_frame + static_cast<int>(row) * g.stride + tap;
+        int at = x + g.iw * (y + g.ih * static_cast<int>(p0 + plane));
+        if (by_scan || best == -INFINITY) scan_window(in, g, p0 + plane, oy0 + row, ox, best, at);
+        out[out0 + j] = best;
+        indexes[out0 + j] = at;
+    }
 }
 
 // 2x2 / stride 2 windows that all lie inside the input: VX outputs per lane from two
@@ -157,6 +267,101 @@ __global__ __launch_bounds__(kBlock) void maxpool_bwd_generic_kernel(const float
             }
         }
     if (touched) grad[cell] = acc;
+}
+
+// Backward through LDS.  A lane per cell that looks at all k * k windows of its cell reads k * k indexes to
+// find one on average (8192 planes of 19 x 19: k = 5 75 us, k = 13 274 us; here 19 and 56).  Here each output of the tile sets ONE bit, in
+// the mask of the cell its index names, at the output's position among the cell's windows in ascending
+// order; the cells with a bit (one in nine for k = 5) are then listed, so that lanes are not idle, and each
+// adds its deltas in that order.  An index that names no cell of the output's own window is ignored, as it
+// is by the kernel above.
+struct PoolWindows {
+    int along;              // windows over a cell along one axis: ceil(kernel / stride)
+    uint32_t words;         // of a cell's mask
+    FastDiv by_stride, by_along;
+};
+
+__global__ __launch_bounds__(kBlock) void maxpool_bwd_tile_kernel(const float* delta, const int* indexes, float* grad,
+                                                                  PoolTile tile, PoolGeom g, PoolWindows w,
+                                                                  FastDiv by_strips, FastDiv by_ow, FastDiv by_oh,
+                                                                  FastDiv by_iw, FastDiv by_ih, uint32_t tile_cells,
+                                                                  uint32_t tile_outputs)
+{
+    extern __shared__ float lds[];
+    uint32_t* masks = reinterpret_cast<uint32_t*>(lds);                      // [word][tile_cells]
+    float* deltas = lds + w.words * tile_cells;                              // [tile_outputs]
+    uint16_t* listed = reinterpret_cast<uint16_t*>(deltas + tile_outputs);   // [tile_cells]
+    __shared__ uint32_t listed_count;
+    uint32_t group, strip;
+    by_strips.divmod(blockIdx.x, group, strip);
+    const uint32_t p0 = group * tile.per_tile;
+    const uint32_t planes = min(tile.per_tile, tile.planes - p0);
+    const int y_lo = static_cast<int>(strip * tile.rows);
+    const int rows_in = min(static_cast<int>(tile.rows), g.ih - y_lo);
+    int oy_lo = 0, rows_out = g.oh;
+    if (tile.strips > 1) {
+        // windows that reach row y_lo or later and begin no later than the last row
+        const int reach = y_lo - g.origin - g.kernel + 1;
+        oy_lo = min(reach <= 0 ? 0 : static_cast<int>(w.by_stride.div(reach + g.stride - 1)), g.oh);
+        const int last = static_cast<int>(w.by_stride.div(y_lo + rows_in - 1 - g.origin));
+        rows_out = max(0, min(g.oh, last + 1) - oy_lo);
+    }
+    const uint32_t cells = planes * rows_in * g.iw;
+    for (uint32_t i = threadIdx.x; i < w.words * tile_cells; i += kBlock) masks[i] = 0;
+    if (threadIdx.x == 0) listed_count = 0;
+    __syncthreads();
+    const uint32_t cell0 = (p0 * g.ih + y_lo) * g.iw, out0 = (p0 * g.oh + oy_lo) * g.ow;
+    for (uint32_t j = threadIdx.x; j < planes * rows_out * g.ow; j += kBlock) {
+        deltas[j] = delta[out0 + j];
+        const uint32_t cell = static_cast<uint32_t>(indexes[out0 + j]) - cell0;     // negative: beyond any tile
+        if (cell >= cells) continue;
+        uint32_t row, ox, plane = 0, y, x, cell_plane = 0;
+        by_ow.divmod(j, row, ox);
+        by_iw.divmod(cell, y, x);
+        if (tile.strips == 1) {
+            by_oh.divmod(row, plane, row);
+            by_ih.divmod(y, cell_plane, y);
+        }
+        const int ty = y_lo + static_cast<int>(y) - g.origin - (oy_lo + static_cast<int>(row)) * g.stride;
+        const int tx = static_cast<int>(x) - g.origin - static_cast<int>(ox) * g.stride;
+        if (plane != cell_plane || ty < 0 || ty >= g.kernel || tx < 0 || tx >= g.kernel) continue;
+        const uint32_t bit = w.by_stride.div(g.kernel - 1 - ty) * w.along + w.by_stride.div(g.kernel - 1 - tx);
+        atomicOr(&masks[(bit >> 5) * tile_cells + cell], 1u << (bit & 31));
+    }
+    __syncthreads();
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    for (uint32_t i0 = threadIdx.x - lane; i0 < cells; i0 += kBlock) {
+        const uint32_t i = i0 + lane;
+        uint32_t any = 0;
+        if (i < cells)
+            for (uint32_t word = 0; word < w.words; ++word) any |= masks[word * tile_cells + i];
+        const uint64_t hit = __ballot(any != 0);
+        if (hit == 0) continue;
+        uint32_t at = 0;
+        if (lane == 0) at = atomicAdd(&listed_count, static_cast<uint32_t>(__popcll(hit)));
+        at = __builtin_amdgcn_readfirstlane(at);
+        if (any) listed[at + __popcll(hit & ((1ull << lane) - 1))] = static_cast<uint16_t>(i);
+    }
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < listed_count; k += kBlock) {
+        const uint32_t cell = listed[k];
+        uint32_t y, x, plane = 0;
+        by_iw.divmod(cell, y, x);
+        if (tile.strips == 1) by_ih.divmod(y, plane, y);
+        // the first window that reaches the cell along each axis (it may lie before the first output)
+        const int lift = g.kernel * g.stride;
+        const int oy = static_cast<int>(w.by_stride.div(y_lo + y - g.origin - g.kernel + g.stride + lift)) - g.kernel;
+        const int ox = static_cast<int>(w.by_stride.div(x - g.origin - g.kernel + g.stride + lift)) - g.kernel;
+        const int first = (static_cast<int>(plane) * rows_out + oy - oy_lo) * g.ow + ox;
+        float acc = grad[cell0 + cell];
+        for (uint32_t word = 0; word < w.words; ++word)
+            for (uint32_t bits = masks[word * tile_cells + cell]; bits; bits &= bits - 1) {
+                uint32_t wy, wx;
+                w.by_along.divmod(word * 32 + __builtin_ctz(bits), wy, wx);
+                acc += deltas[first + static_cast<int>(wy) * g.ow + static_cast<int>(wx)];
+            }
+        grad[cell0 + cell] = acc;
+    }
 }
 
 // Backward for the 2x2 / stride 2 in-bounds case: one window per output, VX windows per lane,
@@ -359,6 +564,91 @@ bool is_2x2_inbounds(int ih, int iw, int oh, int ow, int kernel, int stride, int
     return kernel == 2 && stride == 2 && padding <= 1 && ih % 2 == 0 && iw % 2 == 0 && oh == ih / 2 && ow == iw / 2;
 }
 
+// Tiles of about `target` cells: whole planes while one fits, else strips.  `rows` and `width` are those of the
+// tensor that is tiled.
+PoolTile pool_tile(uint32_t planes, int rows, int width, uint32_t target)
+{
+    PoolTile t{ planes, 1, 1, static_cast<uint32_t>(rows) };
+    const uint32_t plane = static_cast<uint32_t>(rows) * width;
+    if (plane <= target) {
+        t.per_tile = target / plane;
+        // enough workgroups for the chip before larger ones
+        const uint32_t spread = planes / 1024 > 0 ? planes / 1024 : 1;
+        if (t.per_tile > spread) t.per_tile = spread;
+        return t;
+    }
+    t.rows = target / width > 0 ? target / width : 1;
+    t.strips = (rows + t.rows - 1) / t.rows;
+    return t;
+}
+
+constexpr size_t kPoolLds = 40u << 10;      // four workgroups per compute unit
+constexpr uint32_t kPoolCells = 2048;       // eight per lane; halved until the tile fits
+
+// Launches the tiled forward pass; false when the geometry does not suit it.
+bool launch_fwd_tile(const float* in, float* out, int* indexes, uint32_t planes, const PoolGeom& g, hipStream_t s)
+{
+    // Every input is a tap of (k / stride)^2 windows.  Measured, us one lane per output -> tiled: 3 / 1, 64 planes
+    // of 300 x 300, 45 -> 26; 5 / 1, 8192 of 19 x 19, 44 -> 17; 13 / 1 190 -> 24; but 3 / 2, 64 of 300 x 300,
+    // 13.3 -> 18.8 and 2 / 1, 32768 of 13 x 13, level: with so few taps the detour through LDS costs more.
+    if (g.kernel > 64 || g.kernel * g.kernel < 8 * g.stride * g.stride) return false;
+    for (uint32_t target = kPoolCells; target >= 256; target /= 2) {
+        const PoolTile t = pool_tile(planes, g.oh, g.ow, target);
+        // strips of few rows read most of their input for the rows of the next one
+        if (t.strips > 1 && t.rows * g.stride < static_cast<uint32_t>(g.kernel)) return false;
+        const size_t frame_h = static_cast<size_t>(t.rows - 1) * g.stride + g.kernel;
+        const size_t frame_w = static_cast<size_t>(g.ow - 1) * g.stride + g.kernel;
+        const size_t rows_in = t.strips == 1 ? g.ih : std::min<size_t>(g.ih, frame_h);
+        const size_t cells = t.per_tile * rows_in * frame_w, segments = t.per_tile * frame_h * g.ow;
+        const size_t bytes = cells * 4 + segments * 5;
+        if (bytes > kPoolLds) continue;
+        const dim3 grid((planes + t.per_tile - 1) / t.per_tile * t.strips);
+#define PXH_POOL_TILE(K)                                                                                       \
+        hipLaunchKernelGGL((maxpool_fwd_tile_kernel<K>), grid, dim3(kBlock), bytes, s, in, out, indexes, t, g, \
+                           FastDiv(t.strips), FastDiv(g.iw), FastDiv(g.ih), FastDiv(g.ow), FastDiv(g.oh),      \
+                           static_cast<uint32_t>(cells), static_cast<uint32_t>(segments))
+        switch (g.kernel) {
+        case 2: PXH_POOL_TILE(2); break;
+        case 3: PXH_POOL_TILE(3); break;
+        case 5: PXH_POOL_TILE(5); break;
+        case 9: PXH_POOL_TILE(9); break;
+        case 13: PXH_POOL_TILE(13); break;
+        default: PXH_POOL_TILE(0);
+        }
+#undef PXH_POOL_TILE
+        return true;
+    }
+    return false;
+}
+
+bool launch_bwd_tile(const float* delta, const int* indexes, float* grad, uint32_t planes, const PoolGeom& g,
+                     hipStream_t s)
+{
+    // masks of up to eight words; few windows per cell gain less (2 / 2, 1024 planes of 151 x 151, 86 -> 53 us; 3 / 2,
+    // 64 of 300 x 300, 38 -> 19), and launches too small to matter stay level
+    if (g.kernel > 16 || g.stride > 16) return false;
+    PoolWindows w;
+    w.along = (g.kernel + g.stride - 1) / g.stride;
+    w.words = static_cast<uint32_t>(w.along * w.along + 31) / 32;
+    w.by_stride = FastDiv(g.stride);
+    w.by_along = FastDiv(w.along);
+    for (uint32_t target = kPoolCells; target >= 256; target /= 2) {
+        const PoolTile t = pool_tile(planes, g.ih, g.iw, target);
+        if (t.strips > 1 && t.rows < static_cast<uint32_t>(g.kernel)) return false;
+        const size_t cells = static_cast<size_t>(t.per_tile) * t.rows * g.iw;
+        const size_t rows_out = t.strips == 1 ? g.oh : std::min<size_t>(g.oh, (t.rows + g.kernel - 2) / g.stride + 2);
+        const size_t outputs = t.per_tile * rows_out * g.ow;
+        const size_t bytes = cells * (4 * w.words + 2) + outputs * 4;
+        if (bytes > kPoolLds) continue;
+        const dim3 grid((planes + t.per_tile - 1) / t.per_tile * t.strips);
+        hipLaunchKernelGGL(maxpool_bwd_tile_kernel, grid, dim3(kBlock), bytes, s, delta, indexes, grad, t, g, w,
+                           FastDiv(t.strips), FastDiv(g.ow), FastDiv(g.oh), FastDiv(g.iw), FastDiv(g.ih),
+                           static_cast<uint32_t>(cells), static_cast<uint32_t>(outputs));
+        return true;
+    }
+    return false;
+}
+
 }  // namespace
 }  // namespace pxh
 
@@ -404,6 +694,7 @@ int pxh_maxpool_forward(const float* in, float* out, int* indexes, int batch, in
         return check_launch("pxh_maxpool_forward");
     }
     const PoolGeom g{ ih, iw, oh, ow, kernel, stride, -padding / 2 };
+    if (launch_fwd_tile(in, out, indexes, planes, g, s)) return check_launch("pxh_maxpool_forward");
     hipLaunchKernelGGL(maxpool_fwd_generic_kernel, dim3(grid_for(total, kBlock)), dim3(kBlock), 0, s, in, out, indexes,
                        total, g, FastDiv(ow), FastDiv(oh));
     return check_launch("pxh_maxpool_forward");
@@ -446,6 +737,7 @@ int pxh_maxpool_backward(const float* delta, const int* indexes, float* grad, in
         return check_launch("pxh_maxpool_backward");
     }
     const PoolGeom g{ ih, iw, oh, ow, kernel, stride, -padding / 2 };
+    if (launch_bwd_tile(delta, indexes, grad, planes, g, s)) return check_launch("pxh_maxpool_backward");
     const uint32_t in_total = planes * ih * iw;
     hipLaunchKernelGGL(maxpool_bwd_generic_kernel, dim3(grid_for(in_total, kBlock)), dim3(kBlock), 0, s, delta,
                        indexes, grad, in_total, g, FastDiv(iw), FastDiv(ih));

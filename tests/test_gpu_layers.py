@@ -84,6 +84,43 @@ def test_maxpool_special_values(ops, oracle):
     run_maxpool(ops, oracle, x, 2, 1, 1, 1402)
 
 
+# whole planes in one tile and one more, more planes per tile than are left, strips with a remainder, masks
+# of 1 to 8 words, windows wider than the plane; the last three are beyond one or both tiled kernels
+@pytest.mark.parametrize("shape,k,s,p", [
+    ((1, 1, 32, 64), 2, 1, 1), ((1, 2, 33, 64), 2, 1, 1), ((3, 1031, 5, 7), 3, 1, 2), ((5, 1024, 3, 3), 3, 2, 2),
+    ((1, 2, 101, 67), 3, 1, 2), ((1, 2, 101, 67), 3, 2, 2), ((2, 2, 151, 75), 2, 2, 1), ((1, 3, 19, 19), 5, 1, 4),
+    ((1, 2, 38, 38), 9, 1, 8), ((1, 2, 38, 38), 13, 1, 12), ((1, 2, 47, 53), 13, 1, 12), ((1, 2, 9, 6), 13, 1, 12),
+    ((1, 2, 40, 37), 16, 1, 15), ((1, 2, 21, 20), 6, 4, 5), ((1, 1, 3, 1200), 3, 1, 2), ((1, 1, 4, 12000), 3, 1, 2),
+    ((1, 1, 30, 30), 17, 1, 16)], ids=lambda v: str(v))
+def test_maxpool_tiles(ops, oracle, shape, k, s, p):
+    x = wl.normal(1600 + shape[2] + k, shape)
+    run_maxpool(ops, oracle, x, k, s, p, 1700)
+    # ties, and the values that compare unlike others, often the first tap of a window
+    x = np.round(x).astype(F)
+    flat = x.reshape(-1)
+    flat[::11] = np.nan
+    flat[::13] = -np.inf
+    flat[::17] = np.finfo(F).min
+    flat[::19] = -0.0
+    flat[::23] = np.inf
+    run_maxpool(ops, oracle, x, k, s, p, 1701)
+
+
+def test_maxpool_backward_ignores_foreign_indexes(ops):
+    """An index that names no cell of its own window adds nothing, whatever it holds."""
+    import torch
+    delta = torch.ones(2, 3, 8, 8, device="cuda")
+    own = torch.arange(delta.numel(), device="cuda", dtype=torch.int32).view_as(delta)
+    for foreign in (own * 0 - 1, (own + 64) % own.numel(), own * 0 + 2**31 - 1, own * 0 - 2**31, own.flip(-1) // 8 * 8):
+        idx = own.clone()
+        idx[:, :, 3:6, 4] = foreign[:, :, 3:6, 4]
+        grad = torch.zeros(2, 3, 8, 8, device="cuda")
+        ops.maxpool_backward(delta, idx, grad, 3, 1, 2)
+        want = torch.ones_like(grad)
+        want[:, :, 3:6, 4] = 0
+        assert torch.equal(grad, want)
+
+
 def test_maxpool_scatter_signature(ops, oracle):
     x = wl.normal(1500, (2, 3, 12, 12))
     idx_w, delta, grad0, grad_w = run_maxpool(ops, oracle, x, 2, 2, 1, 1501)
