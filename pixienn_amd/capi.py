@@ -171,7 +171,7 @@ def act_id(act):
 
 def call(name, *args):
     """Calls an int-returning entry point and raises PxError on a non-zero status."""
-    rc = getattr(load(), name)(*args)
+    rc = getattr(_lib or load(), name)(*args)
     if rc != 0:
         raise PxError("%s failed (status %d): %s" % (name, rc, last_error()))
     return rc

@@ -4,6 +4,7 @@ Every function launches on torch's current HIP stream and returns without synchr
 Tensors must be fp32 (int32 for indices), contiguous and on a HIP device.
 """
 import ctypes
+import functools
 
 import numpy as np
 import torch
@@ -12,8 +13,16 @@ from . import capi, workloads
 from .capi import PxError, act_id, call, ptr
 
 
+# A network at a small batch is a few hundred calls of a few microseconds each on the GPU: what a call costs
+# here is then its time.  The current stream's handle comes without a Stream object around it (0.3 us in
+# place of 2), and a tensor that is as it should be passes its check in one expression.
+_F32 = torch.float32
+_current_device = torch.cuda.current_device
+_raw_stream = torch._C._cuda_getCurrentRawStream
+
+
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_current_device())
 
 
 def _chk(t, dtype=torch.float32, name="tensor"):
@@ -31,14 +40,32 @@ def _chk(t, dtype=torch.float32, name="tensor"):
 
 def _chk_all(*ts):
     for t in ts:
+        if t is None or (isinstance(t, torch.Tensor) and t.dtype is _F32 and t.is_cuda and t.is_contiguous()):
+            continue
         _chk(t)
 
 
 def _nchw(x):
-    if x.dim() != 4:
-        raise PxError("NCHW tensor expected, got %d dims" % x.dim())
-    n, c, h, w = x.shape
+    shape = x.shape
+    if len(shape) != 4:
+        raise PxError("NCHW tensor expected, got %d dims" % len(shape))
+    n, c, h, w = shape
     return n, c, h * w
+
+
+@functools.lru_cache(maxsize=64)
+def _int_array(values):
+    """A C array of the integers of a tuple (masks, anchors): the same for every call with the same values."""
+    return (ctypes.c_int * len(values))(*values)
+
+
+def _ints(values):
+    """(address, length, keep-alive) of int32 values in a list, tuple or array."""
+    if isinstance(values, (list, tuple)) and all(type(v) is int and -2**31 <= v < 2**31 for v in values):
+        array = _int_array(tuple(values))
+        return ctypes.addressof(array), len(values), array
+    array = np.ascontiguousarray(values, dtype=np.int32)
+    return array.ctypes.data, len(array), array
 
 
 # ---------------------------------------------------------------- epilogue forward
@@ -353,11 +380,11 @@ def yolo_forward_train(inp, out, delta, truths, truth_counts, max_truth, masks, 
                        object_scale=1.0, noobject_scale=1.0, class_scale=1.0, workspace=None):
     _chk_all(inp, out, delta, truths, stats, cost)
     _chk(truth_counts, torch.int32, "truth_counts")
-    m = np.ascontiguousarray(masks, dtype=np.int32)
-    a = np.ascontiguousarray(anchors, dtype=np.int32)
+    m, m_count, m_keep = _ints(masks)
+    a, a_count, a_keep = _ints(anchors)
     wb = 0 if workspace is None else workspace.numel() * workspace.element_size()
     call("pxh_yolo_forward_train", ptr(inp), ptr(out), ptr(delta), ptr(truths), ptr(truth_counts), int(max_truth),
-         m.ctypes.data, a.ctypes.data, ptr(stats), ptr(cost), batch, len(m), len(a) // 2, classes, width, height,
+         m, a, ptr(stats), ptr(cost), batch, m_count, a_count // 2, classes, width, height,
          net_width, net_height, float(ignore_thresh), float(truth_thresh), float(coord_scale), float(object_scale),
          float(noobject_scale), float(class_scale), ptr(workspace), wb, _stream())
 
@@ -391,10 +418,10 @@ def yolo_forward_train_heads(heads, truths, truth_counts, max_truth, anchors, ba
     keep = None
     if table is None:
         table, keep = yolo_head_table(heads)
-    a = np.ascontiguousarray(anchors, dtype=np.int32)
+    a, a_count, a_keep = _ints(anchors)
     wb = 0 if workspace is None else workspace.numel() * workspace.element_size()
     call("pxh_yolo_forward_train_heads", len(table), ctypes.addressof(table), ptr(truths), ptr(truth_counts),
-         int(max_truth), a.ctypes.data, len(a) // 2, batch, classes, net_width, net_height, ptr(workspace), wb, _stream())
+         int(max_truth), a, a_count // 2, batch, classes, net_width, net_height, ptr(workspace), wb, _stream())
     del keep
 
 
@@ -601,9 +628,9 @@ def yolo_detections_append(predictions, batch, masks, anchors, classes, width, h
     _chk_all(predictions)
     _chk(records, torch.int32, "records")
     _chk(count, torch.int32, "count")
-    m = np.ascontiguousarray(masks, dtype=np.int32)
-    a = np.ascontiguousarray(anchors, dtype=np.int32)
-    call("pxh_yolo_detections_append", ptr(predictions), batch, m.ctypes.data, len(m), a.ctypes.data, len(a) // 2,
+    m, m_count, m_keep = _ints(masks)
+    a, a_count, a_keep = _ints(anchors)
+    call("pxh_yolo_detections_append", ptr(predictions), batch, m, m_count, a, a_count // 2,
          classes, width, height, net_width, net_height, int(image_width), int(image_height), float(threshold),
          int(order_base), ptr(records), int(records.shape[0]), ptr(count), _stream())
 
@@ -623,11 +650,25 @@ def nms(records, count, batch, classes, threshold, workspace=None):
     return kept, kept_count
 
 
+_FIRST_COPY = 4096       # survivors that travel with their count, 128 KB
+
+
 def nms_to_host(kept, kept_count):
     """Blocking copy of the survivors as a numpy structured array."""
+    # The count and as many records as a call usually leaves go to pinned memory behind the launches, and the
+    # host waits once: asking for the count first is a second round trip (25 us) before the records' own.
+    first = min(kept.shape[0], _FIRST_COPY)
+    count = torch.empty(1, dtype=torch.int32, pin_memory=True)
+    records = torch.empty((first, *kept.shape[1:]), dtype=kept.dtype, pin_memory=True)
+    count.copy_(kept_count, non_blocking=True)
+    records.copy_(kept[:first], non_blocking=True)
     torch.cuda.current_stream().synchronize()
-    n = int(kept_count.item())
-    return kept[:n].cpu().numpy().view(DETECTION_DTYPE).reshape(-1)
+    n = int(count[0])
+    if n <= first:
+        rows = records[:n].numpy().copy()
+    else:
+        rows = np.concatenate([records.numpy(), kept[first:n].cpu().numpy()])
+    return rows.view(DETECTION_DTYPE).reshape(-1)
 
 
 def records_to_device(rec, capacity=None, device="cuda"):
