@@ -1095,7 +1095,7 @@ constexpr int kResidualAhead = 4;
 
 // V = 4 needs spatial % 4 == 0 and 16-byte aligned tensors.  R + L vectors per thread at most.
 template<int ACT, int V, int R, int L, int T = kResidentThreads, bool RES = false>
-__global__ __launch_bounds__(T, L == 0 && V * R <= 32 ? 8 : 4) void bn_resident_fwd_kernel(ResidentFwdArgs a)
+__global__ __launch_bounds__(T, L == 0 && V * R <= (V == 1 ? (RES ? 8 : 16) : 32) ? 8 : 4) void bn_resident_fwd_kernel(ResidentFwdArgs a)
 {
     static_assert(L == 0 || T == kResidentThreads, "the LDS part is laid out for the full workgroup");
     extern __shared__ __align__(16) float resident_lds[];
@@ -1160,7 +1160,7 @@ __global__ __launch_bounds__(T, L == 0 && V * R <= 32 ? 8 : 4) void bn_resident_
     // (16 x 1024 x 19^2: 19.9 us against 25.6 us with every step's load behind the reduction).
     // (the half-size workgroups of the 128-bit form have 128 registers: eight of twelve steps, four of sixteen)
     constexpr int kAhead = !RES ? 0 : V * (R + L) <= 8 ? R + L : L > 0 ? kResidualAhead
-                                : T < kResidentThreads ? (R <= 12 ? 8 : 4) : 0;
+                                : T < kResidentThreads ? (R <= 12 ? 8 : 4) : V == 1 && R >= 16 ? 4 : 0;
     [[maybe_unused]] Pack<V> ahead[kAhead > 0 ? kAhead : 1];
     if constexpr (RES) {
 #pragma unroll
@@ -1507,7 +1507,7 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
 // the first launch and leave at once when nothing has to change; the forms without an LDS part run it
 // as a capped grid that walks the channels otherwise.
 template<int ACT, int V, int R, int L, int MODE = kPlain, int T = kResidentThreads>
-__global__ __launch_bounds__(T, L == 0 && MODE != kRedo ? 8 : 4) void bn_resident_bwd_kernel(ResidentBwdArgs a)
+__global__ __launch_bounds__(T, L == 0 && MODE != kRedo && !(V == 1 && R > 16) ? 8 : 4) void bn_resident_bwd_kernel(ResidentBwdArgs a)
 {
     static_assert(L == 0 || T == kResidentThreads, "the LDS part is laid out for the full workgroup");
     if constexpr (MODE == kRedo) {
@@ -1542,15 +1542,43 @@ constexpr int kResidentVectors = 8;
 // the large form (128-bit vectors only): 16 vectors in registers + 8 in LDS (128 KB of the CU's 160)
 constexpr int kResidentLargeRegs = 16, kResidentLargeLds = 8;
 constexpr size_t kResidentLargeLdsBytes = static_cast<size_t>(kResidentLargeLds) * kResidentThreads * 16;
+// The scalar forms (odd planes) with more values per lane: 16 in 64 registers, two workgroups per compute unit
+// (one with a shortcut's source on top); the backward also 24 in 128 registers.  Against the three launches, us:
+//                       forward        + shortcut     backward
+//   64 x 256 x 13^2     15.1 ->  8.7   15.9 -> 11.4   21.9 -> 11.6   leaky
+//   64 x 512 x 13^2     22.1 -> 14.4   24.3 -> 22.2   32.2 -> 17.8
+//   64 x 1024 x 13^2    36.5 -> 27.6   41.3 -> 43.8   49.7 -> 37.9
+//   64 x 512 x 19^2     29.7 -> 28.3   38.9 -> 54.0   49.6 -> 36.6   24 values
+//   64 x 256 x 13^2     15.8 -> 11.9   16.4 -> 13.1   28.5 -> 20.7   mish
+//   64 x 512 x 13^2     22.7 -> 18.5   24.9 -> 24.5   40.6 -> 35.4
+//   32 x 1024 x 19^2    30.8 -> 37.1   39.6 -> 52.4   64.8 -> 66.5
+//   64 x 512 x 19^2     30.1 -> 34.7   40.3 -> 64.3   64.5 -> 61.8   24 values
+// An activation with an exponential, or a second tensor, leaves a workgroup that waits for its own channel more to do
+// after the wait, and a thousand channels keep the three launches' many small workgroups busy: those take the
+// one-launch form only up to 512 channels, and 24 values only where the backward's gradient is a select.
+// (Forward with 24 values the shortcut would lose, and a layer below 512 channels has the same statistics to the
+// bit with and without one: no such form.)
+constexpr int kResidentScalarMid = 16, kResidentScalarWide = 24;
+constexpr int kResidentScalarFew = 512;
 
-int resident_vectors(int batch, int channels, int spatial, bool vec)
+constexpr bool selects(int activation)
+{
+    return activation == PXH_LEAKY || activation == PXH_RELU || activation == PXH_LINEAR;
+}
+
+enum class Pass { Forward, ForwardShortcut, Backward };
+
+int resident_vectors(int batch, int channels, int spatial, bool vec, int activation, Pass pass)
 {
     if (channels < 96) return 0;
     const size_t per_channel = static_cast<size_t>(batch) * spatial;
     const size_t vectors = (per_channel + (vec ? 3 : 0)) / (vec ? 4 : 1);
     const size_t per_thread = (vectors + kResidentThreads - 1) / kResidentThreads;
     if (per_thread <= kResidentVectors) return kResidentVectors;
-    if (vec && per_thread <= kResidentLargeRegs + kResidentLargeLds) return kResidentLargeRegs + kResidentLargeLds;
+    if (vec) return per_thread <= kResidentLargeRegs + kResidentLargeLds ? kResidentLargeRegs + kResidentLargeLds : 0;
+    const bool light = selects(activation) && pass != Pass::ForwardShortcut;
+    if (per_thread <= kResidentScalarMid && (light || channels <= kResidentScalarFew)) return kResidentScalarMid;
+    if (per_thread <= kResidentScalarWide && light && pass == Pass::Backward) return kResidentScalarWide;
     return 0;
 }
 
@@ -1559,12 +1587,11 @@ int resident_vectors(int batch, int channels, int spatial, bool vec)
 // forward 14.6 against 16.3 us, backward 23.1 against 26.5; at 512 channels the forward gains 5 %, the
 // backward loses 20 %.
 constexpr int kResidentNarrowVectors = 2 * kResidentVectors;
-bool resident_narrow(int batch, int channels, int spatial, bool vec, bool backward)
+bool resident_narrow(int batch, int channels, int spatial, int per_thread, bool vec, bool backward)
 {
-    if (vec || channels < (backward ? 1024 : 512)) return false;
+    if (vec || per_thread != kResidentVectors || channels < (backward ? 1024 : 512)) return false;
     const size_t per_channel = static_cast<size_t>(batch) * spatial;
-    return (per_channel + kResidentNarrowThreads - 1) / kResidentNarrowThreads <= kResidentNarrowVectors &&
-           resident_vectors(batch, channels, spatial, vec) == kResidentVectors;
+    return (per_channel + kResidentNarrowThreads - 1) / kResidentNarrowThreads <= kResidentNarrowVectors;
 }
 
 // A kernel that asks for more than 64 KB of dynamic LDS has to be allowed to, once.
@@ -1698,13 +1725,20 @@ int bn_train_forward(const char* who, const float* x, float* y, float* pre_activ
     {
         const bool vec = spatial % 4 == 0 && aligned16(x) && aligned16(y) && aligned16(pre_activation) &&
                          aligned16(x_saved) && aligned16(x_norm) && aligned16(res.from);
-        const int per_thread = resident_vectors(batch, channels, spatial, vec);
+        const int per_thread = resident_vectors(batch, channels, spatial, vec, activation,
+                                                res.from ? Pass::ForwardShortcut : Pass::Forward);
         if (per_thread) {
             const ResidentFwdArgs r{ x, y, pre_activation, x_saved, x_norm, mean, var, rolling_mean, rolling_var,
                                      scale, bias, resident_geom(batch, channels, spatial), res.from, res.alpha, res.beta };
+            if (!vec && per_thread > kResidentVectors) {
+                // the workspace that the three launches need is still the caller's part of this shape
+                void* unused;
+                rc = get_workspace(workspace_bytes(batch, channels, spatial), &unused);
+                if (rc) return rc;
+            }
             // (with the shortcut's source on top, sixteen values per lane no longer fit the registers of four
             // workgroups per compute unit: that form keeps the full workgroups)
-            const bool narrow = !res.from && resident_narrow(batch, channels, spatial, vec, false);
+            const bool narrow = !res.from && resident_narrow(batch, channels, spatial, per_thread, vec, false);
             const dim3 grid(channels), block(narrow ? kResidentNarrowThreads : kResidentThreads);
             int large_lds_rc = PXH_OK;
             const auto launch = [&]<int ACT, bool RES>() {
@@ -1732,7 +1766,9 @@ int bn_train_forward(const char* who, const float* x, float* y, float* pre_activ
                         return;
                     }
                 }
-                if (per_thread > kResidentVectors) {
+                if (!vec && per_thread == kResidentScalarMid) {
+                    hipLaunchKernelGGL((bn_resident_fwd_kernel<ACT, 1, kResidentScalarMid, 0, kT, RES>), grid, block, 0, s, r);
+                } else if (per_thread > kResidentVectors) {
                     auto kernel = bn_resident_fwd_kernel<ACT, 4, kResidentLargeRegs, kResidentLargeLds, kT, RES>;
                     large_lds_rc = allow_large_lds(reinterpret_cast<const void*>(kernel));
                     if (large_lds_rc == PXH_OK)
@@ -1986,7 +2022,7 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
     if (rc) return rc;
     hipStream_t s = as_stream(stream);
     const bool rvec = spatial % 4 == 0 && aligned16(delta) && aligned16(x) && aligned16(pre_activation);
-    const int per_thread = resident_vectors(batch, channels, spatial, rvec);
+    const int per_thread = resident_vectors(batch, channels, spatial, rvec, activation, Pass::Backward);
     void* ws = nullptr;
     ClippedRegions region{};
     ClipArgs clip{};
@@ -1997,19 +2033,29 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
         clip = ClipArgs{ region.norm_partial, region.plan, cs.threshold, cs.clip, cs.norm_out };
     }
     if (per_thread) {
+        if (!cs.on && !rvec && per_thread > kResidentVectors) {
+            // the workspace that the three launches need is still the caller's part of this shape
+            rc = resolve_workspace(workspace, workspace_bytes_given, workspace_bytes(batch, channels, spatial), &ws, s);
+            if (rc) return rc;
+        }
         const ResidentBwdArgs r{ BackwardArgs{ delta, x, pre_activation, mean, var, scale, bias }, scale_updates,
                                  bias_updates, mean_delta, var_delta, resident_geom(batch, channels, spatial),
                                  region.channel_norm, region.channel_sums, region.channel_done, clip };
-        const bool narrow = resident_narrow(batch, channels, spatial, rvec, true);
+        const bool narrow = resident_narrow(batch, channels, spatial, per_thread, rvec, true);
         const dim3 block(narrow ? kResidentNarrowThreads : kResidentThreads);
         int large_lds_rc = PXH_OK;
         const auto launch = [&]<int ACT, int MODE>() {
             // the launch that follows the plan: one workgroup per compute unit at most, each walks channels
-            const bool walks = MODE == kRedo && per_thread <= kResidentVectors && channels > kRedoWorkgroups;
+            const bool walks = MODE == kRedo && !(rvec && per_thread > kResidentVectors) && channels > kRedoWorkgroups;
             const dim3 grid(walks ? kRedoWorkgroups : channels);
             if (narrow) {
                 hipLaunchKernelGGL((bn_resident_bwd_kernel<ACT, 1, kResidentNarrowVectors, 0, MODE, kResidentNarrowThreads>),
                                    grid, block, 0, s, r);
+            } else if (!rvec && per_thread == kResidentScalarWide) {
+                if constexpr (selects(ACT))
+                    hipLaunchKernelGGL((bn_resident_bwd_kernel<ACT, 1, kResidentScalarWide, 0, MODE>), grid, block, 0, s, r);
+            } else if (!rvec && per_thread == kResidentScalarMid) {
+                hipLaunchKernelGGL((bn_resident_bwd_kernel<ACT, 1, kResidentScalarMid, 0, MODE>), grid, block, 0, s, r);
             } else if (per_thread > kResidentVectors) {
                 auto kernel = bn_resident_bwd_kernel<ACT, 4, kResidentLargeRegs, kResidentLargeLds, MODE>;
                 large_lds_rc = allow_large_lds(reinterpret_cast<const void*>(kernel));
