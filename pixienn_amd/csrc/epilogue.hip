@@ -364,17 +364,24 @@ int launch_epilogue_fwd(const char* who, EpilogueArgs a, int activation, hipStre
 // Per-channel reductions.
 //
 // Channel c owns `batch` planes of `spatial` contiguous floats.  A plane is cut into segments of
-// kSeg floats; the (image, segment) items of a channel are dealt kItemsPerBlock to a workgroup,
+// kSeg floats; the (image, segment) items of a channel are dealt ReduceGeom::per_block to a workgroup,
 // one item per wavefront at a time (64 lanes x 128-bit x 4 loads = one segment).  Lanes sum a
 // segment in fp32, carry across segments in double; the workgroup's pair of sums goes to
 // partial[c][j] and a second kernel adds the partials of a channel in a fixed order.
 // ------------------------------------------------------------------------------------------
 constexpr int kSegLoads = 4;                  // 128-bit loads in flight per lane
 constexpr int kSeg = kWave * 4 * kSegLoads;   // 1024 floats
+// Items of a workgroup: as many as kItemsPerBlock, four to a wavefront, where that leaves kFillBlocks workgroups
+// (four to a compute unit); fewer, down to one a wavefront, where it does not.  A wavefront takes its items one
+// after the other, so a small grid is bound by that chain and not by memory.  Sixteen items everywhere against this
+// rule, backward, us: 6 x 72 x 135 x 77 (360 workgroups) leaky 26.1 -> 24.2, mish 42.1 -> 33.7; 64 x 64 x 13^2 (256)
+// mish 18.6 -> 15.3; 64 x 96 x 19^2 (384) mish 27.4 -> 23.8.  The forward's sums gain 1 us.  A full grid keeps sixteen:
+// more workgroups there only add partials to finish.
 constexpr int kItemsPerBlock = 16;
+constexpr int kFillBlocks = 1024;
 
 struct ReduceGeom {
-    int channels, spatial, parts, items, blocks;
+    int channels, spatial, parts, items, per_block, blocks;
     FastDiv by_parts;
     FastDiv by_blocks;
 };
@@ -386,7 +393,10 @@ ReduceGeom make_geom(int batch, int channels, int spatial)
     g.spatial = spatial;
     g.parts = (spatial + kSeg - 1) / kSeg;
     g.items = batch * g.parts;
-    g.blocks = (g.items + kItemsPerBlock - 1) / kItemsPerBlock;
+    g.per_block = kItemsPerBlock;
+    const auto blocks = [&] { return (g.items + g.per_block - 1) / g.per_block; };
+    while (g.per_block > kBlock / kWave && static_cast<long long>(channels) * blocks() < kFillBlocks) g.per_block /= 2;
+    g.blocks = blocks();
     g.by_parts = FastDiv(static_cast<uint32_t>(g.parts));
     g.by_blocks = FastDiv(static_cast<uint32_t>(g.blocks));
     return g;
@@ -399,8 +409,8 @@ __device__ __forceinline__ void for_each_item(const ReduceGeom& g, uint32_t c, u
 {
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
-    const int first = j * kItemsPerBlock;
-    const int last = min(first + kItemsPerBlock, g.items);
+    const int first = j * g.per_block;
+    const int last = min(first + g.per_block, g.items);
     for (int it = first + wave; it < last; it += kBlock / kWave) {
         uint32_t n, part;
         g.by_parts.divmod(static_cast<uint32_t>(it), n, part);

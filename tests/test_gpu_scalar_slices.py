@@ -31,3 +31,13 @@ def test_scalar_slices(ops, oracle, monkeypatch, shape, act):
     clipped.test_bn_backward_clipped_matches_rescale_clip_then_backward(ops, oracle, act, False)
     if shape[1] < 300:
         shortcut.test_training_epilogue_with_shortcut_is_the_two_calls_to_the_bit(ops, act)
+
+
+# partial sums with 4, 4, 8 and 16 segments to a workgroup, ragged and 128-bit, the last workgroup of a channel short
+@pytest.mark.parametrize("shape", [(1, 5, 4100), (3, 90, 10245), (24, 80, 4099), (24, 80, 8200)])
+def test_split_of_a_channel(ops, oracle, monkeypatch, shape):
+    for module in (epilogue, clipped):
+        monkeypatch.setattr(module, "TRAIN_SHAPES", [shape])
+    epilogue.test_bn_train_forward_matches_oracle(ops, oracle, "leaky")
+    epilogue.test_bn_backward_matches_oracle(ops, oracle, "mish", False)
+    clipped.test_bn_backward_clipped_matches_rescale_clip_then_backward(ops, oracle, "leaky", False)
