@@ -657,12 +657,17 @@ def nms_to_host(kept, kept_count):
     """Blocking copy of the survivors as a numpy structured array."""
     # The count and as many records as a call usually leaves go to pinned memory behind the launches, and the
     # host waits once: asking for the count first is a second round trip (25 us) before the records' own.
+    # A copy goes to the current stream of its tensor's device, which need not be the current device: those are
+    # the streams to wait for, and launches of another device that the records may come from end before them.
+    if kept.device.index != _current_device():
+        torch.cuda.current_stream().synchronize()
     first = min(kept.shape[0], _FIRST_COPY)
     count = torch.empty(1, dtype=torch.int32, pin_memory=True)
     records = torch.empty((first, *kept.shape[1:]), dtype=kept.dtype, pin_memory=True)
     count.copy_(kept_count, non_blocking=True)
     records.copy_(kept[:first], non_blocking=True)
-    torch.cuda.current_stream().synchronize()
+    for device in {t.device for t in (kept, kept_count) if t.is_cuda}:
+        torch.cuda.current_stream(device).synchronize()
     n = int(count[0])
     if n <= first:
         rows = records[:n].numpy().copy()
