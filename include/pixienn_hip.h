@@ -93,7 +93,8 @@ int pxh_bn_folded_act_forward(const float* x, float* y, float* pre_activation, c
 int pxh_bias_act_forward(const float* x, float* y, float* pre_activation, const float* bias,
                          int batch, int channels, int spatial, int activation, void* stream);
 
-/* Bytes of device workspace the BN training entry points need for this shape. */
+/* Bytes of device workspace that serve the BN training entry points for this shape and for every shape with no
+ * more images, channels or values per plane. */
 size_t pxh_bn_workspace_bytes(int batch, int channels, int spatial);
 
 /* BN-training forward + activation:
@@ -208,7 +209,8 @@ int pxh_bias_act_backward(float* delta, const float* pre_activation, float* bias
  * are linear in the delta and are multiplied by the factor instead -- within rounding of the two-call
  * sequence, not bit-identical to it.  When nothing changes the results are those of
  * pxh_bn_act_backward to the bit.
- * workspace: pxh_bn_clipped_workspace_bytes(), or NULL for the library's. */
+ * workspace: pxh_bn_clipped_workspace_bytes() (enough, like the plain one, for every smaller shape too), or
+ * NULL for the library's. */
 size_t pxh_bn_clipped_workspace_bytes(int batch, int channels, int spatial);
 int pxh_bn_act_backward_clipped(float* delta, const float* x, const float* pre_activation,
                                 const float* mean, const float* var, const float* scale, const float* bias,

@@ -1628,17 +1628,38 @@ ResidentGeom resident_geom(int batch, int channels, int spatial)
                          FastDiv(static_cast<uint32_t>(spatial)) };
 }
 
+constexpr size_t align256(size_t b) { return (b + 255) & ~static_cast<size_t>(255); }
+
 // workspace: [partial sums][per-channel constants]
 size_t partial_bytes(int batch, int channels, int spatial)
 {
     const ReduceGeom g = make_geom(batch, channels, spatial);
-    const size_t b = static_cast<size_t>(channels) * g.blocks * sizeof(double2);
-    return (b + 255) & ~static_cast<size_t>(255);
+    return align256(static_cast<size_t>(channels) * g.blocks * sizeof(double2));
+}
+
+// The most that partial_bytes() comes to for any shape up to this one: what the size functions report, so that a
+// workspace sized once for the largest batch or plane serves every smaller one (the last, shorter batch of an epoch).
+// partial_bytes() itself steps up where a smaller grid is split more finely: by halves of kItemsPerBlock, each time from
+// fewer than kFillBlocks workgroups to less than twice as many, and never beyond one item to a wavefront.
+size_t partial_bytes_up_to(int batch, int channels, int spatial)
+{
+    const ReduceGeom g = make_geom(batch, channels, spatial);
+    const size_t c = static_cast<size_t>(channels), items = static_cast<size_t>(g.items);
+    const auto blocks = [&](size_t per_block) { return c * ((items + per_block - 1) / per_block); };
+    const size_t full = blocks(kItemsPerBlock), finest = blocks(kBlock / kWave);
+    constexpr size_t kMostSplit = 2 * (kFillBlocks - 1);
+    const size_t split = finest < kMostSplit ? finest : kMostSplit;
+    return align256((full > split ? full : split) * sizeof(double2));
+}
+
+size_t workspace_bytes_with(size_t partial, int channels)
+{
+    return partial + static_cast<size_t>(channels) * sizeof(DxCoef);
 }
 
 size_t workspace_bytes(int batch, int channels, int spatial)
 {
-    return partial_bytes(batch, channels, spatial) + static_cast<size_t>(channels) * sizeof(DxCoef);
+    return workspace_bytes_with(partial_bytes(batch, channels, spatial), channels);
 }
 
 void* coef_region(void* ws, int batch, int channels, int spatial)
@@ -1648,8 +1669,6 @@ void* coef_region(void* ws, int batch, int channels, int spatial)
 
 // The clipped backward: [partial sums][per-channel constants][norm partials][plan] for the three
 // launches, [per-channel norm figures][per-channel sums][per-channel flags][plan] for the one-launch form.
-constexpr size_t align256(size_t b) { return (b + 255) & ~static_cast<size_t>(255); }
-
 struct ClippedRegions {
     double2* partial;
     DxCoef* coef;
@@ -1660,12 +1679,17 @@ struct ClippedRegions {
     ClipPlan* plan;
 };
 
-size_t clipped_workspace_bytes(int batch, int channels, int spatial)
+size_t clipped_workspace_bytes_with(size_t partial, int channels)
 {
     const size_t c = static_cast<size_t>(channels);
-    const size_t three = 2 * partial_bytes(batch, channels, spatial) + align256(c * sizeof(DxCoef)) + 256;
+    const size_t three = 2 * partial + align256(c * sizeof(DxCoef)) + 256;
     const size_t one = 2 * align256(c * sizeof(double2)) + align256(c * sizeof(int)) + 256;
     return three > one ? three : one;
+}
+
+size_t clipped_workspace_bytes(int batch, int channels, int spatial)
+{
+    return clipped_workspace_bytes_with(partial_bytes(batch, channels, spatial), channels);
 }
 
 ClippedRegions clipped_regions(void* ws, int batch, int channels, int spatial)
@@ -1822,7 +1846,7 @@ extern "C" {
 size_t pxh_bn_workspace_bytes(int batch, int channels, int spatial)
 {
     if (batch <= 0 || channels <= 0 || spatial <= 0) return 0;
-    return workspace_bytes(batch, channels, spatial);
+    return workspace_bytes_with(partial_bytes_up_to(batch, channels, spatial), channels);
 }
 
 size_t pxh_bn_folded_bytes(int channels)
@@ -2176,7 +2200,7 @@ int pxh_bn_act_backward(float* delta, const float* x, const float* pre_activatio
 size_t pxh_bn_clipped_workspace_bytes(int batch, int channels, int spatial)
 {
     if (batch <= 0 || channels <= 0 || spatial <= 0) return 0;
-    return clipped_workspace_bytes(batch, channels, spatial);
+    return clipped_workspace_bytes_with(partial_bytes_up_to(batch, channels, spatial), channels);
 }
 
 int pxh_bn_act_backward_clipped(float* delta, const float* x, const float* pre_activation, const float* mean,

@@ -98,6 +98,44 @@ def test_workspace_sizes():
     assert lib.pxh_bn_folded_bytes(1024) == 1024 * 32 and lib.pxh_bn_folded_bytes(0) == 0
 
 
+def needed(name, *args):
+    """The bytes an entry point asks for, from its refusal of a workspace of 16 (nothing is launched)."""
+    assert capi.call_raw(name, *args, 256, 16, None) == -3
+    return int(re.search(r"(\d+) needed", capi.last_error()).group(1))
+
+
+def test_bn_workspace_serves_every_smaller_shape():
+    """A workspace of the size reported for a batch, a number of channels and a plane is taken for any fewer."""
+    lib = capi.load()
+    p = 256
+    sizes = {"pxh_bn_stats": lib.pxh_bn_workspace_bytes, "pxh_bn_act_backward": lib.pxh_bn_workspace_bytes,
+             "pxh_bn_act_backward_clipped": lib.pxh_bn_clipped_workspace_bytes}
+
+    def need(name, n, c, s):
+        if name == "pxh_bn_stats":
+            return needed(name, p, p, p, n, c, s)
+        clip = (1e5, 100.0, None) if name.endswith("clipped") else ()
+        return needed(name, p, p, None, p, p, p, p, p, p, None, None, n, c, s, 0, *clip)
+
+    for name, size in sizes.items():
+        # batch by batch, where the split of a channel changes with the number of workgroups
+        for c, s in ((64, 92416), (128, 23104), (72, 10395), (95, 1025), (8, 4099), (90, 700), (1, 65537)):
+            if c >= 96 and name == "pxh_bn_act_backward":
+                continue                      # its one-launch form asks for nothing and would be launched
+            most = 0
+            for n in range(1, 40):
+                most = max(most, need(name, n, c, s))
+                assert size(n, c, s) >= most, (name, n, c, s)
+        # shape against shape
+        import random
+        r = random.Random(7)
+        for _ in range(4000):
+            big = r.randint(1, 64), r.randint(1, 95), r.randint(1, 20000)
+            n, c, s = (r.randint(1, v) for v in big)
+            assert need(name, n, c, s) <= size(*big), (name, n, c, s, big)
+            assert size(n, c, s) <= size(*big)
+
+
 def test_ops_refuse_cpu_tensors():
     import torch
     from pixienn_amd import ops
