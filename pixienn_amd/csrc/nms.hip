@@ -623,7 +623,7 @@ __global__ __launch_bounds__(kWide) void nms_small_kernel(const pxh_detection* r
 //   6. a survivor's place in the whole list is the number of survivors before it in each image, found
 //      by bisection, one lane per image.
 // A mask has 64 words, of which as many that are not empty are stored as 10 MB hold for the whole list (all
-// of them up to 8738 records, eight for 65536), so that the longest list fits the library's first workspace.
+// of them up to 9102 records, eight for 65536), so that the longest list fits the library's first workspace.
 // Step 5 looks at the pairs of a further one again, and at those of a set bit in an image of more than 4096
 // records, where a bit stands for 2, 4, ... 16 neighbouring places.
 constexpr int kImageCapacity = 65536;                 // longest list: a state bit set is 8 KB of LDS
@@ -631,11 +631,15 @@ constexpr int kImageBatch = kWide;                    // most images: one lane e
 constexpr int kMaskWords = 64;
 constexpr size_t kMaskBytes = 10u << 20;
 
-// words of a mask that are stored, each with the byte that says which one it is
+// words of one pass's masks for the whole list, each with the byte that says which one it is
+constexpr size_t kMaskListWords = kMaskBytes / (2 * 9);
+static_assert(kMaskListWords / kImageCapacity >= 8, "the longest list stores some");
+
+// words of a mask that are stored
 int mask_slots(int capacity)
 {
-    const size_t fit = kMaskBytes / (2 * 9 * static_cast<size_t>(capacity));
-    return fit < 8 ? 8 : fit > kMaskWords ? kMaskWords : static_cast<int>(fit);
+    const size_t fit = kMaskListWords / static_cast<size_t>(capacity);
+    return fit > kMaskWords ? kMaskWords : static_cast<int>(fit);
 }
 constexpr int kBitSetWords = kImageCapacity / 64;
 
@@ -1108,8 +1112,8 @@ bool by_image(int capacity, int batch)
     return batch <= kImageBatch && capacity <= kImageCapacity && (capacity <= 8192 || capacity / 2048 <= batch);
 }
 
-// The same for the launches by image; `args` gets every pointer.
-size_t carve_images(void* base, int capacity, int batch, ImageArgs& args)
+// The same for the launches by image; `args` gets every pointer.  `mask_words`: of one pass's masks.
+size_t carve_images(void* base, int capacity, int batch, size_t mask_words, ImageArgs& args)
 {
     const size_t cap = static_cast<size_t>(capacity);
     const size_t tiles = (cap + kWide - 1) / kWide, images = static_cast<size_t>(batch);
@@ -1134,14 +1138,19 @@ size_t carve_images(void* base, int capacity, int batch, ImageArgs& args)
     take(args.group_index, cap);
     take(args.slots, cap);
     for (int k = 0; k < 2; ++k) {
-        take(args.ids[k], cap * args.mask_slots);
+        take(args.ids[k], mask_words);
         take(args.beyond[k], cap);
-        take(args.masks[k], cap * args.mask_slots);
+        take(args.masks[k], mask_words);
     }
     take(args.kept_key, cap);
     take(args.kept_source, cap);
     take(args.kept_images, images);
     return at;
+}
+
+size_t carve_images(void* base, int capacity, int batch, ImageArgs& args)
+{
+    return carve_images(base, capacity, batch, static_cast<size_t>(capacity) * mask_slots(capacity), args);
 }
 
 std::atomic<int> g_sweeps{ 6 };      // parallel sweeps of the duplicate pass before the per-image loop takes over
@@ -1158,9 +1167,12 @@ size_t pxh_nms_workspace_bytes(int capacity)
     if (capacity <= 0) return 0;
     const size_t sorted = carve(nullptr, capacity).bytes;
     if (capacity <= kSmall) return sorted;
-    // the most that any batch asks for; a longer list's bytes also serve every shorter one
+    // The most that any batch and any shorter list ask for, so that a longer list's bytes serve every shorter one:
+    // a list whose records store fewer mask words can need less than a shorter one, but none more than fills kMaskBytes.
+    const int most = capacity < kImageCapacity ? capacity : kImageCapacity;
+    const size_t every_word = static_cast<size_t>(most) * kMaskWords;
     ImageArgs args{};
-    const size_t by_image = carve_images(nullptr, capacity < kImageCapacity ? capacity : kImageCapacity, kImageBatch, args);
+    const size_t by_image = carve_images(nullptr, most, kImageBatch, every_word < kMaskListWords ? every_word : kMaskListWords, args);
     return by_image > sorted ? by_image : sorted;
 }
 

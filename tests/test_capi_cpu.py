@@ -136,6 +136,19 @@ def test_bn_workspace_serves_every_smaller_shape():
             assert size(n, c, s) <= size(*big)
 
 
+def test_nms_workspace_serves_every_shorter_list():
+    """Also where a record of a longer list stores fewer mask words (9102 / 9103, 64726 / 65536), and any batch."""
+    lib = capi.load()
+    sizes = sorted({c for edge in range(8, 65) for c in (582542 // edge, 582542 // edge + 1)} |
+                   {513, 1024, 1025, 8192, 8193, 16384, 16385, 32768, 58254, 65535, 65536, 65537, 100000})
+    most = 0
+    for capacity in sizes:
+        for batch in (1, 4, 32, 1024, 1025):
+            most = max(most, needed("pxh_nms", 256, 256, capacity, batch, 80, 0.45, 512, 512))
+        assert lib.pxh_nms_workspace_bytes(capacity) >= most, capacity
+    assert lib.pxh_nms_workspace_bytes(65536) <= 16 << 20          # the library's first buffer
+
+
 def test_ops_refuse_cpu_tensors():
     import torch
     from pixienn_amd import ops
