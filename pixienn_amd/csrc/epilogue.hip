@@ -10,6 +10,7 @@
 #include "stream.h"
 
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 // Device memory for pxh_bn_train_act_forward_static, the entry point for callers that must not
@@ -969,6 +970,7 @@ constexpr int kResidentThreads = 1024;
 // The scalar forms also come with workgroups of half the size, four to a compute unit instead of two:
 // for the layers with a thousand channels of 19 x 19, whose workgroups would otherwise run in two rounds.
 constexpr int kResidentNarrowThreads = 512;
+constexpr int kResidentVectors = 8;            // per lane of the small forms
 
 // Sum of two doubles over the workgroup; every thread returns both totals.
 template<int T>
@@ -1072,6 +1074,28 @@ struct ResidentGeom {
     }
 };
 
+// The sums of a slice: fp32 per lane, except in the scalar forms that hold more than kResidentVectors values per lane.
+// Those shapes otherwise take three launches, which add a lane's share of one image in fp32 (three values of a 13 x 13
+// plane, one of a plane of up to 64) and carry on in doubles; sixteen or twenty-four values in fp32 lose two to three
+// times as much.  Here two values are added in fp32 where the three launches add as many or more, none where they add
+// fewer, and everything beyond in doubles.  Against fp32 throughout, forward and backward, us: 64 x 256 x 13^2 8.5 -> 8.7
+// and 11.6 -> 11.8, 64 x 1024 x 13^2 27.6 -> 27.7 and 37.3 -> 38.6.  (Every value into a double of its own: 9.1 and 12.1,
+// 28.2 and 39.0.)
+template<int V, int R, int L, int T>
+constexpr bool kWideSlice = V == 1 && (R + L) * T > kResidentVectors * kResidentThreads;
+constexpr int kPairSpatial = 2 * kWave;        // from this plane on a lane of the three launches adds two values and more
+
+__device__ __forceinline__ void add_two(double& sum, float v, float w, bool pair)
+{
+    if (pair) {
+        sum += static_cast<double>(v + w);
+    } else {
+        asm volatile("" : "+v"(v));     // a branch, not both ways and a choice: `pair` is the same for every lane
+        sum += static_cast<double>(v);
+        sum += static_cast<double>(w);
+    }
+}
+
 struct ResidentFwdArgs {
     const float* x;
     float* y;
@@ -1120,6 +1144,8 @@ __global__ __launch_bounds__(T, L == 0 && V * R <= (V == 1 ? (RES ? 8 : 16) : 32
     const float shift = a.x[static_cast<size_t>(c) * a.g.spatial];
     // issued now, needed after the reduction
     const float rm_in = a.rolling_mean[c], rv_in = a.rolling_var[c], scale_in = a.scale[c], bias_in = a.bias[c];
+    constexpr bool kWide = kWideSlice<V, R, L, T>;
+    static_assert(!kWide || (L == 0 && R % 2 == 0), "values are taken in pairs");
     Pack<V> v[R];
     float a1 = 0.0f, a2 = 0.0f;
     [[maybe_unused]] float b1 = 0.0f, b2 = 0.0f;
@@ -1179,13 +1205,27 @@ __global__ __launch_bounds__(T, L == 0 && V * R <= (V == 1 ? (RES ? 8 : 16) : 32
             ahead[i] = ld<V, true>(a.residual, a.g.at(c, e < a.g.per_channel ? e : 0u));
         }
     }
+    double t1, t2;
+    if constexpr (kWide) {
+        t1 = t2 = 0.0;
+        const bool pair = a.g.spatial >= kPairSpatial;
 #pragma unroll
-    for (int r = R - 1; r >= 0; --r) add(r, v[r]);
-    double s1 = static_cast<double>(a1), s2 = static_cast<double>(a2);
-    if constexpr (kTwin) resident_sum2_twin<T>(s1, s2, static_cast<double>(b1), static_cast<double>(b2), slots);
-    else resident_sum2<T>(s1, s2, slots);
+        for (int r = R - 1; r >= 0; r -= 2) {
+            const float d = element(r) < a.g.per_channel ? v[r].v[0] - shift : 0.0f;
+            const float f = element(r - 1) < a.g.per_channel ? v[r - 1].v[0] - shift : 0.0f;
+            add_two(t1, d, f, pair);
+            add_two(t2, d * d, f * f, pair);
+        }
+    } else {
+#pragma unroll
+        for (int r = R - 1; r >= 0; --r) add(r, v[r]);
+        t1 = static_cast<double>(a1);
+        t2 = static_cast<double>(a2);
+    }
+    if constexpr (kTwin) resident_sum2_twin<T>(t1, t2, static_cast<double>(b1), static_cast<double>(b2), slots);
+    else resident_sum2<T>(t1, t2, slots);
     if (threadIdx.x == 0) {
-        const ChannelStats st = channel_stats(s1, s2, shift, static_cast<double>(a.g.per_channel), rm_in, rv_in);
+        const ChannelStats st = channel_stats(t1, t2, shift, static_cast<double>(a.g.per_channel), rm_in, rv_in);
         a.mean[c] = st.mean;
         a.var[c] = st.var;
         a.rolling_mean[c] = st.rolling_mean;
@@ -1342,8 +1382,10 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
     };
     const bool recompute = a.b.pre == nullptr;
     Pack<V> d[R];
-    float fa = 0.0f, fb = 0.0f;
-    [[maybe_unused]] float fq = 0.0f, peak = 0.0f;
+    constexpr bool kWide = kWideSlice<V, R, L, T>;
+    std::conditional_t<kWide, double, float> fa = 0, fb = 0;
+    [[maybe_unused]] std::conditional_t<kWide, double, float> fq = 0;
+    [[maybe_unused]] float peak = 0.0f;
     // Two shapes of the first pass.  Grouped: no branch around the loads (see the forward kernel), lanes
     // past the end read the first vector; kGroup steps at a time, their loads go out together, then each
     // is used as it arrives.  The large form (part of the slice in LDS) is bound by its loads and takes
@@ -1367,7 +1409,7 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
     // rescale + clamp (kRedo), then the activation's gradient
     const auto prepared = [&](float t, float pre, bool valid) {
         if constexpr (MODE == kFirst) {
-            fq += valid ? t * t : 0.0f;
+            if constexpr (!kWide) fq += valid ? t * t : 0.0f;
             peak = fmaxf(peak, valid ? fabsf(t) : 0.0f);
         }
         if constexpr (MODE == kRedo) t = rescaled_clipped(t, factor, limit);
@@ -1382,10 +1424,13 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
             for (int q = 0; q < V; ++q) {
                 const float t = prepared(dv.v[q], ACT != PXH_LINEAR ? pv.v[q] : 0.0f, valid);
                 dv.v[q] = t;
-                fa += valid ? t : 0.0f;
-                fb += valid ? t * (xv.v[q] - k.mean) : 0.0f;
+                if constexpr (!kWide) {
+                    fa += valid ? t : 0.0f;
+                    fb += valid ? t * (xv.v[q] - k.mean) : 0.0f;
+                }
             }
         };
+        [[maybe_unused]] const bool pair = a.g.spatial >= kPairSpatial;
 #pragma unroll
         for (int top = R + L - 1; top >= 0; top -= kGroup) {
             Pack<V> dv[kGroup], xv[kGroup], pv[kGroup];
@@ -1409,10 +1454,29 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
                     }
                 }
             }
+            if constexpr (kWide) {
+#pragma unroll
+                for (int i = 0; i < kGroup; i += 2) {
+                    const bool valid[2] = { element(top - i) < a.g.per_channel, element(top - i - 1) < a.g.per_channel };
+                    float va[2], vb[2], vq[2];
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        const float raw = dv[i + u].v[0];
+                        take(top - i - u, dv[i + u], xv[i + u], pv[i + u]);
+                        const float t = dv[i + u].v[0];
+                        va[u] = valid[u] ? t : 0.0f;
+                        vb[u] = valid[u] ? t * (xv[i + u].v[0] - k.mean) : 0.0f;
+                        vq[u] = valid[u] ? raw * raw : 0.0f;
+                    }
+                    add_two(fa, va[0], va[1], pair);
+                    add_two(fb, vb[0], vb[1], pair);
+                    if constexpr (MODE == kFirst) add_two(fq, vq[0], vq[1], pair);
+                }
+            }
 #pragma unroll
             for (int i = 0; i < kGroup; ++i) {
                 const int r = top - i;
-                take(r, dv[i], xv[i], pv[i]);
+                if constexpr (!kWide) take(r, dv[i], xv[i], pv[i]);
                 if (r < R) d[r < R ? r : 0] = dv[i];
                 else *resident_lds_slot<V, R>(resident_lds, r) = dv[i];
             }
@@ -1548,8 +1612,8 @@ __global__ __launch_bounds__(T, L == 0 && MODE != kRedo && !(V == 1 && R > 16) ?
 // the channel slice must fit, and there must be enough channels to occupy the machine.  (Measured
 // with 24 vectors per thread: the registers spill and 128 workgroups of 16x128x76^2 are slower than
 // the three launches; with a third of them in LDS they do not.)
-constexpr int kResidentVectors = 8;
-// the large form (128-bit vectors only): 16 vectors in registers + 8 in LDS (128 KB of the CU's 160)
+// The small forms hold kResidentVectors (above);
+// the large form (128-bit vectors only) 16 vectors in registers + 8 in LDS (128 KB of the CU's 160)
 constexpr int kResidentLargeRegs = 16, kResidentLargeLds = 8;
 constexpr size_t kResidentLargeLdsBytes = static_cast<size_t>(kResidentLargeLds) * kResidentThreads * 16;
 // The scalar forms (odd planes) with more values per lane: 16 in 64 registers, two workgroups per compute unit
