@@ -1128,9 +1128,11 @@ __device__ __forceinline__ Pack<V>* resident_lds_slot(float* lds, int r)
 constexpr int kResidualAhead = 4;
 
 // V = 4 needs spatial % 4 == 0 and 16-byte aligned tensors.  R + L vectors per thread at most.
-template<int ACT, int V, int R, int L, int T = kResidentThreads, bool RES = false>
-__global__ __launch_bounds__(T, L == 0 && V * R <= (V == 1 ? (RES ? 8 : 16) : 32) ? 8 : 4) void bn_resident_fwd_kernel(ResidentFwdArgs a)
+// TIGHT: the scalar form with the shortcut's source on top in 64 registers, two workgroups per compute unit.
+template<int ACT, int V, int R, int L, int T = kResidentThreads, bool RES = false, bool TIGHT = false>
+__global__ __launch_bounds__(T, L == 0 && V * R <= (V == 1 ? (RES && !TIGHT ? 8 : 16) : 32) ? 8 : 4) void bn_resident_fwd_kernel(ResidentFwdArgs a)
 {
+    static_assert(!TIGHT || (RES && V == 1 && L == 0), "a form of the riding shortcut");
     static_assert(L == 0 || T == kResidentThreads, "the LDS part is laid out for the full workgroup");
     extern __shared__ __align__(16) float resident_lds[];
     // The 128-bit form with workgroups of half the size adds a channel up exactly as the full workgroups do,
@@ -1155,7 +1157,8 @@ __global__ __launch_bounds__(T, L == 0 && V * R <= (V == 1 ? (RES ? 8 : 16) : 32
     // No branch around a load: a lane past the end of the slice reads the slice's first vector and
     // adds nothing, so that the loads of a lane are in flight together (behind a branch each one is
     // waited for before the next is issued, and a wave then has one kilobyte on its way at a time).
-    const auto element = [&](int r) { return static_cast<uint32_t>(r * T + threadIdx.x) * V; };
+    uint32_t lane = threadIdx.x;
+    const auto element = [&](int r) { return (static_cast<uint32_t>(r * T) + lane) * V; };
     const auto fetch = [&](int r) {
         const uint32_t e = element(r);
         return ld<V, true>(a.x, a.g.at(c, e < a.g.per_channel ? e : 0u));
@@ -1196,7 +1199,7 @@ __global__ __launch_bounds__(T, L == 0 && V * R <= (V == 1 ? (RES ? 8 : 16) : 32
     // (16 x 1024 x 19^2: 19.9 us against 25.6 us with every step's load behind the reduction).
     // (the half-size workgroups of the 128-bit form have 128 registers: eight of twelve steps, four of sixteen)
     constexpr int kAhead = !RES ? 0 : V * (R + L) <= 8 ? R + L : L > 0 ? kResidualAhead
-                                : T < kResidentThreads ? (R <= 12 ? 8 : 4) : V == 1 && R >= 16 ? 4 : 0;
+                                : T < kResidentThreads ? (R <= 12 ? 8 : 4) : V == 1 && R >= 16 ? (TIGHT ? 8 : 4) : 0;
     [[maybe_unused]] Pack<V> ahead[kAhead > 0 ? kAhead : 1];
     if constexpr (RES) {
 #pragma unroll
@@ -1234,8 +1237,9 @@ __global__ __launch_bounds__(T, L == 0 && V * R <= (V == 1 ? (RES ? 8 : 16) : 32
     }
     __syncthreads();
     const FoldCoef k = shared_coef;
+    if constexpr (TIGHT) asm volatile("" : "+v"(lane));      // addresses formed again, not kept: 60 registers, not 112
     const auto apply = [&](int r, [[maybe_unused]] const Pack<V>& from) {
-        const uint32_t e = (r * T + threadIdx.x) * V;
+        const uint32_t e = element(r);
         if (e < a.g.per_channel) {
             const size_t where = a.g.at(c, e);
             const Pack<V> t = r < R ? v[r < R ? r : 0] : *resident_lds_slot<V, R>(resident_lds, r);
@@ -1616,33 +1620,36 @@ __global__ __launch_bounds__(T, L == 0 && MODE != kRedo && !(V == 1 && R > 16) ?
 // the large form (128-bit vectors only) 16 vectors in registers + 8 in LDS (128 KB of the CU's 160)
 constexpr int kResidentLargeRegs = 16, kResidentLargeLds = 8;
 constexpr size_t kResidentLargeLdsBytes = static_cast<size_t>(kResidentLargeLds) * kResidentThreads * 16;
-// The scalar forms (odd planes) with more values per lane: 16 in 64 registers, two workgroups per compute unit
-// (one with a shortcut's source on top); the backward also 24 in 128 registers.  Against the three launches, us:
+// The scalar forms (odd planes) with more values per lane: 16 in 64 registers, two workgroups per compute unit; the
+// backward also 24 in 128 registers.  Against the three launches, us:
 //                       forward        + shortcut     backward
-//   64 x 256 x 13^2     15.1 ->  8.7   15.9 -> 11.4   21.9 -> 11.6   leaky
-//   64 x 512 x 13^2     22.1 -> 14.4   24.3 -> 22.2   32.2 -> 17.8
-//   64 x 1024 x 13^2    36.5 -> 27.6   41.3 -> 43.8   49.7 -> 37.9
-//   64 x 512 x 19^2     29.7 -> 28.3   38.9 -> 54.0   49.6 -> 36.6   24 values
-//   64 x 256 x 13^2     15.8 -> 11.9   16.4 -> 13.1   28.5 -> 20.7   mish
-//   64 x 512 x 13^2     22.7 -> 18.5   24.9 -> 24.5   40.6 -> 35.4
+//   64 x 256 x 13^2     15.2 ->  8.7   16.0 -> 11.8   21.8 -> 11.8   leaky
+//   64 x 512 x 13^2     22.1 -> 14.4   24.1 -> 17.6   32.0 -> 18.5
+//   49 x 1024 x 13^2    31.4 -> 23.5   35.7 -> 30.0   43.2 -> 32.1
+//   64 x 1024 x 13^2    36.5 -> 27.7   41.7 -> 38.4   49.1 -> 38.6
+//   32 x 1024 x 19^2    29.9 -> 27.4   41.6 -> 35.8   49.7 -> 37.2
+//   64 x 512 x 19^2     29.7 -> 28.3   38.9 -> 54.0   49.9 -> 36.6   24 values
+//   64 x 256 x 13^2     15.7 -> 12.1   16.4 -> 13.4   28.5 -> 20.8   mish
+//   64 x 512 x 13^2     22.7 -> 19.2   25.1 -> 21.4   40.4 -> 35.8
 //   32 x 1024 x 19^2    30.8 -> 37.1   39.6 -> 52.4   64.8 -> 66.5
 //   64 x 512 x 19^2     30.1 -> 34.7   40.3 -> 64.3   64.5 -> 61.8   24 values
-// An activation with an exponential, or a second tensor, leaves a workgroup that waits for its own channel more to do
-// after the wait, and a thousand channels keep the three launches' many small workgroups busy: those take the
-// one-launch form only up to 512 channels, and 24 values only where the backward's gradient is a select.
-// (Forward with 24 values the shortcut would lose, and a layer below 512 channels has the same statistics to the
-// bit with and without one: no such form.)
+// An activation with an exponential leaves a workgroup that waits for its own channel more to do after the wait, and a
+// thousand channels keep the three launches' many small workgroups busy: it takes the one-launch form only up to 512
+// channels, and 24 values only where the backward's gradient is a select.  (Forward with 24 values the shortcut would
+// lose, and a layer has the same statistics to the bit with and without one: no such form.)
 constexpr int kResidentScalarMid = 16, kResidentScalarWide = 24;
 constexpr int kResidentScalarFew = 512;
+// Beyond this the riding form runs two workgroups to a compute unit (64 x 512 x 13^2, leaky: 17.6 against 20.7 us); up to
+// it every channel finds a compute unit of its own, and the form that keeps its addresses is ahead (64 x 256 x 13^2: 11.2
+// against 11.8, mish 12.6 against 14.2).
+constexpr int kResidentTight = 256;
 
 constexpr bool selects(int activation)
 {
     return activation == PXH_LEAKY || activation == PXH_RELU || activation == PXH_LINEAR;
 }
 
-enum class Pass { Forward, ForwardShortcut, Backward };
-
-int resident_vectors(int batch, int channels, int spatial, bool vec, int activation, Pass pass)
+int resident_vectors(int batch, int channels, int spatial, bool vec, int activation, bool backward)
 {
     if (channels < 96) return 0;
     const size_t per_channel = static_cast<size_t>(batch) * spatial;
@@ -1650,9 +1657,9 @@ int resident_vectors(int batch, int channels, int spatial, bool vec, int activat
     const size_t per_thread = (vectors + kResidentThreads - 1) / kResidentThreads;
     if (per_thread <= kResidentVectors) return kResidentVectors;
     if (vec) return per_thread <= kResidentLargeRegs + kResidentLargeLds ? kResidentLargeRegs + kResidentLargeLds : 0;
-    const bool light = selects(activation) && pass != Pass::ForwardShortcut;
+    const bool light = selects(activation);
     if (per_thread <= kResidentScalarMid && (light || channels <= kResidentScalarFew)) return kResidentScalarMid;
-    if (per_thread <= kResidentScalarWide && light && pass == Pass::Backward) return kResidentScalarWide;
+    if (per_thread <= kResidentScalarWide && light && backward) return kResidentScalarWide;
     return 0;
 }
 
@@ -1823,8 +1830,7 @@ int bn_train_forward(const char* who, const float* x, float* y, float* pre_activ
     {
         const bool vec = spatial % 4 == 0 && aligned16(x) && aligned16(y) && aligned16(pre_activation) &&
                          aligned16(x_saved) && aligned16(x_norm) && aligned16(res.from);
-        const int per_thread = resident_vectors(batch, channels, spatial, vec, activation,
-                                                res.from ? Pass::ForwardShortcut : Pass::Forward);
+        const int per_thread = resident_vectors(batch, channels, spatial, vec, activation, false);
         if (per_thread) {
             const ResidentFwdArgs r{ x, y, pre_activation, x_saved, x_norm, mean, var, rolling_mean, rolling_var,
                                      scale, bias, resident_geom(batch, channels, spatial), res.from, res.alpha, res.beta };
@@ -1864,7 +1870,11 @@ int bn_train_forward(const char* who, const float* x, float* y, float* pre_activ
                         return;
                     }
                 }
-                if (!vec && per_thread == kResidentScalarMid) {
+                if (RES && !vec && per_thread == kResidentScalarMid && channels > kResidentTight) {
+                    if constexpr (RES)
+                        hipLaunchKernelGGL((bn_resident_fwd_kernel<ACT, 1, kResidentScalarMid, 0, kT, true, true>), grid, block,
+                                           0, s, r);
+                } else if (!vec && per_thread == kResidentScalarMid) {
                     hipLaunchKernelGGL((bn_resident_fwd_kernel<ACT, 1, kResidentScalarMid, 0, kT, RES>), grid, block, 0, s, r);
                 } else if (per_thread > kResidentVectors) {
                     auto kernel = bn_resident_fwd_kernel<ACT, 4, kResidentLargeRegs, kResidentLargeLds, kT, RES>;
@@ -2120,7 +2130,7 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
     if (rc) return rc;
     hipStream_t s = as_stream(stream);
     const bool rvec = spatial % 4 == 0 && aligned16(delta) && aligned16(x) && aligned16(pre_activation);
-    const int per_thread = resident_vectors(batch, channels, spatial, rvec, activation, Pass::Backward);
+    const int per_thread = resident_vectors(batch, channels, spatial, rvec, activation, true);
     void* ws = nullptr;
     ClippedRegions region{};
     ClipArgs clip{};
