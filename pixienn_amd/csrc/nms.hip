@@ -611,7 +611,7 @@ __global__ __launch_bounds__(kWide) void nms_small_kernel(const pxh_detection* r
 // Every decision of nms is taken inside one image, so the records are grouped by image first and
 // nothing is sorted: six launches in place of the sorting path's forty-five, whose cost at the few
 // thousand records of a validation batch is the launches and the latency of short dependent steps
-// (7126 records of 16 images in a list for 32768: 440 us in kernels, here 60).
+// (7126 records of 16 images in a list for 32768: 440 us in kernels, here 76).
 //   1. images are counted per tile of 1024 records, 2. the records' keys are laid out image by image,
 //      in any order inside one;
 //   3. a record's place in its image is the number of smaller keys there, counted directly: n^2 of the
@@ -622,13 +622,25 @@ __global__ __launch_bounds__(kWide) void nms_small_kernel(const pxh_detection* r
 //   5. one workgroup per image settles both passes on the masks alone, the states as bit sets in LDS;
 //   6. a survivor's place in the whole list is the number of survivors before it in each image, found
 //      by bisection, one lane per image.
-// A mask has 64 words, of which as many that are not empty are stored as 10 MB hold for the whole list (all
-// of them up to 9102 records, eight for 65536), so that the longest list fits the library's first workspace.
-// Step 5 looks at the pairs of a further one again, and at those of a set bit in an image of more than 4096
-// records, where a bit stands for 2, 4, ... 16 neighbouring places.
-constexpr int kImageCapacity = 65536;                 // longest list: a state bit set is 8 KB of LDS
+// A mask has 16 words, a bit to a place, of which as many that are not empty are stored as 10 MB hold for the whole
+// list (all of them up to 36408 records, eight for 65536), so that the longest list fits the library's first workspace.
+// Step 5 looks at the pairs of a further one again.
+// An image of more than 1024 places has no masks, and more pairs than one workgroup should settle: further workgroups of
+// step 5 settle it block by block, 64 places each, the blocks' pairs all over the chip at once and only the decisions
+// one after the other (further down).
+constexpr int kImageCapacity = 65536;                 // longest list
 constexpr int kImageBatch = kWide;                    // most images: one lane each
-constexpr int kMaskWords = 64;
+constexpr int kMaskWords = 16;
+// Places of an image; larger ones are settled block by block.  Masks against blocks, us: one image of 1100 around 6
+// places 117 -> 78, around 100 80 -> 73; 4000 of one class 243 -> 130; 16 images of 1250 around 100 places 128 -> 132 and
+// 32 of 1875 around 20 304 -> 308; but 64 of 625 around 20 163 -> 235 with the line at 512.
+constexpr uint32_t kLargeImage = 64 * kMaskWords;
+static_assert(kLargeImage <= kGroupVisit, "no place of an image with masks is past those that are visited");
+static_assert(kLargeImage == kWide, "a lane to a place where one workgroup settles an image, a wave to a word of the masks");
+// What a settled block leaves for those behind it: the places that the first pass kept, the kept places of the second
+// that can still suppress one (two words each), the survivors of the image so far.
+constexpr uint32_t kSettledWords = 5, kSettledStride = 8;
+constexpr unsigned kSettleWorkgroups = 256;           // one to a compute unit
 constexpr size_t kMaskBytes = 10u << 20;
 
 // words of one pass's masks for the whole list, each with the byte that says which one it is
@@ -641,7 +653,6 @@ int mask_slots(int capacity)
     const size_t fit = kMaskListWords / static_cast<size_t>(capacity);
     return fit > kMaskWords ? kMaskWords : static_cast<int>(fit);
 }
-constexpr int kBitSetWords = kImageCapacity / 64;
 
 // 64 places of one image
 struct PlaceBlock {
@@ -663,12 +674,14 @@ struct ImageArgs {
     uint32_t* source;
     float4* box;
     uint32_t* cls;
-    uint32_t* group_index;    // earlier records of the same image and class
     int mask_slots;
     uint32_t* slots;          // stored words of a place's masks: [0] other classes, [1] same class << 8
     uint8_t* ids[2];          // [slot][place]: which word it is
     uint64_t* masks[2];       // [slot][place]
     uint64_t* beyond[2];      // words that are not empty and not stored
+    uint32_t* first_block;    // of each image
+    uint32_t* ticket;         // large images: the next block to be settled,
+    uint64_t* settled;        // and what each left for the blocks behind it, [block][kSettledStride]
     uint64_t* kept_key;       // survivors, image by image, in rank order
     uint32_t* kept_source;
     uint32_t* kept_images;    // survivors per image
@@ -677,14 +690,6 @@ struct ImageArgs {
 __device__ __forceinline__ uint32_t image_of(const pxh_detection& d, int batch)
 {
     return static_cast<uint32_t>(min(max(d.batch, 0), batch - 1));
-}
-
-// log2 of the places that a mask bit stands for
-__device__ __forceinline__ int mask_grain(uint32_t places)
-{
-    int g = 0;
-    while ((static_cast<uint32_t>(kMaskWords * 64) << g) < places) ++g;
-    return g;
 }
 
 __global__ __launch_bounds__(kWide) void nms_count_images_kernel(ImageArgs a)
@@ -727,6 +732,10 @@ __global__ __launch_bounds__(kWide) void nms_group_images_kernel(ImageArgs a)
         const uint32_t mine = (all + 63) / 64;
         const uint32_t first_block = wide_exclusive_scan(mine, scan_lds, total);
         if (t <= static_cast<uint32_t>(a.batch) && t < kWide) a.image_begin[t] = begin;
+        if (t < static_cast<uint32_t>(a.batch)) {
+            a.first_block[t] = first_block;
+            a.ticket[t] = 0;
+        }
         if (t == 0) {
             *a.block_count = total;
             a.image_begin[a.batch] = n;
@@ -792,14 +801,17 @@ __global__ __launch_bounds__(kWide) void nms_place_kernel(ImageArgs a)
 }
 
 // One workgroup per 64 places, a lane per place, a wave per word of its masks: the earlier places that
-// the word stands for are loaded 64 at a time and handed round lane by lane.
+// the word stands for are loaded side by side and handed round lane by lane.
 __global__ __launch_bounds__(kWide) void nms_conflicts_kernel(ImageArgs a)
 {
     __shared__ uint64_t beyond[2][kWave];
     __shared__ uint32_t slots[2][kWave];
-    __shared__ uint32_t index[kWave];
     if (live_count(a.count, a.capacity) == 0 || blockIdx.x >= *a.block_count) return;
     const PlaceBlock b = a.blocks[blockIdx.x];
+    if (b.image_end - b.image_begin > kLargeImage) {
+        if (threadIdx.x < kSettledWords) a.settled[blockIdx.x * kSettledStride + threadIdx.x] = 0;
+        return;
+    }
     const uint32_t lane = threadIdx.x & (kWave - 1);
     const uint32_t wave = threadIdx.x / kWave;
     if (threadIdx.x < kWave) {
@@ -807,38 +819,28 @@ __global__ __launch_bounds__(kWide) void nms_conflicts_kernel(ImageArgs a)
             beyond[pass][threadIdx.x] = 0;
             slots[pass][threadIdx.x] = 0;
         }
-        index[threadIdx.x] = 0;
     }
     __syncthreads();
     const bool live = b.first + lane < b.image_end;
     const uint32_t p = live ? b.first + lane : b.first;
     const float4 box = a.box[p];
     const uint32_t cls = a.cls[p];
-    const int grain = mask_grain(b.image_end - b.image_begin);
     const uint32_t upto = min(b.first + kWave, b.image_end);
-    uint32_t same_before = 0;
-    for (uint32_t word = wave; ; word += kWide / kWave) {
-        const uint32_t q_first = b.image_begin + ((word * 64u) << grain);
-        if (word >= kMaskWords || q_first >= upto) break;
-        const uint32_t q_end = min(q_first + (64u << grain), upto);
+    const uint32_t word = wave;
+    const uint32_t q_first = b.image_begin + word * 64u;
+    if (q_first < upto) {
+        const uint32_t mine = min(q_first + lane, upto - 1);
+        const float4 their_box = a.box[mine];
+        const int their_class = static_cast<int>(a.cls[mine]);
+        const int here = static_cast<int>(min(static_cast<uint32_t>(kWave), upto - q_first));
         uint64_t found[2] = { 0, 0 };
-        for (uint32_t q0 = q_first; q0 < q_end; q0 += kWave) {
-            const uint32_t mine = min(q0 + lane, q_end - 1);
-            const float4 their_box = a.box[mine];
-            const int their_class = static_cast<int>(a.cls[mine]);
-            const int here = static_cast<int>(min(static_cast<uint32_t>(kWave), q_end - q0));
-            for (int j = 0; j < here; ++j) {
-                const float4 other = make_float4(from_lane(their_box.x, j), from_lane(their_box.y, j),
-                                                 from_lane(their_box.z, j), from_lane(their_box.w, j));
-                const bool same = static_cast<uint32_t>(__builtin_amdgcn_readlane(their_class, j)) == cls;
-                if (q0 + j < p && live) {
-                    same_before += same ? 1u : 0u;
-                    if (overlaps_above(box, other, same ? a.threshold : kDuplicateOverlap)) {
-                        const uint64_t bit = 1ull << ((q0 - q_first + j) >> grain);
-                        if (same) found[1] |= bit;
-                        else found[0] |= bit;
-                    }
-                }
+        for (int j = 0; j < here; ++j) {
+            const float4 other = make_float4(from_lane(their_box.x, j), from_lane(their_box.y, j),
+                                             from_lane(their_box.z, j), from_lane(their_box.w, j));
+            const bool same = static_cast<uint32_t>(__builtin_amdgcn_readlane(their_class, j)) == cls;
+            if (q_first + j < p && live && overlaps_above(box, other, same ? a.threshold : kDuplicateOverlap)) {
+                if (same) found[1] |= 1ull << j;
+                else found[0] |= 1ull << j;
             }
         }
 #pragma unroll
@@ -853,13 +855,11 @@ __global__ __launch_bounds__(kWide) void nms_conflicts_kernel(ImageArgs a)
             }
         }
     }
-    if (same_before) atomicAdd(&index[lane], same_before);
     __syncthreads();
     if (wave != 0 || !live) return;
     for (int pass = 0; pass < 2; ++pass) a.beyond[pass][p] = beyond[pass][lane];
     const uint32_t most = a.mask_slots;
     a.slots[p] = min(slots[0][lane], most) | min(slots[1][lane], most) << 8;
-    a.group_index[p] = index[lane];
 }
 
 __device__ __forceinline__ uint64_t load_bits(const uint64_t* set, uint32_t word)
@@ -873,25 +873,20 @@ __device__ __forceinline__ void set_bit(uint64_t* set, uint32_t at)
 }
 
 // What the records of lower rank say about place p (places are relative to the image here): 1 = a kept
-// one conflicts, 2 = none does but one that may is undecided, 0 = neither.  Every place below `open` is
-// decided; `from`: places below it have been looked at before.
+// one conflicts, 2 = none does but one that may is undecided, 0 = neither.
 struct Standing {
     int pass;
-    uint32_t image_begin, p, from, open;
-    int grain;
+    uint32_t image_begin, p;
     const uint64_t* kept;
     const uint64_t* gone;
 };
 
-// The same for places [first, first + count) of one word of the bit sets, pair by pair.
-__device__ __forceinline__ int recheck(const ImageArgs& a, const Standing& s, uint32_t first, uint32_t count,
-                                       const float4& box, uint32_t cls)
+// The same for the places of one word of the bit sets, pair by pair.
+__device__ __forceinline__ int recheck(const ImageArgs& a, const Standing& s, uint32_t word, const float4& box, uint32_t cls)
 {
-    const uint32_t word = first >> 6;
     // `kept` is read first: a bit that is set in between shows up as undecided, never as absent
     const uint64_t kept = load_bits(s.kept, word);
-    uint64_t bits = first + 64 > s.open ? kept | ~load_bits(s.gone, word) : kept;
-    if (count < 64) bits &= ((1ull << count) - 1) << (first & 63);
+    uint64_t bits = kept | ~load_bits(s.gone, word);
     if (word == s.p >> 6) bits &= (1ull << (s.p & 63)) - 1;
     bool pending = false;
     for (; bits; bits &= bits - 1) {
@@ -914,99 +909,235 @@ __device__ __forceinline__ int conflict_state(const ImageArgs& a, const Standing
     bool pending = false;
     float4 box = make_float4(0, 0, 0, 0);
     uint32_t cls = 0;
-    if (beyond || s.grain) {
+    if (beyond) {
         box = a.box[place];
         cls = a.cls[place];
     }
     for (int slot = 0; slot < stored; ++slot) {
         const size_t at = static_cast<size_t>(slot) * a.capacity + place;
         const uint32_t word = a.ids[s.pass][at];
-        if (((word + 1) * 64) << s.grain <= s.from) continue;
         const uint64_t mask = a.masks[s.pass][at];
-        if (s.grain == 0) {
-            if (mask & load_bits(s.kept, word)) return 1;
-            pending = pending || (mask & ~load_bits(s.gone, word)) != 0;
-            continue;
-        }
-        for (uint64_t bits = mask; bits; bits &= bits - 1) {
-            const uint32_t first = (word * 64 + static_cast<uint32_t>(__builtin_ctzll(bits))) << s.grain;
-            const int state = recheck(a, s, first, 1u << s.grain, box, cls);
-            if (state == 1) return 1;
-            pending = pending || state == 2;
-        }
+        if (mask & load_bits(s.kept, word)) return 1;
+        pending = pending || (mask & ~load_bits(s.gone, word)) != 0;
     }
     for (; beyond; beyond &= beyond - 1) {          // words that were not stored: all of their places
-        const uint32_t first = (static_cast<uint32_t>(__builtin_ctzll(beyond)) * 64) << s.grain;
-        const uint32_t end = min(first + (64u << s.grain), s.p);
-        for (uint32_t q = max(first, s.from & ~63u); q < end; q += 64) {
-            const int state = recheck(a, s, q, 64, box, cls);
-            if (state == 1) return 1;
-            pending = pending || state == 2;
-        }
+        const int state = recheck(a, s, static_cast<uint32_t>(__builtin_ctzll(beyond)), box, cls);
+        if (state == 1) return 1;
+        pending = pending || state == 2;
     }
     return pending ? 2 : 0;
 }
 
-// One workgroup per image, a lane per place, 1024 places at a time in rank order, so that only conflicts
-// among those can be pending.  Rounds until each of them is decided: a round decides at least the
-// undecided place of lowest rank; the bound makes the exit unconditional.
+// ---- large images, block by block
+// A word that a block of 64 places leaves behind: 32 bits, and above them a tag that says they are there, so that they
+// arrive with the look that finds them.
+constexpr uint64_t kSettledTag = 1ull << 32;
+
+// The words of block `at`, one in each of the first lanes (the others hold a tag and nothing).
+__device__ __forceinline__ uint64_t look_at_block(const ImageArgs& a, uint32_t at, uint32_t lane)
+{
+    return lane < kSettledWords ? __hip_atomic_load(a.settled + at * kSettledStride + lane, __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_AGENT)
+                                : kSettledTag;
+}
+
+__device__ __forceinline__ bool block_is_there(uint64_t words) { return __ballot(words < kSettledTag) == 0; }
+
+__device__ __forceinline__ uint64_t two_words(uint64_t words, int first)
+{
+    const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(words), first);
+    const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(words), first + 1);
+    return (static_cast<uint64_t>(hi) << 32) | lo;
+}
+
+// The lanes of `open` that are kept: a lane whose `mask` (bits of lower lanes) meets a kept one is not.  A round decides
+// at least the lowest of them.
+__device__ __forceinline__ uint64_t settle_lanes(uint64_t kept, uint64_t open, uint64_t mask, uint32_t lane)
+{
+    while (open) {
+        const bool mine = (open >> lane) & 1;
+        const uint64_t keep = __ballot(mine && !(mask & (kept | open)));
+        const uint64_t drop = __ballot(mine && (mask & kept));
+        kept |= keep;
+        open &= ~(keep | drop);
+    }
+    return kept;
+}
+
+// A workgroup takes the next block of 64 places, a lane per place in each of its 16 waves, and goes over the blocks
+// before it in the image, the waves side by side: conflicts with the places of a settled block that were kept, or, with
+// one that is not settled yet, with all of its places while it is waited for.  Then the block's own places, and its
+// words for the blocks behind it.  What bounds it is the chain of decisions, one and a half to two microseconds from
+// block to block, and the ranking in front of it (30000 records of one image around 20 places: 1.2 ms, 11.1 on masks in
+// one workgroup, 7.4 on the sorting path; 60000: 2.9, 104 and 18.5).
+// An image's blocks are taken in order and a block waits only for blocks that were taken before it, whose workgroups
+// therefore run: the first that is not settled never waits, so every wait ends.  (The bound on the looks makes the exit
+// unconditional; it is seconds.)
+__device__ void settle_blocks(const ImageArgs& a, uint32_t worker)
+{
+    __shared__ uint64_t dropped[2];            // by earlier blocks, a bit per lane
+    __shared__ uint64_t inner[2][kWave];       // conflicts inside the block: bits of lower lanes
+    __shared__ uint32_t index[kWave];          // earlier records of the same class
+    __shared__ uint32_t large[kImageCapacity / kLargeImage];
+    __shared__ uint32_t scan_lds[kWide / kWave + 1];
+    __shared__ uint32_t taken, before;
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    const uint32_t wave = threadIdx.x / kWave;
+    constexpr uint32_t kWaves = kWide / kWave;
+    constexpr int kOwn = kWave / kWaves;       // of the block's own places, to a wave
+    const bool is_large = threadIdx.x < static_cast<uint32_t>(a.batch) &&
+                          a.image_begin[threadIdx.x + 1] - a.image_begin[threadIdx.x] > kLargeImage;
+    uint32_t images;
+    const uint32_t nth = wide_exclusive_scan(is_large ? 1u : 0u, scan_lds, images);
+    if (images == 0) return;
+    if (is_large) large[nth] = threadIdx.x;
+    uint32_t looks_left = 1u << 22;
+    for (uint32_t turn = 0; turn < images;) {
+        __syncthreads();
+        // the workgroups spread over the images, and move on to the next when one has no more blocks
+        const uint32_t image = large[(worker + turn) % images];
+        if (threadIdx.x == 0) taken = atomicAdd(a.ticket + image, 1u);
+        __syncthreads();
+        const uint32_t earlier = taken;
+        const uint32_t at = a.first_block[image] + earlier;
+        const uint32_t image_begin = a.image_begin[image], image_end = a.image_begin[image + 1];
+        const uint32_t block_begin = image_begin + earlier * kWave;
+        if (block_begin >= image_end) {
+            ++turn;
+            continue;
+        }
+        if (threadIdx.x < kWave) {
+            inner[0][lane] = inner[1][lane] = 0;
+            index[lane] = 0;
+        }
+        if (threadIdx.x < 2) dropped[threadIdx.x] = 0;
+        if (threadIdx.x == 0) before = 0;
+        __syncthreads();
+        const bool live = block_begin + lane < image_end;
+        const uint32_t p = live ? block_begin + lane : block_begin;
+        const float4 box = a.box[p];
+        const uint32_t cls = a.cls[p];
+        // the block's own pairs, and how far down its group each place is: nothing suppresses one past those that are visited
+        uint32_t same_before = 0;
+        for (uint32_t i = wave; i < earlier; i += kWaves) {
+            const int their_class = static_cast<int>(a.cls[image_begin + i * kWave + lane]);
+#pragma unroll 16
+            for (int j = 0; j < static_cast<int>(kWave); ++j)
+                same_before += static_cast<uint32_t>(__builtin_amdgcn_readlane(their_class, j)) == cls ? 1u : 0u;
+        }
+#pragma unroll
+        for (int u = 0; u < kOwn; ++u) {
+            const int j = static_cast<int>(wave) * kOwn + u;
+            const bool same = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(cls), j)) == cls;
+            const float4 other = make_float4(from_lane(box.x, j), from_lane(box.y, j), from_lane(box.z, j), from_lane(box.w, j));
+            same_before += same && static_cast<uint32_t>(j) < lane ? 1u : 0u;
+            if (static_cast<uint32_t>(j) < lane && overlaps_above(box, other, same ? a.threshold : kDuplicateOverlap))
+                atomicOr(reinterpret_cast<unsigned long long*>(&inner[same ? 1 : 0][lane]), 1ull << j);
+        }
+        if (same_before) atomicAdd(&index[lane], same_before);
+        __syncthreads();
+        const bool visited = index[lane] < static_cast<uint32_t>(kGroupVisit);
+        bool drop0 = false, drop1 = false;
+        for (uint32_t i = wave; i < earlier; i += kWaves) {
+            const uint32_t q = image_begin + i * kWave + lane;
+            const float4 their_box = a.box[q];
+            const int their_class = static_cast<int>(a.cls[q]);
+            uint64_t words = look_at_block(a, at - earlier + i, lane);
+            const bool there = block_is_there(words);
+            const uint64_t in_first = there ? two_words(words, 0) : ~0ull, in_second = there ? two_words(words, 2) : ~0ull;
+            uint64_t found[2] = { 0, 0 };
+            for (uint64_t bits = in_first; bits; bits &= bits - 1) {
+                const int j = __builtin_ctzll(bits);
+                const bool same = static_cast<uint32_t>(__builtin_amdgcn_readlane(their_class, j)) == cls;
+                const bool suppresses = (in_second >> j) & 1;
+                if (!__ballot(!same || (suppresses && visited))) continue;
+                const float4 other = make_float4(from_lane(their_box.x, j), from_lane(their_box.y, j),
+                                                 from_lane(their_box.z, j), from_lane(their_box.w, j));
+                if (overlaps_above(box, other, same ? a.threshold : kDuplicateOverlap)) {
+                    if (same) found[1] |= 1ull << j;
+                    else found[0] |= 1ull << j;
+                }
+            }
+            for (; !block_is_there(words) && looks_left; --looks_left) {
+                __builtin_amdgcn_s_sleep(1);
+                words = look_at_block(a, at - earlier + i, lane);
+            }
+            drop0 = drop0 || (found[0] & two_words(words, 0));
+            drop1 = drop1 || (found[1] & two_words(words, 2));
+            const uint32_t survivors = __builtin_amdgcn_readlane(static_cast<uint32_t>(words), 4);
+            if (i + 1 == earlier && lane == 0) before = survivors;
+        }
+        const uint64_t all0 = __ballot(drop0), all1 = __ballot(drop1);
+        if (lane == 0) {
+            if (all0) atomicOr(reinterpret_cast<unsigned long long*>(&dropped[0]), all0);
+            if (all1) atomicOr(reinterpret_cast<unsigned long long*>(&dropped[1]), all1);
+        }
+        __syncthreads();
+        if (wave != 0) continue;
+        const uint64_t first = settle_lanes(0, __ballot(live) & ~dropped[0], inner[0][lane], lane);
+        // the second pass knows only what the first kept; places past the first 1024 of a group are never visited and stay
+        const uint64_t reached = __ballot(visited);
+        const uint64_t second = settle_lanes(first & ~reached, first & reached & ~dropped[1], inner[1][lane], lane);
+        const uint32_t upto = before + static_cast<uint32_t>(__popcll(second));
+        if (lane < kSettledWords) {
+            const uint64_t bits = lane < 2 ? first : second & reached;
+            const uint32_t word = lane == 4 ? upto : static_cast<uint32_t>(bits >> (32 * (lane & 1)));
+            __hip_atomic_store(a.settled + at * kSettledStride + lane, kSettledTag | word, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if ((second >> lane) & 1) {
+            const uint32_t to = image_begin + before + __popcll(second & ((1ull << lane) - 1));
+            a.kept_key[to] = a.key[p];
+            a.kept_source[to] = a.source[p];
+        }
+        if (block_begin + kWave >= image_end && lane == 0) a.kept_images[image] = upto;
+    }
+}
+
+// One workgroup per image, a lane per place; those behind them settle the large images.  Rounds until each place is
+// decided: a round decides at least the undecided place of lowest rank; the bound makes the exit unconditional.
 __global__ __launch_bounds__(kWide) void nms_settle_kernel(ImageArgs a)
 {
-    __shared__ uint64_t kept[kBitSetWords], gone[kBitSetWords];
-    __shared__ uint32_t word_first[kBitSetWords];
+    __shared__ uint64_t kept[kMaskWords], gone[kMaskWords];
     __shared__ uint32_t scan_lds[kWide / kWave + 1];
-    static_assert(kBitSetWords == kWide, "one word of a bit set per lane");
     const uint32_t t = threadIdx.x;
     if (live_count(a.count, a.capacity) == 0) return;
+    if (blockIdx.x >= static_cast<uint32_t>(a.batch)) {
+        settle_blocks(a, blockIdx.x - static_cast<uint32_t>(a.batch));
+        return;
+    }
     const uint32_t begin = a.image_begin[blockIdx.x];
     const uint32_t places = a.image_begin[blockIdx.x + 1] - begin;
-    gone[t] = 0;
+    if (places > kLargeImage) return;
+    if (t < kMaskWords) gone[t] = 0;
     Standing s{};
     s.image_begin = begin;
-    s.grain = mask_grain(places);
+    s.p = t;
     s.kept = kept;
     s.gone = gone;
     for (s.pass = 0; s.pass < 2; ++s.pass) {
         // the second pass starts from what the first dropped: absent there
-        kept[t] = 0;
+        if (t < kMaskWords) kept[t] = 0;
         __syncthreads();
-        for (s.open = 0; s.open < places; s.open += kWide) {
-            s.p = s.open + t;
-            s.from = 0;
-            bool undecided = s.p < places;
-            if (undecided && s.pass == 1) {
-                if ((load_bits(gone, s.p >> 6) >> (s.p & 63)) & 1) {
-                    undecided = false;
-                } else if (a.group_index[begin + s.p] >= static_cast<uint32_t>(kGroupVisit)) {
-                    // places past the first 1024 of a group are never visited: they stay
-                    set_bit(kept, s.p);
+        bool undecided = t < places;
+        if (undecided && s.pass == 1) undecided = !((load_bits(gone, t >> 6) >> (t & 63)) & 1);
+        for (uint32_t round = 0; round <= kWide; ++round) {
+            if (undecided) {
+                const int state = conflict_state(a, s);
+                if (state != 2) {
+                    set_bit(state == 1 ? gone : kept, t);
                     undecided = false;
                 }
             }
-            for (uint32_t round = 0; round <= kWide; ++round) {
-                if (undecided) {
-                    const int state = conflict_state(a, s);
-                    if (state != 2) {
-                        set_bit(state == 1 ? gone : kept, s.p);
-                        undecided = false;
-                    }
-                    s.from = s.open;
-                }
-                if (__syncthreads_or(undecided) == 0) break;
-            }
+            if (__syncthreads_or(undecided) == 0) break;
         }
-        __syncthreads();
     }
-    const uint64_t mine = kept[t];
+    const bool survives = t < places && ((kept[t >> 6] >> (t & 63)) & 1);
     uint32_t total;
-    word_first[t] = wide_exclusive_scan(static_cast<uint32_t>(__popcll(mine)), scan_lds, total);
-    __syncthreads();
-    for (uint32_t p = t; p < places; p += kWide) {
-        const uint64_t word = kept[p >> 6];
-        if (!((word >> (p & 63)) & 1)) continue;
-        const uint32_t at = begin + word_first[p >> 6] + __popcll(word & ((1ull << (p & 63)) - 1));
-        a.kept_key[at] = a.key[begin + p];
-        a.kept_source[at] = a.source[begin + p];
+    const uint32_t nth = wide_exclusive_scan(survives ? 1u : 0u, scan_lds, total);
+    if (survives) {
+        a.kept_key[begin + nth] = a.key[begin + t];
+        a.kept_source[begin + nth] = a.source[begin + t];
     }
     if (t == 0) a.kept_images[blockIdx.x] = total;
 }
@@ -1101,15 +1232,14 @@ Workspace carve(void* base, int capacity)
     return w;
 }
 
-// Which lists go by image.  Measured on both paths, us sorted -> by image: 600 records of 64 images 161 -> 34,
-// 7000 of 16 336 -> 78, 60000 of 32 1172 -> 388, 8000 of one image 1447 -> 674.  One workgroup settles an
-// image, so a list that may all lie in one and is longer than that stays with the sweeps of the sorting
-// path, which spread over the chip (30000 records of one image around 20 places: 8.0 ms, by image 16.9).
-// More than 2048 places per image of the batch make such a list possible by their number; fewer still allow
-// it, at that price, where nearly all records are of one image.
-bool by_image(int capacity, int batch)
+// Which lists go by image: those whose images have a lane each and whose masks and blocks fit the library's first
+// workspace.  Measured on both paths, us sorted -> by image: 600 records of 64 images 161 -> 33, 7000 of 16 400 -> 76,
+// 60000 of 32 1220 -> 308, of 4 4900 -> 990, of 1 18500 -> 2900; 600 of one image in a list for 65536 163 -> 69, 4000
+// 930 -> 205.  One class has no pairs for the duplicate pass, and 1024 places that are visited: a long list of it stays
+// with the sorting path where the batch is too small to spread it (30000 of one image 1800 -> 786, but 60000 2060 -> 2290).
+bool by_image(int capacity, int batch, int classes)
 {
-    return batch <= kImageBatch && capacity <= kImageCapacity && (capacity <= 8192 || capacity / 2048 <= batch);
+    return batch <= kImageBatch && capacity <= kImageCapacity && (classes > 1 || capacity <= 32768 || capacity / 2048 <= batch);
 }
 
 // The same for the launches by image; `args` gets every pointer.  `mask_words`: of one pass's masks.
@@ -1135,13 +1265,15 @@ size_t carve_images(void* base, int capacity, int batch, size_t mask_words, Imag
     take(args.source, cap);
     take(args.box, cap);
     take(args.cls, cap);
-    take(args.group_index, cap);
     take(args.slots, cap);
     for (int k = 0; k < 2; ++k) {
         take(args.ids[k], mask_words);
         take(args.beyond[k], cap);
         take(args.masks[k], mask_words);
     }
+    take(args.first_block, images);
+    take(args.ticket, images);
+    take(args.settled, (cap / 64 + images + 1) * kSettledStride);
     take(args.kept_key, cap);
     take(args.kept_source, cap);
     take(args.kept_images, images);
@@ -1201,7 +1333,7 @@ int pxh_nms(const pxh_detection* records, const int* count, int capacity, int ba
         return check_launch("pxh_nms");
     }
     void* ws;
-    if (by_image(capacity, batch)) {
+    if (by_image(capacity, batch, classes)) {
         ImageArgs a{};
         int rc = resolve_workspace(workspace, workspace_bytes, carve_images(nullptr, capacity, batch, a), &ws,
                                    as_stream(stream));
@@ -1218,7 +1350,8 @@ int pxh_nms(const pxh_detection* records, const int* count, int capacity, int ba
         hipLaunchKernelGGL(nms_group_images_kernel, per_tile, wide, 0, s, a);
         hipLaunchKernelGGL(nms_place_kernel, per_block, wide, 0, s, a);
         hipLaunchKernelGGL(nms_conflicts_kernel, per_block, wide, 0, s, a);
-        hipLaunchKernelGGL(nms_settle_kernel, dim3(batch), wide, 0, s, a);
+        const unsigned helpers = static_cast<uint32_t>(capacity) > kLargeImage ? kSettleWorkgroups : 0;
+        hipLaunchKernelGGL(nms_settle_kernel, dim3(batch + helpers), wide, 0, s, a);
         hipLaunchKernelGGL(nms_merge_images_kernel, per_block, wide, 0, s, a, kept, kept_count);
         return check_launch("pxh_nms");
     }

@@ -187,9 +187,10 @@ def test_detections_of_two_heads_then_nms(ops, oracle):
 
 @pytest.mark.parametrize("n,used,batch,capacity", [
     (513, 1, 1, 513), (1024, 16, 16, 1024), (1025, 1024, 1024, 1025),      # edges of the tiles, most images
-    (4096, 1, 1, 4097), (4097, 1, 1, 4097), (8192, 1, 1, 8192),            # one and two places per mask bit
-    (9000, 1, 16, 32768), (9000, 1, 32, 65536),                            # four, few mask words stored
-    (1025, 1025, 1025, 1025), (8193, 1, 1, 8193), (700, 3, 31, 65536), (6000, 2, 33, 65537),   # the sorting path
+    (1024, 1, 1, 2000), (1025, 1, 1, 1025), (8192, 1, 1, 8192), (8193, 1, 1, 8193),   # on masks, block by block
+    (9000, 1, 16, 32768), (15000, 16, 16, 65536), (1000, 1, 4, 65536), (700, 3, 31, 65536),    # few mask words stored
+    (9000, 1, 32, 65536), (9000, 1, 31, 65536),                            # one class: by image, sorted
+    (1025, 1025, 1025, 1025), (6000, 2, 33, 65537),                        # more images, a longer list: sorted
 ], ids=lambda v: str(v))
 @pytest.mark.parametrize("classes,clusters,thr", [(1, 40, 0.5), (7, 3, 0.3)])
 def test_nms_by_image_and_by_sorting(ops, oracle, n, used, batch, capacity, classes, clusters, thr):
@@ -200,6 +201,33 @@ def test_nms_by_image_and_by_sorting(ops, oracle, n, used, batch, capacity, clas
     rec["prob"][::7] = rec["prob"][0]                             # ties keep the order
     want = oracle.nms(rec[np.argsort(rec["order"])], thr)
     same(run(ops, rec, batch, classes, thr, capacity), want, "%d of %d images" % (n, used))
+
+
+@pytest.mark.parametrize("sizes,classes,thr", [
+    ([20000, 1024, 1, 1025, 700, 0, 5000], 40, 0.45),       # large images among others, and an empty one
+    ([30000], 2, 0.4), ([12000, 12000], 12000, 0.0)], ids=str)
+def test_nms_large_images(ops, oracle, sizes, classes, thr):
+    """Images settled block by block, twice in a row: what a call leaves in the workspace is nothing to the next."""
+    parts = []
+    for b, n in enumerate(sizes):
+        part = random_detections(oracle, 900 + b, n, 1, classes, 5) if n else random_detections(oracle, 900, 1, 1, 1, 1)[:0]
+        part["batch"] = b
+        parts.append(part)
+    rec = np.concatenate(parts)
+    rec["order"] = np.random.Generator(np.random.Philox(key=len(rec))).permutation(len(rec))
+    want = oracle.nms(rec[np.argsort(rec["order"])], thr)
+    for _ in range(2):
+        same(run(ops, rec, len(sizes), classes, thr, 40000), want, str(sizes))
+    # chains across the edges of the blocks: every decision hangs on the one before it
+    long = 9000
+    rows = np.zeros(long, oracle.DETECTION_DTYPE)
+    rows["w"], rows["h"] = 100.0, 100.0
+    rows["prob"] = 1.0 - 1e-4 * np.arange(long)
+    rows["order"] = np.arange(long)
+    for step, cut, groups in ((4.0, 0.95, 2), (30.0, 0.5, 9)):
+        rows["x"] = step * np.arange(long)
+        rows["class_index"] = np.arange(long) % 2 if groups == 2 else np.arange(long) * groups // long
+        same(run(ops, rows, 1, 12, cut, 9000), oracle.nms(rows, cut), "chain of %g" % step)
 
 
 @pytest.mark.parametrize("capacity,batch", [(70000, 5), (2000, 1025)])
