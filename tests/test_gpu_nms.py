@@ -28,8 +28,9 @@ def same(got, want, what):
     assert got.tobytes() == want.tobytes(), what
 
 
-# A capacity of at most 512 takes the one-workgroup kernel, a larger one the sorting path.
-PATHS = pytest.mark.parametrize("capacity", [None, 3000], ids=["one-workgroup", "sorted"])
+# A capacity of at most 512 takes the one-workgroup kernel, one of at most 65536 goes image by image, a larger one takes
+# the sorting path.
+PATHS = pytest.mark.parametrize("capacity", [None, 3000, 70000], ids=["one-workgroup", "by-image", "sorted"])
 
 
 @PATHS
@@ -73,10 +74,11 @@ def test_nms_hand_worked_scenarios(ops, oracle, capacity):
         same(got, oracle.nms(rec, thr), name)
 
 
-def test_nms_empty_and_capacity(ops, oracle):
+@pytest.mark.parametrize("room", [5000, 70000], ids=["by-image", "sorted"])
+def test_nms_empty_and_capacity(ops, oracle, room):
     import torch
-    got = run(ops, _records(oracle, []), 1, 1, 0.5, capacity=16)
-    assert len(got) == 0
+    for capacity in (16, room):
+        assert len(run(ops, _records(oracle, []), 1, 1, 0.5, capacity)) == 0
     # a counter above the capacity (a detection pass that overflowed) means "capacity records"
     rec = random_detections(oracle, 11, 300, 2, 3, 2)
     records, count = ops.records_to_device(rec, 300)
@@ -84,9 +86,9 @@ def test_nms_empty_and_capacity(ops, oracle):
     kept, kept_count = ops.nms(records, count, 2, 3, 0.45)
     same(ops.nms_to_host(kept, kept_count), oracle.nms(rec, 0.45), "overflowed counter")
     # capacity far above the live count, a caller-owned workspace, a negative counter
-    need = ops.capi.load().pxh_nms_workspace_bytes(5000)
+    need = ops.capi.load().pxh_nms_workspace_bytes(room)
     ws = torch.empty(need, dtype=torch.uint8, device="cuda")
-    records, count = ops.records_to_device(rec, 5000)
+    records, count = ops.records_to_device(rec, room)
     kept, kept_count = ops.nms(records, count, 2, 3, 0.45, workspace=ws)
     same(ops.nms_to_host(kept, kept_count), oracle.nms(rec, 0.45), "capacity above count")
     count.fill_(-5)
@@ -121,11 +123,11 @@ def chain(oracle, length, ratio, classes):
     return _records(oracle, rows)
 
 
-@PATHS
-@pytest.mark.parametrize("sweeps", [1, 3])
+# (the sweeps are the sorting path's)
+@pytest.mark.parametrize("capacity,sweeps", [(None, 6), (3000, 6), (70000, 1), (70000, 3), (70000, 6)])
 def test_nms_long_dependency_chains(ops, oracle, sweeps, capacity):
     """Chains as long as the list: alternating classes exercise the duplicate step's repeated sweeps
-    and its per-image loop, one class the greedy step's loop."""
+    and its per-image loop (or the rounds in which an image is settled), one class the greedy step's loop."""
     lib = ops.capi.load()
     before = lib.pxh_debug_nms_sweeps(sweeps)
     try:
