@@ -608,7 +608,6 @@ bool launch_fwd_tile(const float* in, float* out, int* indexes, uint32_t planes,
                            FastDiv(t.strips), FastDiv(g.iw), FastDiv(g.ih), FastDiv(g.ow), FastDiv(g.oh),      \
                            static_cast<uint32_t>(cells), static_cast<uint32_t>(segments))
         switch (g.kernel) {
-        case 2: PXH_POOL_TILE(2); break;
         case 3: PXH_POOL_TILE(3); break;
         case 5: PXH_POOL_TILE(5); break;
         case 9: PXH_POOL_TILE(9); break;

@@ -85,9 +85,10 @@ def test_maxpool_special_values(ops, oracle):
 
 
 # whole planes in one tile and one more, more planes per tile than are left, strips with a remainder, masks
-# of 1 to 8 words, windows wider than the plane; the last three are beyond one or both tiled kernels
+# of 1 to 8 words, windows wider than the plane; the last three are beyond one or both tiled kernels (as are windows
+# of 2, and of 3 at stride 2, forward: theirs is the tiled backward alone)
 @pytest.mark.parametrize("shape,k,s,p", [
-    ((1, 1, 32, 64), 2, 1, 1), ((1, 2, 33, 64), 2, 1, 1), ((3, 1031, 5, 7), 3, 1, 2), ((5, 1024, 3, 3), 3, 2, 2),
+    ((1, 1, 32, 64), 2, 1, 1), ((1, 2, 33, 64), 2, 1, 1), ((1, 1, 32, 64), 3, 1, 2), ((1, 2, 33, 64), 3, 1, 2), ((3, 1031, 5, 7), 3, 1, 2), ((5, 1024, 3, 3), 3, 2, 2),
     ((1, 2, 101, 67), 3, 1, 2), ((1, 2, 101, 67), 3, 2, 2), ((2, 2, 151, 75), 2, 2, 1), ((1, 3, 19, 19), 5, 1, 4),
     ((1, 2, 38, 38), 9, 1, 8), ((1, 2, 38, 38), 13, 1, 12), ((1, 2, 47, 53), 13, 1, 12), ((1, 2, 9, 6), 13, 1, 12),
     ((1, 2, 40, 37), 16, 1, 15), ((1, 2, 21, 20), 6, 4, 5), ((1, 1, 3, 1200), 3, 1, 2), ((1, 1, 4, 12000), 3, 1, 2),
