@@ -1812,8 +1812,10 @@ struct Residual {
     float alpha = 1.0f, beta = 1.0f;
 };
 
-// BN training forward + activation.  `get_workspace(need, &ws)` is asked for the `need` bytes of the
-// three-launch form only when the shape does not take the one-launch form, which uses none.
+// BN training forward + activation.  `get_workspace(need, &ws)` is asked for the `need` bytes of the three-launch form
+// where the shape takes that, and where it takes a scalar one-launch form of more than kResidentVectors values per lane:
+// those use none of it, but their limits are measured ones that may move, also between activations, and a workspace that
+// is too small for a shape is refused on either side of them (as is growth in a capture).
 template<typename GetWorkspace>
 int bn_train_forward(const char* who, const float* x, float* y, float* pre_activation, float* x_saved, float* x_norm,
                      float* mean, float* var, float* rolling_mean, float* rolling_var, const float* scale,
@@ -1835,7 +1837,7 @@ int bn_train_forward(const char* who, const float* x, float* y, float* pre_activ
             const ResidentFwdArgs r{ x, y, pre_activation, x_saved, x_norm, mean, var, rolling_mean, rolling_var,
                                      scale, bias, resident_geom(batch, channels, spatial), res.from, res.alpha, res.beta };
             if (!vec && per_thread > kResidentVectors) {
-                // the workspace that the three launches need is still the caller's part of this shape
+                // not used, but still the caller's part of this shape (see above)
                 void* unused;
                 rc = get_workspace(workspace_bytes(batch, channels, spatial), &unused);
                 if (rc) return rc;
@@ -2142,7 +2144,7 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
     }
     if (per_thread) {
         if (!cs.on && !rvec && per_thread > kResidentVectors) {
-            // the workspace that the three launches need is still the caller's part of this shape
+            // not used, but still the caller's part of this shape (as in the forward)
             rc = resolve_workspace(workspace, workspace_bytes_given, workspace_bytes(batch, channels, spatial), &ws, s);
             if (rc) return rc;
         }

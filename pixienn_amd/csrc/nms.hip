@@ -611,7 +611,7 @@ __global__ __launch_bounds__(kWide) void nms_small_kernel(const pxh_detection* r
 // Every decision of nms is taken inside one image, so the records are grouped by image first and
 // nothing is sorted: six launches in place of the sorting path's forty-five, whose cost at the few
 // thousand records of a validation batch is the launches and the latency of short dependent steps
-// (7126 records of 16 images in a list for 32768: 440 us in kernels, here 76).
+// (7126 records of 16 images in a list for 32768: 440 us in kernels, here 73).
 //   1. images are counted per tile of 1024 records, 2. the records' keys are laid out image by image,
 //      in any order inside one;
 //   3. a record's place in its image is the number of smaller keys there, counted directly: n^2 of the
