@@ -659,15 +659,21 @@ def nms_to_host(kept, kept_count):
     # host waits once: asking for the count first is a second round trip (25 us) before the records' own.
     # A copy goes to the current stream of its tensor's device, which need not be the current device: those are
     # the streams to wait for, and launches of another device that the records may come from end before them.
-    if kept.device.index != _current_device():
+    here = _current_device()
+    elsewhere = kept.device.index != here or kept_count.device.index != here
+    if elsewhere:
         torch.cuda.current_stream().synchronize()
     first = min(kept.shape[0], _FIRST_COPY)
     count = torch.empty(1, dtype=torch.int32, pin_memory=True)
     records = torch.empty((first, *kept.shape[1:]), dtype=kept.dtype, pin_memory=True)
     count.copy_(kept_count, non_blocking=True)
     records.copy_(kept[:first], non_blocking=True)
-    for device in {t.device for t in (kept, kept_count) if t.is_cuda}:
-        torch.cuda.current_stream(device).synchronize()
+    if elsewhere:
+        for t in (kept, kept_count):
+            if t.is_cuda:
+                torch.cuda.current_stream(t.device).synchronize()
+    else:
+        torch.cuda.current_stream().synchronize()
     n = int(count[0])
     if n <= first:
         rows = records[:n].numpy().copy()
