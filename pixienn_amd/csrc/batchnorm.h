@@ -191,24 +191,39 @@ struct FinishedChannel {
     float bias_add, scale_add, mean_delta, var_delta;
 };
 
+// What the finish takes from the variance alone.
+struct VarianceTerms {
+    double denom, mean_factor, rroot;
+    float power;
+};
+
+__device__ __forceinline__ VarianceTerms variance_terms(float v)
+{
+    const float ve = v + kEps;
+    VarianceTerms t;
+    t.denom = sqrt(static_cast<double>(v)) + static_cast<double>(kEps);
+    t.mean_factor = -1. / static_cast<double>(sqrtf(ve));
+    t.rroot = 1.0 / sqrt(static_cast<double>(ve));
+    t.power = -.5f * powf(ve, -3.0f / 2.0f);
+    return t;
+}
+
 template<bool BN>
-__device__ __forceinline__ FinishedChannel finished_channel(double sa, double sb, int count, const FoldCoef& f, float v,
-                                                            float s)
+__device__ __forceinline__ FinishedChannel finished_channel(double sa, double sb, int count, const FoldCoef& f,
+                                                            const VarianceTerms& t, float s)
 {
     FinishedChannel r{};
     r.bias_add = static_cast<float>(sa);
     if constexpr (BN) {
         // sum d' * x_hat with x_hat = (x - mean) / (sqrt(var) + eps)
-        const double denom = sqrt(static_cast<double>(v)) + static_cast<double>(kEps);
-        r.scale_add = static_cast<float>(sb / denom);
+        r.scale_add = static_cast<float>(sb / t.denom);
         // sums of d'' = d' * scale
         const float sum_dd = static_cast<float>(sa * static_cast<double>(s));
         const float sum_ddx = static_cast<float>(sb * static_cast<double>(s));
-        const float ve = v + kEps;
-        r.mean_delta = static_cast<float>(static_cast<double>(sum_dd) * (-1. / static_cast<double>(sqrtf(ve))));
-        r.var_delta = sum_ddx * (-.5f * powf(ve, -3.0f / 2.0f));
+        r.mean_delta = static_cast<float>(static_cast<double>(sum_dd) * t.mean_factor);
+        r.var_delta = sum_ddx * t.power;
         r.k.f = f;
-        r.k.rroot = 1.0 / sqrt(static_cast<double>(ve));
+        r.k.rroot = t.rroot;
         r.k.c2 = static_cast<double>(r.var_delta) * 2. / static_cast<double>(count);
         r.k.md_term = static_cast<double>(r.mean_delta / static_cast<float>(count));
         r.k.pad = 0.0;

@@ -564,7 +564,7 @@ __device__ __forceinline__ DxCoef finish_backward(double sa, double sb, int c, i
         s = scale[c];
         f = make_coef(mean[c], v, s, bias[c]);
     }
-    const FinishedChannel r = finished_channel<BN>(sa, sb, count, f, v, s);
+    const FinishedChannel r = finished_channel<BN>(sa, sb, count, f, BN ? variance_terms(v) : VarianceTerms{}, s);
     bias_updates[c] = bias_updates_in + r.bias_add;
     if constexpr (BN) {
         scale_updates[c] = scale_updates_in + r.scale_add;
@@ -850,9 +850,10 @@ struct Residual {
 };
 
 // BN training forward + activation.  `get_workspace(need, &ws)` is asked for the `need` bytes of the three-launch form
-// where the shape takes that, and where it takes a scalar one-launch form of more than kResidentVectors values per lane:
-// those use none of it, but their limits are measured ones that may move, also between activations, and a workspace that
-// is too small for a shape is refused on either side of them (as is growth in a capture).
+// where the shape takes that, and where it takes a scalar one-launch form of more than kResidentVectors values per lane
+// or a small form below kResidentChannels: those use none of it, but their limits are measured ones that may move, also
+// between activations, and a workspace that is too small for a shape is refused on either side of them (as is growth in a
+// capture).
 template<typename GetWorkspace>
 int bn_train_forward(const char* who, const float* x, float* y, float* pre_activation, float* x_saved, float* x_norm,
                      float* mean, float* var, float* rolling_mean, float* rolling_var, const float* scale,
@@ -870,16 +871,17 @@ int bn_train_forward(const char* who, const float* x, float* y, float* pre_activ
         const bool vec = spatial % 4 == 0 && aligned16(x) && aligned16(y) && aligned16(pre_activation) &&
                          aligned16(x_saved) && aligned16(x_norm) && aligned16(res.from);
         const int per_thread = resident_vectors(batch, channels, spatial, vec, activation, false);
-        if (per_thread) {
+        const uint32_t small = small_slice(batch, channels, spatial, vec, activation, false);
+        if (per_thread || small) {
             const ResidentFwdArgs r{ x, y, pre_activation, x_saved, x_norm, mean, var, rolling_mean, rolling_var,
                                      scale, bias, resident_geom(batch, channels, spatial), res.from, res.alpha, res.beta };
-            if (!vec && per_thread > kResidentVectors) {
+            if (!per_thread || (!vec && per_thread > kResidentVectors)) {
                 // not used, but still the caller's part of this shape (see above)
                 void* unused;
                 rc = get_workspace(workspace_bytes(batch, channels, spatial), &unused);
                 if (rc) return rc;
             }
-            return launch_resident_forward(who, r, vec, per_thread, activation, s);
+            return launch_resident_forward(who, r, vec, per_thread, small, activation, s);
         }
     }
     void* ws;
@@ -1117,6 +1119,7 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
     hipStream_t s = as_stream(stream);
     const bool rvec = spatial % 4 == 0 && aligned16(delta) && aligned16(x) && aligned16(pre_activation);
     const int per_thread = resident_vectors(batch, channels, spatial, rvec, activation, true);
+    const uint32_t small = small_slice(batch, channels, spatial, rvec, activation, true);
     void* ws = nullptr;
     ClippedRegions region{};
     ClipArgs clip{};
@@ -1126,8 +1129,8 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
         region = clipped_regions(ws, batch, channels, spatial);
         clip = ClipArgs{ region.norm_partial, region.plan, cs.threshold, cs.clip, cs.norm_out };
     }
-    if (per_thread) {
-        if (!cs.on && !rvec && per_thread > kResidentVectors) {
+    if (per_thread || small) {
+        if (!cs.on && (!per_thread || (!rvec && per_thread > kResidentVectors))) {
             // not used, but still the caller's part of this shape (as in the forward)
             rc = resolve_workspace(workspace, workspace_bytes_given, workspace_bytes(batch, channels, spatial), &ws, s);
             if (rc) return rc;
@@ -1135,7 +1138,7 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
         const ResidentBwdArgs r{ BackwardArgs{ delta, x, pre_activation, mean, var, scale, bias }, scale_updates,
                                  bias_updates, mean_delta, var_delta, resident_geom(batch, channels, spatial),
                                  region.channel_norm, region.channel_sums, region.channel_done, clip };
-        return launch_resident_backward(who, r, cs.on, rvec, per_thread, activation, s);
+        return launch_resident_backward(who, r, cs.on, rvec, per_thread, small, activation, s);
     }
     if (!cs.on) {
         rc = resolve_workspace(workspace, workspace_bytes_given, workspace_bytes(batch, channels, spatial), &ws, s);

@@ -14,7 +14,7 @@ constexpr int kResidentThreads = 1024;
 // The scalar forms also come with workgroups of half the size, four to a compute unit instead of two:
 // for the layers with a thousand channels of 19 x 19, whose workgroups would otherwise run in two rounds.
 constexpr int kResidentNarrowThreads = 512;
-constexpr int kResidentVectors = 8;            // per lane of the small forms
+constexpr int kResidentVectors = 8;            // per lane of the forms without an LDS part
 
 // Sum of two doubles over the workgroup; every thread returns both totals.
 template<int T>
@@ -140,6 +140,11 @@ __device__ __forceinline__ void add_two(double& sum, float v, float w, bool pair
     }
 }
 
+// The small forms (small_slice below): a lane adds the values of a vector in fp32 and its vectors in doubles -- no further
+// from 64 bits than a lane of the other forms that holds one vector -- and the backward keeps x beside the delta.
+template<int V, int R, int L, int T>
+constexpr bool kSmallSlice = L == 0 && T < kResidentThreads && V * R <= (V == 4 ? 32 : 12);
+
 // A thread keeps R vectors in registers and L more in LDS (dynamic, L * kResidentThreads vectors:
 // thread-major, so every access is the conflict-free 128-bit one).
 template<int V, int R>
@@ -185,7 +190,7 @@ struct ResidentBwdArgs {
 // the channel slice must fit, and there must be enough channels to occupy the machine.  (Measured
 // with 24 vectors per thread: the registers spill and 128 workgroups of 16x128x76^2 are slower than
 // the three launches; with a third of them in LDS they do not.)
-// The small forms hold kResidentVectors (above);
+// The forms without an LDS part hold kResidentVectors (above);
 // the large form (128-bit vectors only) 16 vectors in registers + 8 in LDS (128 KB of the CU's 160)
 constexpr int kResidentLargeRegs = 16, kResidentLargeLds = 8;
 constexpr size_t kResidentLargeLdsBytes = static_cast<size_t>(kResidentLargeLds) * kResidentThreads * 16;
@@ -218,9 +223,66 @@ constexpr bool selects(int activation)
     return activation == PXH_LEAKY || activation == PXH_RELU || activation == PXH_LINEAR;
 }
 
+constexpr int kResidentChannels = 96;
+
+// The small forms.  A launch over short slices is one chain -- the loads, the sums across the workgroup, the thread that
+// finishes the channel, the stores -- and a workgroup of 1024 lanes that holds 50 vectors walks it at the pace of its
+// sixteen waves: seven of the eight steps of a lane are loads of nothing, and a thousand such workgroups run in two rounds.
+// Few lanes with two to eight steps each shorten every link; what the backward's finish takes from the variance alone is
+// formed while the slice is on its way (0.5 us of each backward).  Against workgroups of 1024 lanes (from 96 channels on)
+// or three launches, us, leaky: forward, forward + shortcut, backward, backward with rescale + clip
+//   2 x 1024 x 10^2    12.8 -> 4.1   12.4 -> 4.2   11.3 -> 4.9   20.0 ->  8.0     64 lanes, 2 vectors
+//   2 x 512 x 20^2      7.9 -> 4.0    7.7 -> 4.3    7.1 -> 4.7   13.0 ->  7.8    128 lanes, 2
+//   2 x 256 x 40^2      6.1 -> 4.5    6.4 -> 4.7    6.7 -> 5.4   11.2 ->  8.1    256 lanes, 4
+//   8 x 512 x 26^2      9.2 -> 6.6    9.6 -> 7.8   10.7 -> 9.0   16.4 -> 12.4    512 lanes, 4
+//   2 x 128 x 80^2      6.8 -> 6.0    7.7 -> 6.2    9.0 -> 8.0   13.4 -> 11.1    512 lanes, 8
+//   1 x 64 x 104^2      9.6 -> 5.5   10.8 -> 5.6   13.4 -> 7.3   19.1 -> 10.6    (three launches before)
+//   1 x 1024 x 13^2     8.4 -> 3.9   11.2 -> 4.0   11.9 -> 4.8   17.7 ->  8.3     64 lanes, 4 values
+//   4 x 1024 x 13^2     9.0 -> 5.3   11.8 -> 5.4   12.8 -> 6.1   17.5 ->  9.6    256 lanes, 4
+//   8 x 512 x 19^2      7.1 -> 6.0    8.3 -> 6.7   10.1 -> 7.9   14.8 -> 11.2    512 lanes, 8
+//   16 x 512 x 19^2     8.3 -> 7.7   10.5 -> 10.3  11.2 -> 10.6  16.3 -> 13.8    512 lanes, 12
+//   16 x 1024 x 19^2   14.1 -> 13.8  19.5 -> 19.6  19.1 -> 19.3  23.2 -> 23.3
+// With more lanes at the same capacity each is slower (2 x 1024 x 10^2 in 128, 256, 512 lanes: backward 4.7, 6.5, 10.0).
+// Eight vectors a lane take a workgroup's 256 registers a lane, one to a compute unit: up to as many channels only
+// (4 x 512 x 52^2, leaky: backward 16.5 us against 14.2).  An activation with an exponential is bound by its gradient, and
+// there the waves count: beyond 512 vectors a slice its backward keeps the full workgroups where it has them
+// (8 x 256 x 38^2, mish: 15.5 us against 13.4; 2 x 256 x 40^2: 8.5 against 8.0; 2 x 512 x 20^2: 6.4 against 7.8).
+constexpr uint32_t kSmallVectors = 4096, kSmallScalars = 6144;
+constexpr uint32_t kSmallVectorsMany = 2048;      // beyond kSmallChannels channels
+constexpr int kSmallChannels = 256;
+constexpr uint32_t kSmallVectorsSmooth = 512;
+
+// The vectors (or scalars) of a channel's slice where the shape takes a small form, else 0.
+inline uint32_t small_slice(int batch, int channels, int spatial, bool vec, int activation, bool backward)
+{
+    const size_t per_channel = static_cast<size_t>(batch) * spatial;
+    const size_t items = vec ? per_channel / 4 : per_channel;
+    size_t most = !vec ? kSmallScalars : channels <= kSmallChannels ? kSmallVectors : kSmallVectorsMany;
+    if (vec && backward && !selects(activation) && channels >= kResidentChannels) most = kSmallVectorsSmooth;
+    return items <= most ? static_cast<uint32_t>(items) : 0;
+}
+
+// Calls launch.operator()<V, R, T>() with the form for `items`: vectors or scalars, steps per lane, lanes.
+template<typename F>
+void dispatch_small_form(bool vec, uint32_t items, F&& launch)
+{
+    if (vec) {
+        if (items <= 64 * 2) return launch.template operator()<4, 2, 64>();
+        if (items <= 128 * 2) return launch.template operator()<4, 2, 128>();
+        if (items <= 256 * 4) return launch.template operator()<4, 4, 256>();
+        if (items <= 512 * 4) return launch.template operator()<4, 4, 512>();
+        return launch.template operator()<4, 8, 512>();
+    }
+    if (items <= 64 * 4) return launch.template operator()<1, 4, 64>();
+    if (items <= 256 * 4) return launch.template operator()<1, 4, 256>();
+    if (items <= 256 * 8) return launch.template operator()<1, 8, 256>();
+    if (items <= 512 * 8) return launch.template operator()<1, 8, 512>();
+    return launch.template operator()<1, 12, 512>();
+}
+
 inline int resident_vectors(int batch, int channels, int spatial, bool vec, int activation, bool backward)
 {
-    if (channels < 96) return 0;
+    if (channels < kResidentChannels) return 0;
     const size_t per_channel = static_cast<size_t>(batch) * spatial;
     const size_t vectors = (per_channel + (vec ? 3 : 0)) / (vec ? 4 : 1);
     const size_t per_thread = (vectors + kResidentThreads - 1) / kResidentThreads;
@@ -252,10 +314,10 @@ inline ResidentGeom resident_geom(int batch, int channels, int spatial)
 // A kernel that asks for more than 64 KB of dynamic LDS has to be allowed to, once.
 int allow_large_lds(const void* kernel);
 
-// `per_thread`: resident_vectors() of the shape.
-int launch_resident_forward(const char* who, const ResidentFwdArgs& r, bool vec, int per_thread, int activation,
-                            hipStream_t s);
+// `per_thread`: resident_vectors() of the shape, `small`: small_slice().
+int launch_resident_forward(const char* who, const ResidentFwdArgs& r, bool vec, int per_thread, uint32_t small,
+                            int activation, hipStream_t s);
 int launch_resident_backward(const char* who, const ResidentBwdArgs& r, bool clipped, bool vec, int per_thread,
-                             int activation, hipStream_t s);
+                             uint32_t small, int activation, hipStream_t s);
 
 }  // namespace pxh

@@ -80,11 +80,16 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
         early[1] = a.scale_updates[c];
         early[2] = a.b.var[c];
     }
+    // the small forms, whose time is one chain, also form what the finish takes from the variance while the slice is on
+    // its way (the first wave: it is the one that finishes the channel)
+    [[maybe_unused]] VarianceTerms terms{};
+    const auto early_terms = [&] { if (threadIdx.x < kWave) terms = variance_terms(early[2]); };
     const auto finish = [&](double sa, double sb) {
         const float bias_updates_in = kEarly ? early[0] : a.bias_updates[c];
         const float scale_updates_in = kEarly ? early[1] : a.scale_updates[c];
         const float var_in = kEarly ? early[2] : a.b.var[c];
-        const FinishedChannel r = finished_channel<true>(sa, sb, static_cast<int>(a.g.per_channel), k, var_in, k.scale);
+        const FinishedChannel r = finished_channel<true>(sa, sb, static_cast<int>(a.g.per_channel), k,
+                                                         kSmallSlice<V, R, L, T> ? terms : variance_terms(var_in), k.scale);
         a.bias_updates[c] = bias_updates_in + r.bias_add;
         a.scale_updates[c] = scale_updates_in + r.scale_add;
         if (a.mean_delta) a.mean_delta[c] = r.mean_delta;
@@ -93,9 +98,10 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
     };
     const bool recompute = a.b.pre == nullptr;
     Pack<V> d[R];
+    constexpr bool kSmall = kSmallSlice<V, R, L, T>;
     constexpr bool kWide = kWideSlice<V, R, L, T>;
-    std::conditional_t<kWide, double, float> fa = 0, fb = 0;
-    [[maybe_unused]] std::conditional_t<kWide, double, float> fq = 0;
+    std::conditional_t<kWide || kSmall, double, float> fa = 0, fb = 0;
+    [[maybe_unused]] std::conditional_t<kWide || kSmall, double, float> fq = 0;
     [[maybe_unused]] float peak = 0.0f;
     // Two shapes of the first pass.  Grouped: no branch around the loads (see the forward kernel), lanes
     // past the end read the first vector; kGroup steps at a time, their loads go out together, then each
@@ -106,7 +112,8 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
     // registers, where a group of two already spills (18.3 against 16.4 us at 16 x 256 x 38^2): it skips a step
     // past the end of the slice outright, as every form does in the second pass, which finds x in the cache.
     constexpr int kGroup = L > 0 ? 4 : 8;
-    constexpr bool kGrouped = L > 0 || V == 1;
+    constexpr bool kGrouped = !kSmall && (L > 0 || V == 1);
+    [[maybe_unused]] Pack<V> kept[kSmall ? R : 1];       // x, which the small forms hold on to
     static_assert(!kGrouped || (R % kGroup == 0 && L % kGroup == 0), "steps come in whole groups");
     // `lane` is the thread index; the second pass takes it through an empty asm statement, so that
     // its addresses are formed again there instead of being held in registers (48 of them) from the first
@@ -120,14 +127,59 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
     // rescale + clamp (kRedo), then the activation's gradient
     const auto prepared = [&](float t, float pre, bool valid) {
         if constexpr (MODE == kFirst) {
-            if constexpr (!kWide) fq += valid ? t * t : 0.0f;
+            if constexpr (!kWide && !kSmall) fq += valid ? t * t : 0.0f;
             peak = fmaxf(peak, valid ? fabsf(t) : 0.0f);
         }
         if constexpr (MODE == kRedo) t = rescaled_clipped(t, factor, limit);
         if constexpr (ACT != PXH_LINEAR) t = t * act_grad<ACT>(pre);
         return t;
     };
-    if constexpr (kGrouped) {
+    if constexpr (kSmall) {
+        // every load of the slice at once, no branch around them; the pre-activations four steps at a time
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const size_t where = place(r);
+            d[r] = ld<V, true>(a.b.delta, where);
+            kept[r] = ld<V, false>(a.b.x, where);
+        }
+        early_terms();
+        constexpr int kFour = R < 4 ? R : 4;
+        static_assert(R % kFour == 0, "steps come in whole groups");
+#pragma unroll
+        for (int first = 0; first < R; first += kFour) {
+            Pack<V> pv[kFour];
+            if constexpr (ACT != PXH_LINEAR) {
+                if (!recompute) {
+#pragma unroll
+                    for (int i = 0; i < kFour; ++i) pv[i] = ld<V, true>(a.b.pre, place(first + i));
+                } else {
+#pragma unroll
+                    for (int i = 0; i < kFour; ++i) {
+#pragma unroll
+                        for (int q = 0; q < V; ++q) pv[i].v[q] = affine(normalize(kept[first + i].v[q], k), k);
+                    }
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < kFour; ++i) {
+                const int r = first + i;
+                const bool valid = element(r) < a.g.per_channel;
+                float va = 0.0f, vb = 0.0f, vq = 0.0f;
+#pragma unroll
+                for (int q = 0; q < V; ++q) {
+                    const float raw = valid ? d[r].v[q] : 0.0f;
+                    const float t = valid ? prepared(raw, ACT != PXH_LINEAR ? pv[i].v[q] : 0.0f, valid) : 0.0f;
+                    d[r].v[q] = t;
+                    va += t;
+                    vb += valid ? t * (kept[r].v[q] - k.mean) : 0.0f;
+                    vq += raw * raw;
+                }
+                fa += static_cast<double>(va);
+                fb += static_cast<double>(vb);
+                if constexpr (MODE == kFirst) fq += static_cast<double>(vq);
+            }
+        }
+    } else if constexpr (kGrouped) {
         // delta * f'(pre) in dv, and the step's share of the sums
         const auto take = [&](int r, Pack<V>& dv, const Pack<V>& xv, const Pack<V>& pv) {
             const bool valid = element(r) < a.g.per_channel;
@@ -276,7 +328,9 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
             const uint32_t e = (r * T + lane) * V;
             if (e < a.g.per_channel) {
                 const size_t where = a.g.at(c, e);
-                const Pack<V> xv = ld<V, false>(a.b.x, where);
+                Pack<V> xv;
+                if constexpr (kSmall) xv = kept[r];
+                else xv = ld<V, false>(a.b.x, where);
                 const Pack<V> dv = r < R ? d[r < R ? r : 0] : *resident_lds_slot<V, R>(resident_lds, r);
                 Pack<V> out;
 #pragma unroll
@@ -286,13 +340,19 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
         }
     }
 }
-// One workgroup per channel.  (The forms without an LDS part are held to 64 registers, two workgroups
+
+// Waves per SIMD that the registers are held to.
+template<int V, int R, int L, int MODE, int T>
+constexpr int kBwdWaves = kSmallSlice<V, R, L, T> ? (MODE == kRedo || V * R >= 32 ? 2 : V * R >= 12 ? 4 : V * R == 8 ? 6 : 8)
+                          : L == 0 && MODE != kRedo && !(V == 1 && R > 16) ? 8 : 4;
+
+// One workgroup per channel.  (The forms of 1024 lanes without an LDS part are held to 64 registers, two workgroups
 // per compute unit: they run the 19 x 19 and 38 x 38 layers, whose launches are too short to fill the
 // machine with one.)  The workgroups of the kRedo launch form the plan from the per-channel figures of
 // the first launch and leave at once when nothing has to change; the forms without an LDS part run it
 // as a capped grid that walks the channels otherwise.
 template<int ACT, int V, int R, int L, int MODE = kPlain, int T = kResidentThreads>
-__global__ __launch_bounds__(T, L == 0 && MODE != kRedo && !(V == 1 && R > 16) ? 8 : 4) void bn_resident_bwd_kernel(ResidentBwdArgs a)
+__global__ __launch_bounds__(T, (kBwdWaves<V, R, L, MODE, T>)) void bn_resident_bwd_kernel(ResidentBwdArgs a)
 {
     static_assert(L == 0 || T == kResidentThreads, "the LDS part is laid out for the full workgroup");
     if constexpr (MODE == kRedo) {
@@ -323,15 +383,22 @@ __global__ __launch_bounds__(T, L == 0 && MODE != kRedo && !(V == 1 && R > 16) ?
 }  // namespace
 
 int launch_resident_backward(const char* who, const ResidentBwdArgs& r, bool clipped, bool vec, int per_thread,
-                             int activation, hipStream_t s)
+                             uint32_t small, int activation, hipStream_t s)
 {
     const bool narrow = resident_narrow(r.g, per_thread, vec, true);
     const dim3 block(narrow ? kResidentNarrowThreads : kResidentThreads);
     int large_lds_rc = PXH_OK;
     const auto launch = [&]<int ACT, int MODE>() {
         // the launch that follows the plan: one workgroup per compute unit at most, each walks channels
-        const bool walks = MODE == kRedo && !(vec && per_thread > kResidentVectors) && r.g.channels > kRedoWorkgroups;
+        const bool large = !small && vec && per_thread > kResidentVectors;
+        const bool walks = MODE == kRedo && !large && r.g.channels > kRedoWorkgroups;
         const dim3 grid(walks ? kRedoWorkgroups : r.g.channels);
+        if (small) {
+            dispatch_small_form(vec, small, [&]<int V, int R, int T>() {
+                hipLaunchKernelGGL((bn_resident_bwd_kernel<ACT, V, R, 0, MODE, T>), grid, dim3(T), 0, s, r);
+            });
+            return;
+        }
         if (narrow) {
             hipLaunchKernelGGL((bn_resident_bwd_kernel<ACT, 1, kResidentNarrowVectors, 0, MODE, kResidentNarrowThreads>),
                                grid, block, 0, s, r);

@@ -12,10 +12,15 @@ namespace {
 // 16 x 512 x 38^2 takes 32.9 us with four steps ahead against 31.0 us with none.)
 constexpr int kResidualAhead = 4;
 
+// Waves per SIMD that the registers are held to: a vector a step, two with a shortcut.
+template<int V, int R, int L, int T, bool RES, bool TIGHT>
+constexpr int kFwdWaves = kSmallSlice<V, R, L, T> ? (V * R >= 32 ? 2 : RES && V * R >= 12 ? 4 : 8)
+                          : L == 0 && V * R <= (V == 1 ? (RES && !TIGHT ? 8 : 16) : 32) ? 8 : 4;
+
 // V = 4 needs spatial % 4 == 0 and 16-byte aligned tensors.  R + L vectors per thread at most.
 // TIGHT: the scalar form with the shortcut's source on top in 64 registers, two workgroups per compute unit.
 template<int ACT, int V, int R, int L, int T = kResidentThreads, bool RES = false, bool TIGHT = false>
-__global__ __launch_bounds__(T, L == 0 && V * R <= (V == 1 ? (RES && !TIGHT ? 8 : 16) : 32) ? 8 : 4) void bn_resident_fwd_kernel(ResidentFwdArgs a)
+__global__ __launch_bounds__(T, (kFwdWaves<V, R, L, T, RES, TIGHT>)) void bn_resident_fwd_kernel(ResidentFwdArgs a)
 {
     static_assert(!TIGHT || (RES && V == 1 && L == 0), "a form of the riding shortcut");
     static_assert(L == 0 || T == kResidentThreads, "the LDS part is laid out for the full workgroup");
@@ -23,7 +28,8 @@ __global__ __launch_bounds__(T, L == 0 && V * R <= (V == 1 ? (RES && !TIGHT ? 8 
     // The 128-bit form with workgroups of half the size adds a channel up exactly as the full workgroups do,
     // so that a layer gives the same statistics to the bit with and without a shortcut riding on it: thread t
     // keeps the sums of the full form's threads t (even steps) and t + T (odd steps) apart.
-    constexpr bool kTwin = V == 4 && T < kResidentThreads;
+    constexpr bool kSmall = kSmallSlice<V, R, L, T>;
+    constexpr bool kTwin = V == 4 && T < kResidentThreads && !kSmall;
     static_assert(!kTwin || 2 * T == kResidentThreads, "half the size");
     __shared__ double slots[2][(kTwin ? 2 : 1) * T / kWave];
     __shared__ FoldCoef shared_coef;
@@ -83,7 +89,7 @@ __global__ __launch_bounds__(T, L == 0 && V * R <= (V == 1 ? (RES && !TIGHT ? 8 
     // slice's own loads, and arrive while the sums are formed -- all of them where a lane holds few values
     // (16 x 1024 x 19^2: 19.9 us against 25.6 us with every step's load behind the reduction).
     // (the half-size workgroups of the 128-bit form have 128 registers: eight of twelve steps, four of sixteen)
-    constexpr int kAhead = !RES ? 0 : V * (R + L) <= 8 ? R + L : L > 0 ? kResidualAhead
+    constexpr int kAhead = !RES ? 0 : kSmall || V * (R + L) <= 8 ? R + L : L > 0 ? kResidualAhead
                                 : T < kResidentThreads ? (R <= 12 ? 8 : 4) : V == 1 && R >= 16 ? (TIGHT ? 8 : 4) : 0;
     [[maybe_unused]] Pack<V> ahead[kAhead > 0 ? kAhead : 1];
     if constexpr (RES) {
@@ -94,7 +100,22 @@ __global__ __launch_bounds__(T, L == 0 && V * R <= (V == 1 ? (RES && !TIGHT ? 8 
         }
     }
     double t1, t2;
-    if constexpr (kWide) {
+    if constexpr (kSmall) {
+        t1 = t2 = 0.0;
+#pragma unroll
+        for (int r = R - 1; r >= 0; --r) {
+            const bool valid = element(r) < a.g.per_channel;
+            float p1 = 0.0f, p2 = 0.0f;
+#pragma unroll
+            for (int k = 0; k < V; ++k) {
+                const float d = valid ? v[r].v[k] - shift : 0.0f;
+                p1 += d;
+                p2 += d * d;
+            }
+            t1 += static_cast<double>(p1);
+            t2 += static_cast<double>(p2);
+        }
+    } else if constexpr (kWide) {
         t1 = t2 = 0.0;
         const bool pair = a.g.spatial >= kPairSpatial;
 #pragma unroll
@@ -144,7 +165,7 @@ __global__ __launch_bounds__(T, L == 0 && V * R <= (V == 1 ? (RES && !TIGHT ? 8 
     };
     if constexpr (RES) {
         // the rest of the shortcut's source four steps at a time, no branch around its loads (see above)
-        constexpr int kGroup = 4;
+        constexpr int kGroup = kSmall ? R : 4;
         static_assert((R + L) % kGroup == 0 && kAhead % kGroup == 0, "steps come in whole groups");
 #pragma unroll
         for (int first = 0; first < R + L; first += kGroup) {
@@ -186,8 +207,8 @@ int allow_large_lds(const void* kernel)
     return PXH_OK;
 }
 
-int launch_resident_forward(const char* who, const ResidentFwdArgs& r, bool vec, int per_thread, int activation,
-                            hipStream_t s)
+int launch_resident_forward(const char* who, const ResidentFwdArgs& r, bool vec, int per_thread, uint32_t small,
+                            int activation, hipStream_t s)
 {
     // (with the shortcut's source on top, sixteen values per lane no longer fit the registers of four
     // workgroups per compute unit: that form keeps the full workgroups)
@@ -196,6 +217,12 @@ int launch_resident_forward(const char* who, const ResidentFwdArgs& r, bool vec,
     int large_lds_rc = PXH_OK;
     const auto launch = [&]<int ACT, bool RES>() {
         constexpr int kT = kResidentThreads;
+        if (small) {
+            dispatch_small_form(vec, small, [&]<int V, int R, int T>() {
+                hipLaunchKernelGGL((bn_resident_fwd_kernel<ACT, V, R, 0, T, RES>), grid, dim3(T), 0, s, r);
+            });
+            return;
+        }
         if constexpr (!RES) {
             if (narrow) {
                 hipLaunchKernelGGL((bn_resident_fwd_kernel<ACT, 1, kResidentNarrowVectors, 0, kResidentNarrowThreads>),
