@@ -1,6 +1,6 @@
 // Conv-layer epilogue for gfx950: batch-norm (inference and training) + bias + activation,
 // forward and backward, as one-pass NCHW streaming kernels and per-channel reductions.
-#include "resident.h"
+#include "grouped.h"
 
 #include <mutex>
 
@@ -787,11 +787,25 @@ struct ClippedRegions {
     ClipPlan* plan;
 };
 
+// per-channel norm figures, sums and flags of the one-launch clipped backward
+size_t figure_bytes(int channels)
+{
+    const size_t c = static_cast<size_t>(channels);
+    return 2 * align256(c * sizeof(double2)) + align256(c * sizeof(int));
+}
+
+// the same of a group: its members' words hold the sums
+size_t group_figure_bytes(int channels)
+{
+    const size_t c = static_cast<size_t>(channels);
+    return align256(c * sizeof(double2)) + align256(c * sizeof(int));
+}
+
 size_t clipped_workspace_bytes_with(size_t partial, int channels)
 {
     const size_t c = static_cast<size_t>(channels);
     const size_t three = 2 * partial + align256(c * sizeof(DxCoef)) + 256;
-    const size_t one = 2 * align256(c * sizeof(double2)) + align256(c * sizeof(int)) + 256;
+    const size_t one = figure_bytes(channels) + 256;
     return three > one ? three : one;
 }
 
@@ -813,6 +827,39 @@ ClippedRegions clipped_regions(void* ws, int batch, int channels, int spatial)
     r.channel_done = reinterpret_cast<int*>(base + 2 * align256(c * sizeof(double2)));
     r.plan = reinterpret_cast<ClipPlan*>(base + clipped_workspace_bytes(batch, channels, spatial) - 256);
     return r;
+}
+
+constexpr int kResidentPlaces = 256;                  // of the workgroups that have a compute unit to themselves
+constexpr size_t kGroupScalars = 7u << 20;
+
+// The groups of a backward (members 0: none).  A plain call and a clipped one take the same form, so that they agree to
+// the bit where nothing is rescaled or clamped, and what they exchange has to fit the workspaces they ask for.
+//
+// `per_thread` is what a workgroup of 1024 lanes would hold of a channel (0: more than it can).  Where it can, one such
+// workgroup per channel is as fast or faster when the channels fill its places: 256 channels of more than kResidentVectors
+// vectors a lane (figures at the kernel; 16 x 192 x 76^2 47 us against 54 in groups, 16 x 320 x 76^2 89 against 80, mish 140
+// against 98), up to 512 of fewer (16 x 384 x 38^2 22.3, 22.6), or any with an exponential to compute.  Odd planes, whose
+// values come one at a time, gain only past the last-level cache's easy reach and with a gradient that is a select:
+// 6 x 72 x 135 x 77 25 -> 27 us, 8 x 96 x 135 x 77 41 -> 37, 32 x 64 x 75^2 48 -> 41; mish 35 -> 41, 54 -> 55, 65 -> 62.
+GroupPlan grouped_backward(int batch, int channels, int spatial, bool vec, int per_thread, int activation)
+{
+    const size_t total = static_cast<size_t>(batch) * channels * spatial;
+    if (!vec && (per_thread || !selects(activation) || total < kGroupScalars)) return GroupPlan{};
+    if (per_thread > kResidentVectors) {
+        const int rounds = (channels + kResidentPlaces - 1) / kResidentPlaces;
+        if (channels * 8 > rounds * kResidentPlaces * 5) return GroupPlan{};
+    } else if (per_thread && (!selects(activation) || channels < 2 * kResidentPlaces)) {
+        return GroupPlan{};
+    }
+    for (const size_t workgroups: { kGroupFill, static_cast<size_t>(1) }) {
+        const GroupPlan p = group_plan(batch, channels, spatial, vec, workgroups);
+        if (p.members <= 1 ||
+            (group_bytes(channels, p.members, kSumWords, false) <= workspace_bytes(batch, channels, spatial) &&
+             group_figure_bytes(channels) + group_bytes(channels, p.members, kFirstWords, true) + 256 <=
+                 clipped_workspace_bytes(batch, channels, spatial)))
+            return p;
+    }
+    return GroupPlan{};
 }
 
 // A tensor this large cannot stay in the last-level cache between two passes over it.
@@ -1128,6 +1175,29 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
         if (rc) return rc;
         region = clipped_regions(ws, batch, channels, spatial);
         clip = ClipArgs{ region.norm_partial, region.plan, cs.threshold, cs.clip, cs.norm_out };
+    }
+    GroupPlan group{};
+    // (a saved pre-activation is a third stream, which no register is left for)
+    if (!small && !pre_activation) group = grouped_backward(batch, channels, spatial, rvec, per_thread, activation);
+    if (group.members) {
+        const bool exchanges = group.members > 1;
+        if (exchanges && !cs.on) {
+            rc = resolve_workspace(workspace, workspace_bytes_given, workspace_bytes(batch, channels, spatial), &ws, s);
+            if (rc && !per_thread) return rc;
+            if (rc) group.members = 0;      // the other form needs no workspace: what it was given is not looked at
+        }
+        if (group.members) {
+            GroupGeom g = group_geom(group, batch, channels, spatial);
+            if (exchanges) {
+                rc = start_exchange(who, g, static_cast<char*>(ws) + (cs.on ? group_figure_bytes(channels) : 0), cs.on ? kFirstWords : kSumWords, cs.on, s);
+                if (rc) return rc;
+            }
+            const ResidentBwdArgs r{ BackwardArgs{ delta, x, nullptr, mean, var, scale, bias }, scale_updates,
+                                     bias_updates, mean_delta, var_delta, g.g, region.channel_norm, region.channel_sums,
+                                     exchanges && cs.on ? reinterpret_cast<int*>(region.channel_sums) : region.channel_done,
+                                     clip };
+            return launch_grouped_backward(who, r, g, cs.on, rvec, activation, s);
+        }
     }
     if (per_thread || small) {
         if (!cs.on && (!per_thread || (!rvec && per_thread > kResidentVectors))) {

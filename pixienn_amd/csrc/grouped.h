@@ -1,0 +1,159 @@
+// The one-launch training passes for slices that one workgroup cannot hold: a channel's slice is shared by the
+// workgroups of a group, which exchange their sums inside the launch.
+#pragma once
+
+#include "resident.h"
+
+namespace pxh {
+
+constexpr int kGroupThreads = 512;
+
+// What a member leaves for the others: up to four doubles, read as soon as they are there.  A word that is not there yet
+// holds kNotThere, a NaN that no sum comes out as (canonical_word below); a launch in front puts it there.
+constexpr uint64_t kNotThere = ~0ull;
+constexpr int kFirstWords = 4;      // sums A and B, the squares, the largest magnitude
+constexpr int kSumWords = 2;
+
+struct GroupGeom {
+    ResidentGeom g;
+    uint32_t items;         // vectors (or values) of a channel's slice
+    uint32_t span;          // of a member: a whole number of wavefronts
+    uint32_t members;       // of a channel
+    uint32_t image_skip;    // values between the end of a channel's plane and its plane in the next image
+    FastDiv by_members;
+    uint64_t* words;        // [channel][member][kFirstWords or kSumWords]; null with one member
+    uint64_t* redo_words;   // [channel][member][kSumWords], of a clipped backward's second launch
+    uint32_t* tickets;      // [2]
+};
+
+__device__ __forceinline__ float* at_byte(float* p, uint32_t bytes)
+{
+    return reinterpret_cast<float*>(reinterpret_cast<char*>(p) + bytes);
+}
+
+__device__ __forceinline__ const float* at_byte(const float* p, uint32_t bytes)
+{
+    return reinterpret_cast<const float*>(reinterpret_cast<const char*>(p) + bytes);
+}
+
+// The workgroups of a launch take numbers, and a channel's members have consecutive ones.  A workgroup waits only for
+// members of its own channel.  Those with lower numbers are running; of those with higher ones some may still have to
+// start, in the one channel whose numbers are not all taken.  Every workgroup of another channel finishes without them and
+// gives up its place, so they start as long as the device has more places than that one channel has waiting members, and
+// every wait ends.  kGroupShare below keeps a launch's waiting members to an eighth of the places of the device.
+__device__ __forceinline__ uint32_t take_ticket(uint32_t* counter, uint32_t& shared)
+{
+    __syncthreads();
+    if (threadIdx.x == 0) shared = atomicAdd(counter, 1u);
+    __syncthreads();
+    return shared;
+}
+
+__device__ __forceinline__ uint64_t canonical_word(double v)
+{
+    const uint64_t bits = __double_as_longlong(v);
+    return bits == kNotThere ? 0x7FF8000000000000ull : bits;
+}
+
+// About the time in which one half of the machine loads its shares (16 x 64 x 152^2: 62 us with it, 67 without, 64 with twice
+// as long; 16 x 128 x 152^2: 120, 123, 122).
+__device__ __forceinline__ void head_start() { __builtin_amdgcn_s_sleep(127); }
+
+// Leaves a member's figures for the others (every thread calls it with the same ones).
+template<int WORDS>
+__device__ __forceinline__ void leave_figures(uint64_t* channel_words, uint32_t member, const double (&figures)[WORDS])
+{
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int w = 0; w < WORDS; ++w)
+            __hip_atomic_store(channel_words + member * WORDS + w, canonical_word(figures[w]), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+// The figures of all members in every thread, added up in an order of the members alone (the last of four: the largest).
+// The bound on the looks makes the exit unconditional; it is seconds.
+template<int WORDS>
+__device__ __forceinline__ void collect_figures(const uint64_t* channel_words, uint32_t members, double (&figures)[WORDS])
+{
+    __shared__ double theirs[kGroupThreads];
+    const uint32_t t = threadIdx.x;
+    if (t < members * WORDS) {
+        uint64_t word = __hip_atomic_load(channel_words + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (uint32_t looks = 1u << 22; word == kNotThere && looks; --looks) {
+            __builtin_amdgcn_s_sleep(1);
+            word = __hip_atomic_load(channel_words + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        theirs[t] = __longlong_as_double(static_cast<long long>(word));
+    }
+    __syncthreads();
+    // a lane per member in every wave
+    const uint32_t lane = t & (kWave - 1);
+#pragma unroll
+    for (int w = 0; w < WORDS; ++w) {
+        const double v = lane < members ? theirs[lane * WORDS + w] : 0.0;
+        if (w < 3) figures[w] = wave_sum(v);
+        else figures[w] = static_cast<double>(wave_max(static_cast<float>(v)));
+    }
+}
+
+// ---- the rules
+// Members at most: a lane each, and their words a thread each.
+constexpr uint32_t kGroupMost = kWave;
+static_assert(kGroupMost * kFirstWords <= kGroupThreads, "a thread per word");
+constexpr uint32_t kGroupShare = 8;
+
+constexpr uint32_t kGroupItems = 12 * kGroupThreads;      // vectors that a member holds, or four times as many values
+constexpr size_t kGroupFill = 512;
+
+// Workgroups of these launches that the current device runs at once.
+uint32_t group_places();
+
+struct GroupPlan {
+    uint32_t items, span, members;      // members 0: another form takes the call
+};
+
+// How a slice is split over workgroups that hold `per_member` vectors (or values) each.
+inline GroupPlan split_slice(size_t items, uint32_t per_member, size_t channels, size_t workgroups)
+{
+    size_t least = (items + per_member - 1) / per_member;
+    const size_t fill = (workgroups + channels - 1) / channels, shortest = items / (4 * kGroupThreads);
+    const size_t more = fill < shortest ? fill : shortest;
+    if (least < more) least = more;
+    const size_t span = ((items + least - 1) / least + kWave - 1) / kWave * kWave;
+    const size_t members = (items + span - 1) / span;
+    if (members > kGroupMost || members * kGroupShare > group_places()) return GroupPlan{};
+    return GroupPlan{ static_cast<uint32_t>(items), static_cast<uint32_t>(span), static_cast<uint32_t>(members) };
+}
+
+inline GroupPlan group_plan(int batch, int channels, int spatial, bool vec, size_t workgroups)
+{
+    const size_t per_channel = static_cast<size_t>(batch) * spatial;
+    if (per_channel * channels >= 1ull << 30) return GroupPlan{};      // places are 32-bit byte offsets
+    return split_slice(vec ? per_channel / 4 : per_channel, vec ? kGroupItems : 4 * kGroupItems, channels, workgroups);
+}
+
+inline GroupGeom group_geom(const GroupPlan& p, int batch, int channels, int spatial)
+{
+    return GroupGeom{ resident_geom(batch, channels, spatial), p.items, p.span, p.members,
+                      static_cast<uint32_t>(channels - 1) * static_cast<uint32_t>(spatial), FastDiv(p.members), nullptr, nullptr,
+                      nullptr };
+}
+
+// Bytes of the words of `count` members, and of everything a launch (with `redo`: and the one behind it) exchanges.
+constexpr size_t group_align(size_t b) { return (b + 255) & ~static_cast<size_t>(255); }
+inline size_t group_bytes(uint32_t channels, uint32_t members, int words, bool redo)
+{
+    const size_t count = static_cast<size_t>(channels) * members;
+    return group_align(count * words * 8) + (redo ? group_align(count * kSumWords * 8) : 0) + 256;
+}
+
+constexpr size_t kGroupLdsBytes = 64u << 10;
+
+// Places GroupGeom's buffers in `at` and queues the launch that empties them.
+int start_exchange(const char* who, GroupGeom& g, void* at, int words, bool redo, hipStream_t s);
+
+int launch_grouped_backward(const char* who, const ResidentBwdArgs& r, const GroupGeom& g, bool clipped, bool vec,
+                            int activation, hipStream_t s);
+
+}  // namespace pxh

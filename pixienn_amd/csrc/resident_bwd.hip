@@ -4,26 +4,6 @@
 namespace pxh {
 namespace {
 
-// A channel that was finished with the sums (sa, sb) of its unscaled delta, after the plan turned out
-// to rescale by `factor` (and its clamp to move nothing in this channel): everything the backward left
-// is linear in the delta, so the accumulated updates get the difference and the two per-channel deltas
-// are formed again.  The dx values are scaled by the caller.
-__device__ __forceinline__ void rescale_finished_channel(double sa, double sb, double factor, int c, const float* var,
-                                                         const float* scale, float* scale_updates,
-                                                         float* bias_updates, float* mean_delta, float* var_delta)
-{
-    bias_updates[c] += static_cast<float>((factor - 1.0) * sa);
-    const float v = var[c];
-    const float s = scale[c];
-    const double denom = sqrt(static_cast<double>(v)) + static_cast<double>(kEps);
-    scale_updates[c] += static_cast<float>((factor - 1.0) * sb / denom);
-    const float sum_dd = static_cast<float>(factor * sa * static_cast<double>(s));
-    const float sum_ddx = static_cast<float>(factor * sb * static_cast<double>(s));
-    const float ve = v + kEps;
-    if (mean_delta) mean_delta[c] = static_cast<float>(static_cast<double>(sum_dd) * (-1. / static_cast<double>(sqrtf(ve))));
-    if (var_delta) var_delta[c] = sum_ddx * (-.5f * powf(ve, -3.0f / 2.0f));
-}
-
 // The workgroup keeps d' = delta * act'(pre) (registers + LDS); x is read again for the dx phase
 // (it is still in the cache: one channel's slice is a few hundred KB).
 //

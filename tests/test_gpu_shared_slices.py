@@ -1,0 +1,106 @@
+"""GPU parity of the training passes whose workgroups share a channel's slice: the checks of the other geometries, with
+their tolerances, at the sizes where the split changes; then under graph replay and on two streams at once."""
+import numpy as np
+import pytest
+
+import test_gpu_clipped_backward as clipped
+import test_gpu_epilogue as epilogue
+from pixienn_amd import workloads as wl
+from util import F, assert_bit_exact, gpu, host
+
+pytestmark = pytest.mark.gpu
+
+# vectors of a slice: 4097 (the first that the small forms leave), a member's 6144 and one more, a last member of one
+# wavefront, planes that end inside a share, 64 members and one more (three launches), 130 channels of two rounds,
+# channels on both sides of five eighths of the places, 512 channels of one member
+VECTORS = [(1, 3, 16388), (4, 2, 6144), (1, 1, 24580), (3, 2, 32772), (7, 5, 10012), (16, 1, 98304), (16, 1, 98308),
+           (3, 130, 32772), (9, 160, 3644), (9, 161, 3644), (4, 512, 4112)]
+# values: of two streams' worth of odd planes, with and without a last share that is short
+SCALARS = [(8, 96, 10395), (32, 41, 5625), (1, 5, 1572863)]
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from pixienn_amd import ops as o
+    return o
+
+
+@pytest.mark.parametrize("act", ["leaky", "mish"])
+@pytest.mark.parametrize("shape", VECTORS + SCALARS, ids=str)
+def test_shared_slices_backward(ops, oracle, monkeypatch, shape, act):
+    for module in (epilogue, clipped):
+        monkeypatch.setattr(module, "TRAIN_SHAPES", [shape])
+    epilogue.test_bn_backward_matches_oracle(ops, oracle, act, False)
+    clipped.test_bn_backward_clipped_matches_rescale_clip_then_backward(ops, oracle, act, False)
+
+
+class Layer:
+    """A layer's tensors, and both passes over them with a workspace of its own."""
+
+    def __init__(self, ops, torch, seed, shape):
+        from pixienn_amd import capi
+        lib = capi.load()
+        N, C, H, W = shape
+        self.ops = ops
+        self.x, self.delta = gpu(wl.normal(seed, shape)), gpu(wl.normal(seed + 1, shape))
+        scale, bias, rmean, rvar = wl.bn_params(seed + 2, C)
+        self.scale, self.bias, self.rolling0 = gpu(scale), gpu(bias), (gpu(rmean), gpu(rvar))
+        self.mean, self.var, self.rm, self.rv, self.su, self.bu = (torch.zeros(C, device="cuda") for _ in range(6))
+        self.y, self.d = torch.empty_like(self.x), torch.empty_like(self.x)
+        need = max(lib.pxh_bn_workspace_bytes(N, C, H * W), lib.pxh_bn_clipped_workspace_bytes(N, C, H * W))
+        self.workspace = torch.zeros(need // 4 + 4, device="cuda")
+
+    def run(self, clip):
+        self.d.copy_(self.delta)
+        self.rm.copy_(self.rolling0[0]); self.rv.copy_(self.rolling0[1])
+        self.su.zero_(); self.bu.zero_()
+        self.ops.bn_train_act_forward(self.x, self.y, self.mean, self.var, self.rm, self.rv, self.scale, self.bias, "leaky",
+                                      workspace=self.workspace)
+        self.ops.bn_act_backward_clipped(self.d, self.x, self.mean, self.var, self.scale, self.bias, self.su, self.bu, "leaky",
+                                         1e6, clip, workspace=self.workspace)
+
+    def results(self):
+        return [host(t) for t in (self.y, self.mean, self.var, self.rm, self.rv, self.d, self.su, self.bu)]
+
+
+@pytest.mark.parametrize("clip", [100.0, 3.0])      # nothing to clamp; some channels gone over again by the second launch
+def test_shared_slices_in_a_replayed_graph(ops, clip):
+    import torch
+    layer = Layer(ops, torch, 9100, (4, 24, 104, 104))
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        layer.run(clip)
+        stream.synchronize()
+        want = layer.results()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            layer.run(clip)
+        for _ in range(4):
+            layer.y.zero_(); layer.d.zero_()
+            graph.replay()
+            stream.synchronize()
+            for got, expected in zip(layer.results(), want):
+                assert_bit_exact(got, expected, "replay")
+            layer.run(clip)                         # eager work on the same workspace in between
+            stream.synchronize()
+
+
+def test_shared_slices_on_two_streams(ops):
+    import torch
+    layers = [Layer(ops, torch, 9200 + 10 * i, shape) for i, shape in enumerate([(4, 40, 104, 104), (8, 64, 152, 152)])]
+    want = []
+    for layer in layers:
+        layer.run(3.0)
+        torch.cuda.synchronize()
+        want.append(layer.results())
+    streams = [torch.cuda.Stream() for _ in layers]
+    for _ in range(3):
+        for layer, stream in zip(layers, streams):
+            stream.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(stream):
+                for _ in range(4):
+                    layer.run(3.0)
+        torch.cuda.synchronize()
+        for layer, expected in zip(layers, want):
+            for got, w in zip(layer.results(), expected):
+                assert_bit_exact(got, w, "two streams")
