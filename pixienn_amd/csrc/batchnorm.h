@@ -233,17 +233,18 @@ __device__ __forceinline__ FinishedChannel finished_channel(double sa, double sb
 
 // A channel that was finished with the sums (sa, sb) of its unscaled delta, after the plan turned out
 // to rescale by `factor` (and its clamp to move nothing in this channel): everything the backward left
-// is linear in the delta, so the accumulated updates get the difference and the two per-channel deltas
-// are formed again.  The dx values are scaled by the caller.
-__device__ __forceinline__ void rescale_finished_channel(double sa, double sb, double factor, int c, const float* var,
-                                                         const float* scale, float* scale_updates,
+// is linear in the delta, so the accumulated updates are formed again from what they were `before` (bias,
+// scale), with one rounding as everywhere, and so are the two per-channel deltas.  The dx values are scaled
+// by the caller.
+__device__ __forceinline__ void rescale_finished_channel(double sa, double sb, double factor, float2 before, int c,
+                                                         const float* var, const float* scale, float* scale_updates,
                                                          float* bias_updates, float* mean_delta, float* var_delta)
 {
-    bias_updates[c] += static_cast<float>((factor - 1.0) * sa);
+    bias_updates[c] = before.x + static_cast<float>(factor * sa);
     const float v = var[c];
     const float s = scale[c];
     const double denom = sqrt(static_cast<double>(v)) + static_cast<double>(kEps);
-    scale_updates[c] += static_cast<float>((factor - 1.0) * sb / denom);
+    scale_updates[c] = before.y + static_cast<float>(factor * sb / denom);
     const float sum_dd = static_cast<float>(factor * sa * static_cast<double>(s));
     const float sum_ddx = static_cast<float>(factor * sb * static_cast<double>(s));
     const float ve = v + kEps;

@@ -776,29 +776,30 @@ void* coef_region(void* ws, int batch, int channels, int spatial)
 }
 
 // The clipped backward: [partial sums][per-channel constants][norm partials][plan] for the three
-// launches, [per-channel norm figures][per-channel sums][per-channel flags][plan] for the one-launch form.
+// launches, [per-channel norm figures][per-channel sums][updates before][per-channel flags][plan] for the one-launch form.
 struct ClippedRegions {
     double2* partial;
     DxCoef* coef;
     double2* norm_partial;
     double2* channel_norm;
     double2* channel_sums;
+    float2* channel_before;
     int* channel_done;
     ClipPlan* plan;
 };
 
-// per-channel norm figures, sums and flags of the one-launch clipped backward
+// per-channel norm figures, sums, updates before and flags of the one-launch clipped backward
 size_t figure_bytes(int channels)
 {
     const size_t c = static_cast<size_t>(channels);
-    return 2 * align256(c * sizeof(double2)) + align256(c * sizeof(int));
+    return 2 * align256(c * sizeof(double2)) + align256(c * (sizeof(float2) + sizeof(int)));
 }
 
 // the same of a group: its members' words hold the sums
 size_t group_figure_bytes(int channels)
 {
     const size_t c = static_cast<size_t>(channels);
-    return align256(c * sizeof(double2)) + align256(c * sizeof(int));
+    return align256(c * sizeof(double2)) + align256(c * (sizeof(float2) + sizeof(int)));
 }
 
 size_t clipped_workspace_bytes_with(size_t partial, int channels)
@@ -824,7 +825,8 @@ ClippedRegions clipped_regions(void* ws, int batch, int channels, int spatial)
     r.norm_partial = reinterpret_cast<double2*>(reinterpret_cast<char*>(r.coef) + align256(c * sizeof(DxCoef)));
     r.channel_norm = reinterpret_cast<double2*>(base);
     r.channel_sums = reinterpret_cast<double2*>(base + align256(c * sizeof(double2)));
-    r.channel_done = reinterpret_cast<int*>(base + 2 * align256(c * sizeof(double2)));
+    r.channel_before = reinterpret_cast<float2*>(base + 2 * align256(c * sizeof(double2)));
+    r.channel_done = reinterpret_cast<int*>(base + 2 * align256(c * sizeof(double2)) + c * sizeof(float2));
     r.plan = reinterpret_cast<ClipPlan*>(base + clipped_workspace_bytes(batch, channels, spatial) - 256);
     return r;
 }
@@ -1192,10 +1194,15 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
                 rc = start_exchange(who, g, static_cast<char*>(ws) + (cs.on ? group_figure_bytes(channels) : 0), cs.on ? kFirstWords : kSumWords, cs.on, s);
                 if (rc) return rc;
             }
+            if (exchanges && cs.on) {
+                // no sums: the members' words hold them
+                char* const base = reinterpret_cast<char*>(region.channel_sums);
+                region.channel_before = reinterpret_cast<float2*>(base);
+                region.channel_done = reinterpret_cast<int*>(base + static_cast<size_t>(channels) * sizeof(float2));
+            }
             const ResidentBwdArgs r{ BackwardArgs{ delta, x, nullptr, mean, var, scale, bias }, scale_updates,
                                      bias_updates, mean_delta, var_delta, g.g, region.channel_norm, region.channel_sums,
-                                     exchanges && cs.on ? reinterpret_cast<int*>(region.channel_sums) : region.channel_done,
-                                     clip };
+                                     region.channel_before, region.channel_done, clip };
             return launch_grouped_backward(who, r, g, cs.on, rvec, activation, s);
         }
     }
@@ -1207,7 +1214,8 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
         }
         const ResidentBwdArgs r{ BackwardArgs{ delta, x, pre_activation, mean, var, scale, bias }, scale_updates,
                                  bias_updates, mean_delta, var_delta, resident_geom(batch, channels, spatial),
-                                 region.channel_norm, region.channel_sums, region.channel_done, clip };
+                                 region.channel_norm, region.channel_sums, region.channel_before, region.channel_done,
+                                 clip };
         return launch_resident_backward(who, r, cs.on, rvec, per_thread, small, activation, s);
     }
     if (!cs.on) {

@@ -140,6 +140,7 @@ __device__ __forceinline__ void grouped_bwd_member(const ResidentBwdArgs& a, con
             a.scale_updates[c] = scale_updates_in + r.scale_add;
             if (a.mean_delta) a.mean_delta[c] = r.mean_delta;
             if (a.var_delta) a.var_delta[c] = r.var_delta;
+            if constexpr (MODE == kFirst) a.channel_before[c] = make_float2(bias_updates_in, scale_updates_in);
         }
         if constexpr (MODE == kFirst) {
             if (member == 0) {
@@ -192,7 +193,7 @@ __device__ __forceinline__ void grouped_rescale_member(const ResidentBwdArgs& a,
         figures[1] = sums.y;
     }
     if (threadIdx.x == 0) {
-        rescale_finished_channel(figures[0], figures[1], static_cast<double>(factor), c, a.b.var, a.b.scale, a.scale_updates,
+        rescale_finished_channel(figures[0], figures[1], static_cast<double>(factor), a.channel_before[c], c, a.b.var, a.b.scale, a.scale_updates,
                                  a.bias_updates, a.mean_delta, a.var_delta);
     }
 }

@@ -179,9 +179,11 @@ struct ResidentBwdArgs {
     float* var_delta;    // nullable
     ResidentGeom g;
     // the clipped form (else null): per channel the (sum of squares, largest magnitude) of its delta,
-    // the two sums it was finished with, and whether it was finished at all
+    // the two sums it was finished with, its bias and scale updates before that, and whether it was
+    // finished at all
     double2* channel_norm;
     double2* channel_sums;
+    float2* channel_before;
     int* channel_done;
     ClipArgs clip;
 };

@@ -34,7 +34,7 @@ __device__ __forceinline__ void resident_rescale_channel(const ResidentBwdArgs& 
     }
     if (threadIdx.x == 0) {
         const double2 sums = a.channel_sums[c];
-        rescale_finished_channel(sums.x, sums.y, static_cast<double>(factor), c, a.b.var, a.b.scale, a.scale_updates,
+        rescale_finished_channel(sums.x, sums.y, static_cast<double>(factor), a.channel_before[c], c, a.b.var, a.b.scale, a.scale_updates,
                                  a.bias_updates, a.mean_delta, a.var_delta);
     }
 }
@@ -74,6 +74,7 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
         a.scale_updates[c] = scale_updates_in + r.scale_add;
         if (a.mean_delta) a.mean_delta[c] = r.mean_delta;
         if (a.var_delta) a.var_delta[c] = r.var_delta;
+        if constexpr (MODE == kFirst) a.channel_before[c] = make_float2(bias_updates_in, scale_updates_in);
         return r.k;
     };
     const bool recompute = a.b.pre == nullptr;
