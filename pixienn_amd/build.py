@@ -9,6 +9,7 @@ ROOT = os.path.dirname(PKG)
 CSRC = os.path.join(PKG, "csrc")
 OBJ = os.path.join(PKG, "build")
 LIB = os.path.join(PKG, "libpixienn_hip.so")
+CALLS = os.path.join(PKG, "_calls.so")
 
 SOURCES = ["runtime.hip", "epilogue.hip", "resident_fwd.hip", "resident_bwd.hip", "grouped_bwd.hip", "elementwise.hip", "pool.hip", "yolo.hip", "nms.hip"]
 
@@ -53,6 +54,21 @@ def build_library(verbose=True):
     return LIB
 
 
+def build_calls():
+    """Compiles csrc/calls.cpp, the extension module that calls the C ABI with torch tensors (host code)."""
+    import sysconfig
+
+    import torch
+    root = os.path.dirname(torch.__file__)
+    include = os.path.join(root, "include")
+    cmd = ["g++", "-shared", "-fPIC", "-std=c++17", "-O2", "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI),
+           "-I" + sysconfig.get_paths()["include"], "-isystem", include, "-isystem",
+           os.path.join(include, "torch", "csrc", "api", "include"), "-I" + os.path.join(ROOT, "include"),
+           os.path.join(CSRC, "calls.cpp"), "-o", CALLS, "-L" + os.path.join(root, "lib"), "-ltorch_python", "-lc10"]
+    subprocess.check_call(cmd)
+    return CALLS
+
+
 def build_host(verbose=True):
     """Compiles the C++ layer interface (host/pixienn/*.h, header-only) as a translation unit of
     its own: the check that it builds against the C ABI alone."""
@@ -74,4 +90,5 @@ def build_host(verbose=True):
 
 if __name__ == "__main__":
     print(build_library())
+    print(build_calls())
     print(build_host())

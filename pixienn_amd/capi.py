@@ -121,6 +121,10 @@ class PxError(RuntimeError):
 
 _lib = None
 
+# The entry points that csrc/calls.cpp calls: name -> (callable that takes tensors for float buffers and answers None for a
+# call it does not make, which arguments are tensors).  Filled by load().
+native = {}
+
 
 def load():
     """Loads the built library; raises PxError when it has not been built."""
@@ -139,6 +143,13 @@ def load():
         fn = getattr(lib, name)
         fn.argtypes = args
         fn.restype = res
+    try:
+        from . import _calls
+    except ImportError as e:
+        raise PxError("the calls of %s are not built (%s); run `python -m pixienn_amd.build` or "
+                      "__graft_entry__.build()" % (LIB_PATH, e)) from e
+    for name in _calls.names():
+        native[name] = _calls.bind(name, ctypes.cast(getattr(lib, name), ctypes.c_void_p).value)
     _lib = lib
     return lib
 

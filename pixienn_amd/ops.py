@@ -17,8 +17,16 @@ from .capi import PxError, act_id, call, ptr
 # here is then its time.  The current stream's handle comes without a Stream object around it (0.3 us in
 # place of 2), and a tensor that is as it should be passes its check in one expression.
 _F32 = torch.float32
-_current_device = torch.cuda.current_device
 _raw_stream = torch._C._cuda_getCurrentRawStream
+
+
+def _current_device():
+    """The current device's index; the first call sets torch's side of the device up, the later ones go past the check
+    that it is (0.1 us in place of 0.7)."""
+    global _current_device
+    index = torch.cuda.current_device()
+    _current_device = torch._C._cuda_getDevice
+    return index
 
 
 def _stream():
@@ -45,8 +53,43 @@ def _chk_all(*ts):
         _chk(t)
 
 
+def _run(name, *args):
+    """call() on the current stream, with tensors themselves, or None, for the float buffers among the arguments."""
+    if capi._lib is None:
+        capi.load()
+    make, tensors = capi.native[name]
+    try:
+        stream = _raw_stream(_current_device())
+        rc = make(*args, stream)
+        if rc == 0:
+            return
+        if rc is not None:
+            raise PxError("%s failed (status %d): %s" % (name, rc, capi.last_error()))
+    except PxError:
+        raise
+    except Exception:
+        _pointers(tensors, args)      # without a device: what is wrong with the tensors comes first
+        raise
+    # not plain tensors and numbers: one by one, each with its own error
+    call(name, *_pointers(tensors, args), stream)
+
+
+def _pointers(tensors, args):
+    for t, is_tensor in zip(args, tensors):
+        if is_tensor:
+            _chk(t)
+    return [ptr(a) if is_tensor else a for a, is_tensor in zip(args, tensors)]
+
+
+def _tensor(t):
+    """A first look at an argument whose sizes are asked for before the call looks at it."""
+    if t.__class__ is not torch.Tensor and not isinstance(t, torch.Tensor):
+        _chk(t)
+    return t
+
+
 def _nchw(x):
-    shape = x.shape
+    shape = _tensor(x).shape
     if len(shape) != 4:
         raise PxError("NCHW tensor expected, got %d dims" % len(shape))
     n, c, h, w = shape
@@ -92,18 +135,16 @@ def bn_fold(rolling_mean, rolling_var, scale, bias, folded=None):
 
 
 def bn_folded_act_forward(x, y, folded, activation, pre_activation=None):
-    _chk_all(x, y, folded, pre_activation)
+    _chk(folded)
     n, c, s = _nchw(x)
-    call("pxh_bn_folded_act_forward", ptr(x), ptr(y), ptr(pre_activation), ptr(folded), n, c, s,
-         act_id(activation), _stream())
+    _run("pxh_bn_folded_act_forward", x, y, pre_activation, ptr(folded), n, c, s,
+         act_id(activation))
     return y
 
 
 def bias_act_forward(x, y, bias, activation, pre_activation=None):
-    _chk_all(x, y, bias, pre_activation)
     n, c, s = _nchw(x)
-    call("pxh_bias_act_forward", ptr(x), ptr(y), ptr(pre_activation), ptr(bias), n, c, s, act_id(activation),
-         _stream())
+    _run("pxh_bias_act_forward", x, y, pre_activation, bias, n, c, s, act_id(activation))
     return y
 
 
@@ -113,12 +154,11 @@ def bn_workspace_bytes(batch, channels, spatial):
 
 def bn_train_act_forward(x, y, mean, var, rolling_mean, rolling_var, scale, bias, activation,
                          pre_activation=None, x_saved=None, x_norm=None, workspace=None):
-    _chk_all(x, y, mean, var, rolling_mean, rolling_var, scale, bias, pre_activation, x_saved, x_norm)
     n, c, s = _nchw(x)
     wb = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    call("pxh_bn_train_act_forward", ptr(x), ptr(y), ptr(pre_activation), ptr(x_saved), ptr(x_norm), ptr(mean),
-         ptr(var), ptr(rolling_mean), ptr(rolling_var), ptr(scale), ptr(bias), n, c, s, act_id(activation),
-         ptr(workspace), wb, _stream())
+    _run("pxh_bn_train_act_forward", x, y, pre_activation, x_saved, x_norm, mean,
+         var, rolling_mean, rolling_var, scale, bias, n, c, s, act_id(activation),
+         ptr(workspace), wb)
     return y
 
 
@@ -133,71 +173,62 @@ def bn_stats(x, mean, var, workspace=None):
 def bn_train_act_shortcut_forward(x, y, mean, var, rolling_mean, rolling_var, scale, bias, activation, from_, alpha=1.0,
                                   beta=1.0, pre_activation=None, x_saved=None, x_norm=None, workspace=None):
     """bn_train_act_forward with the linear shortcut that follows the layer: y = alpha*act(pre) + beta*from_."""
-    _chk_all(x, y, mean, var, rolling_mean, rolling_var, scale, bias, from_, pre_activation, x_saved, x_norm)
     n, c, s = _nchw(x)
     wb = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    call("pxh_bn_train_act_shortcut_forward", ptr(x), ptr(y), ptr(pre_activation), ptr(x_saved), ptr(x_norm), ptr(mean),
-         ptr(var), ptr(rolling_mean), ptr(rolling_var), ptr(scale), ptr(bias), ptr(from_), float(alpha), float(beta),
-         n, c, s, act_id(activation), ptr(workspace), wb, _stream())
+    _run("pxh_bn_train_act_shortcut_forward", x, y, pre_activation, x_saved, x_norm, mean,
+         var, rolling_mean, rolling_var, scale, bias, from_, float(alpha), float(beta),
+         n, c, s, act_id(activation), ptr(workspace), wb)
 
 
 def bn_folded_act_shortcut_forward(x, y, folded, activation, from_, alpha=1.0, beta=1.0, pre_activation=None):
     """bn_folded_act_forward with the linear shortcut that follows the layer."""
-    _chk_all(x, y, from_, pre_activation)
     n, c, s = _nchw(x)
-    call("pxh_bn_folded_act_shortcut_forward", ptr(x), ptr(y), ptr(pre_activation), ptr(folded), ptr(from_),
-         float(alpha), float(beta), n, c, s, act_id(activation), _stream())
+    _run("pxh_bn_folded_act_shortcut_forward", x, y, pre_activation, ptr(folded), from_,
+         float(alpha), float(beta), n, c, s, act_id(activation))
 
 
 def bn_folded_act_maxpool_forward(x, pooled, folded, activation, y=None):
     """bn_folded_act_forward with the 2x2 / 2 max-pool that follows the layer; x is [N, C, H, W]."""
-    _chk_all(x, pooled, y)
-    n, c, h, w = x.shape
-    call("pxh_bn_folded_act_maxpool_forward", ptr(x), ptr(y), ptr(pooled), ptr(folded), n, c, h, w, act_id(activation),
-         _stream())
+    n, c, h, w = _tensor(x).shape
+    _run("pxh_bn_folded_act_maxpool_forward", x, y, pooled, ptr(folded), n, c, h, w, act_id(activation))
 
 
 def bn_act_backward(delta, x, mean, var, scale, bias, scale_updates, bias_updates, activation,
                     pre_activation=None, mean_delta=None, var_delta=None, workspace=None):
-    _chk_all(delta, x, mean, var, scale, bias, scale_updates, bias_updates, pre_activation, mean_delta, var_delta)
     n, c, s = _nchw(delta)
     wb = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    call("pxh_bn_act_backward", ptr(delta), ptr(x), ptr(pre_activation), ptr(mean), ptr(var), ptr(scale), ptr(bias),
-         ptr(scale_updates), ptr(bias_updates), ptr(mean_delta), ptr(var_delta), n, c, s, act_id(activation),
-         ptr(workspace), wb, _stream())
+    _run("pxh_bn_act_backward", delta, x, pre_activation, mean, var, scale, bias,
+         scale_updates, bias_updates, mean_delta, var_delta, n, c, s, act_id(activation),
+         ptr(workspace), wb)
     return delta
 
 
 def bias_act_backward(delta, pre_activation, bias_updates, activation, workspace=None):
-    _chk_all(delta, pre_activation, bias_updates)
     n, c, s = _nchw(delta)
     wb = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    call("pxh_bias_act_backward", ptr(delta), ptr(pre_activation), ptr(bias_updates), n, c, s, act_id(activation),
-         ptr(workspace), wb, _stream())
+    _run("pxh_bias_act_backward", delta, pre_activation, bias_updates, n, c, s, act_id(activation),
+         ptr(workspace), wb)
     return delta
 
 
 def bn_act_backward_clipped(delta, x, mean, var, scale, bias, scale_updates, bias_updates, activation, threshold,
                             clip, norm_out=None, pre_activation=None, mean_delta=None, var_delta=None, workspace=None):
     """rescale_clip(delta, threshold, clip) then bn_act_backward, without the read of delta for its norm."""
-    _chk_all(delta, x, mean, var, scale, bias, scale_updates, bias_updates, pre_activation, mean_delta, var_delta,
-             norm_out)
     n, c, s = _nchw(delta)
     wb = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    call("pxh_bn_act_backward_clipped", ptr(delta), ptr(x), ptr(pre_activation), ptr(mean), ptr(var), ptr(scale),
-         ptr(bias), ptr(scale_updates), ptr(bias_updates), ptr(mean_delta), ptr(var_delta), n, c, s,
-         act_id(activation), float(threshold), float(clip), ptr(norm_out), ptr(workspace), wb, _stream())
+    _run("pxh_bn_act_backward_clipped", delta, x, pre_activation, mean, var, scale,
+         bias, scale_updates, bias_updates, mean_delta, var_delta, n, c, s,
+         act_id(activation), float(threshold), float(clip), norm_out, ptr(workspace), wb)
     return delta
 
 
 def bias_act_backward_clipped(delta, pre_activation, bias_updates, activation, threshold, clip, norm_out=None,
                               workspace=None):
     """rescale_clip(delta, threshold, clip) then bias_act_backward, without the read of delta for its norm."""
-    _chk_all(delta, pre_activation, bias_updates, norm_out)
     n, c, s = _nchw(delta)
     wb = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    call("pxh_bias_act_backward_clipped", ptr(delta), ptr(pre_activation), ptr(bias_updates), n, c, s,
-         act_id(activation), float(threshold), float(clip), ptr(norm_out), ptr(workspace), wb, _stream())
+    _run("pxh_bias_act_backward_clipped", delta, pre_activation, bias_updates, n, c, s,
+         act_id(activation), float(threshold), float(clip), norm_out, ptr(workspace), wb)
     return delta
 
 
@@ -229,8 +260,7 @@ def fill(x, value):
         _chk(x, torch.int32)
         call("pxh_fill_i32", ptr(x), x.numel(), int(value), _stream())
     else:
-        _chk(x)
-        call("pxh_fill_f32", ptr(x), x.numel(), float(value), _stream())
+        _run("pxh_fill_f32", x, x.numel(), float(value))
     return x
 
 
@@ -245,25 +275,22 @@ def mul(x, y):
 
 
 def axpy(alpha, x, y):
-    _chk_all(x, y)
-    call("pxh_axpy", x.numel(), float(alpha), ptr(x), ptr(y), _stream())
+    _run("pxh_axpy", _tensor(x).numel(), float(alpha), x, y)
 
 
 def route_forward(layer_output, route_output, offset):
     """Copies one source layer into its slice of a concatenation (include/RouteLayer.h:91-113).
     layer_output [N, ...] packed; route_output [N, ...]; offset in floats within a route image."""
-    _chk_all(layer_output, route_output)
-    batch = layer_output.shape[0]
-    call("pxh_route_forward", ptr(layer_output), ptr(route_output), batch, layer_output.numel() // max(1, batch),
-         route_output.numel() // max(1, batch), int(offset), _stream())
+    batch = _tensor(layer_output).shape[0]
+    _run("pxh_route_forward", layer_output, route_output, batch, layer_output.numel() // max(1, batch),
+         route_output.numel() // max(1, batch), int(offset))
 
 
 def route_backward(route_delta, layer_delta, offset):
     """layer_delta += the layer's slice of route_delta (include/RouteLayer.h:115-137)."""
-    _chk_all(route_delta, layer_delta)
-    batch = layer_delta.shape[0]
-    call("pxh_route_backward", ptr(route_delta), ptr(layer_delta), batch, layer_delta.numel() // max(1, batch),
-         route_delta.numel() // max(1, batch), int(offset), _stream())
+    batch = _tensor(layer_delta).shape[0]
+    _run("pxh_route_backward", route_delta, layer_delta, batch, layer_delta.numel() // max(1, batch),
+         route_delta.numel() // max(1, batch), int(offset))
 
 
 # ---------------------------------------------------------------- max-pool / upsample / shortcut
@@ -273,21 +300,17 @@ def maxpool_out_dim(n, kernel, stride, padding):
 
 
 def maxpool_forward(x, out, indexes, kernel, stride, padding):
-    _chk_all(x, out)
     _chk(indexes, torch.int32, "indexes")
-    n, c, ih, iw = x.shape
-    oh, ow = out.shape[2], out.shape[3]
-    call("pxh_maxpool_forward", ptr(x), ptr(out), ptr(indexes), n, c, ih, iw, oh, ow, kernel, stride, padding,
-         _stream())
+    n, c, ih, iw = _tensor(x).shape
+    oh, ow = _tensor(out).shape[2:4]
+    _run("pxh_maxpool_forward", x, out, ptr(indexes), n, c, ih, iw, oh, ow, kernel, stride, padding)
 
 
 def maxpool_backward(delta, indexes, grad, kernel, stride, padding):
-    _chk_all(delta, grad)
     _chk(indexes, torch.int32, "indexes")
-    n, c, ih, iw = grad.shape
-    oh, ow = delta.shape[2], delta.shape[3]
-    call("pxh_maxpool_backward", ptr(delta), ptr(indexes), ptr(grad), n, c, ih, iw, oh, ow, kernel, stride, padding,
-         _stream())
+    n, c, ih, iw = _tensor(grad).shape
+    oh, ow = _tensor(delta).shape[2:4]
+    _run("pxh_maxpool_backward", delta, ptr(indexes), grad, n, c, ih, iw, oh, ow, kernel, stride, padding)
 
 
 def maxpool_backward_scatter(delta, indexes, grad):
@@ -362,17 +385,16 @@ def shortcut_backward_first(delta, from_delta, grad=None, activation="linear", a
 def shortcut_backward_clipped(delta, from_delta, grad=None, activation="linear", alpha=1.0, beta=1.0,
                               pre_activation=None, first=True, threshold=0.0, clip=0.0, norm_out=None, workspace=None):
     """rescale_clip(delta, threshold, clip, norm_out), then the shortcut's backward (first writer or accumulating)."""
-    _chk_all(delta, from_delta, grad, pre_activation, norm_out, workspace)
+    _chk(workspace)
     wb = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    call("pxh_shortcut_backward_clipped", ptr(delta), ptr(pre_activation), ptr(from_delta), ptr(grad), delta.numel(),
-         float(alpha), float(beta), act_id(activation), int(bool(first)), float(threshold), float(clip), ptr(norm_out),
-         ptr(workspace), wb, _stream())
+    _run("pxh_shortcut_backward_clipped", delta, pre_activation, from_delta, grad, _tensor(delta).numel(),
+         float(alpha), float(beta), act_id(activation), int(bool(first)), float(threshold), float(clip), norm_out,
+         ptr(workspace), wb)
 
 
 # ---------------------------------------------------------------- YOLO head
 def yolo_activate(inp, out, batch, masks, classes, area):
-    _chk_all(inp, out)
-    call("pxh_yolo_activate", ptr(inp), ptr(out), batch, masks, classes, area, _stream())
+    _run("pxh_yolo_activate", inp, out, batch, masks, classes, area)
 
 
 def yolo_forward_train(inp, out, delta, truths, truth_counts, max_truth, masks, anchors, stats, cost, batch, classes,
@@ -448,9 +470,8 @@ def adam(x, m, v, beta1, beta2, rate, eps, t):
 
 def adam_update(w, d, m, v, batch, t, lr, beta1=0.9, beta2=0.999, eps=1e-8, decay=0.0, apply_decay=False):
     """apply_decay: False / 0 none, True / 1 the reference's L2 term, 2 decoupled decay."""
-    _chk_all(w, d, m, v)
-    call("pxh_adam_update", w.numel(), ptr(w), ptr(d), ptr(m), ptr(v), int(batch), int(t), float(lr), float(beta1),
-         float(beta2), float(eps), float(decay), int(apply_decay), _stream())
+    _run("pxh_adam_update", _tensor(w).numel(), w, d, m, v, int(batch), int(t), float(lr), float(beta1),
+         float(beta2), float(eps), float(decay), int(apply_decay))
 
 
 def _pointer_table(tensors):
@@ -494,9 +515,8 @@ def sgd_update_multi(ws, ds, batch, lr, momentum, decay=0.0, apply_decay=None):
 
 def sgd_update(w, d, batch, lr, momentum, decay=0.0, apply_decay=False):
     """include/ConvLayer.h:309-311 of the reference for one parameter tensor."""
-    _chk_all(w, d)
-    call("pxh_sgd_update", w.numel(), ptr(w), ptr(d), int(batch), float(lr), float(momentum), float(decay),
-         int(bool(apply_decay)), _stream())
+    _run("pxh_sgd_update", _tensor(w).numel(), w, d, int(batch), float(lr), float(momentum), float(decay),
+         int(bool(apply_decay)))
 
 
 class TensorTable:
@@ -562,8 +582,7 @@ def rescale_clip_multi(xs, threshold=0.0, clip=0.0, norms=None):
 
 def rescale_clip(x, threshold=0.0, clip=0.0, norm_out=None):
     """Gradient rescale to a norm threshold, then clamp (include/Layer.h:385-397 of the reference)."""
-    _chk_all(x, norm_out)
-    call("pxh_rescale_clip", ptr(x), x.numel(), float(threshold), float(clip), ptr(norm_out), None, 0, _stream())
+    _run("pxh_rescale_clip", x, _tensor(x).numel(), float(threshold), float(clip), norm_out, None, 0)
 
 
 def norm_groups_like(x):
@@ -625,14 +644,13 @@ def yolo_detections_append(predictions, batch, masks, anchors, classes, width, h
                            threshold, order_base, records, count, image_width=0, image_height=0):
     """Adds the detections of one more head behind those already in `records` (an int32 tensor
     [capacity, 8] on the device); `count` is the device counter both heads share."""
-    _chk_all(predictions)
     _chk(records, torch.int32, "records")
     _chk(count, torch.int32, "count")
     m, m_count, m_keep = _ints(masks)
     a, a_count, a_keep = _ints(anchors)
-    call("pxh_yolo_detections_append", ptr(predictions), batch, m, m_count, a, a_count // 2,
+    _run("pxh_yolo_detections_append", predictions, batch, m, m_count, a, a_count // 2,
          classes, width, height, net_width, net_height, int(image_width), int(image_height), float(threshold),
-         int(order_base), ptr(records), int(records.shape[0]), ptr(count), _stream())
+         int(order_base), ptr(records), int(records.shape[0]), ptr(count))
 
 
 def nms(records, count, batch, classes, threshold, workspace=None):
