@@ -1582,9 +1582,9 @@ __global__ __launch_bounds__(kBlock) void yolo_heads_patch_kernel(PatchHeadsArgs
 }  // namespace all_heads
 
 // ---------------------------------------------------------------- detections
-// Thresholded compaction of a decoded head (include/YoloLayer.h:601-698): one lane per slot; a slot
-// whose objectness passes walks its class rows, and all lanes of a workgroup that found detections
-// in the same class step reserve their output places with one atomic between them: the counter is
+// Thresholded compaction of a decoded head (include/YoloLayer.h:601-698): one lane per slot, then a wave
+// per slot whose objectness passes or, where many pass, each on its lane; the hits of a workgroup (in the
+// same class step) reserve their output places with one atomic between them: the counter is
 // one address for the whole grid, takes about 15 ns per atomic, and at one atomic per wave that
 // was most of the kernel's time when half the slots pass.  The records carry their position in the
 // reference's emission order, so sorting by it restores that order.
