@@ -480,10 +480,18 @@ __device__ __forceinline__ RescalePlan rescale_plan(const double2* partial, int 
     __shared__ double sums[kBlock / kWave];
     __shared__ double tops[kBlock / kWave];
     double s = 0.0, top = 0.0;
-    for (int j = threadIdx.x; j < partials; j += kBlock) {
-        const double2 p = partial[j];
-        s += p.x;
-        top = fmax(top, p.y);
+    // four partials of a thread in flight together: at most kNormBlocks of them are one trip to memory
+    constexpr int kLoads = kNormBlocks / kBlock;
+    for (int base = threadIdx.x; base < partials; base += kLoads * kBlock) {
+        double2 p[kLoads];
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) p[u] = partial[min(base + u * kBlock, partials - 1)];
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) {
+            const bool valid = base + u * kBlock < partials;
+            s += valid ? p[u].x : 0.0;
+            top = fmax(top, valid ? p[u].y : 0.0);
+        }
     }
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) {
@@ -505,16 +513,11 @@ __device__ __forceinline__ RescalePlan rescale_plan(const double2* partial, int 
     return plan_from_totals(total, peak, threshold, clip);
 }
 
-// x = clamp(factor * x); leaves without touching the tensor when there is nothing to do.  The grid
-// is the reduction's capped one and strides over the tensor.
+// Workgroup `block`'s share of x = clamp(factor * x).
 template<int V, bool NT, typename Sink = NoSink>
-__device__ __forceinline__ void rescale_walk(float* x, size_t n_vec, const double2* partial, int partials,
-                                             uint32_t block, uint32_t blocks, float threshold, float clip,
-                                             float* norm_out, const Sink& sink = Sink{})
+__device__ __forceinline__ void rescale_share(float* x, size_t n_vec, const RescalePlan& plan, uint32_t block, uint32_t blocks,
+                                              float clip, const Sink& sink = Sink{})
 {
-    const RescalePlan plan = rescale_plan(partial, partials, threshold, clip);
-    if (norm_out && block == 0 && threadIdx.x == 0) *norm_out = plan.norm;
-    if (!plan.work) return;
     const float factor = plan.factor;
     const size_t per_step = static_cast<size_t>(kBlock) * V * kNormLoads;
     for (size_t base = static_cast<size_t>(block) * per_step; base < n_vec;
@@ -547,6 +550,18 @@ __device__ __forceinline__ void rescale_walk(float* x, size_t n_vec, const doubl
             }
         }
     }
+}
+
+// x = clamp(factor * x); leaves without touching the tensor when there is nothing to do.  The grid
+// is the reduction's capped one and strides over the tensor.
+template<int V, bool NT, typename Sink = NoSink>
+__device__ __forceinline__ void rescale_walk(float* x, size_t n_vec, const double2* partial, int partials,
+                                             uint32_t block, uint32_t blocks, float threshold, float clip,
+                                             float* norm_out, const Sink& sink = Sink{})
+{
+    const RescalePlan plan = rescale_plan(partial, partials, threshold, clip);
+    if (norm_out && block == 0 && threadIdx.x == 0) *norm_out = plan.norm;
+    if (plan.work) rescale_share<V, NT>(x, n_vec, plan, block, blocks, clip, sink);
 }
 
 template<int V, bool NT>
@@ -938,20 +953,32 @@ __global__ __launch_bounds__(kBlock) void table_sumsq_kernel(TableView t)
     else sumsq_walk<4, false>(r.stream[0], r.n, block, blocks, out);
 }
 
-__global__ __launch_bounds__(kBlock) void table_rescale_kernel(TableView t, float threshold, float clip, float* norms)
+// A workgroup takes `per` of the norm pass's shares one after the other.  What a share costs where nothing changes -- the
+// tensor is found, its partials are added up again -- is paid once for those of one tensor; where something does change
+// there are still four workgroups to a compute unit.  7706 shares of the 222 tensors of YOLOv3: 15.1 us with a workgroup for
+// each, 10.8 with four shares to one and its partials in one trip.
+__global__ __launch_bounds__(kBlock) void table_rescale_kernel(TableView t, float threshold, float clip, float* norms,
+                                                               uint32_t shares, uint32_t per)
 {
     __shared__ uint32_t firsts[kMaxTableTensors + 1];
-    const int i = table_tensor_of_block(t.first_norm_block, t.count, blockIdx.x, firsts);
-    const TensorRecord r = t.records[i];
-    const uint32_t block = blockIdx.x - firsts[i], blocks = firsts[i + 1] - firsts[i];
-    const double2* mine = t.partial + firsts[i];
-    float* norm_out = norms ? norms + i : nullptr;
-    if (!r.norm_vector)
-        rescale_walk<1, false>(r.stream[0], r.n, mine, static_cast<int>(blocks), block, blocks, threshold, clip, norm_out);
-    else if (r.n * 4 >= kStreamingBytes)
-        rescale_walk<4, true>(r.stream[0], r.n, mine, static_cast<int>(blocks), block, blocks, threshold, clip, norm_out);
-    else
-        rescale_walk<4, false>(r.stream[0], r.n, mine, static_cast<int>(blocks), block, blocks, threshold, clip, norm_out);
+    uint32_t share = blockIdx.x * per;
+    const uint32_t end = min(share + per, shares);
+    int i = table_tensor_of_block(t.first_norm_block, t.count, share, firsts);
+    for (; share < end; ++i) {
+        const TensorRecord r = t.records[i];
+        const uint32_t blocks = firsts[i + 1] - firsts[i], last = min(end, firsts[i + 1]);
+        const double2* mine = t.partial + firsts[i];
+        const RescalePlan plan = rescale_plan(mine, static_cast<int>(blocks), threshold, clip);
+        if (norms && share == firsts[i] && threadIdx.x == 0) norms[i] = plan.norm;
+        for (; share < last; ++share) {
+            if (!plan.work) continue;
+            const uint32_t block = share - firsts[i];
+            if (!r.norm_vector) rescale_share<1, false>(r.stream[0], r.n, plan, block, blocks, clip);
+            else if (r.n * 4 >= kStreamingBytes) rescale_share<4, true>(r.stream[0], r.n, plan, block, blocks, clip);
+            else rescale_share<4, false>(r.stream[0], r.n, plan, block, blocks, clip);
+        }
+        __syncthreads();       // the sums of the next tensor's plan go where this one's were
+    }
 }
 
 struct AdamStepOp {
@@ -1669,8 +1696,10 @@ int pxh_rescale_clip_table(const pxh_tensor_table* table, float threshold, float
     hipLaunchKernelGGL(table_sumsq_kernel, dim3(table->norm_blocks), dim3(kBlock), 0, s, table->view);
     int rc = check_launch("pxh_rescale_clip_table");
     if (rc) return rc;
-    hipLaunchKernelGGL(table_rescale_kernel, dim3(table->norm_blocks), dim3(kBlock), 0, s, table->view, threshold, clip,
-                       norms);
+    const uint32_t shares = table->norm_blocks;
+    const uint32_t per = shares >= 4 * kNormBlocks ? 4 : shares >= 2 * kNormBlocks ? 2 : 1;
+    hipLaunchKernelGGL(table_rescale_kernel, dim3(grid_for(shares, per)), dim3(kBlock), 0, s, table->view, threshold, clip,
+                       norms, shares, per);
     return check_launch("pxh_rescale_clip_table");
 }
 

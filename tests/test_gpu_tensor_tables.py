@@ -115,6 +115,32 @@ def test_rescale_clip_table_leaves_every_tensor_as_the_single_call_does(ops, thr
         assert_bit_exact(host(a_), host(b_), "second rescale, tensor %d" % i)
 
 
+# Shares of the launch behind the norms: one to a workgroup below 2048, two, four from 4096 on; a last workgroup that is not
+# full, workgroups that end one tensor and begin others.
+@pytest.mark.parametrize("big", [2, 3, 6])
+def test_rescale_clip_table_by_shares(ops, big):
+    import torch
+    sizes = [5, 1027]
+    for k in range(big):
+        sizes += [3 << 20 | 4 * k, 4096, 9 + k, 3 * 4096 + 4]
+    g = torch.Generator(device="cuda")
+    g.manual_seed(6900 + big)
+    many = [torch.empty(n, device="cuda").normal_(0.0, 0.01 * (1 + i % 7), generator=g) for i, n in enumerate(sizes)]
+    one = [t.clone() for t in many]
+    table = ops.TensorTable([many])
+    norms = torch.zeros(table.count, device="cuda")
+    for threshold, clip in ((1e9, 1e9), (40.0, 0.0), (30.0, 0.05)):
+        table.rescale_clip(threshold, clip, norms)
+        want = []
+        for t in one:
+            norm = torch.zeros(1, device="cuda")
+            ops.rescale_clip(t, threshold, clip, norm)
+            want.append(float(norm))
+        assert host(norms).tolist() == want
+        for i, (a_, b_) in enumerate(zip(many, one)):
+            assert torch.equal(a_, b_), "tensor %d of %d values" % (i, sizes[i])
+
+
 def test_table_of_a_whole_model_and_edge_cases(ops):
     import torch
     from pixienn_amd import capi
