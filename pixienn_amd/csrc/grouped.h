@@ -49,6 +49,23 @@ __device__ __forceinline__ uint32_t take_ticket(uint32_t* counter, uint32_t& sha
     return shared;
 }
 
+// A workgroup's way through the shares, from number to number below `all`, as one of its threads sees it.  `wg` is that
+// thread's side of the workgroup: sync() is its barrier, ask() has one thread take the next number into the word that next()
+// reads.  share(number) answers whether it has asked already, behind barriers of its own that follow the reading of
+// `number`; where it has not, a wave may still have to read the word, and only a barrier tells that none has.
+template<typename Workgroup, typename Share>
+__host__ __device__ __forceinline__ void walk_shares(Workgroup& wg, uint32_t number, uint32_t all, Share&& share)
+{
+    while (number < all) {
+        if (!share(number)) {
+            wg.sync();
+            wg.ask();
+        }
+        wg.sync();       // the number is there; and the next share reuses the workgroup's LDS
+        number = wg.next();
+    }
+}
+
 __device__ __forceinline__ uint64_t canonical_word(double v)
 {
     const uint64_t bits = __double_as_longlong(v);

@@ -198,6 +198,17 @@ __device__ __forceinline__ void grouped_rescale_member(const ResidentBwdArgs& a,
     }
 }
 
+// The numbers of a workgroup (walk_shares): taken one by one, or, where a channel has one member and nobody waits, a grid
+// apart.
+struct ShareNumbers {
+    uint32_t* counter;      // null: a grid apart
+    uint32_t& taken;
+    uint32_t number;
+    __device__ __forceinline__ void sync() const { __syncthreads(); }
+    __device__ __forceinline__ void ask() const { if (counter && threadIdx.x == 0) taken = atomicAdd(counter, 1u); }
+    __device__ __forceinline__ uint32_t next() { return number = counter ? taken : number + gridDim.x; }
+};
+
 // The first launch of a clipped backward and the one behind it share the work as those of resident_bwd.hip do.
 template<int ACT, int V, int R, int L, int MODE>
 __global__ __launch_bounds__(kGroupThreads, L > 0 ? 4 : 6) void bn_grouped_bwd_kernel(ResidentBwdArgs a, GroupGeom gg)
@@ -223,18 +234,18 @@ __global__ __launch_bounds__(kGroupThreads, L > 0 ? 4 : 6) void bn_grouped_bwd_k
         if (all >= 2 * gridDim.x && blockIdx.x >= gridDim.x / 2) head_start();
         number = take_ticket(tickets, taken);
     }
-    while (number < all) {
+    const auto share = [&](uint32_t mine) {
         uint32_t c, member;
-        gg.by_members.divmod(__builtin_amdgcn_readfirstlane(number), c, member);      // the same in every lane
+        gg.by_members.divmod(__builtin_amdgcn_readfirstlane(mine), c, member);      // the same in every lane
         if (MODE != kRedo || !a.channel_done[c]) {
             grouped_bwd_member<ACT, V, R, L, MODE>(a, gg, c, member, taken, factor, limit);
-        } else {
-            if (factor != 1.0f) grouped_rescale_member<V, R>(a, gg, c, member, factor);
-            if (gg.members > 1 && threadIdx.x == 0) taken = atomicAdd(tickets, 1u);
+            return true;
         }
-        __syncthreads();       // the next share reuses the workgroup's LDS
-        number = gg.members > 1 ? taken : number + gridDim.x;
-    }
+        if (factor != 1.0f) grouped_rescale_member<V, R>(a, gg, c, member, factor);
+        return false;
+    };
+    ShareNumbers numbers{ gg.members > 1 ? tickets : nullptr, taken, number };
+    walk_shares(numbers, number, all, share);
 }
 
 __global__ __launch_bounds__(kBlock) void empty_words_kernel(uint64_t* words, uint32_t count, uint32_t* tickets)
