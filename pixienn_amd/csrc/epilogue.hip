@@ -831,30 +831,27 @@ ClippedRegions clipped_regions(void* ws, int batch, int channels, int spatial)
     return r;
 }
 
-constexpr int kResidentPlaces = 256;                  // of the workgroups that have a compute unit to themselves
 constexpr size_t kGroupScalars = 7u << 20;
+constexpr int kGroupAlone = 512;
 
 // The groups of a backward (members 0: none).  A plain call and a clipped one take the same form, so that they agree to
 // the bit where nothing is rescaled or clamped, and what they exchange has to fit the workspaces they ask for.
 //
-// `per_thread` is what a workgroup of 1024 lanes would hold of a channel (0: more than it can).  Where it can, one such
-// workgroup per channel is as fast or faster when the channels fill its places: 256 channels of more than kResidentVectors
-// vectors a lane (figures at the kernel; 16 x 192 x 76^2 47 us against 54 in groups, 16 x 320 x 76^2 89 against 80, mish 140
-// against 98), up to 512 of fewer (16 x 384 x 38^2 22.3, 22.6), or any with an exponential to compute.  Odd planes, whose
-// values come one at a time, gain only past the last-level cache's easy reach and with a gradient that is a select:
+// `per_thread` is what a workgroup of 1024 lanes would hold of a channel (0: more than it can).  Where it can, a plain call
+// needs no workspace, and callers on several streams may pass none: groups that exchange something are not for those slices
+// (16 x 128 x 76^2: 37 us where groups would take 33, mish 66 and 47).  A group of one member exchanges nothing, and from
+// kGroupAlone channels on, two to a compute unit, it is ahead (16 x 512 x 38^2: 29 -> 27 us; 16 x 384 x 38^2 22.3, 22.6), except
+// where an exponential has to be computed (37 -> 41).  Odd planes, whose values come one at a time, gain only where the
+// tensors are large and the gradient is a select; the line lies between the first two of
 // 6 x 72 x 135 x 77 25 -> 27 us, 8 x 96 x 135 x 77 41 -> 37, 32 x 64 x 75^2 48 -> 41; mish 35 -> 41, 54 -> 55, 65 -> 62.
 GroupPlan grouped_backward(int batch, int channels, int spatial, bool vec, int per_thread, int activation)
 {
     const size_t total = static_cast<size_t>(batch) * channels * spatial;
     if (!vec && (per_thread || !selects(activation) || total < kGroupScalars)) return GroupPlan{};
-    if (per_thread > kResidentVectors) {
-        const int rounds = (channels + kResidentPlaces - 1) / kResidentPlaces;
-        if (channels * 8 > rounds * kResidentPlaces * 5) return GroupPlan{};
-    } else if (per_thread && (!selects(activation) || channels < 2 * kResidentPlaces)) {
-        return GroupPlan{};
-    }
+    if (per_thread && (!selects(activation) || channels < kGroupAlone)) return GroupPlan{};
     for (const size_t workgroups: { kGroupFill, static_cast<size_t>(1) }) {
         const GroupPlan p = group_plan(batch, channels, spatial, vec, workgroups);
+        if (per_thread && p.members > 1) return GroupPlan{};
         if (p.members <= 1 ||
             (group_bytes(channels, p.members, kSumWords, false) <= workspace_bytes(batch, channels, spatial) &&
              group_figure_bytes(channels) + group_bytes(channels, p.members, kFirstWords, true) + 256 <=
@@ -1183,28 +1180,26 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
     if (!small && !pre_activation) group = grouped_backward(batch, channels, spatial, rvec, per_thread, activation);
     if (group.members) {
         const bool exchanges = group.members > 1;
-        if (exchanges && !cs.on) {
+        if (!cs.on && !per_thread) {
             rc = resolve_workspace(workspace, workspace_bytes_given, workspace_bytes(batch, channels, spatial), &ws, s);
-            if (rc && !per_thread) return rc;
-            if (rc) group.members = 0;      // the other form needs no workspace: what it was given is not looked at
+            if (rc) return rc;
         }
-        if (group.members) {
-            GroupGeom g = group_geom(group, batch, channels, spatial);
-            if (exchanges) {
-                rc = start_exchange(who, g, static_cast<char*>(ws) + (cs.on ? group_figure_bytes(channels) : 0), cs.on ? kFirstWords : kSumWords, cs.on, s);
-                if (rc) return rc;
-            }
-            if (exchanges && cs.on) {
-                // no sums: the members' words hold them
-                char* const base = reinterpret_cast<char*>(region.channel_sums);
-                region.channel_before = reinterpret_cast<float2*>(base);
-                region.channel_done = reinterpret_cast<int*>(base + static_cast<size_t>(channels) * sizeof(float2));
-            }
-            const ResidentBwdArgs r{ BackwardArgs{ delta, x, nullptr, mean, var, scale, bias }, scale_updates,
-                                     bias_updates, mean_delta, var_delta, g.g, region.channel_norm, region.channel_sums,
-                                     region.channel_before, region.channel_done, clip };
-            return launch_grouped_backward(who, r, g, cs.on, rvec, activation, s);
+        GroupGeom g = group_geom(group, batch, channels, spatial);
+        if (exchanges) {
+            rc = start_exchange(who, g, static_cast<char*>(ws) + (cs.on ? group_figure_bytes(channels) : 0),
+                                cs.on ? kFirstWords : kSumWords, cs.on, s);
+            if (rc) return rc;
         }
+        if (exchanges && cs.on) {
+            // no sums: the members' words hold them
+            char* const base = reinterpret_cast<char*>(region.channel_sums);
+            region.channel_before = reinterpret_cast<float2*>(base);
+            region.channel_done = reinterpret_cast<int*>(base + static_cast<size_t>(channels) * sizeof(float2));
+        }
+        const ResidentBwdArgs r{ BackwardArgs{ delta, x, nullptr, mean, var, scale, bias }, scale_updates,
+                                 bias_updates, mean_delta, var_delta, g.g, region.channel_norm, region.channel_sums,
+                                 region.channel_before, region.channel_done, clip };
+        return launch_grouped_backward(who, r, g, cs.on, rvec, activation, s);
     }
     if (per_thread || small) {
         if (!cs.on && (!per_thread || (!rvec && per_thread > kResidentVectors))) {

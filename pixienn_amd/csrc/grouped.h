@@ -1,5 +1,5 @@
-// The one-launch training passes for slices that one workgroup cannot hold: a channel's slice is shared by the
-// workgroups of a group, which exchange their sums inside the launch.
+// The one-launch training passes for slices that one workgroup of 1024 lanes cannot hold: a channel's slice is shared by the
+// workgroups of a group, which exchange their sums inside the launch.  (Groups of one workgroup: where grouped_backward says.)
 #pragma once
 
 #include "resident.h"

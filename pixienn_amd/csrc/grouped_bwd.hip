@@ -16,11 +16,8 @@ namespace {
 //   4 x 16 x 416^2      52 ->  33    59 ->  38       65 ->  48    72 ->  54
 //   2 x 32 x 320^2      33 ->  25    40 ->  30       44 ->  37    50 ->  43
 //   2 x 32 x 160^2      17 ->  13    23 ->  17       24 ->  19    29 ->  24
-// and against one workgroup of 1024 lanes a channel (the limits are grouped_backward's):
-//   16 x 128 x 76^2     37 ->  33    43 ->  38       66 ->  47    72 ->  53
+// and, a group of one member, against one workgroup of 1024 lanes a channel (the limits are grouped_backward's):
 //   16 x 512 x 38^2     29 ->  27    34 ->  31       37 ->  41    45 ->  46
-//   16 x 256 x 76^2     61 ->  63    69 ->  67       82 ->  78    89 ->  85
-//   16 x 256 x 38^2     16 ->  23    20 ->  28       22 ->  33    27 ->  40
 // Loads kept in flight over fewer than two steps, or over four (spills), are slower.
 //
 // One member's share of channel c; `factor` and `limit` are the plan's (kRedo only).  It keeps d' = delta * act'(pre) in

@@ -104,3 +104,25 @@ def test_shared_slices_on_two_streams(ops):
         for layer, expected in zip(layers, want):
             for got, w in zip(layer.results(), expected):
                 assert_bit_exact(got, w, "two streams")
+
+
+# Slices that a workgroup of 1024 lanes holds: a plain call needs no workspace and never looks at the one it is given, so it
+# leaves the same bits whatever that is, and a clipped call that changes nothing leaves them too.
+@pytest.mark.parametrize("shape", [(9, 160, 3644), (1, 512, 24800), (4, 512, 4112)], ids=str)
+def test_slices_of_one_workgroup_need_no_workspace(ops, shape):
+    import torch
+    N, C, HW = shape
+    layer = Layer(ops, torch, 9300, (N, C, HW, 1))
+    layer.run(100.0)                       # statistics to go by
+    outcomes = []
+    for workspace in (None, torch.zeros(4, device="cuda"), layer.workspace):
+        d, su, bu = layer.delta.clone(), torch.ones(C, device="cuda"), torch.ones(C, device="cuda")
+        ops.bn_act_backward(d, layer.x, layer.mean, layer.var, layer.scale, layer.bias, su, bu, "leaky", workspace=workspace)
+        outcomes.append([host(t) for t in (d, su, bu)])
+    d, su, bu = layer.delta.clone(), torch.ones(C, device="cuda"), torch.ones(C, device="cuda")
+    ops.bn_act_backward_clipped(d, layer.x, layer.mean, layer.var, layer.scale, layer.bias, su, bu, "leaky", 1e6, 100.0,
+                                workspace=layer.workspace)
+    outcomes.append([host(t) for t in (d, su, bu)])
+    for outcome in outcomes[1:]:
+        for got, want in zip(outcome, outcomes[0]):
+            assert_bit_exact(got, want, "workspace")
