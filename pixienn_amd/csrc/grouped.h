@@ -14,6 +14,9 @@ constexpr uint64_t kNotThere = ~0ull;
 constexpr int kFirstWords = 4;      // sums A and B, the squares, the largest magnitude
 constexpr int kSumWords = 2;
 
+// Next numbers of the first launch and of the second, and whether a wait of the first gave up.
+constexpr int kLost = 2, kTickets = 3;
+
 struct GroupGeom {
     ResidentGeom g;
     uint32_t items;         // vectors (or values) of a channel's slice
@@ -23,7 +26,8 @@ struct GroupGeom {
     FastDiv by_members;
     uint64_t* words;        // [channel][member][kFirstWords or kSumWords]; null with one member
     uint64_t* redo_words;   // [channel][member][kSumWords], of a clipped backward's second launch
-    uint32_t* tickets;      // [2]
+    uint32_t* tickets;      // [kTickets]
+    uint32_t looks;         // at a word that is not there yet, before a member goes on without it
 };
 
 __device__ __forceinline__ float* at_byte(float* p, uint32_t bytes)
@@ -89,15 +93,17 @@ __device__ __forceinline__ void leave_figures(uint64_t* channel_words, uint32_t 
 }
 
 // The figures of all members in every thread, added up in an order of the members alone (the last of four: the largest).
-// The bound on the looks makes the exit unconditional; it is seconds.
+// The bound on the looks makes the exit unconditional (kLooks: seconds).  Where it was reached, what is missing was never
+// formed: every figure is a NaN and the answer is false, in every thread.
 template<int WORDS>
-__device__ __forceinline__ void collect_figures(const uint64_t* channel_words, uint32_t members, double (&figures)[WORDS])
+__device__ __forceinline__ bool collect_figures(const uint64_t* channel_words, uint32_t members, uint32_t most_looks,
+                                                double (&figures)[WORDS])
 {
     __shared__ double theirs[kGroupThreads];
     const uint32_t t = threadIdx.x;
     if (t < members * WORDS) {
         uint64_t word = __hip_atomic_load(channel_words + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        for (uint32_t looks = 1u << 22; word == kNotThere && looks; --looks) {
+        for (uint32_t looks = most_looks; word == kNotThere && looks; --looks) {
             __builtin_amdgcn_s_sleep(1);
             word = __hip_atomic_load(channel_words + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
@@ -106,12 +112,18 @@ __device__ __forceinline__ void collect_figures(const uint64_t* channel_words, u
     __syncthreads();
     // a lane per member in every wave
     const uint32_t lane = t & (kWave - 1);
+    bool missing = false;
 #pragma unroll
     for (int w = 0; w < WORDS; ++w) {
         const double v = lane < members ? theirs[lane * WORDS + w] : 0.0;
+        missing = missing || static_cast<uint64_t>(__double_as_longlong(v)) == kNotThere;
         if (w < 3) figures[w] = wave_sum(v);
         else figures[w] = static_cast<double>(wave_max(static_cast<float>(v)));
     }
+    if (!__any(missing)) return true;
+#pragma unroll
+    for (int w = 0; w < WORDS; ++w) figures[w] = __longlong_as_double(0x7FF8000000000000ll);
+    return false;
 }
 
 // ---- the rules
@@ -122,6 +134,9 @@ constexpr uint32_t kGroupShare = 8;
 
 constexpr uint32_t kGroupItems = 12 * kGroupThreads;      // vectors that a member holds, or four times as many values
 constexpr size_t kGroupFill = 512;
+
+constexpr uint32_t kLooks = 1u << 22;
+uint32_t group_looks();      // kLooks, or what a test has set
 
 // Workgroups of these launches that the current device runs at once.
 uint32_t group_places();
@@ -154,7 +169,7 @@ inline GroupGeom group_geom(const GroupPlan& p, int batch, int channels, int spa
 {
     return GroupGeom{ resident_geom(batch, channels, spatial), p.items, p.span, p.members,
                       static_cast<uint32_t>(channels - 1) * static_cast<uint32_t>(spatial), FastDiv(p.members), nullptr, nullptr,
-                      nullptr };
+                      nullptr, group_looks() };
 }
 
 // Bytes of the words of `count` members, and of everything a launch (with `redo`: and the one behind it) exchanges.

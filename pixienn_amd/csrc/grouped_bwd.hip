@@ -1,5 +1,6 @@
 // Batch-norm training backward in one launch where a group of workgroups shares a channel's slice.
 #include "grouped.h"
+#include "pixienn_hip_test.h"
 
 #include <atomic>
 
@@ -117,14 +118,20 @@ __device__ __forceinline__ void grouped_bwd_member(const ResidentBwdArgs& a, con
     uint64_t* const words = (MODE == kRedo ? gg.redo_words : gg.words) + static_cast<size_t>(c) * gg.members * kWords;
     if (gg.members > 1) leave_figures<kWords>(words, member, figures);
     early_terms();
+    bool whole = true;
     if (gg.members > 1) {
-        collect_figures<kWords>(words, gg.members, figures);
+        whole = collect_figures<kWords>(words, gg.members, gg.looks, figures);
         // The next share's number, by a thread that does not finish the channel.  Not before the others' figures are
         // there: until then it could be the number of a member that this one waits for.
         if (threadIdx.x == T - 1) next_ticket = atomicAdd(gg.tickets + (MODE == kRedo ? 1 : 0), 1u);
     }
     bool within = true;
     if constexpr (MODE == kFirst) {
+        if (!whole) {
+            // (not NaNs into the share, as in the other passes: the clamp of the second launch would make numbers of them)
+            if (threadIdx.x == 0) __hip_atomic_store(gg.tickets + kLost, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return;
+        }
         const float lim = a.clip.clip;
         within = !(lim > 0.0f) || (figures[3] <= static_cast<double>(lim) && figures[2] == figures[2]);
     }
@@ -183,7 +190,8 @@ __device__ __forceinline__ void grouped_rescale_member(const ResidentBwdArgs& a,
     if (member != 0) return;
     double figures[kFirstWords];
     if (gg.members > 1) {
-        collect_figures<kFirstWords>(gg.words + static_cast<size_t>(c) * gg.members * kFirstWords, gg.members, figures);
+        collect_figures<kFirstWords>(gg.words + static_cast<size_t>(c) * gg.members * kFirstWords, gg.members, gg.looks,
+                                     figures);
     } else {
         const double2 sums = a.channel_sums[c];
         figures[0] = sums.x;
@@ -192,6 +200,28 @@ __device__ __forceinline__ void grouped_rescale_member(const ResidentBwdArgs& a,
     if (threadIdx.x == 0) {
         rescale_finished_channel(figures[0], figures[1], static_cast<double>(factor), a.channel_before[c], c, a.b.var, a.b.scale, a.scale_updates,
                                  a.bias_updates, a.mean_delta, a.var_delta);
+    }
+}
+
+// What the second launch leaves where a wait of the first gave up: NaNs everywhere.
+template<int V>
+__device__ __forceinline__ void leave_lost(const ResidentBwdArgs& a, const GroupGeom& gg, uint32_t all)
+{
+    const float nan = __int_as_float(0x7FC00000);
+    if (blockIdx.x == 0 && threadIdx.x == 0 && a.clip.norm_out) *a.clip.norm_out = nan;
+    Pack<V> nans;
+#pragma unroll
+    for (int q = 0; q < V; ++q) nans.v[q] = nan;
+    for (uint32_t number = blockIdx.x; number < all; number += gridDim.x) {
+        uint32_t c, member;
+        gg.by_members.divmod(number, c, member);
+        const uint32_t begin = member * gg.span, end = min(gg.items, begin + gg.span);
+        for (uint32_t i = begin + threadIdx.x; i < end; i += kGroupThreads) st<V, true>(a.b.delta, gg.g.at(c, i * V), nans);
+        if (member == 0 && threadIdx.x == 0) {
+            a.bias_updates[c] = a.scale_updates[c] = nan;
+            if (a.mean_delta) a.mean_delta[c] = nan;
+            if (a.var_delta) a.var_delta[c] = nan;
+        }
     }
 }
 
@@ -212,7 +242,9 @@ __global__ __launch_bounds__(kGroupThreads, L > 0 ? 4 : 6) void bn_grouped_bwd_k
 {
     __shared__ uint32_t taken;
     float factor = 1.0f, limit = 0.0f;
+    const uint32_t all = static_cast<uint32_t>(gg.g.channels) * gg.members;
     if constexpr (MODE == kRedo) {
+        if (gg.members > 1 && gg.tickets[kLost]) return leave_lost<V>(a, gg, all);
         const ClipPlan plan = clip_plan_from<kGroupThreads>(a.channel_norm, gg.g.channels, a.clip.threshold, a.clip.clip);
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             *a.clip.plan = plan;
@@ -222,7 +254,6 @@ __global__ __launch_bounds__(kGroupThreads, L > 0 ? 4 : 6) void bn_grouped_bwd_k
         factor = plan.factor;
         limit = plan.clip;
     }
-    const uint32_t all = static_cast<uint32_t>(gg.g.channels) * gg.members;
     uint32_t* const tickets = gg.tickets + (MODE == kRedo ? 1 : 0);
     uint32_t number = blockIdx.x;
     if (gg.members > 1) {
@@ -245,11 +276,13 @@ __global__ __launch_bounds__(kGroupThreads, L > 0 ? 4 : 6) void bn_grouped_bwd_k
     walk_shares(numbers, number, all, share);
 }
 
+std::atomic<uint32_t> looks_of_a_wait{ kLooks };
+
 __global__ __launch_bounds__(kBlock) void empty_words_kernel(uint64_t* words, uint32_t count, uint32_t* tickets)
 {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i < count) words[i] = kNotThere;
-    if (i < 2) tickets[i] = 0;
+    if (i < kTickets) tickets[i] = 0;
 }
 
 }  // namespace
@@ -268,6 +301,8 @@ uint32_t group_places()
     }
     return places;
 }
+
+uint32_t group_looks() { return looks_of_a_wait.load(std::memory_order_relaxed); }
 
 int start_exchange(const char* who, GroupGeom& g, void* at, int words, bool redo, hipStream_t s)
 {
@@ -307,3 +342,5 @@ int launch_grouped_backward(const char* who, const ResidentBwdArgs& r, const Gro
 }
 
 }  // namespace pxh
+
+extern "C" unsigned pxh_debug_group_looks(unsigned looks) { return pxh::looks_of_a_wait.exchange(looks); }

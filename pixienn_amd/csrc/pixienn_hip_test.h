@@ -30,6 +30,10 @@ void* pxh_debug_library_workspace(size_t bytes);
  * the order of a few fp32 additions.  Returns 0. */
 int pxh_debug_yolo_tuning(int form, int lanes_per_slot, int head_workers);
 
+/* How often a workgroup of the batch-norm backward that waits for the sums of others looks before it goes on without them;
+ * returns the previous value.  With the usual value (2^22) that is seconds, and nobody has to. */
+unsigned pxh_debug_group_looks(unsigned looks);
+
 /* A kernel with no arithmetic to speak of that reads `reads` and writes `writes` streams of n floats each
  * (1 <= reads, writes <= 4; every pointer 16-byte aligned; n % 4 == 0), launched as the library launches
  * its streaming kernels: what that mix of reads and writes costs on the device whatever is computed.

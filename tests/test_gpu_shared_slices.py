@@ -126,3 +126,39 @@ def test_slices_of_one_workgroup_need_no_workspace(ops, shape):
     for outcome in outcomes[1:]:
         for got, want in zip(outcome, outcomes[0]):
             assert_bit_exact(got, want, "workspace")
+
+
+# A member that stops looking (never, within seconds) before the others' figures are there says so in everything it leaves:
+# each value is the right one or a NaN, and none is the delta as it came.
+@pytest.mark.parametrize("clip", [None, 100.0, 3.0])
+def test_a_wait_that_gives_up_leaves_nothing_plausible(ops, clip):
+    import torch
+    from pixienn_amd import capi
+    lib = capi.load()
+    layer = Layer(ops, torch, 9400, (16, 6, 152, 152))
+    layer.run(100.0)                       # statistics to go by
+    norm = torch.zeros(1, device="cuda")
+
+    def backward():
+        layer.d.copy_(layer.delta); layer.su.zero_(); layer.bu.zero_(); norm.zero_()
+        args = (layer.d, layer.x, layer.mean, layer.var, layer.scale, layer.bias, layer.su, layer.bu, "leaky")
+        if clip is None:
+            ops.bn_act_backward(*args, workspace=layer.workspace)
+        else:
+            ops.bn_act_backward_clipped(*args, 1e6, clip, norm, workspace=layer.workspace)
+        return [host(t) for t in (layer.d, layer.su, layer.bu, norm)]
+
+    want = backward()
+    before = lib.pxh_debug_group_looks(0)
+    try:
+        got = backward()
+    finally:
+        lib.pxh_debug_group_looks(before)
+    lost = [np.isnan(g) for g in got]
+    for g, w, nan in zip(got, want, lost):
+        assert_bit_exact(g[~nan], w[~nan], "what was left")
+    # where the second launch has nothing else to do, it sees to it that all is lost where anything is
+    if clip == 100.0:
+        assert len({bool(n) for nan in lost for n in nan.reshape(-1)}) == 1
+    for again, w in zip(backward(), want):
+        assert_bit_exact(again, w, "the next call")
