@@ -89,8 +89,9 @@ __device__ __forceinline__ ChannelStats channel_stats(double s1, double s2, floa
 struct __attribute__((aligned(16))) ClipPlan {
     float norm, factor, clip;
     int work;       // 0: no value of the delta changes; kChanges: some do; | kClamps: and the clamp may move one
+                    // | kBeyond: and some were beyond the clamp as they came (in the channels that a first launch left)
 };
-enum { kChanges = 1, kClamps = 2 };
+enum { kChanges = 1, kClamps = 2, kBeyond = 4 };
 
 // The plan from `count` partial (sum of squares, largest magnitude) pairs, added in an order that
 // depends on THREADS alone: every workgroup that forms it arrives at the same one.  All THREADS
@@ -141,7 +142,8 @@ __device__ __forceinline__ ClipPlan clip_plan_from(const double2* part, int coun
         peak = fmaxf(peak, plan_tops[w]);
     }
     const RescalePlan r = plan_from_totals(total, peak, threshold, clip);
-    return ClipPlan{ r.norm, r.factor, clip, (r.work ? kChanges : 0) | (r.clamps ? kClamps : 0) };
+    const bool beyond = clip > 0.0f && (!(peak <= clip) || total != total);
+    return ClipPlan{ r.norm, r.factor, clip, (r.work ? kChanges : 0) | (r.clamps ? kClamps : 0) | (r.work && beyond ? kBeyond : 0) };
 }
 
 // What the clipped forms add to a launch: where the first pass leaves its norm partials, and the
