@@ -105,6 +105,7 @@ _TEST_HOOKS = {
     "pxh_debug_library_workspace": (P, [Z]),
     "pxh_debug_yolo_tuning": (I, [I, I, I]),
     "pxh_debug_group_looks": (ctypes.c_uint, [ctypes.c_uint]),
+    "pxh_debug_group_places": (ctypes.c_uint, [P]),
     "pxh_debug_stream_mix": (I, [I, I, Z, P, P, P]),
 }
 

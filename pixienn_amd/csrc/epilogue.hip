@@ -844,13 +844,14 @@ constexpr int kGroupAlone = 512;
 // where an exponential has to be computed (37 -> 41).  Odd planes, whose values come one at a time, gain only where the
 // tensors are large and the gradient is a select; the line lies between the first two of
 // 6 x 72 x 135 x 77 25 -> 27 us, 8 x 96 x 135 x 77 41 -> 37, 32 x 64 x 75^2 48 -> 41; mish 35 -> 41, 54 -> 55, 65 -> 62.
-GroupPlan grouped_backward(int batch, int channels, int spatial, bool vec, int per_thread, int activation)
+GroupPlan grouped_backward(int batch, int channels, int spatial, bool vec, int per_thread, int activation, hipStream_t s)
 {
     const size_t total = static_cast<size_t>(batch) * channels * spatial;
     if (!vec && (per_thread || !selects(activation) || total < kGroupScalars)) return GroupPlan{};
     if (per_thread && (!selects(activation) || channels < kGroupAlone)) return GroupPlan{};
+    const uint32_t places = group_places(s);
     for (const size_t workgroups: { kGroupFill, static_cast<size_t>(1) }) {
-        const GroupPlan p = group_plan(batch, channels, spatial, vec, workgroups);
+        const GroupPlan p = group_plan(batch, channels, spatial, vec, workgroups, places);
         if (per_thread && p.members > 1) return GroupPlan{};
         if (p.members <= 1 ||
             (group_bytes(channels, p.members, kSumWords, false) <= workspace_bytes(batch, channels, spatial) &&
@@ -1177,7 +1178,7 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
     }
     GroupPlan group{};
     // (a saved pre-activation is a third stream, which no register is left for)
-    if (!small && !pre_activation) group = grouped_backward(batch, channels, spatial, rvec, per_thread, activation);
+    if (!small && !pre_activation) group = grouped_backward(batch, channels, spatial, rvec, per_thread, activation, s);
     if (group.members) {
         const bool exchanges = group.members > 1;
         if (!cs.on && !per_thread) {
@@ -1199,7 +1200,7 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
         const ResidentBwdArgs r{ BackwardArgs{ delta, x, nullptr, mean, var, scale, bias }, scale_updates,
                                  bias_updates, mean_delta, var_delta, g.g, region.channel_norm, region.channel_sums,
                                  region.channel_before, region.channel_done, clip };
-        return launch_grouped_backward(who, r, g, cs.on, rvec, activation, s);
+        return launch_grouped_backward(who, r, g, group.places, cs.on, rvec, activation, s);
     }
     if (per_thread || small) {
         if (!cs.on && (!per_thread || (!rvec && per_thread > kResidentVectors))) {

@@ -44,8 +44,11 @@ __device__ __forceinline__ const float* at_byte(const float* p, uint32_t bytes)
 // The workgroups of a launch take numbers, and a channel's members have consecutive ones.  A workgroup waits only for
 // members of its own channel.  Those with lower numbers are running; of those with higher ones some may still have to
 // start, in the one channel whose numbers are not all taken.  Every workgroup of another channel finishes without them and
-// gives up its place, so they start as long as the device has more places than that one channel has waiting members, and
-// every wait ends.  kGroupShare below keeps a launch's waiting members to an eighth of the places of the device.
+// gives up its place, so they start as long as the stream has more places than waiting members hold.  A launch has fewer
+// waiting members than kGroupShare's part of the places (an eighth), so that up to eight launches may run at once on the
+// units of a stream's mask, beside anything that ends by itself.  More of them than that, less than that left by a kernel
+// that stays for seconds, units that the environment takes away without the runtime's knowledge, or two launches at once on
+// one workspace, which the interface forbids: there a wait may reach its bound (kLooks below).
 __device__ __forceinline__ uint32_t take_ticket(uint32_t* counter, uint32_t& shared)
 {
     __syncthreads();
@@ -139,15 +142,24 @@ constexpr size_t kGroupFill = 512;
 constexpr uint32_t kLooks = 1u << 22;
 uint32_t group_looks();      // kLooks, or what a test has set
 
-// Workgroups of these launches that the current device runs at once.
-uint32_t group_places();
+// Compute units of a stream: those of its mask (a bit each), or all of the device's where it has none.
+inline uint32_t units_of_mask(const uint32_t* mask, int words, uint32_t units)
+{
+    uint32_t enabled = 0;
+    for (int w = 0; w < words; ++w) enabled += static_cast<uint32_t>(__builtin_popcount(mask[w]));
+    return enabled && enabled < units ? enabled : units;
+}
+
+// Workgroups of these launches that the current device runs at once for a stream.
+uint32_t group_places(hipStream_t s);
 
 struct GroupPlan {
     uint32_t items, span, members;      // members 0: another form takes the call
+    uint32_t places;
 };
 
-// How a slice is split over workgroups that hold `per_member` vectors (or values) each.
-inline GroupPlan split_slice(size_t items, uint32_t per_member, size_t channels, size_t workgroups)
+// How a slice is split over workgroups that hold `per_member` vectors (or values) each, on a stream of `places`.
+inline GroupPlan split_slice(size_t items, uint32_t per_member, size_t channels, size_t workgroups, uint32_t places)
 {
     size_t least = (items + per_member - 1) / per_member;
     const size_t fill = (workgroups + channels - 1) / channels, shortest = items / (4 * kGroupThreads);
@@ -155,15 +167,15 @@ inline GroupPlan split_slice(size_t items, uint32_t per_member, size_t channels,
     if (least < more) least = more;
     const size_t span = ((items + least - 1) / least + kWave - 1) / kWave * kWave;
     const size_t members = (items + span - 1) / span;
-    if (members > kGroupMost || members * kGroupShare > group_places()) return GroupPlan{};
-    return GroupPlan{ static_cast<uint32_t>(items), static_cast<uint32_t>(span), static_cast<uint32_t>(members) };
+    if (members > kGroupMost || members * kGroupShare > places) return GroupPlan{};
+    return GroupPlan{ static_cast<uint32_t>(items), static_cast<uint32_t>(span), static_cast<uint32_t>(members), places };
 }
 
-inline GroupPlan group_plan(int batch, int channels, int spatial, bool vec, size_t workgroups)
+inline GroupPlan group_plan(int batch, int channels, int spatial, bool vec, size_t workgroups, uint32_t places)
 {
     const size_t per_channel = static_cast<size_t>(batch) * spatial;
     if (per_channel * channels >= 1ull << 30) return GroupPlan{};      // places are 32-bit byte offsets
-    return split_slice(vec ? per_channel / 4 : per_channel, vec ? kGroupItems : 4 * kGroupItems, channels, workgroups);
+    return split_slice(vec ? per_channel / 4 : per_channel, vec ? kGroupItems : 4 * kGroupItems, channels, workgroups, places);
 }
 
 inline GroupGeom group_geom(const GroupPlan& p, int batch, int channels, int spatial)
@@ -186,7 +198,7 @@ constexpr size_t kGroupLdsBytes = 64u << 10;
 // Places GroupGeom's buffers in `at` and queues the launch that empties them.
 int start_exchange(const char* who, GroupGeom& g, void* at, int words, bool redo, hipStream_t s);
 
-int launch_grouped_backward(const char* who, const ResidentBwdArgs& r, const GroupGeom& g, bool clipped, bool vec,
-                            int activation, hipStream_t s);
+int launch_grouped_backward(const char* who, const ResidentBwdArgs& r, const GroupGeom& g, uint32_t places, bool clipped,
+                            bool vec, int activation, hipStream_t s);
 
 }  // namespace pxh

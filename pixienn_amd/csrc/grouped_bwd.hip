@@ -341,19 +341,22 @@ __global__ __launch_bounds__(kBlock) void empty_words_kernel(uint64_t* words, ui
 
 }  // namespace
 
-uint32_t group_places()
+uint32_t group_places(hipStream_t s)
 {
-    // two to a compute unit (their LDS and registers); asked once for each device
+    // two to a compute unit (their LDS and registers); the device's units are asked for once, a stream's mask each time
     static std::atomic<uint32_t> known[16];
-    int device = 0, units = 0;
+    int device = 0, count = 0;
     if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 16) return 0;
-    uint32_t places = known[device].load(std::memory_order_relaxed);
-    if (places == 0) {
-        if (hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || units <= 0) return 0;
-        places = 2 * static_cast<uint32_t>(units);
-        known[device].store(places, std::memory_order_relaxed);
+    uint32_t units = known[device].load(std::memory_order_relaxed);
+    if (units == 0) {
+        if (hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || count <= 0) return 0;
+        units = static_cast<uint32_t>(count);
+        known[device].store(units, std::memory_order_relaxed);
     }
-    return places;
+    constexpr int kWords = 32;
+    uint32_t mask[kWords] = {};
+    if (hipExtStreamGetCUMask(s, kWords, mask) != hipSuccess) (void) hipGetLastError();
+    return 2 * units_of_mask(mask, kWords, units);
 }
 
 uint32_t group_looks() { return looks_of_a_wait.load(std::memory_order_relaxed); }
@@ -371,10 +374,10 @@ int start_exchange(const char* who, GroupGeom& g, void* at, int words, bool redo
     return check_launch(who);
 }
 
-int launch_grouped_backward(const char* who, const ResidentBwdArgs& r, const GroupGeom& g, bool clipped, bool vec,
-                            int activation, hipStream_t s)
+int launch_grouped_backward(const char* who, const ResidentBwdArgs& r, const GroupGeom& g, uint32_t places, bool clipped,
+                            bool vec, int activation, hipStream_t s)
 {
-    const uint32_t all = static_cast<uint32_t>(g.g.channels) * g.members, places = group_places();
+    const uint32_t all = static_cast<uint32_t>(g.g.channels) * g.members;
     int rc = PXH_OK;
     const auto launch = [&]<int ACT, int MODE>() {
         const dim3 grid(all < places ? all : places), block(kGroupThreads);
@@ -398,3 +401,5 @@ int launch_grouped_backward(const char* who, const ResidentBwdArgs& r, const Gro
 }  // namespace pxh
 
 extern "C" unsigned pxh_debug_group_looks(unsigned looks) { return pxh::looks_of_a_wait.exchange(looks); }
+
+extern "C" unsigned pxh_debug_group_places(void* stream) { return pxh::group_places(pxh::as_stream(stream)); }

@@ -34,6 +34,9 @@ int pxh_debug_yolo_tuning(int form, int lanes_per_slot, int head_workers);
  * returns the previous value.  With the usual value (2^22) that is seconds, and nobody has to. */
 unsigned pxh_debug_group_looks(unsigned looks);
 
+/* Workgroups of the batch-norm backward that exchange sums which the current device runs at once for `stream`. */
+unsigned pxh_debug_group_places(void* stream);
+
 /* A kernel with no arithmetic to speak of that reads `reads` and writes `writes` streams of n floats each
  * (1 <= reads, writes <= 4; every pointer 16-byte aligned; n % 4 == 0), launched as the library launches
  * its streaming kernels: what that mix of reads and writes costs on the device whatever is computed.

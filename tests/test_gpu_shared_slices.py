@@ -162,3 +162,12 @@ def test_a_wait_that_gives_up_leaves_nothing_plausible(ops, clip):
         assert len({bool(n) for nan in lost for n in nan.reshape(-1)}) == 1
     for again, w in zip(backward(), want):
         assert_bit_exact(again, w, "the next call")
+
+
+def test_streams_without_a_mask_have_the_whole_device():
+    import torch
+    from pixienn_amd import capi
+    lib = capi.load()
+    all_places = 2 * torch.cuda.get_device_properties(0).multi_processor_count
+    for stream in (torch.cuda.default_stream(), torch.cuda.Stream()):
+        assert lib.pxh_debug_group_places(stream.cuda_stream) == all_places
