@@ -6,6 +6,7 @@ failed call raises PxError.
 """
 import ctypes
 import os
+import sys
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libpixienn_hip.so")
@@ -124,36 +125,51 @@ class PxError(RuntimeError):
 _lib = None
 
 # The entry points that csrc/calls.cpp calls: name -> (callable that takes tensors for float buffers and answers None for a
-# call it does not make, which arguments are tensors).  Filled by load().
+# call it does not make, which arguments are tensors).  Filled by bind_calls().
 native = {}
 
 
 def load():
-    """Loads the built library; raises PxError when it has not been built."""
+    """Loads the built library; raises PxError when it has not been built.  Needs no torch; where that is imported, the
+    native calls are bound as well."""
     global _lib
-    if _lib is not None:
-        return _lib
-    if not os.path.exists(LIB_PATH):
-        raise PxError("libpixienn_hip.so is not built (%s); run `python -m pixienn_amd.build` "
-                      "or __graft_entry__.build()" % LIB_PATH)
-    lib = ctypes.CDLL(LIB_PATH)
-    for name, args in SIGNATURES.items():
-        fn = getattr(lib, name)
-        fn.argtypes = args
-        fn.restype = I
-    for name, (res, args) in list(_OTHER_RETURNS.items()) + list(_TEST_HOOKS.items()):
-        fn = getattr(lib, name)
-        fn.argtypes = args
-        fn.restype = res
+    if _lib is None:
+        if not os.path.exists(LIB_PATH):
+            raise PxError("libpixienn_hip.so is not built (%s); run `python -m pixienn_amd.build` "
+                          "or __graft_entry__.build()" % LIB_PATH)
+        lib = ctypes.CDLL(LIB_PATH)
+        for name, args in SIGNATURES.items():
+            fn = getattr(lib, name)
+            fn.argtypes = args
+            fn.restype = I
+        for name, (res, args) in list(_OTHER_RETURNS.items()) + list(_TEST_HOOKS.items()):
+            fn = getattr(lib, name)
+            fn.argtypes = args
+            fn.restype = res
+        _lib = lib
+    if not native and "torch" in sys.modules:
+        try:
+            bind_calls()
+        except PxError:
+            pass        # said by the first call that wants them
+    return _lib
+
+
+def bind_calls():
+    """Fills `native`.  The extension module is linked with torch's libraries, which are found once torch is imported."""
+    lib = _lib or load()
+    if native:
+        return
     try:
         from . import _calls
+    except ModuleNotFoundError as e:
+        raise PxError("pixienn_amd/_calls.so is not built (%s); run `python -m pixienn_amd.build` or "
+                      "__graft_entry__.build()" % e) from e
     except ImportError as e:
-        raise PxError("the calls of %s are not built (%s); run `python -m pixienn_amd.build` or "
-                      "__graft_entry__.build()" % (LIB_PATH, e)) from e
-    for name in _calls.names():
-        native[name] = _calls.bind(name, ctypes.cast(getattr(lib, name), ctypes.c_void_p).value)
-    _lib = lib
-    return lib
+        raise PxError("pixienn_amd/_calls.so does not load (%s): torch has to be imported before it, and be the one that it "
+                      "was built with" % e) from e
+    native.update({name: _calls.bind(name, ctypes.cast(getattr(lib, name), ctypes.c_void_p).value)
+                   for name in _calls.names()})
 
 
 def declared_symbols():

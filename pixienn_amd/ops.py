@@ -55,8 +55,8 @@ def _chk_all(*ts):
 
 def _run(name, *args):
     """call() on the current stream, with tensors themselves, or None, for the float buffers among the arguments."""
-    if capi._lib is None:
-        capi.load()
+    if not capi.native:
+        capi.bind_calls()
     make, tensors = capi.native[name]
     try:
         stream = _raw_stream(_current_device())

@@ -1,6 +1,9 @@
 """The native calls of the C ABI against the ctypes binding: what they cover, what they leave to it, and that both refuse
 the same.  No device: every call here ends at an argument check."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -42,3 +45,41 @@ def test_what_is_no_tensor_of_the_device_is_named(bad, message):
               lambda: ops.rescale_clip(bad), lambda: ops.sgd_update(bad, good, 1, 0.1, 0.9)):
         with pytest.raises(capi.PxError, match=message):
             f()
+
+
+def child(source):
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    proc = subprocess.run([sys.executable, "-c", source], cwd=root, capture_output=True, text=True, timeout=300)
+    assert proc.returncode == 0, proc.stderr
+
+
+def test_the_binding_loads_without_torch():
+    child("""
+import sys
+from pixienn_amd import capi
+assert capi.load().pxh_abi_version() == 2 and capi.call_raw("pxh_axpy", 4, 1.0, None, None, None) != 0
+assert "torch" not in sys.modules and not capi.native
+from pixienn_amd import ops
+try:
+    ops.axpy(1.0, 7, 7)
+except capi.PxError as e:
+    assert "torch.Tensor expected" in str(e)
+ops.torch.zeros(1)
+capi.bind_calls()
+assert "pxh_axpy" in capi.native
+""")
+
+
+def test_a_missing_extension_is_named_by_the_first_call_that_wants_it():
+    child("""
+import sys, torch
+sys.modules["pixienn_amd._calls"] = None
+from pixienn_amd import capi, ops
+assert capi.load().pxh_abi_version() == 2 and not capi.native
+try:
+    ops.axpy(1.0, torch.zeros(4), torch.zeros(4))
+except capi.PxError as e:
+    assert "not built" in str(e)
+else:
+    raise SystemExit("no error")
+""")
