@@ -850,6 +850,7 @@ GroupPlan grouped_backward(int batch, int channels, int spatial, bool vec, int p
     if (!vec && (per_thread || !selects(activation) || total < kGroupScalars)) return GroupPlan{};
     if (per_thread && (!selects(activation) || channels < kGroupAlone)) return GroupPlan{};
     const uint32_t places = group_places(s);
+    // (as few members as hold the slice where the words of more would not fit: up to three channels of a few thousand vectors)
     for (const size_t workgroups: { kGroupFill, static_cast<size_t>(1) }) {
         const GroupPlan p = group_plan(batch, channels, spatial, vec, workgroups, places);
         if (per_thread && p.members > 1) return GroupPlan{};

@@ -32,6 +32,19 @@ int main()
                     check(static_cast<size_t>(p.span) * (p.members - 1) < items, "every member has items", items, channels, places);
                 }
 
+    // the splits that the shapes of tests/test_gpu_shared_slices.py are chosen for
+    const struct { size_t items, channels; uint32_t per_member, members, span; } named[] = {
+        { 4097, 3, kGroupItems, 2, 2112 }, { 6144, 2, kGroupItems, 3, 2048 }, { 17521, 5, kGroupItems, 8, 2240 },
+        { 24579, 2, kGroupItems, 12, 2112 }, { 133120, 8, kGroupItems, 64, 2112 }, { 133120, 7, kGroupItems, 0, 0 },
+        { 98304, 32, kGroupItems, 16, kGroupItems }, { 24579, 130, kGroupItems, 5, 4928 }, { 4112, 512, kGroupItems, 1, 4160 },
+        { 83160, 96, 4 * kGroupItems, 6, 13888 }, { 180000, 41, 4 * kGroupItems, 13, 13888 },
+        { 393215, 32, 4 * kGroupItems, 16, 4 * kGroupItems },
+    };
+    for (const auto& n: named) {
+        const GroupPlan p = split_slice(n.items, n.per_member, n.channels, kGroupFill, 512);
+        check(p.members == n.members && p.span == n.span, "the split of a named slice", n.items, n.channels, 512);
+    }
+
     uint32_t mask[4] = {};
     check(units_of_mask(mask, 4, 256) == 256, "no mask", 0, 0, 0);
     mask[0] = 0x0F0Fu;

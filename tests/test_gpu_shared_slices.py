@@ -10,13 +10,14 @@ from util import F, assert_bit_exact, gpu, host
 
 pytestmark = pytest.mark.gpu
 
-# vectors of a slice: 4097 (the first that the small forms leave), a member's 6144 and one more, a last member of one
-# wavefront, planes that end inside a share, 64 members and one more (three launches), 130 channels of two rounds,
-# channels on both sides of five eighths of the places, 512 channels of one member
-VECTORS = [(1, 3, 16388), (4, 2, 6144), (1, 1, 24580), (3, 2, 32772), (7, 5, 10012), (16, 1, 98304), (16, 1, 98308),
-           (3, 130, 32772), (9, 160, 3644), (9, 161, 3644), (4, 512, 4112)]
-# values: of two streams' worth of odd planes, with and without a last share that is short
-SCALARS = [(8, 96, 10395), (32, 41, 5625), (1, 5, 1572863)]
+# vectors of a slice: 4097 (the first that the small forms leave) in two members; three members of 2048; planes that end
+# inside a share, in eight and in twelve; 64 members, the last of one wavefront, and 65 (three launches); members that are
+# full, sixteen of 6144; more shares than the device runs at once; 512 channels of one member.  How they are split is held by
+# tests/host/split_check.cpp.
+VECTORS = [(1, 3, 16388), (4, 2, 6144), (7, 5, 10012), (3, 2, 32772), (1, 8, 532480), (1, 7, 532480), (4, 32, 98304),
+           (3, 130, 32772), (4, 512, 4112)]
+# values of odd planes, past kGroupScalars: six members, thirteen, and sixteen that are full but for the last value
+SCALARS = [(8, 96, 10395), (32, 41, 5625), (1, 32, 393215)]
 
 
 @pytest.fixture(scope="module")
