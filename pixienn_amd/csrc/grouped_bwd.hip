@@ -287,8 +287,10 @@ struct ShareNumbers {
 
 // The first launch of a clipped backward and the one behind it share the work as those of resident_bwd.hip do.
 template<int ACT, int V, int R, int L, int MODE>
-__global__ __launch_bounds__(kGroupThreads, L > 0 ? 4 : 6) void bn_grouped_bwd_kernel(ResidentBwdArgs a, GroupGeom gg)
+__global__ __launch_bounds__(kGroupThreads, 4) void bn_grouped_bwd_kernel(ResidentBwdArgs a, GroupGeom gg)
 {
+    // two workgroups to a compute unit, which group_places() counts on: 128 registers a lane, and this LDS
+    static_assert(static_cast<size_t>(L) * V * 4 * kGroupThreads == kGroupLdsBytes);
     __shared__ uint32_t taken;
     float factor = 1.0f, limit = 0.0f;
     const uint32_t all = static_cast<uint32_t>(gg.g.channels) * gg.members;
