@@ -833,6 +833,7 @@ ClippedRegions clipped_regions(void* ws, int batch, int channels, int spatial)
 
 constexpr size_t kGroupScalars = 7u << 20;
 constexpr int kGroupAlone = 512;
+constexpr size_t kGroupFewest = 1u << 19, kGroupFewestSmooth = 1u << 20;
 
 // The groups of a backward (members 0: none).  A plain call and a clipped one take the same form, so that they agree to
 // the bit where nothing is rescaled or clamped, and what they exchange has to fit the workspaces they ask for.
@@ -844,9 +845,19 @@ constexpr int kGroupAlone = 512;
 // where an exponential has to be computed (37 -> 41).  Odd planes, whose values come one at a time, gain only where the
 // tensors are large and the gradient is a select; the line lies between the first two of
 // 6 x 72 x 135 x 77 25 -> 27 us, 8 x 96 x 135 x 77 41 -> 37, 32 x 64 x 75^2 48 -> 41; mish 35 -> 41, 54 -> 55, 65 -> 62.
+//
+// Small tensors (which the caches hold for the launches that read them twice) stay with those launches: a group's second one
+// costs them more where it has something to do.  Three or five launches -> groups, us: plain; clipped with nothing to change,
+// rescaled, and clamped throughout:
+//   2 x 16 x 104^2  leaky 12.0 -> 11.4; 17.6 -> 15.3, 17.6 -> 19.3, 20.1 -> 22.9   mish 16.1 -> 18.0; 21.4 -> 22.1, 21.5 -> 26.2, 27.2 -> 36.2
+//   2 x 16 x 160^2        13.5 -> 12.1; 18.8 -> 16.0, 18.8 -> 20.1, 21.7 -> 24.3        18.2 -> 18.8; 23.3 -> 23.1, 23.3 -> 27.3, 29.1 -> 37.7
+//   1 x 32 x 208^2        16.1 -> 12.9; 21.5 -> 16.8, 21.5 -> 21.2, 24.4 -> 25.7        22.0 -> 20.1; 27.2 -> 23.9, 27.3 -> 28.6, 33.8 -> 39.9
+//   4 x 32 x 208^2        28.2 -> 23.8; 34.9 -> 28.1, 35.0 -> 36.7, 42.8 -> 45.0        39.7 -> 34.9; 46.7 -> 40.0, 46.8 -> 48.6, 63.6 -> 69.2
+// From there on the usual call gains a tenth to a quarter; one that clamps gains from 16 x 64 x 152^2 on (121 -> 107).
 GroupPlan grouped_backward(int batch, int channels, int spatial, bool vec, int per_thread, int activation, hipStream_t s)
 {
     const size_t total = static_cast<size_t>(batch) * channels * spatial;
+    if (total < (selects(activation) ? kGroupFewest : kGroupFewestSmooth)) return GroupPlan{};
     if (!vec && (per_thread || !selects(activation) || total < kGroupScalars)) return GroupPlan{};
     if (per_thread && (!selects(activation) || channels < kGroupAlone)) return GroupPlan{};
     const uint32_t places = group_places(s);

@@ -34,8 +34,8 @@ int main()
 
     // the splits that the shapes of tests/test_gpu_shared_slices.py are chosen for
     const struct { size_t items, channels; uint32_t per_member, members, span; } named[] = {
-        { 4097, 3, kGroupItems, 2, 2112 }, { 6144, 2, kGroupItems, 3, 2048 }, { 17521, 5, kGroupItems, 8, 2240 },
-        { 24579, 2, kGroupItems, 12, 2112 }, { 133120, 8, kGroupItems, 64, 2112 }, { 133120, 7, kGroupItems, 0, 0 },
+        { 4097, 95, kGroupItems, 2, 2112 }, { 6144, 64, kGroupItems, 3, 2048 }, { 17521, 30, kGroupItems, 8, 2240 },
+        { 24579, 12, kGroupItems, 12, 2112 }, { 133120, 8, kGroupItems, 64, 2112 }, { 133120, 7, kGroupItems, 0, 0 },
         { 98304, 32, kGroupItems, 16, kGroupItems }, { 24579, 130, kGroupItems, 5, 4928 }, { 4112, 512, kGroupItems, 1, 4160 },
         { 83160, 96, 4 * kGroupItems, 6, 13888 }, { 180000, 41, 4 * kGroupItems, 13, 13888 },
         { 393215, 32, 4 * kGroupItems, 16, 4 * kGroupItems },

@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 # inside a share, in eight and in twelve; 64 members, the last of one wavefront, and 65 (three launches); members that are
 # full, sixteen of 6144; more shares than the device runs at once; 512 channels of one member.  How they are split is held by
 # tests/host/split_check.cpp.
-VECTORS = [(1, 3, 16388), (4, 2, 6144), (7, 5, 10012), (3, 2, 32772), (1, 8, 532480), (1, 7, 532480), (4, 32, 98304),
+VECTORS = [(1, 95, 16388), (4, 64, 6144), (7, 30, 10012), (3, 12, 32772), (1, 8, 532480), (1, 7, 532480), (4, 32, 98304),
            (3, 130, 32772), (4, 512, 4112)]
 # values of odd planes, past kGroupScalars: six members, thirteen, and sixteen that are full but for the last value
 SCALARS = [(8, 96, 10395), (32, 41, 5625), (1, 32, 393215)]
