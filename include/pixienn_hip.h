@@ -180,7 +180,9 @@ int pxh_bn_stats(const float* x, float* mean, float* var, int batch, int channel
  *   delta <- d''/sqrt(var+1e-5) + var_delta*2*(x-mean)/(N*HW) + mean_delta/(N*HW)   (in place)
  * x is the saved conv output (x_saved of the forward).  pre_activation may be NULL: it is then
  * recomputed from x exactly as the forward computed it.  mean_delta / var_delta are outputs
- * (nullable).  workspace as for the forward.
+ * (nullable).  workspace as for the forward.  Over large slices the workgroups of a channel wait for each other's sums (up to
+ * eight such calls may run at once on the units of their streams, beside work that ends by itself); a wait that is starved
+ * for seconds ends, and what could not be formed is then NaN.
  * Replaces gradient() + cudnnBatchNormalizationBackward, include/cuda/ConvLayer.h:315-338;
  * CPU semantics include/ConvLayer.h:244-252, src/BatchNorm.cpp:69-96. */
 int pxh_bn_act_backward(float* delta, const float* x, const float* pre_activation,
