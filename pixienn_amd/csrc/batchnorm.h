@@ -254,19 +254,26 @@ __device__ __forceinline__ void rescale_finished_channel(double sa, double sb, d
     if (var_delta) var_delta[c] = sum_ddx * (-.5f * powf(ve, -3.0f / 2.0f));
 }
 
+// dx from d' = delta * act'(pre)
+__device__ __forceinline__ float dx_value(float d, float x, const DxCoef& k)
+{
+    const float dd = d * k.f.scale;
+    const float xm = x - k.f.mean;
+    // src/CpuUtil.cpp:336-338 evaluated in double, stored as float
+    const double v = static_cast<double>(dd) * k.rroot + k.c2 * static_cast<double>(xm) + k.md_term;
+    return static_cast<float>(v);
+}
+
+// ... and from the delta itself
 template<int ACT>
-__device__ __forceinline__ float dx_value(float d, float x, float pre_in, bool recompute, const DxCoef& k)
+__device__ __forceinline__ float dx_of_delta(float d, float x, float pre_in, bool recompute, const DxCoef& k)
 {
     if constexpr (ACT != PXH_LINEAR) {
         float pre = pre_in;
         if (recompute) pre = affine(normalize(x, k.f), k.f);
         d = d * act_grad<ACT>(pre);
     }
-    const float dd = d * k.f.scale;
-    const float xm = x - k.f.mean;
-    // src/CpuUtil.cpp:336-338 evaluated in double, stored as float
-    const double v = static_cast<double>(dd) * k.rroot + k.c2 * static_cast<double>(xm) + k.md_term;
-    return static_cast<float>(v);
+    return dx_value(d, x, k);
 }
 
 }  // namespace pxh

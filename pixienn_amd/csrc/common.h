@@ -118,29 +118,34 @@ __device__ __forceinline__ float softplus_apply(float x)
     return logf(exp_before_one_plus(x) + 1.0f);
 }
 
+// num / den by the hardware's reciprocal (1 ulp) and one correction of the quotient by its remainder: within an ulp of the
+// quotient, mostly its rounded value, in five instructions where the compiler's division takes a dozen.  For den in
+// [1, 2^126): no scaling.
+__device__ __forceinline__ float quotient(float num, float den)
+{
+    const float r = __builtin_amdgcn_rcpf(den);
+    const float q = num * r;
+    return fmaf(fmaf(-q, den, num), r, q);
+}
+
+// 1 / (1 + exp(-x)) for the gradients.  Below -20 it is exp(x), and the other exponential would overflow further down;
+// exponentials below -110 are zero anyway (and infinities would make NaNs in the short form); a NaN stays one.
+__device__ __forceinline__ float sigmoid(float x)
+{
+    const bool low = x < -20.0f;
+    const float a = low ? x : -x;
+    const float e = exp_by_exp2(a < -110.0f ? -110.0f : a);
+    return low ? e : quotient(1.0f, 1.0f + e);
+}
+
 __device__ __forceinline__ float softplus_grad(float x)
 {
-    if (x > 20.0f) return 1.0f;
-    if (x < -20.0f) return expf(x);
-    return 1.0f / (1.0f + expf(-x));
+    return x > 20.0f ? 1.0f : sigmoid(x);
 }
 
-// tanh(softplus(x)) for |x| <= 20.  The CPU functor evaluates tanhf(logf(u)) with
-// u = float(expf(x) + 1); tanh(log u) = (u*u - 1)/(u*u + 1) exactly, and (u - 1) is exact in
-// fp32, so the same rounded u gives the same value to a few ulp with one exp and one division
-// instead of exp + log + tanh.
-__device__ __forceinline__ float tanh_softplus_from_exp(float e)
-{
-    const float u = e + 1.0f;
-    const float num = (u - 1.0f) * (u + 1.0f);
-    const float den = u * u + 1.0f;
-    return num / den;
-}
-
-__device__ __forceinline__ float tanh_softplus_mid(float x)
-{
-    return tanh_softplus_from_exp(exp_before_one_plus(x));
-}
+// tanh(softplus(x)) for |x| <= 20: the CPU functor evaluates tanhf(logf(u)) with u = float(expf(x) + 1);
+// tanh(log u) = (u*u - 1)/(u*u + 1) exactly, and (u - 1) is exact in fp32, so the same rounded u gives
+// the same value to a few ulp with one exp and one division instead of exp + log + tanh.
 
 // Forward mish: one exp (see exp_before_one_plus), the division as a hardware reciprocal and a
 // multiply (2 ulp), the two tails by selection.
@@ -157,19 +162,24 @@ __device__ __forceinline__ float mish_apply(float x)
     return x > 20.0f ? x : x * t;
 }
 
+// The gradient from one exp: e and u = 1 + e give both tanh(softplus) and the logistic e / (1 + e), the latter with what
+// u lost of e (what tanh(softplus) is formed from is the rounded u, as in the forward).  Two exponentials and two divisions
+// per value were what bound the backward of a smooth activation; us: 16 x 128 x 152^2 167 -> 146, 64 x 512 x 13^2 36 -> 25.5,
+// 16 x 256 x 76^2 with rescale + clip 87 -> 73; logistic and swish gain a twentieth.
+template<bool QUICK = false>
 __device__ __forceinline__ float mish_grad(float x)
 {
-    if (x > 20.0f) return 1.0f;              // (1 - 1*1)*1*x + 1
-    float tsp, gsp;
-    if (x < -20.0f) {
-        tsp = expf(x);
-        gsp = tsp;
-    } else {
-        tsp = tanh_softplus_mid(x);
-        gsp = 1.0f / (1.0f + expf(-x));
-    }
+    const float a = x < -110.0f ? -110.0f : x;      // as in sigmoid()
+    const float e = QUICK ? exp_by_exp2(a) : exp_before_one_plus(a);
+    const float u = e + 1.0f;
+    const float v = u - 1.0f;
+    const float mid = quotient(v * (u + 1.0f), u * u + 1.0f);
+    const float tsp = x < -20.0f ? e : mid;
+    const float r = __builtin_amdgcn_rcpf(u);
+    const float q = e * r;
+    const float gsp = fmaf(fmaf(-q, e - v, fmaf(-q, u, e)), r, q);
     const float gtsp = (1.0f - tsp * tsp) * gsp;
-    return x * gtsp + tsp;
+    return x > 20.0f ? 1.0f : x * gtsp + tsp;      // beyond 20: (1 - 1*1)*1*x + 1
 }
 
 template<int ACT>
@@ -222,18 +232,52 @@ __device__ __forceinline__ float act_grad(float x)
         float y = (x + 1.0f) / 2.0f;
         return 2.0f * (1.0f - y) * y;
     } else if constexpr (ACT == PXH_LOGISTIC) {
-        float y = 1.0f / (1.0f + expf(-x));
+        float y = sigmoid(x);
         return y * (1.0f - y);
     } else if constexpr (ACT == PXH_MISH) {
-        return mish_grad(x);
+        return mish_grad<false>(x);
     } else if constexpr (ACT == PXH_RELU) return x > 0.0f ? 1.0f : 0.0f;
     else if constexpr (ACT == PXH_SOFTPLUS) return softplus_grad(x);
     else if constexpr (ACT == PXH_SWISH) {
-        float val = 1.0f / (1.0f + expf(-1.0f * x));
+        float val = sigmoid(x);
         return x * val + 1.0f * val * (1.0f - x * val);
     } else {
         float y = tanhf(x);
         return 1.0f - y * y;
+    }
+}
+
+// V values at once: for mish one branch for the wave, as in act_apply_n, with the results of act_grad value by value.
+template<int ACT, int V>
+__device__ __forceinline__ void act_grad_n(const float (&pre)[V], float (&g)[V])
+{
+    if constexpr (ACT == PXH_MISH) {
+        bool any = false;
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+            g[k] = mish_grad<true>(pre[k]);
+            any = any | one_plus_exp_is_sensitive(pre[k]);
+        }
+        if (__ballot(any)) {
+#pragma unroll
+            for (int k = 0; k < V; ++k)
+                if (one_plus_exp_is_sensitive(pre[k])) g[k] = mish_grad<false>(pre[k]);
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < V; ++k) g[k] = act_grad<ACT>(pre[k]);
+    }
+}
+
+// d times the activation's gradient at pre, V values.
+template<int ACT, int V>
+__device__ __forceinline__ void times_grad(float (&d)[V], const float (&pre)[V])
+{
+    if constexpr (ACT != PXH_LINEAR) {
+        float g[V];
+        act_grad_n<ACT, V>(pre, g);
+#pragma unroll
+        for (int k = 0; k < V; ++k) d[k] = d[k] * g[k];
     }
 }
 

@@ -38,9 +38,8 @@ struct GradientOp {
     }
     template<int V, bool NT> __device__ void finish(size_t e, const Regs<V>& r) const
     {
-        Pack<V> o;
-#pragma unroll
-        for (int k = 0; k < V; ++k) o.v[k] = r.d.v[k] * act_grad<ACT>(r.x.v[k]);
+        Pack<V> o = r.d;
+        times_grad<ACT>(o.v, r.x.v);
         st<V, NT>(delta, e, o);
     }
 };
@@ -234,9 +233,9 @@ struct ShortcutBackwardOp {
     template<int V, bool NT> __device__ Pack<V> finish_value(size_t e, const Regs<V>& r) const
     {
         Pack<V> d = r.d, f, g;
+        if constexpr (ACT != PXH_LINEAR) times_grad<ACT>(d.v, r.p.v);
 #pragma unroll
         for (int k = 0; k < V; ++k) {
-            if constexpr (ACT != PXH_LINEAR) d.v[k] = d.v[k] * act_grad<ACT>(r.p.v[k]);
             const float add = beta * d.v[k];
             const float ga = alpha * d.v[k];
             if constexpr (FIRST) {

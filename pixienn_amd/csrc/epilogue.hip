@@ -499,26 +499,29 @@ __global__ __launch_bounds__(kBlock) void bwd_partial_kernel(BackwardArgs a, Red
         for (int u = 0; u < kLoads; ++u) {
             const int off = seg0 + (u * kWave + lane) * V;
             if (off < seg1) {
+                if constexpr (MODE != kPlain) {
+#pragma unroll
+                    for (int q = 0; q < V; ++q) {
+                        const float dv = d[u].v[q];
+                        if constexpr (MODE == kFirst) {
+                            fq += dv * dv;
+                            peak = fmaxf(peak, fabsf(dv));
+                        } else {
+                            d[u].v[q] = rescaled_clipped(dv, factor, limit);
+                        }
+                    }
+                }
+                if constexpr (ACT != PXH_LINEAR) {
+                    if (recompute) {
+#pragma unroll
+                        for (int q = 0; q < V; ++q) pv[u].v[q] = affine(normalize(xv[u].v[q], k), k);
+                    }
+                    times_grad<ACT>(d[u].v, pv[u].v);
+                }
 #pragma unroll
                 for (int q = 0; q < V; ++q) {
-                    float dv = d[u].v[q];
-                    if constexpr (MODE == kFirst) {
-                        fq += dv * dv;
-                        peak = fmaxf(peak, fabsf(dv));
-                    }
-                    if constexpr (MODE == kRedo) {
-                        dv = rescaled_clipped(dv, factor, limit);
-                        d[u].v[q] = dv;
-                    }
-                    if constexpr (ACT != PXH_LINEAR) {
-                        float pre;
-                        if (recompute) pre = affine(normalize(xv[u].v[q], k), k);
-                        else pre = pv[u].v[q];
-                        dv = dv * act_grad<ACT>(pre);
-                        d[u].v[q] = dv;
-                    }
-                    fa += dv;
-                    if constexpr (BN) fb += dv * (xv[u].v[q] - k.mean);
+                    fa += d[u].v[q];
+                    if constexpr (BN) fb += d[u].v[q] * (xv[u].v[q] - k.mean);
                 }
                 if constexpr (WRITE && (ACT != PXH_LINEAR || MODE == kRedo)) {
                     if (ACT != PXH_LINEAR || changes) st<V, NT>(a.delta, base + off, d[u]);
@@ -679,16 +682,22 @@ __global__ __launch_bounds__(kBlock) void bn_dx_kernel(DxArgs a)
     const bool crosses = !(r + 3 < hw);
     if (!__ballot(crosses)) {
         const DxCoef k = a.coef[c];
+        if constexpr (ACT != PXH_LINEAR) {
+            if (recompute) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) out.v[j] = dx_value<ACT>(din.v[j], xin.v[j], pin.v[j], recompute, k);
+                for (int j = 0; j < 4; ++j) pin.v[j] = affine(normalize(xin.v[j], k.f), k.f);
+            }
+            times_grad<ACT>(din.v, pin.v);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) out.v[j] = dx_value(din.v[j], xin.v[j], k);
     } else if (hw >= 4) {
         // one boundary per vector at most: constants selected per element, one copy of the arithmetic
         // for the wave (see epilogue_fwd_kernel)
         const DxCoef k0 = a.coef[c];
         DxCoef k1 = k0;
         if (crosses) k1 = a.coef[c + 1 == a.by_channels.d ? 0 : c + 1];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        const auto constants = [&](int j) {
             const bool here = r + j < hw;
             DxCoef k;
             k.f.mean = here ? k0.f.mean : k1.f.mean;
@@ -699,8 +708,20 @@ __global__ __launch_bounds__(kBlock) void bn_dx_kernel(DxArgs a)
             k.rroot = here ? k0.rroot : k1.rroot;
             k.c2 = here ? k0.c2 : k1.c2;
             k.md_term = here ? k0.md_term : k1.md_term;
-            out.v[j] = dx_value<ACT>(din.v[j], xin.v[j], pin.v[j], recompute, k);
+            return k;
+        };
+        if constexpr (ACT != PXH_LINEAR) {
+            if (recompute) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const DxCoef k = constants(j);
+                    pin.v[j] = affine(normalize(xin.v[j], k.f), k.f);
+                }
+            }
+            times_grad<ACT>(din.v, pin.v);
         }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) out.v[j] = dx_value(din.v[j], xin.v[j], constants(j));
     } else {
         uint32_t rr = r, cc = c;
 #pragma unroll
@@ -709,7 +730,7 @@ __global__ __launch_bounds__(kBlock) void bn_dx_kernel(DxArgs a)
                 rr = 0;
                 cc = cc + 1 == a.by_channels.d ? 0 : cc + 1;
             }
-            out.v[j] = dx_value<ACT>(din.v[j], xin.v[j], pin.v[j], recompute, a.coef[cc]);
+            out.v[j] = dx_of_delta<ACT>(din.v[j], xin.v[j], pin.v[j], recompute, a.coef[cc]);
             ++rr;
         }
     }
@@ -733,7 +754,7 @@ __global__ __launch_bounds__(kBlock) void bn_dx_scalar_kernel(DxArgs a)
     Pack<1> d;
     d.v[0] = a.delta[e];
     apply_plan<CLIPPED, 1>(a, d);
-    a.delta[e] = dx_value<ACT>(d.v[0], a.x[e], pre, recompute, a.coef[c]);
+    a.delta[e] = dx_of_delta<ACT>(d.v[0], a.x[e], pre, recompute, a.coef[c]);
 }
 
 constexpr size_t align256(size_t b) { return (b + 255) & ~static_cast<size_t>(255); }

@@ -79,10 +79,17 @@ __device__ __forceinline__ void grouped_bwd_member(const ResidentBwdArgs& a, con
                 peak = fmaxf(peak, fabsf(t));
             }
             if constexpr (MODE == kRedo) t = rescaled_clipped(t, factor, limit);
-            if constexpr (ACT != PXH_LINEAR) {
-                const float s = t * act_grad<ACT>(affine(normalize(x[r].v[q], k), k));
-                t = valid ? s : 0.0f;
-            }
+            d[r].v[q] = t;
+        }
+        if constexpr (ACT != PXH_LINEAR) {
+            float pre[V];
+#pragma unroll
+            for (int q = 0; q < V; ++q) pre[q] = affine(normalize(x[r].v[q], k), k);
+            times_grad<ACT>(d[r].v, pre);
+        }
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+            const float t = ACT == PXH_LINEAR || valid ? d[r].v[q] : 0.0f;
             d[r].v[q] = t;
             const float u = t * (x[r].v[q] - k.mean);
             va += t;
@@ -162,7 +169,7 @@ __device__ __forceinline__ void grouped_bwd_member(const ResidentBwdArgs& a, con
         const Pack<V> xv = r < X ? x[r] : lds[(r - X) * T];
         Pack<V> out;
 #pragma unroll
-        for (int q = 0; q < V; ++q) out.v[q] = dx_value<PXH_LINEAR>(d[r].v[q], xv.v[q], 0.0f, false, kd);
+        for (int q = 0; q < V; ++q) out.v[q] = dx_value(d[r].v[q], xv.v[q], kd);
         return out;
     };
 #pragma unroll

@@ -117,16 +117,18 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
         const uint32_t e = element(r);
         return a.g.at(c, e < a.g.per_channel ? e : 0u);
     };
-    // one value of the delta on its way to d': the norm's share of it first (kFirst), or the plan's
+    // a vector of the delta on its way to d': the norm's share of it first (kFirst), or the plan's
     // rescale + clamp (kRedo), then the activation's gradient
-    const auto prepared = [&](float t, float pre, bool valid) {
-        if constexpr (MODE == kFirst) {
-            if constexpr (!kWide && !kSmall) fq += valid ? t * t : 0.0f;
-            peak = fmaxf(peak, valid ? fabsf(t) : 0.0f);
+    const auto prepare = [&](Pack<V>& t, const Pack<V>& pre, bool valid) {
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+            if constexpr (MODE == kFirst) {
+                if constexpr (!kWide && !kSmall) fq += valid ? t.v[q] * t.v[q] : 0.0f;
+                peak = fmaxf(peak, valid ? fabsf(t.v[q]) : 0.0f);
+            }
+            if constexpr (MODE == kRedo) t.v[q] = rescaled_clipped(t.v[q], factor, limit);
         }
-        if constexpr (MODE == kRedo) t = rescaled_clipped(t, factor, limit);
-        if constexpr (ACT != PXH_LINEAR) t = t * act_grad<ACT>(pre);
-        return t;
+        times_grad<ACT>(t.v, pre.v);
     };
     if constexpr (kSmall) {
         // every load of the slice at once, no branch around them; the pre-activations four steps at a time
@@ -161,12 +163,16 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
                 float va = 0.0f, vb = 0.0f, vq = 0.0f;
 #pragma unroll
                 for (int q = 0; q < V; ++q) {
-                    const float raw = valid ? d[r].v[q] : 0.0f;
-                    const float t = valid ? prepared(raw, ACT != PXH_LINEAR ? pv[i].v[q] : 0.0f, valid) : 0.0f;
+                    d[r].v[q] = valid ? d[r].v[q] : 0.0f;
+                    vq += d[r].v[q] * d[r].v[q];
+                }
+                prepare(d[r], pv[i], valid);
+#pragma unroll
+                for (int q = 0; q < V; ++q) {
+                    const float t = valid ? d[r].v[q] : 0.0f;
                     d[r].v[q] = t;
                     va += t;
                     vb += valid ? t * (kept[r].v[q] - k.mean) : 0.0f;
-                    vq += raw * raw;
                 }
                 fa += static_cast<double>(va);
                 fb += static_cast<double>(vb);
@@ -177,13 +183,12 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
         // delta * f'(pre) in dv, and the step's share of the sums
         const auto take = [&](int r, Pack<V>& dv, const Pack<V>& xv, const Pack<V>& pv) {
             const bool valid = element(r) < a.g.per_channel;
+            prepare(dv, pv, valid);
+            if constexpr (!kWide) {
 #pragma unroll
-            for (int q = 0; q < V; ++q) {
-                const float t = prepared(dv.v[q], ACT != PXH_LINEAR ? pv.v[q] : 0.0f, valid);
-                dv.v[q] = t;
-                if constexpr (!kWide) {
-                    fa += valid ? t : 0.0f;
-                    fb += valid ? t * (xv.v[q] - k.mean) : 0.0f;
+                for (int q = 0; q < V; ++q) {
+                    fa += valid ? dv.v[q] : 0.0f;
+                    fb += valid ? dv.v[q] * (xv.v[q] - k.mean) : 0.0f;
                 }
             }
         };
@@ -255,19 +260,18 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
                 const Pack<V> xv = ld<V, false>(a.b.x, where);
                 Pack<V> pv;
                 if constexpr (ACT != PXH_LINEAR) {
-                    if (!recompute) pv = ld<V, true>(a.b.pre, where);
+                    if (!recompute) {
+                        pv = ld<V, true>(a.b.pre, where);
+                    } else {
+#pragma unroll
+                        for (int q = 0; q < V; ++q) pv.v[q] = affine(normalize(xv.v[q], k), k);
+                    }
                 }
+                prepare(dv, pv, true);
 #pragma unroll
                 for (int q = 0; q < V; ++q) {
-                    float pre = 0.0f;
-                    if constexpr (ACT != PXH_LINEAR) {
-                        if (recompute) pre = affine(normalize(xv.v[q], k), k);
-                        else pre = pv.v[q];
-                    }
-                    const float t = prepared(dv.v[q], pre, true);
-                    dv.v[q] = t;
-                    fa += t;
-                    fb += t * (xv.v[q] - k.mean);
+                    fa += dv.v[q];
+                    fb += dv.v[q] * (xv.v[q] - k.mean);
                 }
                 if (r < R) d[r < R ? r : 0] = dv;
                 else *resident_lds_slot<V, R>(resident_lds, r) = dv;
@@ -310,7 +314,7 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
                 const Pack<V> dv = r < R ? d[r < R ? r : 0] : *resident_lds_slot<V, R>(resident_lds, r);
                 Pack<V> out;
 #pragma unroll
-                for (int q = 0; q < V; ++q) out.v[q] = dx_value<PXH_LINEAR>(dv.v[q], xv[i].v[q], 0.0f, false, kd);
+                for (int q = 0; q < V; ++q) out.v[q] = dx_value(dv.v[q], xv[i].v[q], kd);
                 if (element(r) < a.g.per_channel) st<V, true>(a.b.delta, place(r), out);
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -328,7 +332,7 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
                 const Pack<V> dv = r < R ? d[r < R ? r : 0] : *resident_lds_slot<V, R>(resident_lds, r);
                 Pack<V> out;
 #pragma unroll
-                for (int q = 0; q < V; ++q) out.v[q] = dx_value<PXH_LINEAR>(dv.v[q], xv.v[q], 0.0f, false, kd);
+                for (int q = 0; q < V; ++q) out.v[q] = dx_value(dv.v[q], xv.v[q], kd);
                 st<V, true>(a.b.delta, where, out);
             }
         }
