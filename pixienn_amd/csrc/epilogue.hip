@@ -879,7 +879,7 @@ GroupPlan grouped_backward(int batch, int channels, int spatial, bool vec, int p
 {
     const size_t total = static_cast<size_t>(batch) * channels * spatial;
     if (total < (selects(activation) ? kGroupFewest : kGroupFewestSmooth)) return GroupPlan{};
-    if (!vec && (per_thread || !selects(activation) || total < kGroupScalars)) return GroupPlan{};
+    if (!vec && (!selects(activation) || total < kGroupScalars)) return GroupPlan{};
     if (per_thread && (!selects(activation) || channels < kGroupAlone)) return GroupPlan{};
     const uint32_t places = group_places(s);
     // (as few members as hold the slice where the words of more would not fit: up to three channels of a few thousand vectors)
@@ -930,10 +930,7 @@ struct Residual {
 };
 
 // BN training forward + activation.  `get_workspace(need, &ws)` is asked for the `need` bytes of the three-launch form
-// where the shape takes that, and where it takes a scalar one-launch form of more than kResidentVectors values per lane
-// or a small form below kResidentChannels: those use none of it, but their limits are measured ones that may move, also
-// between activations, and a workspace that is too small for a shape is refused on either side of them (as is growth in a
-// capture).
+// where the shape takes that, and where it takes a one-launch form whose limits may move (asks_for_workspace).
 template<typename GetWorkspace>
 int bn_train_forward(const char* who, const float* x, float* y, float* pre_activation, float* x_saved, float* x_norm,
                      float* mean, float* var, float* rolling_mean, float* rolling_var, const float* scale,
@@ -950,18 +947,16 @@ int bn_train_forward(const char* who, const float* x, float* y, float* pre_activ
     {
         const bool vec = spatial % 4 == 0 && aligned16(x) && aligned16(y) && aligned16(pre_activation) &&
                          aligned16(x_saved) && aligned16(x_norm) && aligned16(res.from);
-        const int per_thread = resident_vectors(batch, channels, spatial, vec, activation, false);
-        const uint32_t small = small_slice(batch, channels, spatial, vec, activation, false);
-        if (per_thread || small) {
+        if (const ResidentForm form = resident_form(batch, channels, spatial, vec, activation, false)) {
             const ResidentFwdArgs r{ x, y, pre_activation, x_saved, x_norm, mean, var, rolling_mean, rolling_var,
                                      scale, bias, resident_geom(batch, channels, spatial), res.from, res.alpha, res.beta };
-            if (!per_thread || (!vec && per_thread > kResidentVectors)) {
+            if (asks_for_workspace(batch, channels, spatial, vec)) {
                 // not used, but still the caller's part of this shape (see above)
                 void* unused;
                 rc = get_workspace(workspace_bytes(batch, channels, spatial), &unused);
                 if (rc) return rc;
             }
-            return launch_resident_forward(who, r, vec, per_thread, small, activation, s);
+            return launch_resident_forward(who, r, form, activation, s);
         }
     }
     void* ws;
@@ -1198,8 +1193,8 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
     if (rc) return rc;
     hipStream_t s = as_stream(stream);
     const bool rvec = spatial % 4 == 0 && aligned16(delta) && aligned16(x) && aligned16(pre_activation);
-    const int per_thread = resident_vectors(batch, channels, spatial, rvec, activation, true);
-    const uint32_t small = small_slice(batch, channels, spatial, rvec, activation, true);
+    const ResidentForm form = resident_form(batch, channels, spatial, rvec, activation, true);
+    const bool asks = asks_for_workspace(batch, channels, spatial, rvec);
     void* ws = nullptr;
     ClippedRegions region{};
     ClipArgs clip{};
@@ -1211,10 +1206,11 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
     }
     GroupPlan group{};
     // (a saved pre-activation is a third stream, which no register is left for)
-    if (!small && !pre_activation) group = grouped_backward(batch, channels, spatial, rvec, per_thread, activation, s);
+    if (!form.small && !form.odd && !pre_activation)
+        group = grouped_backward(batch, channels, spatial, rvec, form.per_thread, activation, s);
     if (group.members) {
         const bool exchanges = group.members > 1;
-        if (!cs.on && !per_thread) {
+        if (!cs.on && asks) {
             rc = resolve_workspace(workspace, workspace_bytes_given, workspace_bytes(batch, channels, spatial), &ws, s);
             if (rc) return rc;
         }
@@ -1235,8 +1231,8 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
                                  region.channel_before, region.channel_done, clip };
         return launch_grouped_backward(who, r, g, group.places, cs.on, rvec, activation, s);
     }
-    if (per_thread || small) {
-        if (!cs.on && (!per_thread || (!rvec && per_thread > kResidentVectors))) {
+    if (form) {
+        if (!cs.on && asks) {
             // not used, but still the caller's part of this shape (as in the forward)
             rc = resolve_workspace(workspace, workspace_bytes_given, workspace_bytes(batch, channels, spatial), &ws, s);
             if (rc) return rc;
@@ -1245,7 +1241,7 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
                                  bias_updates, mean_delta, var_delta, resident_geom(batch, channels, spatial),
                                  region.channel_norm, region.channel_sums, region.channel_before, region.channel_done,
                                  clip };
-        return launch_resident_backward(who, r, cs.on, rvec, per_thread, small, activation, s);
+        return launch_resident_backward(who, r, cs.on, form, activation, s);
     }
     if (!cs.on) {
         rc = resolve_workspace(workspace, workspace_bytes_given, workspace_bytes(batch, channels, spatial), &ws, s);

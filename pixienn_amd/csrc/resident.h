@@ -11,8 +11,7 @@ namespace pxh {
 // holds channel c, reduces it, finishes the statistics and applies them.  The tensor is read from
 // memory once, and a small layer costs one launch instead of three.
 constexpr int kResidentThreads = 1024;
-// The scalar forms also come with workgroups of half the size, four to a compute unit instead of two:
-// for the layers with a thousand channels of 19 x 19, whose workgroups would otherwise run in two rounds.
+// Workgroups of half the size: the 128-bit form with a shortcut on top, and odd planes (dispatch_odd_form).
 constexpr int kResidentNarrowThreads = 512;
 constexpr int kResidentVectors = 8;            // per lane of the forms without an LDS part
 
@@ -116,34 +115,63 @@ struct ResidentGeom {
         by_spatial.divmod(e, n, r);
         return (static_cast<size_t>(n) * channels + c) * spatial + r;
     }
+    // Odd planes: vectors of a plane, the last one moved back to end with the plane, and of the slice.
+    FastDiv by_row;
+    uint32_t vectors;
 };
 
-// The sums of a slice: fp32 per lane, except in the scalar forms that hold more than kResidentVectors values per lane.
-// Those shapes otherwise take three launches, which add a lane's share of one image in fp32 (three values of a 13 x 13
-// plane, one of a plane of up to 64) and carry on in doubles; sixteen or twenty-four values in fp32 lose two to three
-// times as much.  Here two values are added in fp32 where the three launches add as many or more, none where they add
-// fewer, and everything beyond in doubles.  Against fp32 throughout, forward and backward, us: 64 x 256 x 13^2 8.5 -> 8.7
-// and 11.6 -> 11.8, 64 x 1024 x 13^2 27.6 -> 27.7 and 37.3 -> 38.6.  (Every value into a double of its own: 9.1 and 12.1,
-// 28.2 and 39.0.)
-template<int V, int R, int L, int T>
-constexpr bool kWideSlice = V == 1 && (R + L) * T > kResidentVectors * kResidentThreads;
-constexpr int kPairSpatial = 2 * kWave;        // from this plane on a lane of the three launches adds two values and more
+// A step of a lane: where its values are, whether the slice has them, and how many of the first ones the vector in front
+// holds too.
+struct Step {
+    size_t at;
+    bool valid;
+    int held;
+};
 
-__device__ __forceinline__ void add_two(double& sum, float v, float w, bool pair)
+template<int V, bool RAGGED>
+__device__ __forceinline__ Step step_of(const ResidentGeom& g, uint32_t c, uint32_t item)
 {
-    if (pair) {
-        sum += static_cast<double>(v + w);
+    if constexpr (RAGGED) {
+        const bool valid = item < g.vectors;
+        uint32_t n, j;
+        g.by_row.divmod(valid ? item : 0u, n, j);
+        const int beyond = static_cast<int>(j) * 4 + 4 - g.spatial;
+        const int held = beyond > 0 ? beyond : 0;
+        return Step{ (static_cast<size_t>(n) * g.channels + c) * g.spatial + (static_cast<int>(j) * 4 - held), valid, held };
     } else {
-        asm volatile("" : "+v"(v));     // a branch, not both ways and a choice: `pair` is the same for every lane
-        sum += static_cast<double>(v);
-        sum += static_cast<double>(w);
+        const uint32_t e = item * V;
+        const bool valid = e < g.per_channel;
+        return Step{ g.at(c, valid ? e : 0u), valid, 0 };
+    }
+}
+
+template<int V, bool NT, bool RAGGED>
+__device__ __forceinline__ Pack<V> ld_step(const float* p, const Step& s)
+{
+    if constexpr (RAGGED) return ld_word(p + s.at);
+    else return ld<V, NT>(p, s.at);
+}
+
+// OWN: without the values that the vector in front holds too.
+template<int V, bool RAGGED, bool OWN = false>
+__device__ __forceinline__ void st_step(float* p, const Step& s, const Pack<V>& v)
+{
+    if constexpr (!RAGGED) {
+        st<V, true>(p, s.at, v);
+    } else if (!OWN || s.held == 0) {
+        st_word(p + s.at, v);
+    } else {
+#pragma unroll
+        for (int q = 1; q < 4; ++q)
+            if (q >= s.held) __builtin_nontemporal_store(v.v[q], p + s.at + q);
     }
 }
 
 // The small forms (small_slice below): a lane adds the values of a vector in fp32 and its vectors in doubles -- no further
-// from 64 bits than a lane of the other forms that holds one vector -- and the backward keeps x beside the delta.
+// from 64 bits than a lane of the other forms that holds one vector -- and the backward keeps x beside the delta.  (Odd
+// planes: every value in doubles.)
 template<int V, int R, int L, int T>
-constexpr bool kSmallSlice = L == 0 && T < kResidentThreads && V * R <= (V == 4 ? 32 : 12);
+constexpr bool kSmallSlice = L == 0 && T < kResidentThreads && V * R <= 32;
 
 // A thread keeps R vectors in registers and L more in LDS (dynamic, L * kResidentThreads vectors:
 // thread-major, so every access is the conflict-free 128-bit one).
@@ -196,30 +224,6 @@ struct ResidentBwdArgs {
 // the large form (128-bit vectors only) 16 vectors in registers + 8 in LDS (128 KB of the CU's 160)
 constexpr int kResidentLargeRegs = 16, kResidentLargeLds = 8;
 constexpr size_t kResidentLargeLdsBytes = static_cast<size_t>(kResidentLargeLds) * kResidentThreads * 16;
-// The scalar forms (odd planes) with more values per lane: 16 in 64 registers, two workgroups per compute unit; the
-// backward also 24 in 128 registers.  Against the three launches, us:
-//                       forward        + shortcut     backward
-//   64 x 256 x 13^2     15.2 ->  8.7   16.0 -> 11.8   21.8 -> 11.8   leaky
-//   64 x 512 x 13^2     22.1 -> 14.4   24.1 -> 17.6   32.0 -> 18.5
-//   49 x 1024 x 13^2    31.4 -> 23.5   35.7 -> 30.0   43.2 -> 32.1
-//   64 x 1024 x 13^2    36.5 -> 27.7   41.7 -> 38.4   49.1 -> 38.6
-//   32 x 1024 x 19^2    29.9 -> 27.4   41.6 -> 35.8   49.7 -> 37.2
-//   64 x 512 x 19^2     29.7 -> 28.3   38.9 -> 54.0   49.9 -> 36.6   24 values
-//   64 x 256 x 13^2     15.7 -> 12.1   16.4 -> 13.4   28.5 -> 20.8   mish
-//   64 x 512 x 13^2     22.7 -> 19.2   25.1 -> 21.4   40.4 -> 35.8
-//   32 x 1024 x 19^2    30.8 -> 37.1   39.6 -> 52.4   64.8 -> 66.5
-//   64 x 512 x 19^2     30.1 -> 34.7   40.3 -> 64.3   64.5 -> 61.8   24 values
-// An activation with an exponential leaves a workgroup that waits for its own channel more to do after the wait, and a
-// thousand channels keep the three launches' many small workgroups busy: it takes the one-launch form only up to 512
-// channels, and 24 values only where the backward's gradient is a select.  (Forward with 24 values the shortcut would
-// lose, and a layer has the same statistics to the bit with and without one: no such form.)
-constexpr int kResidentScalarMid = 16, kResidentScalarWide = 24;
-constexpr int kResidentScalarFew = 512;
-// Beyond this the riding form runs two workgroups to a compute unit (64 x 512 x 13^2, leaky: 17.6 against 20.7 us); up to
-// it every channel finds a compute unit of its own, and the form that keeps its addresses is ahead (64 x 256 x 13^2: 11.2
-// against 11.8, mish 12.6 against 14.2).
-constexpr int kResidentTight = 256;
-
 constexpr bool selects(int activation)
 {
     return activation == PXH_LEAKY || activation == PXH_RELU || activation == PXH_LINEAR;
@@ -239,87 +243,138 @@ constexpr int kResidentChannels = 96;
 //   8 x 512 x 26^2      9.2 -> 6.6    9.6 -> 7.8   10.7 -> 9.0   16.4 -> 12.4    512 lanes, 4
 //   2 x 128 x 80^2      6.8 -> 6.0    7.7 -> 6.2    9.0 -> 8.0   13.4 -> 11.1    512 lanes, 8
 //   1 x 64 x 104^2      9.6 -> 5.5   10.8 -> 5.6   13.4 -> 7.3   19.1 -> 10.6    (three launches before)
-//   1 x 1024 x 13^2     8.4 -> 3.9   11.2 -> 4.0   11.9 -> 4.8   17.7 ->  8.3     64 lanes, 4 values
-//   4 x 1024 x 13^2     9.0 -> 5.3   11.8 -> 5.4   12.8 -> 6.1   17.5 ->  9.6    256 lanes, 4
-//   8 x 512 x 19^2      7.1 -> 6.0    8.3 -> 6.7   10.1 -> 7.9   14.8 -> 11.2    512 lanes, 8
-//   16 x 512 x 19^2     8.3 -> 7.7   10.5 -> 10.3  11.2 -> 10.6  16.3 -> 13.8    512 lanes, 12
-//   16 x 1024 x 19^2   14.1 -> 13.8  19.5 -> 19.6  19.1 -> 19.3  23.2 -> 23.3
 // With more lanes at the same capacity each is slower (2 x 1024 x 10^2 in 128, 256, 512 lanes: backward 4.7, 6.5, 10.0).
 // Eight vectors a lane take a workgroup's 256 registers a lane, one to a compute unit: up to as many channels only
 // (4 x 512 x 52^2, leaky: backward 16.5 us against 14.2).  An activation with an exponential is bound by its gradient, and
 // there the waves count: beyond 512 vectors a slice its backward keeps the full workgroups where it has them
 // (8 x 256 x 38^2, mish: 15.5 us against 13.4; 2 x 256 x 40^2: 8.5 against 8.0; 2 x 512 x 20^2: 6.4 against 7.8).
-constexpr uint32_t kSmallVectors = 4096, kSmallScalars = 6144;
+constexpr uint32_t kSmallVectors = 4096;
 constexpr uint32_t kSmallVectorsMany = 2048;      // beyond kSmallChannels channels
 constexpr int kSmallChannels = 256;
 constexpr uint32_t kSmallVectorsSmooth = 512;
 
-// The vectors (or scalars) of a channel's slice where the shape takes a small form, else 0.
+// The vectors of a channel's slice where the shape takes a small form, else 0.
 inline uint32_t small_slice(int batch, int channels, int spatial, bool vec, int activation, bool backward)
 {
-    const size_t per_channel = static_cast<size_t>(batch) * spatial;
-    const size_t items = vec ? per_channel / 4 : per_channel;
-    size_t most = !vec ? kSmallScalars : channels <= kSmallChannels ? kSmallVectors : kSmallVectorsMany;
-    if (vec && backward && !selects(activation) && channels >= kResidentChannels) most = kSmallVectorsSmooth;
+    if (!vec) return 0;
+    const size_t items = static_cast<size_t>(batch) * spatial / 4;
+    size_t most = channels <= kSmallChannels ? kSmallVectors : kSmallVectorsMany;
+    if (backward && !selects(activation) && channels >= kResidentChannels) most = kSmallVectorsSmooth;
     return items <= most ? static_cast<uint32_t>(items) : 0;
 }
 
-// Calls launch.operator()<V, R, T>() with the form for `items`: vectors or scalars, steps per lane, lanes.
+// Calls launch.operator()<R, T>() with the form for `items` vectors: steps per lane, lanes.
 template<typename F>
-void dispatch_small_form(bool vec, uint32_t items, F&& launch)
+void dispatch_small_form(uint32_t items, F&& launch)
 {
-    if (vec) {
-        if (items <= 64 * 2) return launch.template operator()<4, 2, 64>();
-        if (items <= 128 * 2) return launch.template operator()<4, 2, 128>();
-        if (items <= 256 * 4) return launch.template operator()<4, 4, 256>();
-        if (items <= 512 * 4) return launch.template operator()<4, 4, 512>();
-        return launch.template operator()<4, 8, 512>();
-    }
-    if (items <= 64 * 4) return launch.template operator()<1, 4, 64>();
-    if (items <= 256 * 4) return launch.template operator()<1, 4, 256>();
-    if (items <= 256 * 8) return launch.template operator()<1, 8, 256>();
-    if (items <= 512 * 8) return launch.template operator()<1, 8, 512>();
-    return launch.template operator()<1, 12, 512>();
+    if (items <= 64 * 2) return launch.template operator()<2, 64>();
+    if (items <= 128 * 2) return launch.template operator()<2, 128>();
+    if (items <= 256 * 4) return launch.template operator()<4, 256>();
+    if (items <= 512 * 4) return launch.template operator()<4, 512>();
+    return launch.template operator()<8, 512>();
 }
 
-inline int resident_vectors(int batch, int channels, int spatial, bool vec, int activation, bool backward)
+inline int resident_vectors(int batch, int channels, int spatial, bool vec)
 {
-    if (channels < kResidentChannels) return 0;
-    const size_t per_channel = static_cast<size_t>(batch) * spatial;
-    const size_t vectors = (per_channel + (vec ? 3 : 0)) / (vec ? 4 : 1);
+    if (!vec || channels < kResidentChannels) return 0;
+    const size_t vectors = static_cast<size_t>(batch) * spatial / 4;
     const size_t per_thread = (vectors + kResidentThreads - 1) / kResidentThreads;
     if (per_thread <= kResidentVectors) return kResidentVectors;
-    if (vec) return per_thread <= kResidentLargeRegs + kResidentLargeLds ? kResidentLargeRegs + kResidentLargeLds : 0;
-    const bool light = selects(activation);
-    if (per_thread <= kResidentScalarMid && (light || channels <= kResidentScalarFew)) return kResidentScalarMid;
-    if (per_thread <= kResidentScalarWide && light && backward) return kResidentScalarWide;
-    return 0;
+    return per_thread <= kResidentLargeRegs + kResidentLargeLds ? kResidentLargeRegs + kResidentLargeLds : 0;
 }
 
-// The scalar form with workgroups of kResidentNarrowThreads (twice the values per thread): when the full
-// workgroups would outnumber the two places a compute unit has for them.  Measured at 16 x 1024 x 19^2:
-// forward 14.6 against 16.3 us, backward 23.1 against 26.5; at 512 channels the forward gains 5 %, the
-// backward loses 20 %.
-constexpr int kResidentNarrowVectors = 2 * kResidentVectors;
-inline bool resident_narrow(const ResidentGeom& g, int per_thread, bool vec, bool backward)
+// Odd planes (and tensors off a 16-byte boundary).  A 128-bit access needs the alignment of a word only, so their planes
+// are taken in vectors too, the last of a plane moved back to end with it: the values that it shares with the vector in
+// front are loaded twice, added once, and written twice with the same result, or once where a lane may read what another
+// has written.  One value per access was what bound these layers (a quarter of the bytes on their way per instruction and
+// four times the addresses); a lane that keeps both tensors needs no second read of x either.
+// One value a step, or three launches (*) -> vectors, us, leaky and mish: forward, + shortcut, backward, backward with rescale + clip
+//   64 x 1024 x 13^2  28.4 -> 23.8  39.8 -> 34.3  40.4 -> 35.0  48.0 -> 37.1   6 x 512   38.6*-> 24.0  43.5*-> 33.7  62.6*-> 36.0  72.2*-> 47.6
+//   64 x 512 x 13^2   15.2 -> 11.2  19.0 -> 16.3  19.8 -> 16.8  24.8 -> 19.0   6 x 512   18.5 -> 12.4  22.3 -> 16.6  25.0 -> 19.1  34.0 -> 25.5
+//   64 x 256 x 13^2    9.3 ->  8.0  12.6 ->  8.9  12.3 -> 10.6  16.7 -> 13.8   6 x 512   11.9 ->  8.8  14.1 -> 10.0  15.3 -> 13.0  21.2 -> 17.1
+//   64 x 512 x 19^2   31.9*-> 21.4  38.2*-> 31.9  37.5 -> 35.3  43.5 -> 41.0   6 x 1024  33.2*-> 20.9  41.6*-> 33.5  57.4*-> 40.1  66.0*-> 56.5
+//   16 x 1024 x 19^2  13.3 -> 10.6  19.5 -> 15.7  18.8 -> 16.7  22.5 -> 19.1   6 x 256   17.5 -> 12.6  21.7 -> 16.5  21.9 -> 19.2  29.3 -> 25.1
+//   16 x 512 x 19^2    7.7 ->  7.5   9.4 ->  8.4  10.6 ->  9.4  13.8 -> 12.7   3 x 512   10.8 ->  8.1  12.0 ->  9.3  13.0 -> 11.3  17.4 -> 15.6
+//   8 x 512 x 19^2     5.9 ->  5.7   6.4 ->  6.0   7.7 ->  6.6  10.8 ->  9.8   3 x 256    7.6 ->  6.5   8.0 ->  6.9   9.7 ->  8.0  13.0 -> 11.5
+//   8 x 96 x 45^2      9.2 ->  6.8  12.7 ->  9.0  12.5 ->  9.5  17.2 -> 13.3   4 x 1024  14.3 ->  8.7  15.8 -> 10.8  16.0 -> 12.3  20.7 -> 17.1
+//   4 x 1024 x 13^2    5.1 ->  4.9   5.3 ->  5.2   5.6 ->  5.5   9.3 ->  8.9   2 x 128    5.8 ->  5.4   5.9 ->  5.7   6.7 ->  6.3  10.2 ->  9.7
+//   1 x 1024 x 13^2    4.1 ->  4.3   4.2 ->  4.5   4.4 ->  4.3   7.7 ->  7.8   1 x 64     4.5 ->  4.4   4.5 ->  4.6   5.0 ->  4.5   8.5 ->  8.1
+// (steps x lanes of the form.)  More lanes than the slice needs are slower everywhere (64 x 1024 x 13^2, backward: 4 x 1024
+// 41.4, 8 x 512 43.0; 16 x 512 x 19^2: 3 x 1024 14.3); six steps in workgroups of 256 lanes serve a thousand channels, whose
+// workgroups then run in one round (16 x 1024 x 19^2 16.7 against 18.2 with 3 x 512), three in 512 lanes up to half as many
+// (16 x 512 x 19^2, mish: 11.3 against 12.5).
+constexpr int kOddSpatial = 4;                    // planes below have no vector: one value a step
+constexpr uint32_t kOddVectors = 6144;
+constexpr uint32_t kOddVectorsFew = 4096;         // with fewer than kResidentChannels channels (as kSmallVectors)
+constexpr uint32_t kOddValues = kResidentVectors * kResidentThreads, kOddValuesFew = 1024;
+constexpr int kOddChannels = 512;
+
+// The vectors (values in planes below kOddSpatial) of a channel's slice where such a shape takes a one-launch form, else 0.
+inline uint32_t odd_slice(int batch, int channels, int spatial, bool vec)
 {
-    if (vec || per_thread != kResidentVectors || g.channels < (backward ? 1024 : 512)) return false;
-    return (g.per_channel + kResidentNarrowThreads - 1) / kResidentNarrowThreads <= kResidentNarrowVectors;
+    if (vec) return 0;
+    const bool few = channels < kResidentChannels;
+    const bool values = spatial < kOddSpatial;
+    const size_t items = static_cast<size_t>(batch) * (values ? spatial : (spatial + 3) / 4);
+    const uint32_t most = values ? (few ? kOddValuesFew : kOddValues) : few ? kOddVectorsFew : kOddVectors;
+    return items <= most ? static_cast<uint32_t>(items) : 0;
+}
+
+// Calls launch.operator()<V, R, T>() with the form for `items`: values per step, steps per lane, lanes.
+template<typename F>
+void dispatch_odd_form(uint32_t items, const ResidentGeom& g, F&& launch)
+{
+    if (g.spatial < kOddSpatial) {
+        if (items <= kOddValuesFew) return launch.template operator()<1, 4, 256>();
+        return launch.template operator()<1, kResidentVectors, kResidentThreads>();
+    }
+    if (items <= 64) return launch.template operator()<4, 1, 64>();
+    if (items <= 128 * 2) return launch.template operator()<4, 2, 128>();
+    if (items <= 256 * 3) return launch.template operator()<4, 3, 256>();
+    if (items <= 256 * 6 && g.channels > kOddChannels) return launch.template operator()<4, 6, 256>();
+    if (items <= 512 * 3) return launch.template operator()<4, 3, 512>();
+    if (items <= 512 * 4) return launch.template operator()<4, 4, 512>();
+    if (items <= 512 * 6) return launch.template operator()<4, 6, 512>();
+    if (items <= 1024 * 4) return launch.template operator()<4, 4, 1024>();
+    return launch.template operator()<4, 6, 1024>();
+}
+
+// Whether a plain call of a shape asks for a workspace: unless it takes a one-launch form that never depended on measured
+// limits.  Those of the others may move, also between activations, and a workspace that is too small for a shape is refused
+// on either side of them (as is growth in a capture).
+inline bool asks_for_workspace(int batch, int channels, int spatial, bool vec)
+{
+    if (vec) return resident_vectors(batch, channels, spatial, true) == 0;
+    return channels < kResidentChannels || static_cast<size_t>(batch) * spatial > kResidentVectors * kResidentThreads;
 }
 
 inline ResidentGeom resident_geom(int batch, int channels, int spatial)
 {
     return ResidentGeom{ channels, spatial, static_cast<uint32_t>(batch) * static_cast<uint32_t>(spatial),
-                         FastDiv(static_cast<uint32_t>(spatial)) };
+                         FastDiv(static_cast<uint32_t>(spatial)), FastDiv(static_cast<uint32_t>(spatial + 3) / 4),
+                         static_cast<uint32_t>(batch) * (static_cast<uint32_t>(spatial + 3) / 4) };
 }
 
 // A kernel that asks for more than 64 KB of dynamic LDS has to be allowed to, once.
 int allow_large_lds(const void* kernel);
 
-// `per_thread`: resident_vectors() of the shape, `small`: small_slice().
-int launch_resident_forward(const char* who, const ResidentFwdArgs& r, bool vec, int per_thread, uint32_t small,
-                            int activation, hipStream_t s);
-int launch_resident_backward(const char* who, const ResidentBwdArgs& r, bool clipped, bool vec, int per_thread,
-                             uint32_t small, int activation, hipStream_t s);
+// How a shape takes the one-launch passes: the vectors per lane of the forms of 1024 lanes (resident_vectors), or the vectors of
+// a slice in a small form (small_slice) or of odd planes (odd_slice); all 0 where it does not.
+struct ResidentForm {
+    int per_thread;
+    uint32_t small, odd;
+    explicit operator bool() const { return per_thread || small || odd; }
+};
+
+inline ResidentForm resident_form(int batch, int channels, int spatial, bool vec, int activation, bool backward)
+{
+    return ResidentForm{ resident_vectors(batch, channels, spatial, vec),
+                         small_slice(batch, channels, spatial, vec, activation, backward),
+                         odd_slice(batch, channels, spatial, vec) };
+}
+
+int launch_resident_forward(const char* who, const ResidentFwdArgs& r, const ResidentForm& form, int activation, hipStream_t s);
+int launch_resident_backward(const char* who, const ResidentBwdArgs& r, bool clipped, const ResidentForm& form, int activation,
+                             hipStream_t s);
 
 }  // namespace pxh

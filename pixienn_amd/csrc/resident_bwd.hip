@@ -18,31 +18,29 @@ namespace {
 // clamped delta.
 // Channel c of a backward whose first launch finished it with the sums of its unscaled delta, scaled
 // by the factor the plan arrived at.
-template<int V, int R, int L, int T>
+template<int V, int R, int L, int T, bool RAGGED>
 __device__ __forceinline__ void resident_rescale_channel(const ResidentBwdArgs& a, uint32_t c, float factor)
 {
     // The steps' loads in flight together where a lane has the registers beside the full pass: one after the other they are
     // most of a channel's time (16 x 512 x 19^2 rescaled 29.3 -> 22.0 us, 1 x 1024 x 13^2 16.1 -> 14.4, 64 x 1024 x 13^2 91 -> 77; the
     // 128-bit forms of 1024 lanes spill with eight of them, 16 x 256 x 38^2 28.9 -> 38.6).
-    constexpr bool kTogether = V == 1 || kSmallSlice<V, R, L, T>;
+    constexpr bool kTogether = V == 1 || RAGGED || kSmallSlice<V, R, L, T>;
     constexpr int kLoads = !kTogether ? 1 : (R + L) % 12 == 0 ? 12 : (R + L) % 8 == 0 ? 8 : R + L;
     static_assert((R + L) % kLoads == 0, "steps come in whole groups");
 #pragma unroll 1
     for (int first = 0; first < R + L; first += kLoads) {
         Pack<V> t[kLoads];
-        const auto element = [&](int u) { return static_cast<uint32_t>((first + u) * T + threadIdx.x) * V; };
-        if (!kTogether && element(0) >= a.g.per_channel) break;
+        const auto step = [&](int u) { return step_of<V, RAGGED>(a.g, c, static_cast<uint32_t>((first + u) * T + threadIdx.x)); };
+        if (!kTogether && !step(0).valid) break;
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) t[u] = ld_step<V, true, RAGGED>(a.b.delta, step(u));
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) {
-            const uint32_t e = element(u);
-            t[u] = ld<V, true>(a.b.delta, a.g.at(c, e < a.g.per_channel ? e : 0u));
-        }
-#pragma unroll
-        for (int u = 0; u < kLoads; ++u) {
-            const uint32_t e = element(u);
+            const Step p = step(u);
 #pragma unroll
             for (int q = 0; q < V; ++q) t[u].v[q] = factor * t[u].v[q];
-            if (e < a.g.per_channel) st<V, true>(a.b.delta, a.g.at(c, e), t[u]);
+            // (no barrier between a lane's loads and another's stores: only what is its own)
+            if (p.valid) st_step<V, RAGGED, true>(a.b.delta, p, t[u]);
         }
     }
     if (threadIdx.x == 0) {
@@ -53,12 +51,13 @@ __device__ __forceinline__ void resident_rescale_channel(const ResidentBwdArgs& 
 }
 
 // Channel c by the whole workgroup; `factor` and `limit` are the plan's (kRedo only).
-template<int ACT, int V, int R, int L, int MODE, int T>
+template<int ACT, int V, int R, int L, int MODE, int T, bool RAGGED>
 __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, const uint32_t c,
                                                      [[maybe_unused]] const float factor,
                                                      [[maybe_unused]] const float limit)
 {
     extern __shared__ __align__(16) float resident_lds[];
+    constexpr bool kSmall = RAGGED || kSmallSlice<V, R, L, T>;
     __shared__ double slots[MODE == kFirst ? 3 : 2][T / kWave];
     __shared__ DxCoef shared_coef;
     const FoldCoef k = make_coef(a.b.mean[c], a.b.var[c], a.b.scale[c], a.b.bias[c]);
@@ -82,7 +81,7 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
         const float scale_updates_in = kEarly ? early[1] : a.scale_updates[c];
         const float var_in = kEarly ? early[2] : a.b.var[c];
         const FinishedChannel r = finished_channel<true>(sa, sb, static_cast<int>(a.g.per_channel), k,
-                                                         kSmallSlice<V, R, L, T> ? terms : variance_terms(var_in), k.scale);
+                                                         kSmall ? terms : variance_terms(var_in), k.scale);
         a.bias_updates[c] = bias_updates_in + r.bias_add;
         a.scale_updates[c] = scale_updates_in + r.scale_add;
         if (a.mean_delta) a.mean_delta[c] = r.mean_delta;
@@ -92,10 +91,8 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
     };
     const bool recompute = a.b.pre == nullptr;
     Pack<V> d[R];
-    constexpr bool kSmall = kSmallSlice<V, R, L, T>;
-    constexpr bool kWide = kWideSlice<V, R, L, T>;
-    std::conditional_t<kWide || kSmall, double, float> fa = 0, fb = 0;
-    [[maybe_unused]] std::conditional_t<kWide || kSmall, double, float> fq = 0;
+    std::conditional_t<kSmall, double, float> fa = 0, fb = 0;
+    [[maybe_unused]] std::conditional_t<kSmall, double, float> fq = 0;
     [[maybe_unused]] float peak = 0.0f;
     // Two shapes of the first pass.  Grouped: no branch around the loads (see the forward kernel), lanes
     // past the end read the first vector; kGroup steps at a time, their loads go out together, then each
@@ -113,6 +110,7 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
     // its addresses are formed again there instead of being held in registers (48 of them) from the first
     [[maybe_unused]] uint32_t lane = threadIdx.x;
     [[maybe_unused]] const auto element = [&](int r) { return (static_cast<uint32_t>(r * T) + lane) * V; };
+    const auto step = [&](int r) { return step_of<V, RAGGED>(a.g, c, static_cast<uint32_t>(r * T) + lane); };
     [[maybe_unused]] const auto place = [&](int r) {
         const uint32_t e = element(r);
         return a.g.at(c, e < a.g.per_channel ? e : 0u);
@@ -123,7 +121,7 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
 #pragma unroll
         for (int q = 0; q < V; ++q) {
             if constexpr (MODE == kFirst) {
-                if constexpr (!kWide && !kSmall) fq += valid ? t.v[q] * t.v[q] : 0.0f;
+                if constexpr (!kSmall) fq += valid ? t.v[q] * t.v[q] : 0.0f;
                 peak = fmaxf(peak, valid ? fabsf(t.v[q]) : 0.0f);
             }
             if constexpr (MODE == kRedo) t.v[q] = rescaled_clipped(t.v[q], factor, limit);
@@ -134,12 +132,12 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
         // every load of the slice at once, no branch around them; the pre-activations four steps at a time
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const size_t where = place(r);
-            d[r] = ld<V, true>(a.b.delta, where);
-            kept[r] = ld<V, false>(a.b.x, where);
+            const Step p = step(r);
+            d[r] = ld_step<V, true, RAGGED>(a.b.delta, p);
+            kept[r] = ld_step<V, false, RAGGED>(a.b.x, p);
         }
         early_terms();
-        constexpr int kFour = R < 4 ? R : 4;
+        constexpr int kFour = R < 4 ? R : R % 4 == 0 ? 4 : 3;
         static_assert(R % kFour == 0, "steps come in whole groups");
 #pragma unroll
         for (int first = 0; first < R; first += kFour) {
@@ -147,7 +145,7 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
             if constexpr (ACT != PXH_LINEAR) {
                 if (!recompute) {
 #pragma unroll
-                    for (int i = 0; i < kFour; ++i) pv[i] = ld<V, true>(a.b.pre, place(first + i));
+                    for (int i = 0; i < kFour; ++i) pv[i] = ld_step<V, true, RAGGED>(a.b.pre, step(first + i));
                 } else {
 #pragma unroll
                     for (int i = 0; i < kFour; ++i) {
@@ -159,6 +157,26 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
 #pragma unroll
             for (int i = 0; i < kFour; ++i) {
                 const int r = first + i;
+                if constexpr (RAGGED) {
+                    // every value into a double of its own, and those that the vector in front holds too stay out of the sums
+                    const Step p = step(r);
+                    const int own = p.valid ? p.held : V;
+                    if constexpr (MODE == kFirst) {
+#pragma unroll
+                        for (int q = 0; q < V; ++q) {
+                            const float t = q >= own ? d[r].v[q] : 0.0f;
+                            fq += static_cast<double>(t * t);
+                        }
+                    }
+                    prepare(d[r], pv[i], p.valid);
+#pragma unroll
+                    for (int q = 0; q < V; ++q) {
+                        const float t = d[r].v[q];
+                        fa += static_cast<double>(q >= own ? t : 0.0f);
+                        fb += static_cast<double>(q >= own ? t * (kept[r].v[q] - k.mean) : 0.0f);
+                    }
+                    continue;
+                }
                 const bool valid = element(r) < a.g.per_channel;
                 float va = 0.0f, vb = 0.0f, vq = 0.0f;
 #pragma unroll
@@ -184,15 +202,12 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
         const auto take = [&](int r, Pack<V>& dv, const Pack<V>& xv, const Pack<V>& pv) {
             const bool valid = element(r) < a.g.per_channel;
             prepare(dv, pv, valid);
-            if constexpr (!kWide) {
 #pragma unroll
-                for (int q = 0; q < V; ++q) {
-                    fa += valid ? dv.v[q] : 0.0f;
-                    fb += valid ? dv.v[q] * (xv.v[q] - k.mean) : 0.0f;
-                }
+            for (int q = 0; q < V; ++q) {
+                fa += valid ? dv.v[q] : 0.0f;
+                fb += valid ? dv.v[q] * (xv.v[q] - k.mean) : 0.0f;
             }
         };
-        [[maybe_unused]] const bool pair = a.g.spatial >= kPairSpatial;
 #pragma unroll
         for (int top = R + L - 1; top >= 0; top -= kGroup) {
             Pack<V> dv[kGroup], xv[kGroup], pv[kGroup];
@@ -216,29 +231,10 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
                     }
                 }
             }
-            if constexpr (kWide) {
-#pragma unroll
-                for (int i = 0; i < kGroup; i += 2) {
-                    const bool valid[2] = { element(top - i) < a.g.per_channel, element(top - i - 1) < a.g.per_channel };
-                    float va[2], vb[2], vq[2];
-#pragma unroll
-                    for (int u = 0; u < 2; ++u) {
-                        const float raw = dv[i + u].v[0];
-                        take(top - i - u, dv[i + u], xv[i + u], pv[i + u]);
-                        const float t = dv[i + u].v[0];
-                        va[u] = valid[u] ? t : 0.0f;
-                        vb[u] = valid[u] ? t * (xv[i + u].v[0] - k.mean) : 0.0f;
-                        vq[u] = valid[u] ? raw * raw : 0.0f;
-                    }
-                    add_two(fa, va[0], va[1], pair);
-                    add_two(fb, vb[0], vb[1], pair);
-                    if constexpr (MODE == kFirst) add_two(fq, vq[0], vq[1], pair);
-                }
-            }
 #pragma unroll
             for (int i = 0; i < kGroup; ++i) {
                 const int r = top - i;
-                if constexpr (!kWide) take(r, dv[i], xv[i], pv[i]);
+                take(r, dv[i], xv[i], pv[i]);
                 if (r < R) d[r < R ? r : 0] = dv[i];
                 else *resident_lds_slot<V, R>(resident_lds, r) = dv[i];
             }
@@ -323,34 +319,34 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
         asm volatile("" : "+v"(lane));      // addresses formed again, not kept from the first pass
 #pragma unroll
         for (int r = 0; r < R + L; ++r) {
-            const uint32_t e = (r * T + lane) * V;
-            if (e < a.g.per_channel) {
-                const size_t where = a.g.at(c, e);
+            const Step p = step(r);
+            if (p.valid) {
                 Pack<V> xv;
                 if constexpr (kSmall) xv = kept[r];
-                else xv = ld<V, false>(a.b.x, where);
+                else xv = ld<V, false>(a.b.x, p.at);
                 const Pack<V> dv = r < R ? d[r < R ? r : 0] : *resident_lds_slot<V, R>(resident_lds, r);
                 Pack<V> out;
 #pragma unroll
                 for (int q = 0; q < V; ++q) out.v[q] = dx_value(dv.v[q], xv.v[q], kd);
-                st<V, true>(a.b.delta, where, out);
+                // (a value that two lanes hold is written by both, the same: every delta was read before the sums)
+                st_step<V, RAGGED>(a.b.delta, p, out);
             }
         }
     }
 }
 
 // Waves per SIMD that the registers are held to.
-template<int V, int R, int L, int MODE, int T>
-constexpr int kBwdWaves = kSmallSlice<V, R, L, T> ? (MODE == kRedo || V * R >= 32 ? 2 : V * R >= 12 ? 4 : V * R == 8 ? 6 : 8)
-                          : L == 0 && MODE != kRedo && !(V == 1 && R > 16) ? 8 : 4;
+template<int V, int R, int L, int MODE, int T, bool RAGGED>
+constexpr int kBwdWaves = RAGGED && T == kResidentThreads ? 4 : RAGGED || kSmallSlice<V, R, L, T> ? (MODE == kRedo || V * R >= 32 ? 2 : V * R >= 12 ? 4 : V * R == 8 ? 6 : 8)
+                          : L == 0 && MODE != kRedo ? 8 : 4;
 
 // One workgroup per channel.  (The forms of 1024 lanes without an LDS part are held to 64 registers, two workgroups
 // per compute unit: they run the 19 x 19 and 38 x 38 layers, whose launches are too short to fill the
 // machine with one.)  The workgroups of the kRedo launch form the plan from the per-channel figures of
 // the first launch and leave at once when nothing has to change; the forms without an LDS part run it
 // as a capped grid that walks the channels otherwise.
-template<int ACT, int V, int R, int L, int MODE = kPlain, int T = kResidentThreads>
-__global__ __launch_bounds__(T, (kBwdWaves<V, R, L, MODE, T>)) void bn_resident_bwd_kernel(ResidentBwdArgs a)
+template<int ACT, int V, int R, int L, int MODE = kPlain, int T = kResidentThreads, bool RAGGED = false>
+__global__ __launch_bounds__(T, (kBwdWaves<V, R, L, MODE, T, RAGGED>)) void bn_resident_bwd_kernel(ResidentBwdArgs a)
 {
     static_assert(L == 0 || T == kResidentThreads, "the LDS part is laid out for the full workgroup");
     if constexpr (MODE == kRedo) {
@@ -364,55 +360,46 @@ __global__ __launch_bounds__(T, (kBwdWaves<V, R, L, MODE, T>)) void bn_resident_
         if constexpr (L > 0) {
             // (one workgroup per channel: walking several costs the large form 450 bytes of spills per lane)
             const uint32_t c = blockIdx.x;
-            if (!a.channel_done[c]) resident_bwd_channel<ACT, V, R, L, kRedo, T>(a, c, plan.factor, plan.clip);
-            else if (plan.factor != 1.0f) resident_rescale_channel<V, R, L, T>(a, c, plan.factor);
+            if (!a.channel_done[c]) resident_bwd_channel<ACT, V, R, L, kRedo, T, RAGGED>(a, c, plan.factor, plan.clip);
+            else if (plan.factor != 1.0f) resident_rescale_channel<V, R, L, T, RAGGED>(a, c, plan.factor);
         } else {
             for (uint32_t c = blockIdx.x; c < static_cast<uint32_t>(a.g.channels); c += gridDim.x) {
-                if (!a.channel_done[c]) resident_bwd_channel<ACT, V, R, L, kRedo, T>(a, c, plan.factor, plan.clip);
-                else if (plan.factor != 1.0f) resident_rescale_channel<V, R, L, T>(a, c, plan.factor);
+                if (!a.channel_done[c]) resident_bwd_channel<ACT, V, R, L, kRedo, T, RAGGED>(a, c, plan.factor, plan.clip);
+                else if (plan.factor != 1.0f) resident_rescale_channel<V, R, L, T, RAGGED>(a, c, plan.factor);
                 __syncthreads();       // the next channel reuses the workgroup's LDS
             }
         }
     } else {
-        resident_bwd_channel<ACT, V, R, L, MODE, T>(a, blockIdx.x, 1.0f, 0.0f);
+        resident_bwd_channel<ACT, V, R, L, MODE, T, RAGGED>(a, blockIdx.x, 1.0f, 0.0f);
     }
 }
 
 }  // namespace
 
-int launch_resident_backward(const char* who, const ResidentBwdArgs& r, bool clipped, bool vec, int per_thread,
-                             uint32_t small, int activation, hipStream_t s)
+int launch_resident_backward(const char* who, const ResidentBwdArgs& r, bool clipped, const ResidentForm& form, int activation,
+                             hipStream_t s)
 {
-    const bool narrow = resident_narrow(r.g, per_thread, vec, true);
-    const dim3 block(narrow ? kResidentNarrowThreads : kResidentThreads);
+    const dim3 block(kResidentThreads);
     int large_lds_rc = PXH_OK;
     const auto launch = [&]<int ACT, int MODE>() {
         // the launch that follows the plan: one workgroup per compute unit at most, each walks channels
-        const bool large = !small && vec && per_thread > kResidentVectors;
+        const bool large = !form.odd && !form.small && form.per_thread > kResidentVectors;
         const bool walks = MODE == kRedo && !large && r.g.channels > kRedoWorkgroups;
         const dim3 grid(walks ? kRedoWorkgroups : r.g.channels);
-        if (small) {
-            dispatch_small_form(vec, small, [&]<int V, int R, int T>() {
-                hipLaunchKernelGGL((bn_resident_bwd_kernel<ACT, V, R, 0, MODE, T>), grid, dim3(T), 0, s, r);
+        if (form.odd) {
+            dispatch_odd_form(form.odd, r.g, [&]<int V, int R, int T>() {
+                hipLaunchKernelGGL((bn_resident_bwd_kernel<ACT, V, R, 0, MODE, T, V == 4>), grid, dim3(T), 0, s, r);
             });
-            return;
-        }
-        if (narrow) {
-            hipLaunchKernelGGL((bn_resident_bwd_kernel<ACT, 1, kResidentNarrowVectors, 0, MODE, kResidentNarrowThreads>),
-                               grid, block, 0, s, r);
-        } else if (!vec && per_thread == kResidentScalarWide) {
-            if constexpr (selects(ACT))
-                hipLaunchKernelGGL((bn_resident_bwd_kernel<ACT, 1, kResidentScalarWide, 0, MODE>), grid, block, 0, s, r);
-        } else if (!vec && per_thread == kResidentScalarMid) {
-            hipLaunchKernelGGL((bn_resident_bwd_kernel<ACT, 1, kResidentScalarMid, 0, MODE>), grid, block, 0, s, r);
-        } else if (per_thread > kResidentVectors) {
+        } else if (form.small) {
+            dispatch_small_form(form.small, [&]<int R, int T>() {
+                hipLaunchKernelGGL((bn_resident_bwd_kernel<ACT, 4, R, 0, MODE, T>), grid, dim3(T), 0, s, r);
+            });
+        } else if (large) {
             auto kernel = bn_resident_bwd_kernel<ACT, 4, kResidentLargeRegs, kResidentLargeLds, MODE>;
             large_lds_rc = allow_large_lds(reinterpret_cast<const void*>(kernel));
             if (large_lds_rc == PXH_OK) hipLaunchKernelGGL(kernel, grid, block, kResidentLargeLdsBytes, s, r);
-        } else if (vec) {
-            hipLaunchKernelGGL((bn_resident_bwd_kernel<ACT, 4, kResidentVectors, 0, MODE>), grid, block, 0, s, r);
         } else {
-            hipLaunchKernelGGL((bn_resident_bwd_kernel<ACT, 1, kResidentVectors, 0, MODE>), grid, block, 0, s, r);
+            hipLaunchKernelGGL((bn_resident_bwd_kernel<ACT, 4, kResidentVectors, 0, MODE>), grid, block, 0, s, r);
         }
     };
     const bool known = dispatch_activation(activation, [&]<int ACT>() {

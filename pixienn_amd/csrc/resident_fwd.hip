@@ -13,22 +13,20 @@ namespace {
 constexpr int kResidualAhead = 4;
 
 // Waves per SIMD that the registers are held to: a vector a step, two with a shortcut.
-template<int V, int R, int L, int T, bool RES, bool TIGHT>
-constexpr int kFwdWaves = kSmallSlice<V, R, L, T> ? (V * R >= 32 ? 2 : RES && V * R >= 12 ? 4 : 8)
-                          : L == 0 && V * R <= (V == 1 ? (RES && !TIGHT ? 8 : 16) : 32) ? 8 : 4;
+template<int V, int R, int L, int T, bool RES, bool RAGGED>
+constexpr int kFwdWaves = RAGGED || kSmallSlice<V, R, L, T> ? (RAGGED && T == kResidentThreads ? (RES ? 4 : 8) : V * R >= 32 ? 2 : RES && V * R >= 12 ? 4 : 8)
+                          : L == 0 && V * R <= (V == 1 ? 8 : 32) ? 8 : 4;
 
-// V = 4 needs spatial % 4 == 0 and 16-byte aligned tensors.  R + L vectors per thread at most.
-// TIGHT: the scalar form with the shortcut's source on top in 64 registers, two workgroups per compute unit.
-template<int ACT, int V, int R, int L, int T = kResidentThreads, bool RES = false, bool TIGHT = false>
-__global__ __launch_bounds__(T, (kFwdWaves<V, R, L, T, RES, TIGHT>)) void bn_resident_fwd_kernel(ResidentFwdArgs a)
+// V = 4 needs spatial % 4 == 0 and 16-byte aligned tensors, RAGGED (odd planes) neither.  R + L vectors per thread at most.
+template<int ACT, int V, int R, int L, int T = kResidentThreads, bool RES = false, bool RAGGED = false>
+__global__ __launch_bounds__(T, (kFwdWaves<V, R, L, T, RES, RAGGED>)) void bn_resident_fwd_kernel(ResidentFwdArgs a)
 {
-    static_assert(!TIGHT || (RES && V == 1 && L == 0), "a form of the riding shortcut");
     static_assert(L == 0 || T == kResidentThreads, "the LDS part is laid out for the full workgroup");
     extern __shared__ __align__(16) float resident_lds[];
     // The 128-bit form with workgroups of half the size adds a channel up exactly as the full workgroups do,
     // so that a layer gives the same statistics to the bit with and without a shortcut riding on it: thread t
     // keeps the sums of the full form's threads t (even steps) and t + T (odd steps) apart.
-    constexpr bool kSmall = kSmallSlice<V, R, L, T>;
+    constexpr bool kSmall = RAGGED || kSmallSlice<V, R, L, T>;
     constexpr bool kTwin = V == 4 && T < kResidentThreads && !kSmall;
     static_assert(!kTwin || 2 * T == kResidentThreads, "half the size");
     __shared__ double slots[2][(kTwin ? 2 : 1) * T / kWave];
@@ -37,8 +35,6 @@ __global__ __launch_bounds__(T, (kFwdWaves<V, R, L, T, RES, TIGHT>)) void bn_res
     const float shift = a.x[static_cast<size_t>(c) * a.g.spatial];
     // issued now, needed after the reduction
     const float rm_in = a.rolling_mean[c], rv_in = a.rolling_var[c], scale_in = a.scale[c], bias_in = a.bias[c];
-    constexpr bool kWide = kWideSlice<V, R, L, T>;
-    static_assert(!kWide || (L == 0 && R % 2 == 0), "values are taken in pairs");
     Pack<V> v[R];
     float a1 = 0.0f, a2 = 0.0f;
     [[maybe_unused]] float b1 = 0.0f, b2 = 0.0f;
@@ -48,12 +44,10 @@ __global__ __launch_bounds__(T, (kFwdWaves<V, R, L, T, RES, TIGHT>)) void bn_res
     // No branch around a load: a lane past the end of the slice reads the slice's first vector and
     // adds nothing, so that the loads of a lane are in flight together (behind a branch each one is
     // waited for before the next is issued, and a wave then has one kilobyte on its way at a time).
-    uint32_t lane = threadIdx.x;
+    const uint32_t lane = threadIdx.x;
     const auto element = [&](int r) { return (static_cast<uint32_t>(r * T) + lane) * V; };
-    const auto fetch = [&](int r) {
-        const uint32_t e = element(r);
-        return ld<V, true>(a.x, a.g.at(c, e < a.g.per_channel ? e : 0u));
-    };
+    const auto step = [&](int r) { return step_of<V, RAGGED>(a.g, c, static_cast<uint32_t>(r * T) + lane); };
+    const auto fetch = [&](int r) { return ld_step<V, true, RAGGED>(a.x, step(r)); };
     const auto add = [&](int r, const Pack<V>& t) {
         const bool valid = element(r) < a.g.per_channel;
         const bool second = kTwin && (r & 1);
@@ -90,17 +84,27 @@ __global__ __launch_bounds__(T, (kFwdWaves<V, R, L, T, RES, TIGHT>)) void bn_res
     // (16 x 1024 x 19^2: 19.9 us against 25.6 us with every step's load behind the reduction).
     // (the half-size workgroups of the 128-bit form have 128 registers: eight of twelve steps, four of sixteen)
     constexpr int kAhead = !RES ? 0 : kSmall || V * (R + L) <= 8 ? R + L : L > 0 ? kResidualAhead
-                                : T < kResidentThreads ? (R <= 12 ? 8 : 4) : V == 1 && R >= 16 ? (TIGHT ? 8 : 4) : 0;
+                                : T < kResidentThreads ? (R <= 12 ? 8 : 4) : 0;
     [[maybe_unused]] Pack<V> ahead[kAhead > 0 ? kAhead : 1];
     if constexpr (RES) {
 #pragma unroll
-        for (int i = 0; i < kAhead; ++i) {
-            const uint32_t e = element(i);
-            ahead[i] = ld<V, true>(a.residual, a.g.at(c, e < a.g.per_channel ? e : 0u));
-        }
+        for (int i = 0; i < kAhead; ++i) ahead[i] = ld_step<V, true, RAGGED>(a.residual, step(i));
     }
     double t1, t2;
-    if constexpr (kSmall) {
+    if constexpr (RAGGED) {
+        t1 = t2 = 0.0;
+#pragma unroll
+        for (int r = R - 1; r >= 0; --r) {
+            const Step p = step(r);
+            const int first = p.valid ? p.held : V;
+#pragma unroll
+            for (int k = 0; k < V; ++k) {
+                const float d = k >= first ? v[r].v[k] - shift : 0.0f;
+                t1 += static_cast<double>(d);
+                t2 += static_cast<double>(d * d);
+            }
+        }
+    } else if constexpr (kSmall) {
         t1 = t2 = 0.0;
 #pragma unroll
         for (int r = R - 1; r >= 0; --r) {
@@ -114,16 +118,6 @@ __global__ __launch_bounds__(T, (kFwdWaves<V, R, L, T, RES, TIGHT>)) void bn_res
             }
             t1 += static_cast<double>(p1);
             t2 += static_cast<double>(p2);
-        }
-    } else if constexpr (kWide) {
-        t1 = t2 = 0.0;
-        const bool pair = a.g.spatial >= kPairSpatial;
-#pragma unroll
-        for (int r = R - 1; r >= 0; r -= 2) {
-            const float d = element(r) < a.g.per_channel ? v[r].v[0] - shift : 0.0f;
-            const float f = element(r - 1) < a.g.per_channel ? v[r - 1].v[0] - shift : 0.0f;
-            add_two(t1, d, f, pair);
-            add_two(t2, d * d, f * f, pair);
         }
     } else {
 #pragma unroll
@@ -143,11 +137,12 @@ __global__ __launch_bounds__(T, (kFwdWaves<V, R, L, T, RES, TIGHT>)) void bn_res
     }
     __syncthreads();
     const FoldCoef k = shared_coef;
-    if constexpr (TIGHT) asm volatile("" : "+v"(lane));      // addresses formed again, not kept: 60 registers, not 112
     const auto apply = [&](int r, [[maybe_unused]] const Pack<V>& from) {
-        const uint32_t e = element(r);
-        if (e < a.g.per_channel) {
-            const size_t where = a.g.at(c, e);
+        Step p{};
+        if constexpr (RAGGED) p = step(r);
+        else p.valid = element(r) < a.g.per_channel;
+        if (p.valid) {
+            if constexpr (!RAGGED) p.at = a.g.at(c, element(r));      // (not the load's: it is formed again, not kept)
             const Pack<V> t = r < R ? v[r < R ? r : 0] : *resident_lds_slot<V, R>(resident_lds, r);
             Pack<V> xn, pre, out;
 #pragma unroll
@@ -157,10 +152,12 @@ __global__ __launch_bounds__(T, (kFwdWaves<V, R, L, T, RES, TIGHT>)) void bn_res
                 out.v[q] = act_apply<ACT>(pre.v[q]);
                 if constexpr (RES) out.v[q] = with_residual(out.v[q], from.v[q], a.res_alpha, a.res_beta);
             }
-            if (a.x_saved) st<V, true>(a.x_saved, where, t);
-            if (a.x_norm) st<V, true>(a.x_norm, where, xn);
-            if (a.pre) st<V, true>(a.pre, where, pre);
-            st<V, true>(a.y, where, out);
+            if (a.x_saved) st_step<V, RAGGED>(a.x_saved, p, t);
+            if (a.x_norm) st_step<V, RAGGED>(a.x_norm, p, xn);
+            if (a.pre) st_step<V, RAGGED>(a.pre, p, pre);
+            // (the shortcut's source may be y itself, whose loads nothing here waits for: a value two lanes hold is written
+            // by the one that owns it)
+            st_step<V, RAGGED, RES>(a.y, p, out);
         }
     };
     if constexpr (RES) {
@@ -175,8 +172,7 @@ __global__ __launch_bounds__(T, (kFwdWaves<V, R, L, T, RES, TIGHT>)) void bn_res
                 if (first + i < kAhead) {
                     from[i] = ahead[first + i < kAhead ? first + i : 0];
                 } else {
-                    const uint32_t e = element(first + i);
-                    from[i] = ld<V, true>(a.residual, a.g.at(c, e < a.g.per_channel ? e : 0u));
+                    from[i] = ld_step<V, true, RAGGED>(a.residual, step(first + i));
                 }
             }
 #pragma unroll
@@ -207,60 +203,43 @@ int allow_large_lds(const void* kernel)
     return PXH_OK;
 }
 
-int launch_resident_forward(const char* who, const ResidentFwdArgs& r, bool vec, int per_thread, uint32_t small,
-                            int activation, hipStream_t s)
+int launch_resident_forward(const char* who, const ResidentFwdArgs& r, const ResidentForm& form, int activation, hipStream_t s)
 {
-    // (with the shortcut's source on top, sixteen values per lane no longer fit the registers of four
-    // workgroups per compute unit: that form keeps the full workgroups)
-    const bool narrow = !r.residual && resident_narrow(r.g, per_thread, vec, false);
-    const dim3 grid(r.g.channels), block(narrow ? kResidentNarrowThreads : kResidentThreads);
+    const dim3 grid(r.g.channels), block(kResidentThreads);
     int large_lds_rc = PXH_OK;
     const auto launch = [&]<int ACT, bool RES>() {
         constexpr int kT = kResidentThreads;
-        if (small) {
-            dispatch_small_form(vec, small, [&]<int V, int R, int T>() {
-                hipLaunchKernelGGL((bn_resident_fwd_kernel<ACT, V, R, 0, T, RES>), grid, dim3(T), 0, s, r);
+        if (form.odd) {
+            dispatch_odd_form(form.odd, r.g, [&]<int V, int R, int T>() {
+                hipLaunchKernelGGL((bn_resident_fwd_kernel<ACT, V, R, 0, T, RES, V == 4>), grid, dim3(T), 0, s, r);
             });
             return;
         }
-        if constexpr (!RES) {
-            if (narrow) {
-                hipLaunchKernelGGL((bn_resident_fwd_kernel<ACT, 1, kResidentNarrowVectors, 0, kResidentNarrowThreads>),
-                                   grid, block, 0, s, r);
-                return;
-            }
+        if (form.small) {
+            dispatch_small_form(form.small, [&]<int R, int T>() {
+                hipLaunchKernelGGL((bn_resident_fwd_kernel<ACT, 4, R, 0, T, RES>), grid, dim3(T), 0, s, r);
+            });
+            return;
         }
-        if constexpr (RES) {
-            // The 128-bit form with the shortcut's source on top of eight vectors of the slice spills at
-            // 64 registers: half-size workgroups with twice the vectors per lane and twice the registers
-            // keep the same two workgroups per compute unit (16 x 512 x 38^2: 26.2 against 30.9 us).
-            if (vec && per_thread <= kResidentVectors) {
-                const size_t vectors = (static_cast<size_t>(r.g.per_channel) + 3) / 4;
-                const dim3 half(kResidentNarrowThreads);
-                if (vectors <= 12u * kResidentNarrowThreads)
-                    hipLaunchKernelGGL((bn_resident_fwd_kernel<ACT, 4, 12, 0, kResidentNarrowThreads, true>), grid,
-                                       half, 0, s, r);
-                else
-                    hipLaunchKernelGGL((bn_resident_fwd_kernel<ACT, 4, 16, 0, kResidentNarrowThreads, true>), grid,
-                                       half, 0, s, r);
-                return;
-            }
-        }
-        if (RES && !vec && per_thread == kResidentScalarMid && r.g.channels > kResidentTight) {
-            if constexpr (RES)
-                hipLaunchKernelGGL((bn_resident_fwd_kernel<ACT, 1, kResidentScalarMid, 0, kT, true, true>), grid, block,
-                                   0, s, r);
-        } else if (!vec && per_thread == kResidentScalarMid) {
-            hipLaunchKernelGGL((bn_resident_fwd_kernel<ACT, 1, kResidentScalarMid, 0, kT, RES>), grid, block, 0, s, r);
-        } else if (per_thread > kResidentVectors) {
+        if (form.per_thread > kResidentVectors) {
             auto kernel = bn_resident_fwd_kernel<ACT, 4, kResidentLargeRegs, kResidentLargeLds, kT, RES>;
             large_lds_rc = allow_large_lds(reinterpret_cast<const void*>(kernel));
             if (large_lds_rc == PXH_OK)
                 hipLaunchKernelGGL(kernel, grid, block, kResidentLargeLdsBytes, s, r);
-        } else if (vec) {
-            hipLaunchKernelGGL((bn_resident_fwd_kernel<ACT, 4, kResidentVectors, 0, kT, RES>), grid, block, 0, s, r);
+        } else if constexpr (RES) {
+            // The 128-bit form with the shortcut's source on top of eight vectors of the slice spills at
+            // 64 registers: half-size workgroups with twice the vectors per lane and twice the registers
+            // keep the same two workgroups per compute unit (16 x 512 x 38^2: 26.2 against 30.9 us).
+            const size_t vectors = (static_cast<size_t>(r.g.per_channel) + 3) / 4;
+            const dim3 half(kResidentNarrowThreads);
+            if (vectors <= 12u * kResidentNarrowThreads)
+                hipLaunchKernelGGL((bn_resident_fwd_kernel<ACT, 4, 12, 0, kResidentNarrowThreads, true>), grid,
+                                   half, 0, s, r);
+            else
+                hipLaunchKernelGGL((bn_resident_fwd_kernel<ACT, 4, 16, 0, kResidentNarrowThreads, true>), grid,
+                                   half, 0, s, r);
         } else {
-            hipLaunchKernelGGL((bn_resident_fwd_kernel<ACT, 1, kResidentVectors, 0, kT, RES>), grid, block, 0, s, r);
+            hipLaunchKernelGGL((bn_resident_fwd_kernel<ACT, 4, kResidentVectors, 0, kT, RES>), grid, block, 0, s, r);
         }
     };
     const bool known = dispatch_activation(activation, [&]<int ACT>() {

@@ -96,6 +96,22 @@ __device__ __forceinline__ void sti(int* p, size_t e, const IPack<V>& v)
     st<V, NT>(reinterpret_cast<float*>(p), e, t);
 }
 
+// Four values that start on any of them: a 128-bit access wants the alignment of a word only.
+typedef float f32x4_word __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ Pack<4> ld_word(const float* p)
+{
+    const f32x4_word t = __builtin_nontemporal_load(reinterpret_cast<const f32x4_word*>(p));
+    return Pack<4>{ { t.x, t.y, t.z, t.w } };
+}
+
+__device__ __forceinline__ void st_word(float* p, const Pack<4>& v)
+{
+    f32x4_word t;
+    t.x = v.v[0]; t.y = v.v[1]; t.z = v.v[2]; t.w = v.v[3];
+    __builtin_nontemporal_store(t, reinterpret_cast<f32x4_word*>(p));
+}
+
 // n_vec elements [0, n_vec) are processed V at a time (n_vec % V == 0), one vector per lane.
 template<int V, bool NT, typename Op>
 __global__ __launch_bounds__(kBlock) void stream_kernel(size_t n_vec, Op op)

@@ -1,0 +1,85 @@
+"""GPU parity of the one-launch training passes on odd planes, whose vectors end with their plane: the checks of the other
+geometries, with their tolerances, at the last size of each form and the first of the next, with one, two and three values
+left in a plane's last vector, and on tensors off a 16-byte boundary; then a shortcut whose source is the output itself."""
+import numpy as np
+import pytest
+import torch
+
+import test_gpu_clipped_backward as clipped
+import test_gpu_epilogue as epilogue
+import test_gpu_epilogue_shortcut as shortcut
+from util import F, assert_bit_exact, gpu, host
+
+pytestmark = pytest.mark.gpu
+
+# vectors of a slice: 1, 64 and 65, 256 and 259, 768 and 771, 1536 (up to 512 channels and beyond) and 1539, 2049, 3072 and
+# 3075, 4096 and 4100 (few channels, which leave, and many), 6144 and 6148, 300 channels that are walked; then values of
+# planes below four: 1024 and 1026, 8192 and 8193
+SHAPES = [(1, 3, 4), (1, 5, 5), (32, 97, 7), (13, 97, 17), (128, 96, 6), (37, 96, 25), (256, 97, 9), (257, 96, 9), (512, 96, 10),
+          (384, 520, 13), (513, 96, 9), (683, 96, 11), (1024, 96, 9), (1025, 300, 11), (1024, 5, 14), (1025, 5, 15), (1025, 96, 15),
+          (1536, 96, 15), (1537, 96, 14), (512, 5, 2), (513, 97, 2), (4096, 96, 2), (2731, 96, 3)]
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from pixienn_amd import ops as o
+    return o
+
+
+@pytest.mark.parametrize("act", ["leaky", "mish"])
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_odd_planes(ops, oracle, monkeypatch, shape, act):
+    for module in (epilogue, clipped, shortcut):
+        monkeypatch.setattr(module, "TRAIN_SHAPES", [shape])
+    epilogue.test_bn_train_forward_matches_oracle(ops, oracle, act)
+    epilogue.test_bn_backward_matches_oracle(ops, oracle, act, False)
+    epilogue.test_bn_backward_matches_oracle(ops, oracle, act, True)
+    clipped.test_bn_backward_clipped_matches_rescale_clip_then_backward(ops, oracle, act, False)
+    monkeypatch.setattr(shortcut, "EXTRA_SHAPES", [])
+    shortcut.test_training_epilogue_with_shortcut_is_the_two_calls_to_the_bit(ops, act)
+
+
+def layer(shape, offset, seed=3):
+    """x, y, delta and the parameters of a layer, the tensors `offset` values off a 16-byte boundary."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    n = int(np.prod(shape))
+
+    def tensor():
+        place = torch.empty(n + 4, device="cuda")[offset:offset + n].view(shape)
+        return place.copy_(torch.empty(n, device="cuda").normal_(generator=g).view(shape))
+
+    return [tensor() for _ in range(3)], [torch.empty(shape[1], device="cuda").normal_(generator=g).abs_() + 0.5 for _ in range(6)]
+
+
+@pytest.mark.parametrize("offset", [1, 2, 3])
+@pytest.mark.parametrize("shape", [(6, 100, 4, 4), (40, 96, 13, 13)], ids=str)
+def test_tensors_off_a_boundary(ops, shape, offset):
+    """The same values as from tensors that begin on a word of their own: odd planes to the bit (one form), others within
+    the rounding of sums in another order."""
+    found = []
+    for at in (offset, 0):
+        (x, y, delta), (scale, bias, rm, rv, su, bu) = layer(shape, at)
+        mean, var = torch.zeros_like(rm), torch.zeros_like(rm)
+        source = layer(shape, at)[0][0].clone()
+        ops.bn_train_act_forward(x, y, mean, var, rm, rv, scale, bias, "leaky")
+        ops.bn_act_backward_clipped(delta, x, mean, var, scale, bias, su, bu, "leaky", 1e-3, 0.0)
+        assert torch.equal(x, source)
+        found.append([host(t) for t in (y, mean, var, rm, rv, su, bu, delta)])
+    for a, b in zip(*found):
+        if shape[2] % 2:
+            assert_bit_exact(a, b)
+        else:
+            assert np.max(np.abs(a.astype(np.float64) - b)) <= 1e-5 * np.sqrt(np.mean(b.astype(np.float64) ** 2))
+
+
+@pytest.mark.parametrize("shape", [(64, 100, 5, 5), (33, 520, 13, 13), (40, 100, 19, 19)], ids=str)
+def test_shortcut_source_is_the_output(ops, shape):
+    found = []
+    for alias in (False, True):
+        (x, y, source), (scale, bias, rm, rv, _, _) = layer(shape, 0)
+        mean, var = torch.zeros_like(rm), torch.zeros_like(rm)
+        out = source if alias else y
+        ops.bn_train_act_shortcut_forward(x, out, mean, var, rm, rv, scale, bias, "leaky", source)
+        found.append(host(out))
+    assert_bit_exact(*found)
