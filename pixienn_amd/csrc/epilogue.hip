@@ -370,8 +370,24 @@ __device__ __forceinline__ void for_each_item(const ReduceGeom& g, uint32_t c, u
     }
 }
 
+// Odd planes: the vector at `off` of a plane, the last one moved back to end with it.  The values that it shares with the one
+// in front (of the segment in front, even) stay out of the sums and are not written; every value goes into a double of
+// its own.
+template<bool RAGGED>
+__device__ __forceinline__ int ragged_start(int off, int spatial)
+{
+    return RAGGED && off + 4 > spatial ? spatial - 4 : off;
+}
+
+template<int V, bool NT, bool RAGGED>
+__device__ __forceinline__ Pack<V> ld_at(const float* p, size_t e)
+{
+    if constexpr (RAGGED) return ld_word<NT>(p + e);
+    else return ld<V, NT>(p, e);
+}
+
 // ---- statistics: S1 = sum(x - K), S2 = sum((x - K)^2), K = first element of the channel ----
-template<int V, bool NT>
+template<int V, bool NT, bool RAGGED = false>
 __global__ __launch_bounds__(kBlock) void bn_stats_partial_kernel(const float* x, ReduceGeom g, double2* partial)
 {
     __shared__ double slots[2][kBlock / kWave];
@@ -385,7 +401,21 @@ __global__ __launch_bounds__(kBlock) void bn_stats_partial_kernel(const float* x
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) {
             const int off = seg0 + (u * kWave + lane) * V;
-            if (off < seg1) v[u] = ld<V, NT>(x, base + off);
+            if (off < seg1) v[u] = ld_at<V, NT, RAGGED>(x, base + ragged_start<RAGGED>(off, g.spatial));
+        }
+        if constexpr (RAGGED) {
+#pragma unroll
+            for (int u = 0; u < kLoads; ++u) {
+                const int off = seg0 + (u * kWave + lane) * V;
+                const int own = off < seg1 ? off - ragged_start<RAGGED>(off, g.spatial) : V;
+#pragma unroll
+                for (int k = 0; k < V; ++k) {
+                    const float d = k >= own ? v[u].v[k] - shift : 0.0f;
+                    s1 += static_cast<double>(d);
+                    s2 += static_cast<double>(d * d);
+                }
+            }
+            return;
         }
         float a1 = 0.0f, a2 = 0.0f;
 #pragma unroll
@@ -453,7 +483,7 @@ __global__ __launch_bounds__(kBlock) void bn_stats_finish_kernel(const float* x,
 // WRITE (the bias-only layer, which has no dx pass): d' goes back into delta.  With kFirst nothing is
 // written (the delta is still needed as it came); with kRedo the pass also runs, writing, when nothing
 // has to change but the activation has a gradient to apply.
-template<int ACT, bool BN, bool WRITE, int V, bool NT, int MODE = kPlain>
+template<int ACT, bool BN, bool WRITE, int V, bool NT, int MODE = kPlain, bool RAGGED = false>
 __global__ __launch_bounds__(kBlock) void bwd_partial_kernel(BackwardArgs a, ReduceGeom g, double2* partial,
                                                              ClipArgs clip = ClipArgs{})
 {
@@ -486,10 +516,11 @@ __global__ __launch_bounds__(kBlock) void bwd_partial_kernel(BackwardArgs a, Red
         for (int u = 0; u < kLoads; ++u) {
             const int off = seg0 + (u * kWave + lane) * V;
             if (off < seg1) {
-                d[u] = ld<V, NT>(a.delta, base + off);
-                if constexpr (BN) xv[u] = ld<V, NT>(a.x, base + off);
+                const size_t at = base + ragged_start<RAGGED>(off, g.spatial);
+                d[u] = ld_at<V, NT, RAGGED>(a.delta, at);
+                if constexpr (BN) xv[u] = ld_at<V, NT, RAGGED>(a.x, at);
                 if constexpr (ACT != PXH_LINEAR) {
-                    if (!recompute) pv[u] = ld<V, NT>(a.pre, base + off);
+                    if (!recompute) pv[u] = ld_at<V, NT, RAGGED>(a.pre, at);
                 }
             }
         }
@@ -499,12 +530,14 @@ __global__ __launch_bounds__(kBlock) void bwd_partial_kernel(BackwardArgs a, Red
         for (int u = 0; u < kLoads; ++u) {
             const int off = seg0 + (u * kWave + lane) * V;
             if (off < seg1) {
+                const int start = ragged_start<RAGGED>(off, g.spatial);
                 if constexpr (MODE != kPlain) {
 #pragma unroll
                     for (int q = 0; q < V; ++q) {
                         const float dv = d[u].v[q];
                         if constexpr (MODE == kFirst) {
-                            fq += dv * dv;
+                            if constexpr (RAGGED) sq += static_cast<double>(q >= off - start ? dv * dv : 0.0f);
+                            else fq += dv * dv;
                             peak = fmaxf(peak, fabsf(dv));
                         } else {
                             d[u].v[q] = rescaled_clipped(dv, factor, limit);
@@ -520,11 +553,20 @@ __global__ __launch_bounds__(kBlock) void bwd_partial_kernel(BackwardArgs a, Red
                 }
 #pragma unroll
                 for (int q = 0; q < V; ++q) {
-                    fa += d[u].v[q];
-                    if constexpr (BN) fb += d[u].v[q] * (xv[u].v[q] - k.mean);
+                    if constexpr (RAGGED) {
+                        const float t = d[u].v[q];
+                        sa += static_cast<double>(q >= off - start ? t : 0.0f);
+                        if constexpr (BN) sb += static_cast<double>(q >= off - start ? t * (xv[u].v[q] - k.mean) : 0.0f);
+                    } else {
+                        fa += d[u].v[q];
+                        if constexpr (BN) fb += d[u].v[q] * (xv[u].v[q] - k.mean);
+                    }
                 }
                 if constexpr (WRITE && (ACT != PXH_LINEAR || MODE == kRedo)) {
-                    if (ACT != PXH_LINEAR || changes) st<V, NT>(a.delta, base + off, d[u]);
+                    if (ACT != PXH_LINEAR || changes) {
+                        if constexpr (RAGGED) st_own(a.delta + base + start, d[u], off - start);
+                        else st<V, NT>(a.delta, base + off, d[u]);
+                    }
                 }
             }
         }
@@ -852,9 +894,8 @@ ClippedRegions clipped_regions(void* ws, int batch, int channels, int spatial)
     return r;
 }
 
-constexpr size_t kGroupScalars = 7u << 20;
 constexpr int kGroupAlone = 512;
-constexpr size_t kGroupFewest = 1u << 19, kGroupFewestSmooth = 1u << 20;
+constexpr size_t kGroupFewest = 1u << 19, kGroupFewestSmooth = 1u << 20, kGroupFewestOddSmooth = 7u << 20;
 
 // The groups of a backward (members 0: none).  A plain call and a clipped one take the same form, so that they agree to
 // the bit where nothing is rescaled or clamped, and what they exchange has to fit the workspaces they ask for.
@@ -863,9 +904,21 @@ constexpr size_t kGroupFewest = 1u << 19, kGroupFewestSmooth = 1u << 20;
 // needs no workspace, and callers on several streams may pass none: groups that exchange something are not for those slices
 // (16 x 128 x 76^2: 37 us where groups would take 33, mish 66 and 47).  A group of one member exchanges nothing, and from
 // kGroupAlone channels on, two to a compute unit, it is ahead (16 x 512 x 38^2: 29 -> 27 us; 16 x 384 x 38^2 22.3, 22.6), except
-// where an exponential has to be computed (37 -> 41).  Odd planes, whose values come one at a time, gain only where the
-// tensors are large and the gradient is a select; the line lies between the first two of
-// 6 x 72 x 135 x 77 25 -> 27 us, 8 x 96 x 135 x 77 41 -> 37, 32 x 64 x 75^2 48 -> 41; mish 35 -> 41, 54 -> 55, 65 -> 62.
+// where an exponential has to be computed (37 -> 41).
+//
+// Odd planes take groups by the same line where the gradient is a select.  An exponential moves the line up: below it a call
+// that clamps throughout loses more than the others gain.  Three or five launches -> groups, us: plain; clipped with nothing
+// to change, rescaled, and clamped throughout (the launches with one value per access)
+//   2 x 16 x 151^2       leaky 13.5 -> 11.9; 18.6 -> 16.4, 18.6 -> 16.4, 22.3 -> 24.5
+//   4 x 32 x 207^2             28.4 -> 23.4; 35.8 -> 28.1, 35.8 -> 28.0, 43.8 -> 46.0   mish 33.9 -> 33.2; 41.5 -> 39.0, 41.7 -> 40.2, 54.5 -> 69.7
+//   64 x 24 x 75 x 45          28.4 -> 23.4; 35.8 -> 29.0, 35.7 -> 28.8, 43.5 -> 46.4        33.6 -> 31.8; 41.7 -> 39.1, 41.7 -> 40.4, 54.5 -> 69.2
+//   8 x 96 x 135 x 77          41   -> 26.4; 48   -> 31.2, 48   -> 31.1, 61   -> 52.5        46.4 -> 37.6; 52.6 -> 43.5, 52.8 -> 45.8, 72.3 -> 78.7
+//   16 x 64 x 151^2            88   -> 66.5; 97   -> 73.2, 97   -> 73.3, 124  -> 118         93.2 -> 82.9; 102  -> 91.6, 104  -> 109,  144  -> 164
+// (8 x 96 x 135 x 77 and 16 x 64 x 151^2, mish, in launches of one value per access: 51, 59, 59, 84 and 110, 117, 117, 169.)
+//
+// As many members as make kGroupFill workgroups of a whole number of channels: a few more than the machine holds run in a
+// second round (8 x 96 x 135 x 77 in 576 and in 480: 33.6 -> 26.4, 64 x 200 x 25^2 600 and 400: 34.5 -> 28.8,
+// 9 x 20 x 203 x 251 520 and 500: 37.0 -> 29.3).
 //
 // Small tensors (which the caches hold for the launches that read them twice) stay with those launches: a group's second one
 // costs them more where it has something to do.  Three or five launches -> groups, us: plain; clipped with nothing to change,
@@ -879,11 +932,12 @@ GroupPlan grouped_backward(int batch, int channels, int spatial, bool vec, int p
 {
     const size_t total = static_cast<size_t>(batch) * channels * spatial;
     if (total < (selects(activation) ? kGroupFewest : kGroupFewestSmooth)) return GroupPlan{};
-    if (!vec && (!selects(activation) || total < kGroupScalars)) return GroupPlan{};
+    if (!vec && (spatial < kOddSpatial || (!selects(activation) && total < kGroupFewestOddSmooth))) return GroupPlan{};
     if (per_thread && (!selects(activation) || channels < kGroupAlone)) return GroupPlan{};
     const uint32_t places = group_places(s);
     // (as few members as hold the slice where the words of more would not fit: up to three channels of a few thousand vectors)
-    for (const size_t workgroups: { kGroupFill, static_cast<size_t>(1) }) {
+    const size_t whole = kGroupFill / channels * channels;
+    for (const size_t workgroups: { whole > 0 ? whole : 1, static_cast<size_t>(1) }) {
         const GroupPlan p = group_plan(batch, channels, spatial, vec, workgroups, places);
         if (per_thread && p.members > 1) return GroupPlan{};
         if (p.members <= 1 ||
@@ -913,7 +967,8 @@ int launch_stats(const float* x, float* mean, float* var, float* rolling_mean, f
         if (nt) hipLaunchKernelGGL((bn_stats_partial_kernel<4, true>), grid, dim3(kBlock), 0, stream, x, g, partial);
         else hipLaunchKernelGGL((bn_stats_partial_kernel<4, false>), grid, dim3(kBlock), 0, stream, x, g, partial);
     } else {
-        hipLaunchKernelGGL((bn_stats_partial_kernel<1, false>), grid, dim3(kBlock), 0, stream, x, g, partial);
+        if (spatial >= kOddSpatial) hipLaunchKernelGGL((bn_stats_partial_kernel<4, false, true>), grid, dim3(kBlock), 0, stream, x, g, partial);
+        else hipLaunchKernelGGL((bn_stats_partial_kernel<1, false>), grid, dim3(kBlock), 0, stream, x, g, partial);
     }
     int rc = check_launch("bn_stats_partial");
     if (rc) return rc;
@@ -1264,6 +1319,9 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
         } else if (vec) {
             hipLaunchKernelGGL((bwd_partial_kernel<ACT, true, false, 4, false, MODE>), grid, dim3(kBlock), 0, s, b, g,
                                partial, clip);
+        } else if (spatial >= kOddSpatial) {
+            hipLaunchKernelGGL((bwd_partial_kernel<ACT, true, false, 4, false, MODE, true>), grid, dim3(kBlock), 0, s, b, g,
+                               partial, clip);
         } else {
             hipLaunchKernelGGL((bwd_partial_kernel<ACT, true, false, 1, false, MODE>), grid, dim3(kBlock), 0, s, b, g,
                                partial, clip);
@@ -1375,6 +1433,9 @@ static int bias_backward(const char* who, float* delta, const float* pre_activat
     const auto sums = [&]<int ACT, bool WRITE, int MODE>() {
         if (vec) {
             hipLaunchKernelGGL((bwd_partial_kernel<ACT, false, WRITE, 4, false, MODE>), grid, dim3(kBlock), 0, s, b, g,
+                               partial, clip);
+        } else if (spatial >= kOddSpatial) {
+            hipLaunchKernelGGL((bwd_partial_kernel<ACT, false, WRITE, 4, false, MODE, true>), grid, dim3(kBlock), 0, s, b, g,
                                partial, clip);
         } else {
             hipLaunchKernelGGL((bwd_partial_kernel<ACT, false, WRITE, 1, false, MODE>), grid, dim3(kBlock), 0, s, b, g,

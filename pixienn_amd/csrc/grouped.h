@@ -20,7 +20,7 @@ constexpr int kLost = 32, kTickets = kLost + 1;
 
 struct GroupGeom {
     ResidentGeom g;
-    uint32_t items;         // vectors (or values) of a channel's slice
+    uint32_t items;         // vectors of a channel's slice
     uint32_t span;          // of a member: a whole number of wavefronts
     uint32_t members;       // of a channel
     uint32_t image_skip;    // values between the end of a channel's plane and its plane in the next image
@@ -136,7 +136,7 @@ constexpr uint32_t kGroupMost = kWave;
 static_assert(kGroupMost * kFirstWords <= kGroupThreads, "a thread per word");
 constexpr uint32_t kGroupShare = 8;
 
-constexpr uint32_t kGroupItems = 12 * kGroupThreads;      // vectors that a member holds, or four times as many values
+constexpr uint32_t kGroupItems = 12 * kGroupThreads;      // vectors that a member holds
 constexpr size_t kGroupFill = 512;
 
 constexpr uint32_t kLooks = 1u << 22;
@@ -158,7 +158,7 @@ struct GroupPlan {
     uint32_t places;
 };
 
-// How a slice is split over workgroups that hold `per_member` vectors (or values) each, on a stream of `places`: into as many
+// How a slice is split over workgroups that hold `per_member` vectors each, on a stream of `places`: into as many
 // members as make `workgroups` of them, none of fewer than four vectors a lane.  Where those would be more than kGroupMost
 // (up to seven channels) the launches that wait for nothing keep the slice.  64 members would serve it where nothing is rescaled
 // and lose where something is or is clamped: 4 x 6 x 512^2 36.5 -> 30.6, 36.5 -> 40.5 and 46 -> 49 us, 8 x 4 x 304^2 26 -> 22.8,
@@ -179,7 +179,8 @@ inline GroupPlan group_plan(int batch, int channels, int spatial, bool vec, size
 {
     const size_t per_channel = static_cast<size_t>(batch) * spatial;
     if (per_channel * channels >= 1ull << 30) return GroupPlan{};      // places are 32-bit byte offsets
-    return split_slice(vec ? per_channel / 4 : per_channel, vec ? kGroupItems : 4 * kGroupItems, channels, workgroups, places);
+    const size_t items = vec ? per_channel / 4 : static_cast<size_t>(batch) * ((spatial + 3) / 4);      // vectors, as odd_slice
+    return split_slice(items, kGroupItems, channels, workgroups, places);
 }
 
 inline GroupGeom group_geom(const GroupPlan& p, int batch, int channels, int spatial)

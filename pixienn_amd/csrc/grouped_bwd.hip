@@ -7,6 +7,13 @@
 namespace pxh {
 namespace {
 
+template<bool RAGGED>
+__device__ __forceinline__ Pack<4> load(const float* p)
+{
+    if constexpr (RAGGED) return ld_word<true>(p);
+    else return ld<4, true>(p, 0);
+}
+
 // What bounds these launches is memory: x and the delta are read once and the delta written once, where the three launches
 // read both twice and a workgroup that holds a channel alone reads x twice.  Two workgroups to a compute unit (128
 // registers a lane, 64 KB of LDS each) hold 24 vectors a lane between them; rounds of load, sums, exchange and store cost
@@ -23,12 +30,12 @@ namespace {
 //
 // One member's share of channel c; `factor` and `limit` are the plan's (kRedo only).  It keeps d' = delta * act'(pre) in
 // R steps of a lane and x beside it, the first R - L steps in registers and L in LDS, so that each tensor is read once.
-template<int ACT, int V, int R, int L, int MODE>
+template<int ACT, bool RAGGED, int R, int L, int MODE>
 __device__ __forceinline__ void grouped_bwd_member(const ResidentBwdArgs& a, const GroupGeom& gg, const uint32_t c,
                                                    const uint32_t member, uint32_t& next_ticket,
                                                    [[maybe_unused]] const float factor, [[maybe_unused]] const float limit)
 {
-    constexpr int T = kGroupThreads;
+    constexpr int T = kGroupThreads, V = 4;
     constexpr int X = R - L;
     extern __shared__ __align__(16) float grouped_lds[];
     __shared__ double slots[MODE == kFirst ? 3 : 2][T / kWave];
@@ -41,13 +48,27 @@ __device__ __forceinline__ void grouped_bwd_member(const ResidentBwdArgs& a, con
     const auto item = [&](int r) { return begin + static_cast<uint32_t>(r * T) + lane; };
     // bytes to vector i of the slice (a tensor of these launches has fewer than 2^32: no 64-bit multiplies)
     const auto place = [&](uint32_t i) {
-        const uint32_t e = i * V;
-        return (e + channel_at + gg.g.by_spatial.div(e) * gg.image_skip) * 4u;
+        if constexpr (RAGGED) {
+            uint32_t n, j;
+            gg.g.by_row.divmod(i, n, j);
+            return (n * (gg.image_skip + gg.g.spatial) + channel_at + min(j * V, gg.g.spatial - static_cast<uint32_t>(V))) * 4u;
+        } else {
+            const uint32_t e = i * V;
+            return (e + channel_at + gg.g.by_spatial.div(e) * gg.image_skip) * 4u;
+        }
+    };
+    // values of vector i that the one in front holds too: they stay out of the sums, and are not written (the vector in front
+    // may be another member's)
+    const auto held = [&](uint32_t i) {
+        uint32_t n, j;
+        gg.g.by_row.divmod(i, n, j);
+        const int beyond = static_cast<int>(j) * V + V - gg.g.spatial;
+        return beyond > 0 ? beyond : 0;
     };
     // kStep steps at a time, a group's loads in flight while the sums pass over the group before it; the LDS part first:
     // its registers are free again after that.  Groups past the end of the share are left out, and in the one that holds
     // the end a lane past it reads the share's first vector and adds nothing: no branch around a load.
-    constexpr int kStep = V == 4 ? 2 : 8;
+    constexpr int kStep = 2;
     static_assert(R % kStep == 0 && L % kStep == 0, "steps come in whole groups");
     const auto any = [&](int top) { return begin + static_cast<uint32_t>((top - kStep + 1) * T) < end; };
     Pack<V> d[R], x[R];
@@ -56,8 +77,8 @@ __device__ __forceinline__ void grouped_bwd_member(const ResidentBwdArgs& a, con
         for (int i = 0; i < kStep; ++i) {
             const uint32_t at = item(top - i);
             const uint32_t where = place(at < end ? at : begin);
-            d[top - i] = ld<V, true>(at_byte(a.b.delta, where), 0);
-            x[top - i] = ld<V, true>(at_byte(a.b.x, where), 0);
+            d[top - i] = load<RAGGED>(at_byte(a.b.delta, where));
+            x[top - i] = load<RAGGED>(at_byte(a.b.x, where));
         }
     };
     if (any(R - 1)) fetch(R - 1);
@@ -67,15 +88,16 @@ __device__ __forceinline__ void grouped_bwd_member(const ResidentBwdArgs& a, con
     const auto early_terms = [&] { if (threadIdx.x < kWave) terms = variance_terms(var_in); };
     double figures[MODE == kFirst ? kFirstWords : kSumWords] = {};
     float peak = 0.0f;
-    // a vector in fp32, vectors in doubles, as in the small forms
+    // a vector in fp32, vectors in doubles, as in the small forms; on odd planes every value, as there
     const auto take = [&](int r) {
-        const bool valid = item(r) < end;
+        const int own = item(r) >= end ? V : RAGGED ? held(item(r)) : 0;
         float va = 0.0f, vb = 0.0f, vq = 0.0f;
 #pragma unroll
         for (int q = 0; q < V; ++q) {
-            float t = valid ? d[r].v[q] : 0.0f;
+            float t = q >= own ? d[r].v[q] : 0.0f;
             if constexpr (MODE == kFirst) {
-                vq += t * t;
+                if constexpr (RAGGED) figures[2] += static_cast<double>(t * t);
+                else vq += t * t;
                 peak = fmaxf(peak, fabsf(t));
             }
             if constexpr (MODE == kRedo) t = rescaled_clipped(t, factor, limit);
@@ -89,15 +111,22 @@ __device__ __forceinline__ void grouped_bwd_member(const ResidentBwdArgs& a, con
         }
 #pragma unroll
         for (int q = 0; q < V; ++q) {
-            const float t = ACT == PXH_LINEAR || valid ? d[r].v[q] : 0.0f;
+            const float t = ACT == PXH_LINEAR || q >= own ? d[r].v[q] : 0.0f;
             d[r].v[q] = t;
-            const float u = t * (x[r].v[q] - k.mean);
-            va += t;
-            vb += valid ? u : 0.0f;
+            const float u = q >= own ? t * (x[r].v[q] - k.mean) : 0.0f;
+            if constexpr (RAGGED) {
+                figures[0] += static_cast<double>(t);
+                figures[1] += static_cast<double>(u);
+            } else {
+                va += t;
+                vb += u;
+            }
         }
-        figures[0] += static_cast<double>(va);
-        figures[1] += static_cast<double>(vb);
-        if constexpr (MODE == kFirst) figures[2] += static_cast<double>(vq);
+        if constexpr (!RAGGED) {
+            figures[0] += static_cast<double>(va);
+            figures[1] += static_cast<double>(vb);
+            if constexpr (MODE == kFirst) figures[2] += static_cast<double>(vq);
+        }
         if (r >= X) lds[(r - X) * T] = x[r];
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -176,7 +205,11 @@ __device__ __forceinline__ void grouped_bwd_member(const ResidentBwdArgs& a, con
     for (int r = 0; r < R; ++r) {
         if (r % kStep == 0 && !any(r + kStep - 1)) break;
         const Pack<V> out = leave(r);
-        if (item(r) < end) st<V, true>(at_byte(a.b.delta, place(item(r))), 0, out);
+        if (item(r) < end) {
+            float* const to = at_byte(a.b.delta, place(item(r)));
+            if constexpr (RAGGED) st_own(to, out, held(item(r)));
+            else st<V, true>(to, 0, out);
+        }
     }
 }
 
@@ -199,7 +232,7 @@ __device__ __forceinline__ void grouped_rescale_updates(const ResidentBwdArgs& a
 }
 
 // A member's share of a finished channel where others have to be gone over again.
-template<int V>
+template<bool RAGGED>
 __device__ __forceinline__ void grouped_rescale_member(const ResidentBwdArgs& a, const GroupGeom& gg, uint32_t c,
                                                        uint32_t member, float factor)
 {
@@ -207,11 +240,11 @@ __device__ __forceinline__ void grouped_rescale_member(const ResidentBwdArgs& a,
     const uint32_t end = min(gg.items, begin + gg.span);
 #pragma unroll 1
     for (uint32_t i = begin + threadIdx.x; i < end; i += kGroupThreads) {
-        const size_t where = gg.g.at(c, i * V);
-        Pack<V> t = ld<V, true>(a.b.delta, where);
+        const Step p = step_of<4, RAGGED>(gg.g, c, i);
+        Pack<4> t = ld_step<4, true, RAGGED>(a.b.delta, p);
 #pragma unroll
-        for (int q = 0; q < V; ++q) t.v[q] = factor * t.v[q];
-        st<V, true>(a.b.delta, where, t);
+        for (int q = 0; q < 4; ++q) t.v[q] = factor * t.v[q];
+        st_step<4, RAGGED, true>(a.b.delta, p, t);
     }
     if (member == 0) grouped_rescale_updates(a, gg, c, factor);
 }
@@ -220,28 +253,33 @@ __device__ __forceinline__ void grouped_rescale_member(const ResidentBwdArgs& a,
 // written.  Share by share with a number taken for each, 16 x 128 x 152^2 rescaled 202 -> 191 us, 16 x 64 x 152^2 108 -> 99,
 // 4 x 16 x 416^2 60 -> 53.  (Five launches that read both tensors twice: 164, 91 and 51, but 164, 91 and 51 also where nothing
 // is rescaled, 127, 67 and 38 here; the bytes are the same, and theirs come in one stream.)
-template<int V>
+template<bool RAGGED>
 __device__ __forceinline__ void grouped_rescale_all(const ResidentBwdArgs& a, const GroupGeom& gg, float factor)
 {
-    constexpr int kLoads = V == 4 ? 6 : 12;
-    const uint32_t items = static_cast<uint32_t>(gg.g.channels) * gg.items;
+    constexpr int kLoads = 6;
+    const uint32_t values = static_cast<uint32_t>(gg.g.channels) * gg.g.per_channel;
+    const uint32_t items = values / 4;      // the values of an odd tensor's end one by one, below
     const uint32_t step = gridDim.x * (kLoads * kGroupThreads);
     const auto at = [&](uint32_t first, int u) { return first + static_cast<uint32_t>(u * kGroupThreads) + threadIdx.x; };
-    Pack<V> t[2][kLoads];
-    const auto fetch = [&](Pack<V> (&p)[kLoads], uint32_t first) {
+    Pack<4> t[2][kLoads];
+    const auto fetch = [&](Pack<4> (&p)[kLoads], uint32_t first) {
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) {
             const uint32_t i = at(first, u);
-            p[u] = ld<V, true>(a.b.delta, static_cast<size_t>(i < items ? i : 0) * V);
+            p[u] = load<RAGGED>(a.b.delta + static_cast<size_t>(i < items ? i : 0) * 4);
         }
     };
-    const auto leave = [&](Pack<V> (&p)[kLoads], uint32_t first) {
+    const auto leave = [&](Pack<4> (&p)[kLoads], uint32_t first) {
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) {
             const uint32_t i = at(first, u);
 #pragma unroll
-            for (int q = 0; q < V; ++q) p[u].v[q] = factor * p[u].v[q];
-            if (i < items) st<V, true>(a.b.delta, static_cast<size_t>(i) * V, p[u]);
+            for (int q = 0; q < 4; ++q) p[u].v[q] = factor * p[u].v[q];
+            float* const to = a.b.delta + static_cast<size_t>(i) * 4;
+            if (i < items) {
+                if constexpr (RAGGED) st_word(to, p[u]);
+                else st<4, true>(to, 0, p[u]);
+            }
         }
     };
     uint32_t first = blockIdx.x * (kLoads * kGroupThreads);
@@ -255,24 +293,27 @@ __device__ __forceinline__ void grouped_rescale_all(const ResidentBwdArgs& a, co
         if (first < items) fetch(t[0], first);
         leave(t[1], second);
     }
+    if (RAGGED && blockIdx.x == 0 && threadIdx.x < values - 4 * items) {
+        float* const last = a.b.delta + 4 * static_cast<size_t>(items) + threadIdx.x;
+        *last = factor * *last;
+    }
     for (uint32_t c = blockIdx.x; c < static_cast<uint32_t>(gg.g.channels); c += gridDim.x)
         grouped_rescale_updates(a, gg, c, factor);
 }
 
 // What the second launch leaves where a wait of the first gave up: NaNs everywhere.  By one workgroup.
-template<int V>
+template<bool RAGGED>
 __device__ __forceinline__ void leave_lost(const ResidentBwdArgs& a, const GroupGeom& gg, uint32_t all)
 {
     const float nan = __int_as_float(0x7FC00000);
     if (threadIdx.x == 0 && a.clip.norm_out) *a.clip.norm_out = nan;
-    Pack<V> nans;
-#pragma unroll
-    for (int q = 0; q < V; ++q) nans.v[q] = nan;
+    const Pack<4> nans{ { nan, nan, nan, nan } };
     for (uint32_t number = 0; number < all; ++number) {
         uint32_t c, member;
         gg.by_members.divmod(number, c, member);
         const uint32_t begin = member * gg.span, end = min(gg.items, begin + gg.span);
-        for (uint32_t i = begin + threadIdx.x; i < end; i += kGroupThreads) st<V, true>(a.b.delta, gg.g.at(c, i * V), nans);
+        for (uint32_t i = begin + threadIdx.x; i < end; i += kGroupThreads)
+            st_step<4, RAGGED>(a.b.delta, step_of<4, RAGGED>(gg.g, c, i), nans);
         if (member == 0 && threadIdx.x == 0) {
             a.bias_updates[c] = a.scale_updates[c] = nan;
             if (a.mean_delta) a.mean_delta[c] = nan;
@@ -293,11 +334,11 @@ struct ShareNumbers {
 };
 
 // The first launch of a clipped backward and the one behind it share the work as those of resident_bwd.hip do.
-template<int ACT, int V, int R, int L, int MODE>
+template<int ACT, bool RAGGED, int R, int L, int MODE>
 __global__ __launch_bounds__(kGroupThreads, 4) void bn_grouped_bwd_kernel(ResidentBwdArgs a, GroupGeom gg)
 {
     // two workgroups to a compute unit, which group_places() counts on: 128 registers a lane, and this LDS
-    static_assert(static_cast<size_t>(L) * V * 4 * kGroupThreads == kGroupLdsBytes);
+    static_assert(static_cast<size_t>(L) * 16 * kGroupThreads == kGroupLdsBytes);
     __shared__ uint32_t taken;
     float factor = 1.0f, limit = 0.0f;
     const uint32_t all = static_cast<uint32_t>(gg.g.channels) * gg.members;
@@ -309,13 +350,13 @@ __global__ __launch_bounds__(kGroupThreads, 4) void bn_grouped_bwd_kernel(Reside
         }
         // (one workgroup sees to what never happens: the others leave in the usual case with nothing more to look at)
         if ((plan.work || blockIdx.x == 0) && gg.members > 1 && gg.tickets[kLost]) {
-            if (blockIdx.x == 0) leave_lost<V>(a, gg, all);
+            if (blockIdx.x == 0) leave_lost<RAGGED>(a, gg, all);
             return;
         }
         if (!plan.work) return;
         factor = plan.factor;
         limit = plan.clip;
-        if (!(plan.work & kBeyond)) return grouped_rescale_all<V>(a, gg, factor);
+        if (!(plan.work & kBeyond)) return grouped_rescale_all<RAGGED>(a, gg, factor);
     }
     uint32_t* const tickets = gg.tickets + (MODE == kRedo ? 1 : 0);
     uint32_t number = blockIdx.x;
@@ -329,10 +370,10 @@ __global__ __launch_bounds__(kGroupThreads, 4) void bn_grouped_bwd_kernel(Reside
         uint32_t c, member;
         gg.by_members.divmod(__builtin_amdgcn_readfirstlane(mine), c, member);      // the same in every lane
         if (MODE != kRedo || !a.channel_done[c]) {
-            grouped_bwd_member<ACT, V, R, L, MODE>(a, gg, c, member, taken, factor, limit);
+            grouped_bwd_member<ACT, RAGGED, R, L, MODE>(a, gg, c, member, taken, factor, limit);
             return true;
         }
-        if (factor != 1.0f) grouped_rescale_member<V>(a, gg, c, member, factor);
+        if (factor != 1.0f) grouped_rescale_member<RAGGED>(a, gg, c, member, factor);
         return false;
     };
     ShareNumbers numbers{ gg.members > 1 ? tickets : nullptr, taken, number };
@@ -390,7 +431,7 @@ int launch_grouped_backward(const char* who, const ResidentBwdArgs& r, const Gro
     int rc = PXH_OK;
     const auto launch = [&]<int ACT, int MODE>() {
         const dim3 grid(all < places ? all : places), block(kGroupThreads);
-        const auto kernel = vec ? bn_grouped_bwd_kernel<ACT, 4, 12, 8, MODE> : bn_grouped_bwd_kernel<ACT, 1, 48, 32, MODE>;
+        const auto kernel = vec ? bn_grouped_bwd_kernel<ACT, false, 12, 8, MODE> : bn_grouped_bwd_kernel<ACT, true, 12, 8, MODE>;
         if (!rc) rc = allow_large_lds(reinterpret_cast<const void*>(kernel));
         if (!rc) hipLaunchKernelGGL(kernel, grid, block, kGroupLdsBytes, s, r, g);
     };

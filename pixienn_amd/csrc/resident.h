@@ -148,7 +148,7 @@ __device__ __forceinline__ Step step_of(const ResidentGeom& g, uint32_t c, uint3
 template<int V, bool NT, bool RAGGED>
 __device__ __forceinline__ Pack<V> ld_step(const float* p, const Step& s)
 {
-    if constexpr (RAGGED) return ld_word(p + s.at);
+    if constexpr (RAGGED) return ld_word<NT>(p + s.at);
     else return ld<V, NT>(p, s.at);
 }
 
@@ -158,12 +158,10 @@ __device__ __forceinline__ void st_step(float* p, const Step& s, const Pack<V>& 
 {
     if constexpr (!RAGGED) {
         st<V, true>(p, s.at, v);
-    } else if (!OWN || s.held == 0) {
-        st_word(p + s.at, v);
+    } else if (OWN) {
+        st_own(p + s.at, v, s.held);
     } else {
-#pragma unroll
-        for (int q = 1; q < 4; ++q)
-            if (q >= s.held) __builtin_nontemporal_store(v.v[q], p + s.at + q);
+        st_word(p + s.at, v);
     }
 }
 

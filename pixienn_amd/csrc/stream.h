@@ -99,9 +99,11 @@ __device__ __forceinline__ void sti(int* p, size_t e, const IPack<V>& v)
 // Four values that start on any of them: a 128-bit access wants the alignment of a word only.
 typedef float f32x4_word __attribute__((ext_vector_type(4), aligned(4)));
 
+template<bool NT>
 __device__ __forceinline__ Pack<4> ld_word(const float* p)
 {
-    const f32x4_word t = __builtin_nontemporal_load(reinterpret_cast<const f32x4_word*>(p));
+    const f32x4_word* const q = reinterpret_cast<const f32x4_word*>(p);
+    const f32x4_word t = NT ? __builtin_nontemporal_load(q) : *q;
     return Pack<4>{ { t.x, t.y, t.z, t.w } };
 }
 
@@ -110,6 +112,18 @@ __device__ __forceinline__ void st_word(float* p, const Pack<4>& v)
     f32x4_word t;
     t.x = v.v[0]; t.y = v.v[1]; t.z = v.v[2]; t.w = v.v[3];
     __builtin_nontemporal_store(t, reinterpret_cast<f32x4_word*>(p));
+}
+
+// All but the first `held` of them.
+__device__ __forceinline__ void st_own(float* p, const Pack<4>& v, int held)
+{
+    if (held == 0) {
+        st_word(p, v);
+    } else {
+#pragma unroll
+        for (int q = 1; q < 4; ++q)
+            if (q >= held) __builtin_nontemporal_store(v.v[q], p + q);
+    }
 }
 
 // n_vec elements [0, n_vec) are processed V at a time (n_vec % V == 0), one vector per lane.

@@ -39,6 +39,39 @@ def test_odd_planes(ops, oracle, monkeypatch, shape, act):
     shortcut.test_training_epilogue_with_shortcut_is_the_two_calls_to_the_bit(ops, act)
 
 
+# three launches: a segment of 1024 values that ends one, two and three values behind its last whole vector, and one that
+# holds a plane's last value alone; then groups: two members, the last vector of a plane in another share than the one in
+# front of it, channels that leave workgroups over, and a gradient with an exponential
+SPLIT = [(1, 5, 1025), (3, 7, 2051), (2, 9, 1022), (40, 3, 5003)]
+GROUPS = [(1, 90, 16385), (2, 23, 25 * 1025), (3, 70, 10243), (8, 96, 10395)]
+
+
+@pytest.mark.parametrize("act", ["leaky", "mish"])
+@pytest.mark.parametrize("shape", SPLIT + GROUPS, ids=str)
+def test_longer_slices(ops, oracle, monkeypatch, shape, act):
+    for module in (epilogue, clipped):
+        monkeypatch.setattr(module, "TRAIN_SHAPES", [shape])
+    epilogue.test_bn_train_forward_matches_oracle(ops, oracle, act)
+    epilogue.test_bn_backward_matches_oracle(ops, oracle, act, False)
+    epilogue.test_bn_backward_matches_oracle(ops, oracle, act, True)
+    clipped.test_bn_backward_clipped_matches_rescale_clip_then_backward(ops, oracle, act, False)
+
+
+@pytest.mark.parametrize("shape", [(3, 20, 13, 13), (2, 5, 25, 41), (7, 3, 1, 5), (5, 3, 1, 3)], ids=str)
+@pytest.mark.parametrize("threshold", [1e9, 1e-3])
+def test_bias_backward(ops, shape, threshold):
+    """d' = (rescaled delta) * the gradient in place, and its sums, against 64 bits: a handful of roundings a value."""
+    (x, pre, delta), (_, _, _, _, _, updates) = layer(shape, 1)
+    before = [host(t).astype(np.float64) for t in (delta, pre, updates)]
+    ops.bias_act_backward_clipped(delta, pre, updates, "leaky", threshold, 0.0)
+    norm = np.sqrt(np.sum(before[0] ** 2))
+    want = before[0] * (threshold / norm if norm > threshold else 1.0) * np.where(before[1] > 0, 1.0, np.float64(F(0.1)))
+    assert np.all(np.abs(host(delta) - want) <= 8 * 2.0 ** -24 * np.abs(want))
+    total = before[2] + want.sum((0, 2, 3))
+    room = 8 * 2.0 ** -24 * (np.abs(want).sum((0, 2, 3)) + np.abs(total))
+    assert np.all(np.abs(host(updates) - total) <= room)
+
+
 def layer(shape, offset, seed=3):
     """x, y, delta and the parameters of a layer, the tensors `offset` values off a 16-byte boundary."""
     g = torch.Generator(device="cuda")
