@@ -153,6 +153,159 @@ __global__ __launch_bounds__(kBlock) void maxpool_fwd_tile_kernel(const float* i
     }
 }
 
+// The same for windows that move by one cell, the usual case, with the LDS work of several outputs shared: the tile comes in
+// by 128-bit loads that are in flight while its frame is laid out; a lane takes four neighbouring outputs of a row from one
+// reading of their K + 3 cells (128 bits at a time), then four outputs of a column from one reading of their K + 3 segments.
+// Rows beyond the image are left out by their numbers, so that only columns have a frame.  Against the kernel above, us,
+// 8192 planes of 19 x 19: k = 5 16.8 -> 12.9, 9 20.9 -> 16.2, 13 23.5 -> 19.2; 64 of 300 x 300, k = 3, 25.5 -> 19.9.
+struct SlideTile {
+    uint32_t pitch, groups;     // cells of a framed row; fours of outputs of a row
+};
+
+constexpr int kSlideRun = 4;
+
+constexpr uint32_t slide_pitch(int k, uint32_t groups)
+{
+    return 4 * (groups - 1) + (k + kSlideRun - 1 + 3) / 4 * 4;
+}
+
+template<int K>
+__global__ __launch_bounds__(kBlock) void maxpool_fwd_slide_kernel(const float* in, float* out, int* indexes,
+                                                                   PoolTile tile, PoolGeom g, SlideTile st,
+                                                                   FastDiv by_strips, FastDiv by_iw, FastDiv by_groups,
+                                                                   FastDiv by_ow, FastDiv by_runs)
+{
+    extern __shared__ __align__(16) float lds[];
+    constexpr int kRead = (K + kSlideRun - 1 + 3) / 4 * 4;
+    constexpr int kLoads = 2;       // vectors of a lane on their way at once: what a tile of 2048 cells has
+    uint32_t group, strip;
+    by_strips.divmod(blockIdx.x, group, strip);
+    const uint32_t p0 = group * tile.per_tile;
+    const uint32_t planes = min(tile.per_tile, tile.planes - p0);
+    const int oy0 = static_cast<int>(strip * tile.rows);
+    const int rows_out = min(static_cast<int>(tile.rows), g.oh - oy0);
+    const int y_frame = g.origin + oy0;
+    int y_lo = 0, rows_in = g.ih;
+    if (tile.strips > 1) {
+        y_lo = min(max(0, y_frame), g.ih);
+        rows_in = max(0, min(g.ih, y_frame + rows_out - 1 + K) - y_lo);
+    }
+    const uint32_t all_rows = planes * rows_in, width = 4 * st.groups;
+    float* const cells = lds;                                  // [all_rows][pitch], column 0 at x = g.origin
+    float* const best_of = cells + all_rows * st.pitch;        // [all_rows][width]
+    uint8_t* const tap_of = reinterpret_cast<uint8_t*>(best_of + all_rows * width);
+    const uint32_t in0 = (p0 * g.ih + y_lo) * g.iw;
+    const uint32_t values = all_rows * g.iw, vectors = values / 4;
+    Pack<4> v[kLoads];
+    const auto fetch = [&](uint32_t first) {
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) {
+            const uint32_t i = first + u * kBlock + threadIdx.x;
+            if (i < vectors) v[u] = ld_word<false>(in + in0 + 4 * static_cast<size_t>(i));
+        }
+    };
+    fetch(0);
+    const Pack<4> outside{ { -INFINITY, -INFINITY, -INFINITY, -INFINITY } };
+    for (uint32_t i = threadIdx.x; i < all_rows * (st.pitch / 4); i += kBlock) *reinterpret_cast<Pack<4>*>(cells + 4 * i) = outside;
+    __syncthreads();
+    bool nan = false;
+    const auto put = [&](uint32_t row, uint32_t x, float value) {
+        nan |= value != value;
+        const uint32_t column = x - g.origin;
+        if (column < st.pitch) cells[row * st.pitch + column] = value;
+    };
+    for (uint32_t first = 0; first < vectors; first += kLoads * kBlock) {
+        if (first) fetch(first);
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) {
+            const uint32_t i = first + u * kBlock + threadIdx.x;
+            if (i >= vectors) continue;
+            uint32_t row, x;
+            by_iw.divmod(4 * i, row, x);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                put(row, x, v[u].v[q]);
+                if (++x == static_cast<uint32_t>(g.iw)) {
+                    x = 0;
+                    ++row;
+                }
+            }
+        }
+    }
+    if (threadIdx.x < values - 4 * vectors) {
+        uint32_t row, x;
+        by_iw.divmod(4 * vectors + threadIdx.x, row, x);
+        put(row, x, in[in0 + 4 * vectors + threadIdx.x]);
+    }
+    const bool by_scan = __syncthreads_or(nan) != 0;
+    for (uint32_t j = threadIdx.x; j < all_rows * st.groups; j += kBlock) {
+        uint32_t row, four;
+        by_groups.divmod(j, row, four);
+        const float* const line = cells + row * st.pitch + 4 * four;
+        float w[kRead];
+#pragma unroll
+        for (int q = 0; q < kRead / 4; ++q) {
+            const Pack<4> t = *reinterpret_cast<const Pack<4>*>(line + 4 * q);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) w[4 * q + k] = t.v[k];
+        }
+        Pack<4> best;
+        uint32_t taps = 0;
+#pragma unroll
+        for (int o = 0; o < 4; ++o) {
+            best.v[o] = w[o];
+            uint32_t tap = 0;
+#pragma unroll
+            for (int kx = 1; kx < K; ++kx) {
+                tap = w[o + kx] > best.v[o] ? kx : tap;
+                best.v[o] = w[o + kx] > best.v[o] ? w[o + kx] : best.v[o];      // not fmaxf: of two zeros the first stays
+            }
+            taps |= tap << (8 * o);
+        }
+        *reinterpret_cast<Pack<4>*>(best_of + row * width + 4 * four) = best;
+        *reinterpret_cast<uint32_t*>(tap_of + row * width + 4 * four) = taps;
+    }
+    __syncthreads();
+    // runs of kSlideRun rows
+    for (uint32_t j = threadIdx.x; j < planes * by_runs.d * g.ow; j += kBlock) {
+        uint32_t run, ox, plane;
+        by_ow.divmod(j, run, ox);
+        by_runs.divmod(run, plane, run);
+        const int row0 = static_cast<int>(run) * kSlideRun;
+        const int seg0 = y_frame + row0 - y_lo;       // of the tile's rows of this plane; the first may lie before them
+        const uint32_t column = plane * rows_in * width + ox;
+        float w[K + kSlideRun - 1];
+#pragma unroll
+        for (int q = 0; q < K + kSlideRun - 1; ++q) {
+            const bool inside = static_cast<uint32_t>(seg0 + q) < static_cast<uint32_t>(rows_in);
+            const float value = best_of[column + (inside ? seg0 + q : 0) * width];
+            w[q] = inside ? value : -INFINITY;
+        }
+#pragma unroll
+        for (int o = 0; o < kSlideRun; ++o) {
+            if (row0 + o >= rows_out) break;
+            float best = w[o];
+            int tap = 0;
+#pragma unroll
+            for (int ky = 1; ky < K; ++ky) {
+                tap = w[o + ky] > best ? ky : tap;
+                best = w[o + ky] > best ? w[o + ky] : best;
+            }
+            int at;
+            if (by_scan || best == -INFINITY) {
+                scan_window(in, g, p0 + plane, oy0 + row0 + o, ox, best, at);
+            } else {
+                const int x = g.origin + static_cast<int>(ox) + tap_of[column + (seg0 + o + tap) * width];
+                const int y = y_frame + row0 + o + tap;
+                at = x + g.iw * (y + g.ih * static_cast<int>(p0 + plane));
+            }
+            const size_t to = (static_cast<size_t>(p0 + plane) * g.oh + oy0 + row0 + o) * g.ow + ox;
+            out[to] = best;
+            indexes[to] = at;
+        }
+    }
+}
+
 // 2x2 / stride 2 windows that all lie inside the input: VX outputs per lane from two
 // (2*VX)-wide row loads, stored as VX-wide value and index vectors.
 template<int VX, bool NT>
@@ -270,7 +423,7 @@ __global__ __launch_bounds__(kBlock) void maxpool_bwd_generic_kernel(const float
 }
 
 // Backward through LDS.  A lane per cell that looks at all k * k windows of its cell reads k * k indexes to
-// find one on average (8192 planes of 19 x 19: k = 5 75 us, k = 13 274 us; here 19 and 56).  Here each output of the tile sets ONE bit, in
+// find one on average (8192 planes of 19 x 19: k = 5 75 us, k = 13 274 us; here 14 and 44).  Here each output of the tile sets ONE bit, in
 // the mask of the cell its index names, at the output's position among the cell's windows in ascending
 // order; the cells with a bit (one in nine for k = 5) are then listed, so that lanes are not idle, and each
 // adds its deltas in that order.  An index that names no cell of the output's own window is ignored, as it
@@ -281,15 +434,25 @@ struct PoolWindows {
     FastDiv by_stride, by_along;
 };
 
+// K: the window of a kernel that moves by one cell over rows of at least K, or 0 for any geometry.  There a window's taps are
+// told apart by one division of the distance from its first cell.  The outputs come in by 128-bit loads that are in flight
+// while the masks are cleared.  us, 8192 planes of 19 x 19: k = 5 19.3 -> 14.2, 9 34.3 -> 22.8, 13 55.5 -> 44.0; 64 of 300 x 300,
+// k = 3, 32.8 -> 24.9; 32768 of 13 x 13, k = 2, 30.1 -> 21.3.  (Any geometry, by the loads alone: 1024 of 151 x 151, 3 / 2,
+// 53.2 -> 48.7.)
+template<int K>
 __global__ __launch_bounds__(kBlock) void maxpool_bwd_tile_kernel(const float* delta, const int* indexes, float* grad,
                                                                   PoolTile tile, PoolGeom g, PoolWindows w,
                                                                   FastDiv by_strips, FastDiv by_ow, FastDiv by_oh,
                                                                   FastDiv by_iw, FastDiv by_ih, uint32_t tile_cells,
                                                                   uint32_t tile_outputs)
 {
-    extern __shared__ float lds[];
+    extern __shared__ __align__(16) float lds[];
+    constexpr int kLoads = 2;
+    const int k = K ? K : g.kernel;
+    const uint32_t along = K ? K : w.along, words = K ? (K * K + 31) / 32 : w.words;
+    const auto by_stride = [&](uint32_t n) { return K ? n : w.by_stride.div(n); };
     uint32_t* masks = reinterpret_cast<uint32_t*>(lds);                      // [word][tile_cells]
-    float* deltas = lds + w.words * tile_cells;                              // [tile_outputs]
+    float* deltas = lds + words * tile_cells;                                // [tile_outputs]
     uint16_t* listed = reinterpret_cast<uint16_t*>(deltas + tile_outputs);   // [tile_cells]
     __shared__ uint32_t listed_count;
     uint32_t group, strip;
@@ -301,32 +464,85 @@ __global__ __launch_bounds__(kBlock) void maxpool_bwd_tile_kernel(const float* d
     int oy_lo = 0, rows_out = g.oh;
     if (tile.strips > 1) {
         // windows that reach row y_lo or later and begin no later than the last row
-        const int reach = y_lo - g.origin - g.kernel + 1;
-        oy_lo = min(reach <= 0 ? 0 : static_cast<int>(w.by_stride.div(reach + g.stride - 1)), g.oh);
-        const int last = static_cast<int>(w.by_stride.div(y_lo + rows_in - 1 - g.origin));
+        const int reach = y_lo - g.origin - k + 1;
+        oy_lo = min(reach <= 0 ? 0 : static_cast<int>(by_stride(reach + g.stride - 1)), g.oh);
+        const int last = static_cast<int>(by_stride(y_lo + rows_in - 1 - g.origin));
         rows_out = max(0, min(g.oh, last + 1) - oy_lo);
     }
     const uint32_t cells = planes * rows_in * g.iw;
-    for (uint32_t i = threadIdx.x; i < w.words * tile_cells; i += kBlock) masks[i] = 0;
+    const uint32_t cell0 = (p0 * g.ih + y_lo) * g.iw, out0 = (p0 * g.oh + oy_lo) * g.ow;
+    const uint32_t outputs = planes * rows_out * g.ow, vectors = outputs / 4;
+    Pack<4> d[kLoads], at[kLoads];
+    const auto fetch = [&](uint32_t first) {
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) {
+            const uint32_t i = first + u * kBlock + threadIdx.x;
+            if (i >= vectors) continue;
+            d[u] = ld_word<false>(delta + out0 + 4 * static_cast<size_t>(i));
+            at[u] = ld_word<false>(reinterpret_cast<const float*>(indexes) + out0 + 4 * static_cast<size_t>(i));
+        }
+    };
+    fetch(0);
+    for (uint32_t i = threadIdx.x; i < words * tile_cells; i += kBlock) masks[i] = 0;
     if (threadIdx.x == 0) listed_count = 0;
     __syncthreads();
-    const uint32_t cell0 = (p0 * g.ih + y_lo) * g.iw, out0 = (p0 * g.oh + oy_lo) * g.ow;
-    for (uint32_t j = threadIdx.x; j < planes * rows_out * g.ow; j += kBlock) {
-        deltas[j] = delta[out0 + j];
-        const uint32_t cell = static_cast<uint32_t>(indexes[out0 + j]) - cell0;     // negative: beyond any tile
-        if (cell >= cells) continue;
-        uint32_t row, ox, plane = 0, y, x, cell_plane = 0;
-        by_ow.divmod(j, row, ox);
-        by_iw.divmod(cell, y, x);
-        if (tile.strips == 1) {
-            by_oh.divmod(row, plane, row);
-            by_ih.divmod(y, cell_plane, y);
+    // output (row, ox) of the plane, `j` of the tile
+    const auto take = [&](uint32_t j, uint32_t plane, uint32_t row, uint32_t ox, float value, int index) {
+        deltas[j] = value;
+        const uint32_t cell = static_cast<uint32_t>(index) - cell0;     // negative: beyond any tile
+        if (cell >= cells) return;
+        uint32_t ty, tx;
+        if constexpr (K > 0) {
+            const int y0 = oy_lo + static_cast<int>(row) + g.origin - y_lo, x0 = static_cast<int>(ox) + g.origin;
+            const int from = (static_cast<int>(plane) * rows_in + y0) * g.iw + x0;
+            const int away = static_cast<int>(cell) - from;
+            if (away < 0) return;
+            by_iw.divmod(away, ty, tx);
+            if (ty >= K || tx >= K || static_cast<uint32_t>(x0 + static_cast<int>(tx)) >= static_cast<uint32_t>(g.iw) ||
+                static_cast<uint32_t>(y0 + static_cast<int>(ty)) >= static_cast<uint32_t>(rows_in))
+                return;
+        } else {
+            uint32_t y, x, cell_plane = 0;
+            by_iw.divmod(cell, y, x);
+            if (tile.strips == 1) by_ih.divmod(y, cell_plane, y);
+            ty = y_lo + y - g.origin - (oy_lo + row) * g.stride;
+            tx = x - g.origin - ox * g.stride;
+            if (plane != cell_plane || ty >= static_cast<uint32_t>(k) || tx >= static_cast<uint32_t>(k)) return;
         }
-        const int ty = y_lo + static_cast<int>(y) - g.origin - (oy_lo + static_cast<int>(row)) * g.stride;
-        const int tx = static_cast<int>(x) - g.origin - static_cast<int>(ox) * g.stride;
-        if (plane != cell_plane || ty < 0 || ty >= g.kernel || tx < 0 || tx >= g.kernel) continue;
-        const uint32_t bit = w.by_stride.div(g.kernel - 1 - ty) * w.along + w.by_stride.div(g.kernel - 1 - tx);
+        const uint32_t bit = by_stride(k - 1 - ty) * along + by_stride(k - 1 - tx);
         atomicOr(&masks[(bit >> 5) * tile_cells + cell], 1u << (bit & 31));
+    };
+    const auto place = [&](uint32_t j, uint32_t& plane, uint32_t& row, uint32_t& ox) {
+        by_ow.divmod(j, row, ox);
+        plane = 0;
+        if (tile.strips == 1) by_oh.divmod(row, plane, row);
+    };
+    for (uint32_t first = 0; first < vectors; first += kLoads * kBlock) {
+        if (first) fetch(first);
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) {
+            const uint32_t i = first + u * kBlock + threadIdx.x;
+            if (i >= vectors) continue;
+            uint32_t plane, row, ox;
+            place(4 * i, plane, row, ox);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                take(4 * i + q, plane, row, ox, d[u].v[q], __float_as_int(at[u].v[q]));
+                if (++ox == static_cast<uint32_t>(g.ow)) {
+                    ox = 0;
+                    if (++row == static_cast<uint32_t>(rows_out)) {
+                        row = 0;
+                        ++plane;
+                    }
+                }
+            }
+        }
+    }
+    if (threadIdx.x < outputs - 4 * vectors) {
+        const uint32_t j = 4 * vectors + threadIdx.x;
+        uint32_t plane, row, ox;
+        place(j, plane, row, ox);
+        take(j, plane, row, ox, delta[out0 + j], indexes[out0 + j]);
     }
     __syncthreads();
     const uint32_t lane = threadIdx.x & (kWave - 1);
@@ -334,30 +550,36 @@ __global__ __launch_bounds__(kBlock) void maxpool_bwd_tile_kernel(const float* d
         const uint32_t i = i0 + lane;
         uint32_t any = 0;
         if (i < cells)
-            for (uint32_t word = 0; word < w.words; ++word) any |= masks[word * tile_cells + i];
+            for (uint32_t word = 0; word < words; ++word) any |= masks[word * tile_cells + i];
         const uint64_t hit = __ballot(any != 0);
         if (hit == 0) continue;
-        uint32_t at = 0;
-        if (lane == 0) at = atomicAdd(&listed_count, static_cast<uint32_t>(__popcll(hit)));
-        at = __builtin_amdgcn_readfirstlane(at);
-        if (any) listed[at + __popcll(hit & ((1ull << lane) - 1))] = static_cast<uint16_t>(i);
+        uint32_t next = 0;
+        if (lane == 0) next = atomicAdd(&listed_count, static_cast<uint32_t>(__popcll(hit)));
+        next = __builtin_amdgcn_readfirstlane(next);
+        if (any) listed[next + __popcll(hit & ((1ull << lane) - 1))] = static_cast<uint16_t>(i);
     }
     __syncthreads();
-    for (uint32_t k = threadIdx.x; k < listed_count; k += kBlock) {
-        const uint32_t cell = listed[k];
+    for (uint32_t n = threadIdx.x; n < listed_count; n += kBlock) {
+        const uint32_t cell = listed[n];
+        float acc = grad[cell0 + cell];
         uint32_t y, x, plane = 0;
         by_iw.divmod(cell, y, x);
         if (tile.strips == 1) by_ih.divmod(y, plane, y);
         // the first window that reaches the cell along each axis (it may lie before the first output)
-        const int lift = g.kernel * g.stride;
-        const int oy = static_cast<int>(w.by_stride.div(y_lo + y - g.origin - g.kernel + g.stride + lift)) - g.kernel;
-        const int ox = static_cast<int>(w.by_stride.div(x - g.origin - g.kernel + g.stride + lift)) - g.kernel;
+        const int lift = k * g.stride;
+        const int oy = static_cast<int>(by_stride(y_lo + y - g.origin - k + g.stride + lift)) - k;
+        const int ox = static_cast<int>(by_stride(x - g.origin - k + g.stride + lift)) - k;
         const int first = (static_cast<int>(plane) * rows_out + oy - oy_lo) * g.ow + ox;
-        float acc = grad[cell0 + cell];
-        for (uint32_t word = 0; word < w.words; ++word)
+        for (uint32_t word = 0; word < words; ++word)
             for (uint32_t bits = masks[word * tile_cells + cell]; bits; bits &= bits - 1) {
+                const uint32_t bit = word * 32 + __builtin_ctz(bits);
                 uint32_t wy, wx;
-                w.by_along.divmod(word * 32 + __builtin_ctz(bits), wy, wx);
+                if constexpr (K > 0) {
+                    wy = bit / K;
+                    wx = bit - wy * K;
+                } else {
+                    w.by_along.divmod(bit, wy, wx);
+                }
                 acc += deltas[first + static_cast<int>(wy) * g.ow + static_cast<int>(wx)];
             }
         grad[cell0 + cell] = acc;
@@ -589,7 +811,7 @@ constexpr uint32_t kPoolCells = 2048;       // eight per lane; halved until the 
 bool launch_fwd_tile(const float* in, float* out, int* indexes, uint32_t planes, const PoolGeom& g, hipStream_t s)
 {
     // Every input is a tap of (k / stride)^2 windows.  Measured, us one lane per output -> tiled: 3 / 1, 64 planes
-    // of 300 x 300, 45 -> 26; 5 / 1, 8192 of 19 x 19, 44 -> 17; 13 / 1 190 -> 24; but 3 / 2, 64 of 300 x 300,
+    // of 300 x 300, 45 -> 20; 5 / 1, 8192 of 19 x 19, 44 -> 13; 13 / 1 190 -> 19; but 3 / 2, 64 of 300 x 300,
     // 13.3 -> 18.8 and 2 / 1, 32768 of 13 x 13, level: with so few taps the detour through LDS costs more.
     if (g.kernel > 64 || g.kernel * g.kernel < 8 * g.stride * g.stride) return false;
     for (uint32_t target = kPoolCells; target >= 256; target /= 2) {
@@ -601,8 +823,23 @@ bool launch_fwd_tile(const float* in, float* out, int* indexes, uint32_t planes,
         const size_t rows_in = t.strips == 1 ? g.ih : std::min<size_t>(g.ih, frame_h);
         const size_t cells = t.per_tile * rows_in * frame_w, segments = t.per_tile * frame_h * g.ow;
         const size_t bytes = cells * 4 + segments * 5;
-        if (bytes > kPoolLds) continue;
         const dim3 grid((planes + t.per_tile - 1) / t.per_tile * t.strips);
+        const uint32_t groups = static_cast<uint32_t>(g.ow + 3) / 4;
+        const SlideTile st{ slide_pitch(g.kernel, groups), groups };
+        const size_t slide_bytes = t.per_tile * rows_in * (4 * st.pitch + 5 * 4 * groups);
+        const auto slide = [&]<int K>() {
+            hipLaunchKernelGGL((maxpool_fwd_slide_kernel<K>), grid, dim3(kBlock), slide_bytes, s, in, out, indexes, t, g, st,
+                               FastDiv(t.strips), FastDiv(g.iw), FastDiv(groups), FastDiv(g.ow),
+                               FastDiv((t.rows + kSlideRun - 1) / kSlideRun));
+            return true;
+        };
+        if (g.stride == 1 && slide_bytes <= kPoolLds) {
+            if (g.kernel == 3) return slide.template operator()<3>();
+            if (g.kernel == 5) return slide.template operator()<5>();
+            if (g.kernel == 9) return slide.template operator()<9>();
+            if (g.kernel == 13) return slide.template operator()<13>();
+        }
+        if (bytes > kPoolLds) continue;
 #define PXH_POOL_TILE(K)                                                                                       \
         hipLaunchKernelGGL((maxpool_fwd_tile_kernel<K>), grid, dim3(kBlock), bytes, s, in, out, indexes, t, g, \
                            FastDiv(t.strips), FastDiv(g.iw), FastDiv(g.ih), FastDiv(g.ow), FastDiv(g.oh),      \
@@ -640,9 +877,19 @@ bool launch_bwd_tile(const float* delta, const int* indexes, float* grad, uint32
         const size_t bytes = cells * (4 * w.words + 2) + outputs * 4;
         if (bytes > kPoolLds) continue;
         const dim3 grid((planes + t.per_tile - 1) / t.per_tile * t.strips);
-        hipLaunchKernelGGL(maxpool_bwd_tile_kernel, grid, dim3(kBlock), bytes, s, delta, indexes, grad, t, g, w,
-                           FastDiv(t.strips), FastDiv(g.ow), FastDiv(g.oh), FastDiv(g.iw), FastDiv(g.ih),
-                           static_cast<uint32_t>(cells), static_cast<uint32_t>(outputs));
+        const auto launch = [&]<int K>() {
+            hipLaunchKernelGGL((maxpool_bwd_tile_kernel<K>), grid, dim3(kBlock), bytes, s, delta, indexes, grad, t, g, w,
+                               FastDiv(t.strips), FastDiv(g.ow), FastDiv(g.oh), FastDiv(g.iw), FastDiv(g.ih),
+                               static_cast<uint32_t>(cells), static_cast<uint32_t>(outputs));
+        };
+        switch (g.stride == 1 && g.iw >= g.kernel ? g.kernel : 0) {
+        case 2: launch.template operator()<2>(); break;
+        case 3: launch.template operator()<3>(); break;
+        case 5: launch.template operator()<5>(); break;
+        case 9: launch.template operator()<9>(); break;
+        case 13: launch.template operator()<13>(); break;
+        default: launch.template operator()<0>();
+        }
         return true;
     }
     return false;
