@@ -611,17 +611,17 @@ __global__ __launch_bounds__(kWide) void nms_small_kernel(const pxh_detection* r
 // Every decision of nms is taken inside one image, so the records are grouped by image first and
 // nothing is sorted: six launches in place of the sorting path's forty-five, whose cost at the few
 // thousand records of a validation batch is the launches and the latency of short dependent steps
-// (7126 records of 16 images in a list for 32768: 440 us in kernels, here 73).
+// (7126 records of 16 images in a list for 32768: 440 us in kernels, here 39).
 //   1. images are counted per tile of 1024 records, 2. the records' keys are laid out image by image,
 //      in any order inside one;
 //   3. a record's place in its image is the number of smaller keys there, counted directly: n^2 of the
 //      cheapest comparisons per image, all independent, where a radix sort is a chain of thirty launches;
-//   4. every pair of an image is looked at once, 64 x 64 pairs per wave: bit masks of the earlier
+//   4. every pair of an image is looked at once, 64 pairs per step of a wave: bit masks of the earlier
 //      records that conflict, one for each of the two passes (other class and overlap above 0.9, same
 //      class and overlap above the threshold);
 //   5. one workgroup per image settles both passes on the masks alone, the states as bit sets in LDS;
 //   6. a survivor's place in the whole list is the number of survivors before it in each image, found
-//      by bisection, one lane per image.
+//      by a search of a few lanes per image.
 // A mask has 16 words, a bit to a place, of which as many that are not empty are stored as 10 MB hold for the whole
 // list (all of them up to 36408 records, eight for 65536), so that the longest list fits the library's first workspace.
 // Step 5 looks at the pairs of a further one again.
@@ -757,13 +757,24 @@ __device__ __forceinline__ uint64_t key_of_lane(uint64_t key, int lane)
     return (static_cast<uint64_t>(hi) << 32) | lo;
 }
 
+// Block `at` of 64 places; false where there are no more.  (With no records there are none: the group launch
+// writes that down too.  Both loads are on their way at once: of the steps of these launches, which are short, a trip to
+// memory is the longest.)
+__device__ __forceinline__ bool find_block(const ImageArgs& a, uint32_t at, PlaceBlock& b)
+{
+    const uint32_t blocks = *a.block_count;
+    b = a.blocks[at];
+    return at < blocks;
+}
+
 // One workgroup per 64 records, a lane per record in each of its 16 waves, the waves side by side over
-// the image's keys.  Records of equal key keep their input order.
+// the image's keys.  Records of equal key keep their input order; a record's own key does not count as one (going over its
+// 64 keys again for it, a trip to memory each, was half the launch: 7000 records of 16 images 14.9 -> 7.1 us).
 __global__ __launch_bounds__(kWide) void nms_place_kernel(ImageArgs a)
 {
     __shared__ uint32_t smaller[kWave];
-    if (live_count(a.count, a.capacity) == 0 || blockIdx.x >= *a.block_count) return;
-    const PlaceBlock b = a.blocks[blockIdx.x];
+    PlaceBlock b;
+    if (!find_block(a, blockIdx.x, b)) return;
     const uint32_t lane = threadIdx.x & (kWave - 1);
     const uint32_t wave = threadIdx.x / kWave;
     if (threadIdx.x < kWave) smaller[threadIdx.x] = 0;
@@ -777,16 +788,19 @@ __global__ __launch_bounds__(kWide) void nms_place_kernel(ImageArgs a)
         const uint32_t here = min(static_cast<uint32_t>(kWave), b.image_end - q0);
         // lanes past the end carry the largest key: none is smaller than any record's
         const uint64_t keys = lane < here ? a.loose_key[q0 + lane] : ~0ull;
+        const uint32_t own = p - q0;       // beyond any lane where the record's key is not among these
         bool equal = false;
 #pragma unroll 16
-        for (int j = 0; j < kWave; ++j) {
-            const uint64_t k = key_of_lane(keys, j);
+        for (uint32_t j = 0; j < kWave; ++j) {
+            const uint64_t k = key_of_lane(keys, static_cast<int>(j));
             rank += k < mine ? 1u : 0u;
-            equal |= k == mine;
+            equal |= k == mine && j != own;
         }
         if (__ballot(equal)) {
+            const uint32_t sources = a.loose_source[min(q0 + lane, b.image_end - 1)];
             for (uint32_t j = 0; j < here; ++j)
-                if (key_of_lane(keys, static_cast<int>(j)) == mine && a.loose_source[q0 + j] < source) ++rank;
+                if (key_of_lane(keys, static_cast<int>(j)) == mine && static_cast<uint32_t>(__builtin_amdgcn_readlane(sources, j)) < source)
+                    ++rank;
         }
     }
     if (rank) atomicAdd(&smaller[lane], rank);
@@ -800,66 +814,89 @@ __global__ __launch_bounds__(kWide) void nms_place_kernel(ImageArgs a)
     a.cls[place] = static_cast<uint32_t>(min(max(d.class_index, 0), a.classes - 1));
 }
 
-// One workgroup per 64 places, a lane per place, a wave per word of its masks: the earlier places that
-// the word stands for are loaded side by side and handed round lane by lane.
+// kConflictParts workgroups per block of 64 places, 16 places each: a wave holds them four times over, and its quarters and
+// the 16 waves share out the places in front of them (and the block's own) evenly, from LDS; what they find is put together
+// in the words it belongs to, and a lane per word and place stores them.  A pair is some 90 instructions, the whole overlap
+// test for nearly every step of a wave, so what bounds the launch is how evenly the pairs lie on the compute units: 64
+// places to a workgroup and a wave to a word, 7000 records of 16 images took 26 us, with a word's places shared out over
+// the waves 20, now 8.0.
+constexpr uint32_t kConflictPlaces = 16, kConflictParts = 64 / kConflictPlaces;
+
 __global__ __launch_bounds__(kWide) void nms_conflicts_kernel(ImageArgs a)
 {
-    __shared__ uint64_t beyond[2][kWave];
-    __shared__ uint32_t slots[2][kWave];
-    if (live_count(a.count, a.capacity) == 0 || blockIdx.x >= *a.block_count) return;
-    const PlaceBlock b = a.blocks[blockIdx.x];
+    __shared__ float4 boxes[kLargeImage];
+    __shared__ uint32_t classes[kLargeImage];
+    __shared__ unsigned long long found[2][kMaskWords][kConflictPlaces];
+    __shared__ uint64_t beyond[2][kConflictPlaces];
+    __shared__ uint32_t slots[2][kConflictPlaces];
+    const uint32_t t = threadIdx.x;
+    const uint32_t block = blockIdx.x / kConflictParts, part = blockIdx.x % kConflictParts;
+    PlaceBlock b;
+    if (!find_block(a, block, b)) return;
     if (b.image_end - b.image_begin > kLargeImage) {
-        if (threadIdx.x < kSettledWords) a.settled[blockIdx.x * kSettledStride + threadIdx.x] = 0;
+        if (part == 0 && t < kSettledWords) a.settled[block * kSettledStride + t] = 0;
         return;
     }
-    const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint32_t wave = threadIdx.x / kWave;
-    if (threadIdx.x < kWave) {
-        for (int pass = 0; pass < 2; ++pass) {
-            beyond[pass][threadIdx.x] = 0;
-            slots[pass][threadIdx.x] = 0;
-        }
+    const uint32_t first = b.first + part * kConflictPlaces;
+    if (first >= b.image_end) return;
+    // places of the image from here on: this workgroup's are from `first_place` to `length`
+    const uint32_t first_place = first - b.image_begin;
+    const uint32_t length = min(first + kConflictPlaces, b.image_end) - b.image_begin;
+    if (t < length) {
+        boxes[t] = a.box[b.image_begin + t];
+        classes[t] = a.cls[b.image_begin + t];
+    }
+    if (t < 2 * kMaskWords * kConflictPlaces) (&found[0][0][0])[t] = 0;
+    if (t < 2 * kConflictPlaces) {
+        (&beyond[0][0])[t] = 0;
+        (&slots[0][0])[t] = 0;
     }
     __syncthreads();
-    const bool live = b.first + lane < b.image_end;
-    const uint32_t p = live ? b.first + lane : b.first;
-    const float4 box = a.box[p];
-    const uint32_t cls = a.cls[p];
-    const uint32_t upto = min(b.first + kWave, b.image_end);
-    const uint32_t word = wave;
-    const uint32_t q_first = b.image_begin + word * 64u;
-    if (q_first < upto) {
-        const uint32_t mine = min(q_first + lane, upto - 1);
-        const float4 their_box = a.box[mine];
-        const int their_class = static_cast<int>(a.cls[mine]);
-        const int here = static_cast<int>(min(static_cast<uint32_t>(kWave), upto - q_first));
-        uint64_t found[2] = { 0, 0 };
-        for (int j = 0; j < here; ++j) {
-            const float4 other = make_float4(from_lane(their_box.x, j), from_lane(their_box.y, j),
-                                             from_lane(their_box.z, j), from_lane(their_box.w, j));
-            const bool same = static_cast<uint32_t>(__builtin_amdgcn_readlane(their_class, j)) == cls;
-            if (q_first + j < p && live && overlaps_above(box, other, same ? a.threshold : kDuplicateOverlap)) {
-                if (same) found[1] |= 1ull << j;
-                else found[0] |= 1ull << j;
-            }
-        }
+    constexpr uint32_t kTeams = kWide / kConflictPlaces;
+    const uint32_t column = t % kConflictPlaces;
+    const uint32_t place = first_place + column;
+    const bool live = place < length;
+    const uint32_t share = (length + kTeams - 1) / kTeams;       // 16 at most
+    const uint32_t q_first = t / kConflictPlaces * share, q_last = min(q_first + share, live ? place : 0u);
+    const float4 box = boxes[live ? place : first_place];
+    const uint32_t cls = classes[live ? place : first_place];
+    uint32_t hits[2] = { 0, 0 };       // bit j: place q_first + j
+    for (uint32_t q = q_first; q < q_last; ++q) {
+        const bool same = classes[q] == cls;
+        if (overlaps_above(box, boxes[q], same ? a.threshold : kDuplicateOverlap)) hits[same ? 1 : 0] |= 1u << (q - q_first);
+    }
+    // a share begins anywhere in a word and may end in the next
+    const uint32_t word = q_first >> 6, shift = q_first & 63;
+#pragma unroll
+    for (int pass = 0; pass < 2; ++pass) {
+        if (!hits[pass]) continue;
+        const uint64_t low = static_cast<uint64_t>(hits[pass]) << shift;
+        const uint64_t high = shift ? static_cast<uint64_t>(hits[pass]) >> (64 - shift) : 0ull;
+        if (low) atomicOr(&found[pass][word][column], static_cast<unsigned long long>(low));
+        if (high) atomicOr(&found[pass][word + 1][column], static_cast<unsigned long long>(high));
+    }
+    __syncthreads();
+    const uint32_t most = a.mask_slots;
+    if (t < kMaskWords * kConflictPlaces && live) {
+        const uint32_t mine = t / kConflictPlaces;       // the word; `column` and `place` are those of above
 #pragma unroll
         for (int pass = 0; pass < 2; ++pass) {
-            if (!found[pass]) continue;
-            const uint32_t slot = atomicAdd(&slots[pass][lane], 1u);
-            if (slot < static_cast<uint32_t>(a.mask_slots)) {
-                a.masks[pass][static_cast<size_t>(slot) * a.capacity + p] = found[pass];
-                a.ids[pass][static_cast<size_t>(slot) * a.capacity + p] = static_cast<uint8_t>(word);
+            const uint64_t mask = found[pass][mine][column];
+            if (!mask) continue;
+            const uint32_t slot = atomicAdd(&slots[pass][column], 1u);
+            if (slot < most) {
+                const size_t at = static_cast<size_t>(slot) * a.capacity + b.image_begin + place;
+                a.masks[pass][at] = mask;
+                a.ids[pass][at] = static_cast<uint8_t>(mine);
             } else {
-                atomicOr(reinterpret_cast<unsigned long long*>(&beyond[pass][lane]), 1ull << word);
+                atomicOr(reinterpret_cast<unsigned long long*>(&beyond[pass][column]), 1ull << mine);
             }
         }
     }
     __syncthreads();
-    if (wave != 0 || !live) return;
-    for (int pass = 0; pass < 2; ++pass) a.beyond[pass][p] = beyond[pass][lane];
-    const uint32_t most = a.mask_slots;
-    a.slots[p] = min(slots[0][lane], most) | min(slots[1][lane], most) << 8;
+    if (t >= kConflictPlaces || !live) return;
+    for (int pass = 0; pass < 2; ++pass) a.beyond[pass][b.image_begin + place] = beyond[pass][column];
+    a.slots[b.image_begin + place] = min(slots[0][column], most) | min(slots[1][column], most) << 8;
 }
 
 __device__ __forceinline__ uint64_t load_bits(const uint64_t* set, uint32_t word)
@@ -900,10 +937,34 @@ __device__ __forceinline__ int recheck(const ImageArgs& a, const Standing& s, ui
     return pending ? 2 : 0;
 }
 
-__device__ __forceinline__ int conflict_state(const ImageArgs& a, const Standing& s)
+// The first stored words of a place's mask, which a lane keeps from round to round: read again in each, the rounds of 16
+// images around 445 places took 11.4 us, now 9.4.
+constexpr int kHeldWords = 4;
+
+struct HeldMask {
+    int stored;
+    uint32_t word[kHeldWords];
+    uint64_t mask[kHeldWords];
+};
+
+__device__ __forceinline__ HeldMask held_mask(const ImageArgs& a, uint32_t place, int pass, uint32_t slots)
+{
+    HeldMask h;
+    h.stored = (slots >> (8 * pass)) & 0xFF;
+#pragma unroll
+    for (int slot = 0; slot < kHeldWords; ++slot) {
+        const bool there = slot < h.stored;
+        const size_t at = static_cast<size_t>(there ? slot : 0) * a.capacity + place;
+        h.word[slot] = there ? a.ids[pass][at] : 0;
+        h.mask[slot] = there ? a.masks[pass][at] : 0ull;
+    }
+    return h;
+}
+
+__device__ __forceinline__ int conflict_state(const ImageArgs& a, const Standing& s, const HeldMask& h)
 {
     const uint32_t place = s.image_begin + s.p;
-    const int stored = (a.slots[place] >> (8 * s.pass)) & 0xFF;
+    const int stored = h.stored;
     if (stored == 0) return 0;                      // nothing is kept beyond the stored words either
     uint64_t beyond = stored == a.mask_slots ? a.beyond[s.pass][place] : 0ull;
     bool pending = false;
@@ -913,7 +974,12 @@ __device__ __forceinline__ int conflict_state(const ImageArgs& a, const Standing
         box = a.box[place];
         cls = a.cls[place];
     }
-    for (int slot = 0; slot < stored; ++slot) {
+#pragma unroll
+    for (int slot = 0; slot < kHeldWords; ++slot) {
+        if (h.mask[slot] & load_bits(s.kept, h.word[slot])) return 1;
+        pending = pending || (h.mask[slot] & ~load_bits(s.gone, h.word[slot])) != 0;
+    }
+    for (int slot = kHeldWords; slot < stored; ++slot) {
         const size_t at = static_cast<size_t>(slot) * a.capacity + place;
         const uint32_t word = a.ids[s.pass][at];
         const uint64_t mask = a.masks[s.pass][at];
@@ -1101,7 +1167,6 @@ __global__ __launch_bounds__(kWide) void nms_settle_kernel(ImageArgs a)
     __shared__ uint64_t kept[kMaskWords], gone[kMaskWords];
     __shared__ uint32_t scan_lds[kWide / kWave + 1];
     const uint32_t t = threadIdx.x;
-    if (live_count(a.count, a.capacity) == 0) return;
     if (blockIdx.x >= static_cast<uint32_t>(a.batch)) {
         settle_blocks(a, blockIdx.x - static_cast<uint32_t>(a.batch));
         return;
@@ -1109,6 +1174,7 @@ __global__ __launch_bounds__(kWide) void nms_settle_kernel(ImageArgs a)
     const uint32_t begin = a.image_begin[blockIdx.x];
     const uint32_t places = a.image_begin[blockIdx.x + 1] - begin;
     if (places > kLargeImage) return;
+    const uint32_t slots = t < places ? a.slots[begin + t] : 0;
     if (t < kMaskWords) gone[t] = 0;
     Standing s{};
     s.image_begin = begin;
@@ -1120,10 +1186,11 @@ __global__ __launch_bounds__(kWide) void nms_settle_kernel(ImageArgs a)
         if (t < kMaskWords) kept[t] = 0;
         __syncthreads();
         bool undecided = t < places;
+        const HeldMask held = held_mask(a, begin + (undecided ? t : 0), s.pass, undecided ? slots : 0);
         if (undecided && s.pass == 1) undecided = !((load_bits(gone, t >> 6) >> (t & 63)) & 1);
         for (uint32_t round = 0; round <= kWide; ++round) {
             if (undecided) {
-                const int state = conflict_state(a, s);
+                const int state = conflict_state(a, s, held);
                 if (state != 2) {
                     set_bit(state == 1 ? gone : kept, t);
                     undecided = false;
@@ -1142,48 +1209,73 @@ __global__ __launch_bounds__(kWide) void nms_settle_kernel(ImageArgs a)
     if (t == 0) a.kept_images[blockIdx.x] = total;
 }
 
-// One wave per survivor, a lane per other image: how many of that image's survivors come before it.
-__global__ __launch_bounds__(kWide) void nms_merge_images_kernel(ImageArgs a, pxh_detection* kept, int* kept_count)
+// One wave per survivor, kMergeParts workgroups per block of 64: how many of each other image's survivors come before it.  A power of two of lanes share an image
+// (batches of up to 64; else images take turns): they look at as many places that split what is left evenly, and the part
+// between the last that comes before and the first that does not is what is left of it.  The looks of a step are on their way at
+// once, so that a step costs one trip to memory: with four lanes four steps for 440 survivors, where halving takes nine
+// (7000 records of 16 images, the launch, with four waves to a wave's survivors: 13.7 -> 5.9 us).
+constexpr uint32_t kMergeParts = kWave / (kWide / kWave);
+
+__global__ __launch_bounds__(kWide) void nms_merge_images_kernel(ImageArgs a, pxh_detection* kept, int* kept_count, uint32_t lanes,
+                                                                 FastDiv by_parts)
 {
-    const uint32_t n = live_count(a.count, a.capacity);
     const uint32_t lane = threadIdx.x & (kWave - 1);
     const uint32_t wave = threadIdx.x / kWave;
+    const uint32_t images = static_cast<uint32_t>(a.batch);
     if (blockIdx.x == 0 && wave == 0) {
         uint32_t sum = 0;
-        if (n)
-            for (uint32_t i = lane; i < static_cast<uint32_t>(a.batch); i += kWave) sum += a.kept_images[i];
+        for (uint32_t i = lane; i < images; i += kWave) sum += a.kept_images[i];
 #pragma unroll
         for (int off = kWave / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, kWave);
         if (lane == 0) *kept_count = static_cast<int>(sum);
     }
-    if (n == 0 || blockIdx.x >= *a.block_count) return;
-    const PlaceBlock b = a.blocks[blockIdx.x];
-    const uint32_t end = min(b.first + kWave, b.image_begin + a.kept_images[b.image]);
-    for (uint32_t at = b.first + wave; at < end; at += kWide / kWave) {
-        const uint64_t key = a.kept_key[at];
-        const uint32_t source = a.kept_source[at];
-        uint32_t before = 0;
-        for (uint32_t i = lane; i < static_cast<uint32_t>(a.batch); i += kWave) {
-            if (i == b.image) {
-                before += at - b.image_begin;
-                continue;
-            }
-            const uint32_t first = a.image_begin[i];
-            uint32_t lo = first, hi = first + a.kept_images[i];
-            while (lo < hi) {
-                const uint32_t mid = lo + (hi - lo) / 2;
-                const uint64_t k = a.kept_key[mid];
-                if (k < key || (k == key && a.kept_source[mid] < source)) lo = mid + 1;
-                else hi = mid;
-            }
-            before += lo - first;
+    const uint32_t part = lane & (lanes - 1), per_round = kWave / lanes;
+    const uint64_t team = ((1ull << lanes) - 1) << (lane & ~(lanes - 1));
+    // the first images' tables on their way beside the block
+    const uint32_t nearest = min(lane / lanes, images - 1);
+    const uint32_t near_begin = a.image_begin[nearest], near_kept = a.kept_images[nearest];
+    PlaceBlock b;
+    if (!find_block(a, blockIdx.x / kMergeParts, b)) return;
+    const uint32_t at = b.first + blockIdx.x % kMergeParts * (kWide / kWave) + wave;
+    if (at >= min(b.first + kWave, b.image_begin + a.kept_images[b.image])) return;
+    const uint64_t key = a.kept_key[at];
+    const uint32_t source = a.kept_source[at];
+    constexpr uint32_t kRecordWords = sizeof(pxh_detection) / 4;
+    const uint32_t record = reinterpret_cast<const uint32_t*>(a.records + source)[lane % kRecordWords];
+    uint32_t before = 0;
+    for (uint32_t i0 = 0; i0 < images; i0 += per_round) {
+        const uint32_t i = i0 + lane / lanes;
+        uint32_t lo = 0, hi = 0;
+        if (i < images) {
+            lo = i0 ? a.image_begin[i] : near_begin;
+            hi = lo + (i0 ? a.kept_images[i] : near_kept);
         }
-#pragma unroll
-        for (int off = kWave / 2; off > 0; off >>= 1) before += __shfl_xor(before, off, kWave);
-        constexpr uint32_t kRecordWords = sizeof(pxh_detection) / 4;
-        if (lane < kRecordWords)
-            reinterpret_cast<uint32_t*>(kept + before)[lane] = reinterpret_cast<const uint32_t*>(a.records + source)[lane];
+        const uint32_t first = lo;
+        if (i == b.image) lo = hi = at;       // the survivors of its own image: those in front of it
+        while (__ballot(lo < hi)) {
+            // lane `part` looks at place lo + length * (part + 1) / (lanes + 1): below hi, and in order
+            const uint32_t length = hi - lo;
+            const auto look = [&](uint32_t nth) { return lo + by_parts.div(length * nth); };       // length is kImageCapacity at most
+            const uint32_t place = look(part + 1);
+            bool less = false;
+            if (length) {
+                const uint64_t k = a.kept_key[place];
+                less = k < key || (k == key && a.kept_source[place] < source);
+            }
+            // places that come before are the first ones: as many lanes as say so
+            const uint32_t count = static_cast<uint32_t>(__popcll(__ballot(less) & team));
+            if (length) {
+                const uint32_t from = count == 0 ? lo : look(count) + 1;
+                const uint32_t to = count == lanes ? hi : look(count + 1);
+                lo = from;
+                hi = to;
+            }
+        }
+        if (part == 0 && i < images) before += lo - first;
     }
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) before += __shfl_xor(before, off, kWave);
+    if (lane < kRecordWords) reinterpret_cast<uint32_t*>(kept + before)[lane] = record;
 }
 
 size_t align256(size_t b) { return (b + 255) & ~static_cast<size_t>(255); }
@@ -1349,10 +1441,14 @@ int pxh_nms(const pxh_detection* records, const int* count, int capacity, int ba
         hipLaunchKernelGGL(nms_count_images_kernel, per_tile, wide, 0, s, a);
         hipLaunchKernelGGL(nms_group_images_kernel, per_tile, wide, 0, s, a);
         hipLaunchKernelGGL(nms_place_kernel, per_block, wide, 0, s, a);
-        hipLaunchKernelGGL(nms_conflicts_kernel, per_block, wide, 0, s, a);
+        hipLaunchKernelGGL(nms_conflicts_kernel, dim3(per_block.x * kConflictParts), wide, 0, s, a);
         const unsigned helpers = static_cast<uint32_t>(capacity) > kLargeImage ? kSettleWorkgroups : 0;
         hipLaunchKernelGGL(nms_settle_kernel, dim3(batch + helpers), wide, 0, s, a);
-        hipLaunchKernelGGL(nms_merge_images_kernel, per_block, wide, 0, s, a, kept, kept_count);
+        // as many lanes to an image as leave one for each, sixteen at most: further ones save no step worth a division
+        uint32_t lanes = 1;
+        while (lanes < 16 && 2 * lanes * static_cast<uint32_t>(batch) <= static_cast<uint32_t>(kWave)) lanes *= 2;
+        hipLaunchKernelGGL(nms_merge_images_kernel, dim3(per_block.x * kMergeParts), wide, 0, s, a, kept, kept_count, lanes,
+                           FastDiv(lanes + 1));
         return check_launch("pxh_nms");
     }
     int rc = resolve_workspace(workspace, workspace_bytes, carve(nullptr, capacity).bytes, &ws, as_stream(stream));
