@@ -44,10 +44,15 @@ __global__ __launch_bounds__(T, (kFwdWaves<V, R, L, T, RES, RAGGED>)) void bn_re
     // No branch around a load: a lane past the end of the slice reads the slice's first vector and
     // adds nothing, so that the loads of a lane are in flight together (behind a branch each one is
     // waited for before the next is issued, and a wave then has one kilobyte on its way at a time).
-    const uint32_t lane = threadIdx.x;
+    uint32_t lane = threadIdx.x;
     const auto element = [&](int r) { return (static_cast<uint32_t>(r * T) + lane) * V; };
     const auto step = [&](int r) { return step_of<V, RAGGED>(a.g, c, static_cast<uint32_t>(r * T) + lane); };
     const auto fetch = [&](int r) { return ld_step<V, true, RAGGED>(a.x, step(r)); };
+    const auto ride = [&](int r) {
+        if constexpr (RAGGED) return ld_step<V, true, RAGGED>(a.residual, step(r));
+        const uint32_t e = element(r);
+        return ld<V, true>(a.residual, a.g.at(c, e < a.g.per_channel ? e : 0u));
+    };
     const auto add = [&](int r, const Pack<V>& t) {
         const bool valid = element(r) < a.g.per_channel;
         const bool second = kTwin && (r & 1);
@@ -88,7 +93,7 @@ __global__ __launch_bounds__(T, (kFwdWaves<V, R, L, T, RES, RAGGED>)) void bn_re
     [[maybe_unused]] Pack<V> ahead[kAhead > 0 ? kAhead : 1];
     if constexpr (RES) {
 #pragma unroll
-        for (int i = 0; i < kAhead; ++i) ahead[i] = ld_step<V, true, RAGGED>(a.residual, step(i));
+        for (int i = 0; i < kAhead; ++i) ahead[i] = ride(i);
     }
     double t1, t2;
     if constexpr (RAGGED) {
@@ -137,12 +142,13 @@ __global__ __launch_bounds__(T, (kFwdWaves<V, R, L, T, RES, RAGGED>)) void bn_re
     }
     __syncthreads();
     const FoldCoef k = shared_coef;
+    if constexpr (L > 0 && RES) asm volatile("" : "+v"(lane));      // addresses formed again, not kept: they would spill
     const auto apply = [&](int r, [[maybe_unused]] const Pack<V>& from) {
-        Step p{};
-        if constexpr (RAGGED) p = step(r);
-        else p.valid = element(r) < a.g.per_channel;
-        if (p.valid) {
-            if constexpr (!RAGGED) p.at = a.g.at(c, element(r));      // (not the load's: it is formed again, not kept)
+        const uint32_t e = element(r);
+        const Step kept = RAGGED ? step(r) : Step{ 0, e < a.g.per_channel, 0 };
+        if (kept.valid) {
+            // (not the load's place: it is formed again, not kept)
+            const Step p = RAGGED ? kept : Step{ a.g.at(c, e), true, 0 };
             const Pack<V> t = r < R ? v[r < R ? r : 0] : *resident_lds_slot<V, R>(resident_lds, r);
             Pack<V> xn, pre, out;
 #pragma unroll
@@ -172,7 +178,7 @@ __global__ __launch_bounds__(T, (kFwdWaves<V, R, L, T, RES, RAGGED>)) void bn_re
                 if (first + i < kAhead) {
                     from[i] = ahead[first + i < kAhead ? first + i : 0];
                 } else {
-                    from[i] = ld_step<V, true, RAGGED>(a.residual, step(first + i));
+                    from[i] = ride(first + i);
                 }
             }
 #pragma unroll
