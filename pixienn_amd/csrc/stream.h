@@ -10,7 +10,7 @@
 //     template<int V> struct Regs;                                     // state between the phases
 //     template<int V, bool NT> __device__ void load(size_t e, Regs<V>&) const;   // e = first element
 //     template<int V, bool NT> __device__ void finish(size_t e, const Regs<V>&) const;
-// V is 4 for the 128-bit path and 1 for the scalar path (unaligned pointers and the n % 4 tail).
+// V is 4 for the 128-bit path and 1 for the scalar path (unaligned pointers and the n % 4 elements behind the vectors).
 #pragma once
 
 #include "common.h"
@@ -126,9 +126,22 @@ __device__ __forceinline__ void st_own(float* p, const Pack<4>& v, int held)
     }
 }
 
-// n_vec elements [0, n_vec) are processed V at a time (n_vec % V == 0), one vector per lane.
+// The n % 4 elements behind the vectors, one to a lane of the last workgroup: a launch of their own is 1.3 us, and the host's
+// time for it 3.
+template<typename Op>
+__device__ __forceinline__ void stream_tail(size_t n_vec, size_t n, const Op& op)
+{
+    const size_t e = n_vec + threadIdx.x;
+    if (n_vec != n && blockIdx.x == gridDim.x - 1 && e < n) {
+        typename Op::template Regs<1> r;
+        op.template load<1, false>(e, r);
+        op.template finish<1, false>(e, r);
+    }
+}
+
+// Elements [0, n_vec) are processed V at a time (n_vec % V == 0), one vector per lane, then those up to n.
 template<int V, bool NT, typename Op>
-__global__ __launch_bounds__(kBlock) void stream_kernel(size_t n_vec, Op op)
+__global__ __launch_bounds__(kBlock) void stream_kernel(size_t n_vec, size_t n, Op op)
 {
     const size_t e = (static_cast<size_t>(blockIdx.x) * kBlock + threadIdx.x) * V;
     if (e < n_vec) {
@@ -136,6 +149,7 @@ __global__ __launch_bounds__(kBlock) void stream_kernel(size_t n_vec, Op op)
         op.template load<V, NT>(e, r);
         op.template finish<V, NT>(e, r);
     }
+    if constexpr (V > 1) stream_tail(n_vec, n, op);
 }
 
 // The same with two vectors per lane, a workgroup's width apart, all loads before the first store.  For
@@ -144,7 +158,7 @@ __global__ __launch_bounds__(kBlock) void stream_kernel(size_t n_vec, Op op)
 // this path (1 + 1 up to 3 + 2 streams) is as fast or faster with one.  Lanes past the end load element
 // 0 (no branch between the loads) and store nothing.
 template<bool NT, typename Op>
-__global__ __launch_bounds__(kBlock) void stream_pairs_kernel(size_t n_vec, Op op)
+__global__ __launch_bounds__(kBlock) void stream_pairs_kernel(size_t n_vec, size_t n, Op op)
 {
     const size_t e0 = (static_cast<size_t>(blockIdx.x) * 2 * kBlock + threadIdx.x) * 4;
     const size_t e1 = e0 + static_cast<size_t>(kBlock) * 4;
@@ -154,18 +168,7 @@ __global__ __launch_bounds__(kBlock) void stream_pairs_kernel(size_t n_vec, Op o
     op.template load<4, NT>(in1 ? e1 : 0, r1);
     if (in0) op.template finish<4, NT>(e0, r0);
     if (in1) op.template finish<4, NT>(e1, r1);
-}
-
-// Elements [begin, n) one at a time (the tail of the 128-bit path).
-template<typename Op>
-__global__ __launch_bounds__(kWave) void stream_tail_kernel(size_t begin, size_t n, Op op)
-{
-    const size_t e = begin + threadIdx.x;
-    if (e < n) {
-        typename Op::template Regs<1> r;
-        op.template load<1, false>(e, r);
-        op.template finish<1, false>(e, r);
-    }
+    stream_tail(n_vec, n, op);
 }
 
 // ---------------------------------------------------------------- group sums of a written tensor
@@ -233,19 +236,14 @@ int launch_stream(const char* name, size_t n, bool vector_ok, int bytes_per_elem
     const bool nt = n * static_cast<size_t>(bytes_per_elem) >= streaming_from;
     if (vector_ok) {
         const size_t n4 = n & ~static_cast<size_t>(3);
-        if (n4) {
-            const dim3 grid(grid_for(n4, static_cast<size_t>(kBlock) * 4));
-            if (nt && pairs)
-                hipLaunchKernelGGL((stream_pairs_kernel<true, Op>), dim3(grid_for(n4, static_cast<size_t>(kBlock) * 8)),
-                                   dim3(kBlock), 0, stream, n4, op);
-            else if (nt) hipLaunchKernelGGL((stream_kernel<4, true, Op>), grid, dim3(kBlock), 0, stream, n4, op);
-            else hipLaunchKernelGGL((stream_kernel<4, false, Op>), grid, dim3(kBlock), 0, stream, n4, op);
-        }
-        if (n4 < n) {
-            hipLaunchKernelGGL((stream_tail_kernel<Op>), dim3(1), dim3(kWave), 0, stream, n4, n, op);
-        }
+        const dim3 grid(grid_for(n4 ? n4 : 4, static_cast<size_t>(kBlock) * 4));
+        if (nt && pairs)
+            hipLaunchKernelGGL((stream_pairs_kernel<true, Op>), dim3(grid_for(n4 ? n4 : 4, static_cast<size_t>(kBlock) * 8)),
+                               dim3(kBlock), 0, stream, n4, n, op);
+        else if (nt) hipLaunchKernelGGL((stream_kernel<4, true, Op>), grid, dim3(kBlock), 0, stream, n4, n, op);
+        else hipLaunchKernelGGL((stream_kernel<4, false, Op>), grid, dim3(kBlock), 0, stream, n4, n, op);
     } else {
-        hipLaunchKernelGGL((stream_kernel<1, false, Op>), dim3(grid_for(n, kBlock)), dim3(kBlock), 0, stream, n, op);
+        hipLaunchKernelGGL((stream_kernel<1, false, Op>), dim3(grid_for(n, kBlock)), dim3(kBlock), 0, stream, n, n, op);
     }
     return check_launch(name);
 }
