@@ -388,7 +388,7 @@ __device__ __forceinline__ Pack<V> ld_at(const float* p, size_t e)
 
 // ---- statistics: S1 = sum(x - K), S2 = sum((x - K)^2), K = first element of the channel ----
 template<int V, bool NT, bool RAGGED = false>
-__global__ __launch_bounds__(kBlock) void bn_stats_partial_kernel(const float* x, ReduceGeom g, double2* partial)
+__global__ __launch_bounds__(kBlock) void bn_stats_partial_kernel(const float* x, ReduceGeom g, double2* partial, float* shifts)
 {
     __shared__ double slots[2][kBlock / kWave];
     uint32_t c, j;
@@ -435,7 +435,10 @@ __global__ __launch_bounds__(kBlock) void bn_stats_partial_kernel(const float* x
     });
     const double t1 = block_sum(s1, slots[0]);
     const double t2 = block_sum(s2, slots[1]);
-    if (threadIdx.x == 0) partial[blockIdx.x] = make_double2(t1, t2);
+    if (threadIdx.x == 0) {
+        partial[blockIdx.x] = make_double2(t1, t2);
+        if (shifts && j == 0) shifts[c] = shift;
+    }
 }
 
 // The same for channel c of the tensors: writes the statistics and folds the constants the apply
@@ -799,6 +802,207 @@ __global__ __launch_bounds__(kBlock) void bn_dx_scalar_kernel(DxArgs a)
     a.delta[e] = dx_of_delta<ACT>(d.v[0], a.x[e], pre, recompute, a.coef[c]);
 }
 
+// ------------------------------------------------------------------------------------------
+// The pass behind the partial sums with the finish of the channels inside: a workgroup goes over the same items of a channel
+// as one of the sums' does, its first wave adds the channel's partials up and forms the constants while the loads of the
+// first items are on their way, and the channel's first workgroup writes what is left of it.  A launch that does only that
+// is 4 us, whatever the size: a chain of trips to memory and double-precision roots.  Past a size the flat pass is ahead by
+// more, whose lanes take one vector each and past the caches.  Three launches -> two, us, leaky and mish: forward,
+// + shortcut, backward with the pre-activation kept (one without takes groups in most of these)
+//   2 x 16 x 160^2       9.7 ->  7.8    9.9 ->  7.8   14.4 ->  9.7   10.2 ->  8.7   10.4 ->  8.6   18.9 -> 12.2
+//   4 x 64 x 104^2      13.9 -> 10.7   14.5 -> 11.1   23.2 -> 18.0   14.3 -> 12.2   14.7 -> 12.7   29.0 -> 22.6
+//   6 x 72 x 135 x 77   17.4 -> 13.1   19.8 -> 13.8   32.6 -> 28.0   17.6 -> 14.3   20.1 -> 15.5   40.0 -> 33.7
+//   4 x 32 x 208^2      18.6 -> 14.2   21.4 -> 16.9   37.0 -> 33.1   19.0 -> 17.1   22.0 -> 19.3   43.0 -> 39.2
+//   9 x 20 x 203 x 251  26.4 -> 22.3   31.9 -> 26.7   48.6 -> 51.3   27.2 -> 23.7   32.6 -> 27.6   58.6 -> 61.3
+//   4 x 16 x 416^2      29.0 -> 27.4   35.9 -> 33.1   56.0 -> 60.2   29.3 -> 29.7   36.3 -> 37.9   66.0 -> 69.8
+//   8 x 16 x 416^2      47.0 -> 45.8   60.2 -> 69.2   104  -> 123    47.1 -> 49.6   61.6 -> 77.8   122  -> 136
+// (6 x 72 x 135 x 77, mish, without the pre-activation: 31.5 -> 28.4.)
+// ------------------------------------------------------------------------------------------
+constexpr int kFusedPartials = 4 * kWave;      // of a channel: a lane of the first wave takes four
+constexpr uint32_t kFusedForward = 10u << 20, kFusedBackward = 6u << 20;      // values of a tensor
+constexpr int kFusedSpatial = 4 * kWave;       // a wave's step; planes below leave most of its lanes without a vector
+
+__device__ __forceinline__ double2 channel_sums(const double2* partial, uint32_t c, int blocks)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    double s1 = 0.0, s2 = 0.0;
+    for (int j = lane; j < blocks; j += kWave) {
+        const double2 p = partial[static_cast<size_t>(c) * blocks + j];
+        s1 += p.x;
+        s2 += p.y;
+    }
+    return make_double2(wave_sum(s1), wave_sum(s2));
+}
+
+// The items of a wave, one after the other, and their vectors.
+template<bool RAGGED>
+struct WaveItems {
+    const ReduceGeom& g;
+    uint32_t c;
+    int it, last;
+    size_t base = 0;
+    int seg0 = 0, seg1 = 0;
+    __device__ __forceinline__ WaveItems(const ReduceGeom& geom, uint32_t channel, uint32_t j)
+        : g(geom), c(channel), it(j * geom.per_block + threadIdx.x / kWave), last(min(static_cast<int>((j + 1) * geom.per_block), geom.items))
+    {
+        place();
+    }
+    __device__ __forceinline__ void place()
+    {
+        uint32_t n, part;
+        g.by_parts.divmod(static_cast<uint32_t>(it < last ? it : 0), n, part);
+        base = (static_cast<size_t>(n) * g.channels + c) * g.spatial;
+        seg0 = part * kSeg;
+        seg1 = min(g.spatial, seg0 + kSeg);
+    }
+    __device__ __forceinline__ bool more() const { return it < last; }
+    __device__ __forceinline__ void next()
+    {
+        it += kBlock / kWave;
+        place();
+    }
+    // vector u of the lane: where it begins in its plane, and whether it is one of the item's
+    __device__ __forceinline__ int offset(int u) const { return seg0 + (u * kWave + static_cast<int>(threadIdx.x & (kWave - 1))) * 4; }
+    __device__ __forceinline__ bool has(int u) const { return more() && offset(u) < seg1; }
+    __device__ __forceinline__ size_t at(int u) const { return base + ragged_start<RAGGED>(offset(u), g.spatial); }
+    __device__ __forceinline__ int held(int u) const { return offset(u) - ragged_start<RAGGED>(offset(u), g.spatial); }
+};
+
+template<bool RAGGED>
+__device__ __forceinline__ void st_item(float* p, size_t at, const Pack<4>& v, int held)
+{
+    if constexpr (RAGGED) st_own(p + at, v, held);
+    else st<4, false>(p, at, v);
+}
+
+struct StatsFinish {
+    const double2* partial;
+    const float* shifts;
+    double count;
+    float *mean, *var, *rolling_mean, *rolling_var;
+    const float *scale, *bias;
+};
+
+template<int ACT, bool RES, bool RAGGED>
+__global__ __launch_bounds__(kBlock) void bn_finish_apply_kernel(EpilogueArgs a, ReduceGeom g, StatsFinish f)
+{
+    __shared__ FoldCoef shared_coef;
+    uint32_t c, j;
+    g.by_blocks.divmod(blockIdx.x, c, j);
+    WaveItems<RAGGED> item(g, c, j);
+    Pack<4> x[kSegLoads], r[kSegLoads];
+    const auto fetch = [&] {
+#pragma unroll
+        for (int u = 0; u < kSegLoads; ++u) {
+            if (!item.has(u)) continue;
+            x[u] = ld_at<4, false, RAGGED>(a.x, item.at(u));
+            if constexpr (RES) r[u] = ld_at<4, false, RAGGED>(a.residual, item.at(u));
+        }
+    };
+    fetch();
+    if (threadIdx.x < kWave) {
+        const float shift = f.shifts[c], scale = f.scale[c], bias = f.bias[c];
+        const float rolling_mean = j == 0 ? f.rolling_mean[c] : 0.0f, rolling_var = j == 0 ? f.rolling_var[c] : 0.0f;
+        const double2 sums = channel_sums(f.partial, c, g.blocks);
+        const ChannelStats st = channel_stats(sums.x, sums.y, shift, f.count, rolling_mean, rolling_var);
+        if (threadIdx.x == 0) {
+            shared_coef = make_coef(st.mean, st.var, scale, bias);
+            if (j == 0) {
+                f.mean[c] = st.mean;
+                f.var[c] = st.var;
+                f.rolling_mean[c] = st.rolling_mean;
+                f.rolling_var[c] = st.rolling_var;
+            }
+        }
+    }
+    __syncthreads();
+    const FoldCoef k = shared_coef;
+    while (item.more()) {
+#pragma unroll
+        for (int u = 0; u < kSegLoads; ++u) {
+            if (!item.has(u)) continue;
+            Pack<4> yo, po, no;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) po.v[q] = pre_value<true>(x[u].v[q], k, no.v[q]);
+            act_apply_n<ACT>(po.v, yo.v);
+            if constexpr (RES) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) yo.v[q] = with_residual(yo.v[q], r[u].v[q], a.res_alpha, a.res_beta);
+            }
+            const size_t at = item.at(u);
+            const int held = item.held(u);
+            if (a.x_saved) st_item<RAGGED>(a.x_saved, at, x[u], held);
+            if (a.x_norm) st_item<RAGGED>(a.x_norm, at, no, held);
+            if (a.pre) st_item<RAGGED>(a.pre, at, po, held);
+            st_item<RAGGED>(a.y, at, yo, held);
+        }
+        item.next();
+        fetch();
+    }
+}
+
+struct BackwardFinish {
+    const double2* partial;
+    float *scale_updates, *bias_updates, *mean_delta, *var_delta;
+    int count;
+};
+
+template<int ACT, bool RAGGED>
+__global__ __launch_bounds__(kBlock) void bn_finish_dx_kernel(BackwardArgs a, ReduceGeom g, BackwardFinish f)
+{
+    __shared__ DxCoef shared_coef;
+    uint32_t c, j;
+    g.by_blocks.divmod(blockIdx.x, c, j);
+    WaveItems<RAGGED> item(g, c, j);
+    const bool recompute = a.pre == nullptr;
+    Pack<4> d[kSegLoads], x[kSegLoads], pre[kSegLoads];
+    const auto fetch = [&] {
+#pragma unroll
+        for (int u = 0; u < kSegLoads; ++u) {
+            if (!item.has(u)) continue;
+            d[u] = ld_at<4, false, RAGGED>(a.delta, item.at(u));
+            x[u] = ld_at<4, false, RAGGED>(a.x, item.at(u));
+            if constexpr (ACT != PXH_LINEAR) {
+                if (!recompute) pre[u] = ld_at<4, false, RAGGED>(a.pre, item.at(u));
+            }
+        }
+    };
+    fetch();
+    if (threadIdx.x < kWave) {
+        const double2 sums = channel_sums(f.partial, c, g.blocks);
+        if (threadIdx.x == 0) {
+            if (j == 0) {
+                shared_coef = finish_backward<true>(sums.x, sums.y, c, f.count, a.mean, a.var, a.scale, a.bias, f.scale_updates,
+                                                    f.bias_updates, f.mean_delta, f.var_delta);
+            } else {
+                const float v = a.var[c], s = a.scale[c];
+                shared_coef = finished_channel<true>(sums.x, sums.y, f.count, make_coef(a.mean[c], v, s, a.bias[c]), variance_terms(v), s).k;
+            }
+        }
+    }
+    __syncthreads();
+    const DxCoef k = shared_coef;
+    while (item.more()) {
+#pragma unroll
+        for (int u = 0; u < kSegLoads; ++u) {
+            if (!item.has(u)) continue;
+            if constexpr (ACT != PXH_LINEAR) {
+                if (recompute) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) pre[u].v[q] = affine(normalize(x[u].v[q], k.f), k.f);
+                }
+                times_grad<ACT>(d[u].v, pre[u].v);
+            }
+            Pack<4> out;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) out.v[q] = dx_value(d[u].v[q], x[u].v[q], k);
+            st_item<RAGGED>(a.delta, item.at(u), out, item.held(u));
+        }
+        item.next();
+        fetch();
+    }
+}
+
 constexpr size_t align256(size_t b) { return (b + 255) & ~static_cast<size_t>(255); }
 
 // workspace: [partial sums][per-channel constants]
@@ -955,27 +1159,39 @@ bool streams_past_cache(uint32_t total, int tensors)
     return static_cast<size_t>(total) * 4 * tensors >= kStreamingBytes;
 }
 
+int launch_stats_partial(const float* x, const ReduceGeom& g, double2* partial, float* shifts, uint32_t total, hipStream_t stream)
+{
+    const dim3 grid(static_cast<unsigned>(g.channels) * g.blocks);
+    const bool nt = streams_past_cache(total, 1);
+    if (g.spatial % 4 == 0 && aligned16(x)) {
+        if (nt) hipLaunchKernelGGL((bn_stats_partial_kernel<4, true>), grid, dim3(kBlock), 0, stream, x, g, partial, shifts);
+        else hipLaunchKernelGGL((bn_stats_partial_kernel<4, false>), grid, dim3(kBlock), 0, stream, x, g, partial, shifts);
+    } else if (g.spatial >= kOddSpatial) {
+        hipLaunchKernelGGL((bn_stats_partial_kernel<4, false, true>), grid, dim3(kBlock), 0, stream, x, g, partial, shifts);
+    } else {
+        hipLaunchKernelGGL((bn_stats_partial_kernel<1, false>), grid, dim3(kBlock), 0, stream, x, g, partial, shifts);
+    }
+    return check_launch("bn_stats_partial");
+}
+
 int launch_stats(const float* x, float* mean, float* var, float* rolling_mean, float* rolling_var, const float* scale,
                  const float* bias, FoldCoef* table, int batch, int channels, int spatial, uint32_t total, void* ws,
                  hipStream_t stream)
 {
     const ReduceGeom g = make_geom(batch, channels, spatial);
     double2* partial = static_cast<double2*>(ws);
-    const dim3 grid(static_cast<unsigned>(channels) * g.blocks);
-    const bool nt = streams_past_cache(total, 1);
-    if (spatial % 4 == 0 && aligned16(x)) {
-        if (nt) hipLaunchKernelGGL((bn_stats_partial_kernel<4, true>), grid, dim3(kBlock), 0, stream, x, g, partial);
-        else hipLaunchKernelGGL((bn_stats_partial_kernel<4, false>), grid, dim3(kBlock), 0, stream, x, g, partial);
-    } else {
-        if (spatial >= kOddSpatial) hipLaunchKernelGGL((bn_stats_partial_kernel<4, false, true>), grid, dim3(kBlock), 0, stream, x, g, partial);
-        else hipLaunchKernelGGL((bn_stats_partial_kernel<1, false>), grid, dim3(kBlock), 0, stream, x, g, partial);
-    }
-    int rc = check_launch("bn_stats_partial");
+    const int rc = launch_stats_partial(x, g, partial, nullptr, total, stream);
     if (rc) return rc;
     hipLaunchKernelGGL(bn_stats_finish_kernel, dim3(grid_for(channels, kBlock / kWave)), dim3(kBlock), 0, stream, x,
                        partial, channels, spatial, g.blocks, static_cast<double>(batch) * spatial, mean, var,
                        rolling_mean, rolling_var, scale, bias, table);
     return check_launch("bn_stats_finish");
+}
+
+// Whether the pass behind the partial sums finishes the channels itself.
+bool finishes_inside(const ReduceGeom& g, uint32_t total, bool backward)
+{
+    return total <= (backward ? kFusedBackward : kFusedForward) && g.blocks <= kFusedPartials && g.spatial >= kFusedSpatial;
 }
 
 // The linear shortcut taken into a forward pass (from == nullptr: none).
@@ -999,9 +1215,9 @@ int bn_train_forward(const char* who, const float* x, float* y, float* pre_activ
     int rc = check_shape(who, batch, channels, spatial, &a.total);
     if (rc) return rc;
     hipStream_t s = as_stream(stream);
+    const bool vec = spatial % 4 == 0 && aligned16(x) && aligned16(y) && aligned16(pre_activation) &&
+                     aligned16(x_saved) && aligned16(x_norm) && aligned16(res.from);
     {
-        const bool vec = spatial % 4 == 0 && aligned16(x) && aligned16(y) && aligned16(pre_activation) &&
-                         aligned16(x_saved) && aligned16(x_norm) && aligned16(res.from);
         if (const ResidentForm form = resident_form(batch, channels, spatial, vec, activation, false)) {
             const ResidentFwdArgs r{ x, y, pre_activation, x_saved, x_norm, mean, var, rolling_mean, rolling_var,
                                      scale, bias, resident_geom(batch, channels, spatial), res.from, res.alpha, res.beta };
@@ -1017,14 +1233,34 @@ int bn_train_forward(const char* who, const float* x, float* y, float* pre_activ
     void* ws;
     rc = get_workspace(workspace_bytes(batch, channels, spatial), &ws);
     if (rc) return rc;
+    a.x = x; a.y = y; a.pre = pre_activation; a.x_saved = x_saved; a.x_norm = x_norm;
+    a.residual = res.from; a.res_alpha = res.alpha; a.res_beta = res.beta;
+    const ReduceGeom g = make_geom(batch, channels, spatial);
+    if (finishes_inside(g, a.total, false)) {
+        // (the first value of a channel, which its sums are relative to, is kept: y may be x)
+        float* const shifts = static_cast<float*>(coef_region(ws, batch, channels, spatial));
+        double2* const partial = static_cast<double2*>(ws);
+        rc = launch_stats_partial(x, g, partial, shifts, a.total, s);
+        if (rc) return rc;
+        const StatsFinish f{ partial, shifts, static_cast<double>(batch) * spatial, mean, var, rolling_mean, rolling_var, scale, bias };
+        const dim3 grid(static_cast<unsigned>(channels) * g.blocks);
+        const auto launch = [&]<int ACT, bool RES>() {
+            if (vec) hipLaunchKernelGGL((bn_finish_apply_kernel<ACT, RES, false>), grid, dim3(kBlock), 0, s, a, g, f);
+            else hipLaunchKernelGGL((bn_finish_apply_kernel<ACT, RES, true>), grid, dim3(kBlock), 0, s, a, g, f);
+        };
+        const bool known = dispatch_activation(activation, [&]<int ACT>() {
+            if (res.from) launch.template operator()<ACT, true>();
+            else launch.template operator()<ACT, false>();
+        });
+        if (!known) return fail_invalid("%s: unknown activation %d", who, activation);
+        return check_launch(who);
+    }
     FoldCoef* table = static_cast<FoldCoef*>(coef_region(ws, batch, channels, spatial));
     rc = launch_stats(x, mean, var, rolling_mean, rolling_var, scale, bias, table, batch, channels, spatial, a.total,
                       ws, s);
     if (rc) return rc;
-    a.x = x; a.y = y; a.pre = pre_activation; a.x_saved = x_saved; a.x_norm = x_norm;
     a.table = table;
     a.by_spatial = FastDiv(spatial); a.by_channels = FastDiv(channels);
-    a.residual = res.from; a.res_alpha = res.alpha; a.res_beta = res.beta;
     return launch_epilogue_fwd<true>(who, a, activation, s);
 }
 
@@ -1349,6 +1585,14 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
     if (!known) return fail_invalid("%s: unknown activation %d", who, activation);
     rc = check_launch("bn_backward_partial");
     if (rc) return rc;
+    if (!cs.on && finishes_inside(g, total, true)) {
+        const BackwardFinish f{ partial, scale_updates, bias_updates, mean_delta, var_delta, batch * spatial };
+        dispatch_activation(activation, [&]<int ACT>() {
+            if (vec) hipLaunchKernelGGL((bn_finish_dx_kernel<ACT, false>), grid, dim3(kBlock), 0, s, b, g, f);
+            else hipLaunchKernelGGL((bn_finish_dx_kernel<ACT, true>), grid, dim3(kBlock), 0, s, b, g, f);
+        });
+        return check_launch("bn_backward_finish_dx");
+    }
     if (cs.on) finish.template operator()<kRedo>();
     else finish.template operator()<kPlain>();
     rc = check_launch("bn_backward_finish");

@@ -42,7 +42,10 @@ def test_odd_planes(ops, oracle, monkeypatch, shape, act):
 # three launches: a segment of 1024 values that ends one, two and three values behind its last whole vector, and one that
 # holds a plane's last value alone; then groups: two members, the last vector of a plane in another share than the one in
 # front of it, channels that leave workgroups over, and a gradient with an exponential
-SPLIT = [(1, 5, 1025), (3, 7, 2051), (2, 9, 1022), (40, 3, 5003)]
+# (the pass behind the sums finishes the channels from planes of 256 values on, and up to 256 partial sums a channel: both
+# sides, aligned and odd)
+SPLIT = [(1, 5, 1025), (3, 7, 2051), (2, 9, 1022), (40, 3, 5003), (68, 3, 255), (68, 3, 257), (65, 4, 256), (1030, 2, 260), (1, 1, 4 * 1024 * 257),
+         (1, 9, 16388), (3, 4, 5468)]
 GROUPS = [(1, 90, 16385), (2, 23, 25 * 1025), (3, 70, 10243), (8, 96, 10395)]
 
 
@@ -106,7 +109,25 @@ def test_tensors_off_a_boundary(ops, shape, offset):
             assert np.max(np.abs(a.astype(np.float64) - b)) <= 1e-5 * np.sqrt(np.mean(b.astype(np.float64) ** 2))
 
 
-@pytest.mark.parametrize("shape", [(64, 100, 5, 5), (33, 520, 13, 13), (40, 100, 19, 19)], ids=str)
+@pytest.mark.parametrize("act", ["leaky", "mish"])
+@pytest.mark.parametrize("shape", [(3, 7, 45, 153), (2, 5, 96, 96), (64, 100, 5, 5)], ids=str)
+def test_forward_in_place(ops, shape, act):
+    """y may be x, also with a shortcut on top of it."""
+    found = []
+    for alias in (False, True):
+        (x, y, source), (scale, bias, rm, rv, _, _) = layer(shape, 0)
+        mean, var = torch.zeros_like(rm), torch.zeros_like(rm)
+        out, riding = (x, x.clone()) if alias else (y, torch.empty_like(x))
+        start = x.clone()
+        ops.bn_train_act_forward(x, out, mean, var, rm, rv, scale, bias, act)
+        at = start if not alias else riding
+        ops.bn_train_act_shortcut_forward(at, riding if not alias else at, mean, var, rm, rv, scale, bias, act, source)
+        found.append([host(t) for t in (out, riding, mean, var, rm, rv)])
+    for a, b in zip(*found):
+        assert_bit_exact(a, b)
+
+
+@pytest.mark.parametrize("shape", [(64, 100, 5, 5), (33, 520, 13, 13), (40, 100, 19, 19), (3, 7, 45, 153)], ids=str)
 def test_shortcut_source_is_the_output(ops, shape):
     found = []
     for alias in (False, True):
