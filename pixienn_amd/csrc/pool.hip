@@ -53,6 +53,67 @@ __global__ __launch_bounds__(kBlock) void maxpool_fwd_generic_kernel(const float
     indexes[o] = best_at;
 }
 
+// Windows of 2 that move by one cell over a tensor of the output's size: four outputs of the flat tensor to a lane, whose cells
+// are the five from the first output on and the five a row further, whatever rows they lie in.  One output per lane read
+// each of its cells by itself; us: 32768 planes of 13 x 13 22.5 -> 13.4, 512 level (5.0).
+__global__ __launch_bounds__(kBlock) void maxpool_fwd_step1_kernel(const float* in, float* out, int* indexes, uint32_t total,
+                                                                   PoolGeom g, FastDiv by_w, FastDiv by_h)
+{
+    const uint32_t o = (blockIdx.x * kBlock + threadIdx.x) * 4;
+    if (o >= total) return;
+    uint32_t rows, x, plane, y;
+    by_w.divmod(o, rows, x);
+    by_h.divmod(rows, plane, y);
+    const uint32_t w = by_w.d, h = by_h.d;
+    if (o + w + 5 > total) {
+        // the cells of a row further end with the tensor
+        for (uint32_t q = 0; q < 4 && o + q < total; ++q) {
+            float best;
+            int best_at;
+            scan_window(in, g, plane, y, x, best, best_at);
+            out[o + q] = best;
+            indexes[o + q] = best_at;
+            if (++x == w) {
+                x = 0;
+                if (++y == h) {
+                    y = 0;
+                    ++plane;
+                }
+            }
+        }
+        return;
+    }
+    float a[5], b[5];
+    const Pack<4> a4 = ld_word<false>(in + o), b4 = ld_word<false>(in + o + w);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        a[q] = a4.v[q];
+        b[q] = b4.v[q];
+    }
+    a[4] = in[o + 4];
+    b[4] = in[o + w + 4];
+    Pack<4> value, index;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const bool right = x + 1 < w, below = y + 1 < h;
+        float best = a[q];
+        uint32_t at = o + q;
+        if (right && a[q + 1] > best) { best = a[q + 1]; at = o + q + 1; }
+        if (below && b[q] > best) { best = b[q]; at = o + q + w; }
+        if (right && below && b[q + 1] > best) { best = b[q + 1]; at = o + q + w + 1; }
+        value.v[q] = best;
+        index.v[q] = __int_as_float(static_cast<int>(at));
+        if (!right) {
+            x = 0;
+            y = below ? y + 1 : 0;
+        } else {
+            ++x;
+        }
+    }
+    st_word<false>(out + o, value);
+    st_word<false>(reinterpret_cast<float*>(indexes) + o, index);
+}
+
 // ------------------------------------------------------------------ max-pool through LDS
 // Overlapping windows read every input k * k times; from the caches, at one lane per output, that is what
 // the kernel above costs (8192 planes of 19 x 19: k = 5 44 us, k = 13 191 us, for 36 MB of traffic).  Here a
@@ -812,7 +873,7 @@ bool launch_fwd_tile(const float* in, float* out, int* indexes, uint32_t planes,
 {
     // Every input is a tap of (k / stride)^2 windows.  Measured, us one lane per output -> tiled: 3 / 1, 64 planes
     // of 300 x 300, 45 -> 20; 5 / 1, 8192 of 19 x 19, 44 -> 13; 13 / 1 190 -> 19; but 3 / 2, 64 of 300 x 300,
-    // 13.3 -> 18.8 and 2 / 1, 32768 of 13 x 13, level: with so few taps the detour through LDS costs more.
+    // 13.3 -> 18.8 (and 2 / 1 in a form of its own, above): with so few taps the detour through LDS costs more.
     if (g.kernel > 64 || g.kernel * g.kernel < 8 * g.stride * g.stride) return false;
     for (uint32_t target = kPoolCells; target >= 256; target /= 2) {
         const PoolTile t = pool_tile(planes, g.oh, g.ow, target);
@@ -940,6 +1001,11 @@ int pxh_maxpool_forward(const float* in, float* out, int* indexes, int batch, in
         return check_launch("pxh_maxpool_forward");
     }
     const PoolGeom g{ ih, iw, oh, ow, kernel, stride, -padding / 2 };
+    if (kernel == 2 && stride == 1 && g.origin == 0 && oh == ih && ow == iw) {
+        hipLaunchKernelGGL(maxpool_fwd_step1_kernel, dim3(grid_for(total, static_cast<size_t>(kBlock) * 4)), dim3(kBlock), 0, s,
+                           in, out, indexes, total, g, FastDiv(ow), FastDiv(oh));
+        return check_launch("pxh_maxpool_forward");
+    }
     if (launch_fwd_tile(in, out, indexes, planes, g, s)) return check_launch("pxh_maxpool_forward");
     hipLaunchKernelGGL(maxpool_fwd_generic_kernel, dim3(grid_for(total, kBlock)), dim3(kBlock), 0, s, in, out, indexes,
                        total, g, FastDiv(ow), FastDiv(oh));

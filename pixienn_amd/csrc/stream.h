@@ -107,11 +107,13 @@ __device__ __forceinline__ Pack<4> ld_word(const float* p)
     return Pack<4>{ { t.x, t.y, t.z, t.w } };
 }
 
+template<bool NT = true>
 __device__ __forceinline__ void st_word(float* p, const Pack<4>& v)
 {
     f32x4_word t;
     t.x = v.v[0]; t.y = v.v[1]; t.z = v.v[2]; t.w = v.v[3];
-    __builtin_nontemporal_store(t, reinterpret_cast<f32x4_word*>(p));
+    if constexpr (NT) __builtin_nontemporal_store(t, reinterpret_cast<f32x4_word*>(p));
+    else *reinterpret_cast<f32x4_word*>(p) = t;
 }
 
 // All but the first `held` of them.

@@ -21,7 +21,8 @@ def ops():
 # batch, channels, height, width, window, padding
 CASES = [(1, 1, 1, 1, 3, 2), (3, 1, 1, 3, 3, 2), (1, 5, 2, 2, 5, 4), (1, 3, 13, 13, 13, 12), (1, 2, 12, 12, 13, 12), (2, 1, 40, 9, 9, 8),
          (2, 1, 9, 8, 9, 8), (37, 61, 19, 19, 5, 4), (1, 1300, 13, 13, 3, 2), (2, 3, 17, 18, 5, 0), (1, 4, 30, 30, 13, 0), (2, 3, 61, 47, 3, 1),
-         (1, 2, 91, 130, 9, 8), (1, 2, 300, 301, 3, 2), (1, 2, 67, 95, 5, 4), (5, 7, 14, 15, 2, 1)]
+         (1, 2, 91, 130, 9, 8), (1, 2, 300, 301, 3, 2), (1, 2, 67, 95, 5, 4), (5, 7, 14, 15, 2, 1),
+         (1, 1, 1, 1, 2, 1), (3, 5, 1, 2, 2, 1), (2, 3, 3, 1, 2, 1), (1, 4, 13, 13, 2, 1), (7, 11, 26, 23, 2, 1), (1, 1, 8, 8, 2, 1)]
 
 
 @pytest.mark.parametrize("case", CASES, ids=str)
@@ -39,7 +40,7 @@ def test_slide(ops, oracle, case):
         layers.run_maxpool(ops, oracle, x, k, 1, p, 2203)
 
 
-@pytest.mark.parametrize("k", [3, 5, 13])
+@pytest.mark.parametrize("k", [2, 3, 5, 13])
 def test_off_a_boundary(ops, k):
     """Tensors that begin one value behind a 16-byte boundary: the results of those that begin on one."""
     found = []
