@@ -97,9 +97,8 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
     // Two shapes of the first pass.  Grouped: no branch around the loads (see the forward kernel), lanes
     // past the end read the first vector; kGroup steps at a time, their loads go out together, then each
     // is used as it arrives.  The large form (part of the slice in LDS) is bound by its loads and takes
-    // them so in groups of four; the scalar form in groups of eight (behind a branch a lane waits for
-    // each step's loads before it asks for the next: six trips to memory one after the other at
-    // 16 x 256 x 19^2, 10.4 us against 8.8).  The 128-bit form without an LDS part is held to 64
+    // them so in groups of four; the form with one value a step (planes below four values) in groups of eight (behind a
+    // branch a lane waits for each step's loads before it asks for the next).  The 128-bit form without an LDS part is held to 64
     // registers, where a group of two already spills (18.3 against 16.4 us at 16 x 256 x 38^2): it skips a step
     // past the end of the slice outright, as every form does in the second pass, which finds x in the cache.
     constexpr int kGroup = L > 0 ? 4 : 8;
