@@ -167,7 +167,7 @@ __device__ __forceinline__ void st_step(float* p, const Step& s, const Pack<V>& 
 
 // The small forms (small_slice below): a lane adds the values of a vector in fp32 and its vectors in doubles -- no further
 // from 64 bits than a lane of the other forms that holds one vector -- and the backward keeps x beside the delta.  (Odd
-// planes: every value in doubles.)
+// planes, and one value a step in whatever form: every value in doubles.)
 template<int V, int R, int L, int T>
 constexpr bool kSmallSlice = L == 0 && T < kResidentThreads && V * R <= 32;
 
@@ -301,10 +301,19 @@ inline int resident_vectors(int batch, int channels, int spatial, bool vec)
 // 41.4, 8 x 512 43.0; 16 x 512 x 19^2: 3 x 1024 14.3); six steps in workgroups of 256 lanes serve a thousand channels, whose
 // workgroups then run in one round (16 x 1024 x 19^2 16.7 against 18.2 with 3 x 512), three in 512 lanes up to half as many
 // (16 x 512 x 19^2, mish: 11.3 against 12.5).
-constexpr int kOddSpatial = 4;                    // planes below have no vector: one value a step
+// Planes below kOddSpatial have no vector: one value a step, in forms that hold as much as those of the others.  Three launches
+// give each plane a wave of its own.
+// us, leaky and mish, one launch and (*) several: forward, + shortcut, backward
+//   2731 x 5 x 2       7.7, 9.7, 9.2      8.1, 10.3, 10.6    12 x 512     12.6*, 12.6*, 13.7*   12.8*, 12.8*, 16.0*
+//   2048 x 64 x 3      16.7, 25.8, 24.7   16.9, 25.9, 25.4   12 x 512     34.7*, 34.0*, 37.1*   34.2*, 33.6*, 47.3*
+//   4000 x 256 x 3     59, 93, 92         60, 94, 92         16 x 1024    191*, 192*, 209*      191*, 192*, 292*
+//   8000 x 256 x 3     127, 192, 185      128, 194, 185      24 x 1024    369*, 374*, 402*      369*, 374*, 605*
+// Workgroups of the size that just holds the slice: 64 x 1024 x 1 in 64 lanes 6.7, 7.6, 8.2, in 256 7.2, 8.6, 8.4;
+// 513 x 97 x 2 in 256 lanes 7.9, 8.6, 9.2, in 1024 8.7, 11.1, 11.2.
+constexpr int kOddSpatial = 4;
 constexpr uint32_t kOddVectors = 6144;
 constexpr uint32_t kOddVectorsFew = 4096;         // with fewer than kResidentChannels channels (as kSmallVectors)
-constexpr uint32_t kOddValues = kResidentVectors * kResidentThreads, kOddValuesFew = 1024;
+constexpr uint32_t kOddValues = 4 * kOddVectors, kOddValuesFew = 6144;
 constexpr int kOddChannels = 512;
 
 // The vectors (values in planes below kOddSpatial) of a channel's slice where such a shape takes a one-launch form, else 0.
@@ -323,8 +332,14 @@ template<typename F>
 void dispatch_odd_form(uint32_t items, const ResidentGeom& g, F&& launch)
 {
     if (g.spatial < kOddSpatial) {
-        if (items <= kOddValuesFew) return launch.template operator()<1, 4, 256>();
-        return launch.template operator()<1, kResidentVectors, kResidentThreads>();
+        if (items <= 64 * 4) return launch.template operator()<1, 4, 64>();
+        if (items <= 256 * 4) return launch.template operator()<1, 4, 256>();
+        if (items <= 256 * 8) return launch.template operator()<1, 8, 256>();
+        if (items <= 512 * 8) return launch.template operator()<1, 8, 512>();
+        if (items <= 512 * 12) return launch.template operator()<1, 12, 512>();
+        if (items <= 1024 * 8) return launch.template operator()<1, 8, 1024>();
+        if (items <= 1024 * 16) return launch.template operator()<1, 16, 1024>();
+        return launch.template operator()<1, 24, 1024>();
     }
     if (items <= 64) return launch.template operator()<4, 1, 64>();
     if (items <= 128 * 2) return launch.template operator()<4, 2, 128>();

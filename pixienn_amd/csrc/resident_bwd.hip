@@ -91,8 +91,8 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
     };
     const bool recompute = a.b.pre == nullptr;
     Pack<V> d[R];
-    std::conditional_t<kSmall, double, float> fa = 0, fb = 0;
-    [[maybe_unused]] std::conditional_t<kSmall, double, float> fq = 0;
+    std::conditional_t<kSmall || V == 1, double, float> fa = 0, fb = 0;
+    [[maybe_unused]] std::conditional_t<kSmall || V == 1, double, float> fq = 0;
     [[maybe_unused]] float peak = 0.0f;
     // Two shapes of the first pass.  Grouped: no branch around the loads (see the forward kernel), lanes
     // past the end read the first vector; kGroup steps at a time, their loads go out together, then each
@@ -337,7 +337,7 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
 // Waves per SIMD that the registers are held to.
 template<int V, int R, int L, int MODE, int T, bool RAGGED>
 constexpr int kBwdWaves = RAGGED && T == kResidentThreads ? 4 : RAGGED || kSmallSlice<V, R, L, T> ? (MODE == kRedo || V * R >= 32 ? 2 : V * R >= 12 ? 4 : V * R == 8 ? 6 : 8)
-                          : L == 0 && MODE != kRedo ? 8 : 4;
+                          : L == 0 && MODE != kRedo && !(V == 1 && R > 16) ? 8 : 4;
 
 // One workgroup per channel.  (The forms of 1024 lanes without an LDS part are held to 64 registers, two workgroups
 // per compute unit: they run the 19 x 19 and 38 x 38 layers, whose launches are too short to fill the

@@ -15,7 +15,7 @@ constexpr int kResidualAhead = 4;
 // Waves per SIMD that the registers are held to: a vector a step, two with a shortcut.
 template<int V, int R, int L, int T, bool RES, bool RAGGED>
 constexpr int kFwdWaves = RAGGED || kSmallSlice<V, R, L, T> ? (RAGGED && T == kResidentThreads ? (RES ? 4 : 8) : V * R >= 32 ? 2 : RES && V * R >= 12 ? 4 : 8)
-                          : L == 0 && V * R <= (V == 1 ? 8 : 32) ? 8 : 4;
+                          : L == 0 && V * R <= (V == 1 ? (RES ? 8 : 16) : 32) ? 8 : 4;
 
 // V = 4 needs spatial % 4 == 0 and 16-byte aligned tensors, RAGGED (odd planes) neither.  R + L vectors per thread at most.
 template<int ACT, int V, int R, int L, int T = kResidentThreads, bool RES = false, bool RAGGED = false>
@@ -89,7 +89,7 @@ __global__ __launch_bounds__(T, (kFwdWaves<V, R, L, T, RES, RAGGED>)) void bn_re
     // (16 x 1024 x 19^2: 19.9 us against 25.6 us with every step's load behind the reduction).
     // (the half-size workgroups of the 128-bit form have 128 registers: eight of twelve steps, four of sixteen)
     constexpr int kAhead = !RES ? 0 : kSmall || V * (R + L) <= 8 ? R + L : L > 0 ? kResidualAhead
-                                : T < kResidentThreads ? (R <= 12 ? 8 : 4) : 0;
+                                : T < kResidentThreads ? (R <= 12 ? 8 : 4) : V == 1 ? 4 : 0;
     [[maybe_unused]] Pack<V> ahead[kAhead > 0 ? kAhead : 1];
     if constexpr (RES) {
 #pragma unroll
@@ -109,7 +109,7 @@ __global__ __launch_bounds__(T, (kFwdWaves<V, R, L, T, RES, RAGGED>)) void bn_re
                 t2 += static_cast<double>(d * d);
             }
         }
-    } else if constexpr (kSmall) {
+    } else if constexpr (kSmall || V == 1) {
         t1 = t2 = 0.0;
 #pragma unroll
         for (int r = R - 1; r >= 0; --r) {
@@ -142,7 +142,7 @@ __global__ __launch_bounds__(T, (kFwdWaves<V, R, L, T, RES, RAGGED>)) void bn_re
     }
     __syncthreads();
     const FoldCoef k = shared_coef;
-    if constexpr (L > 0 && RES) asm volatile("" : "+v"(lane));      // addresses formed again, not kept: they would spill
+    if constexpr (RES && (L > 0 || R > 16)) asm volatile("" : "+v"(lane));      // addresses formed again, not kept: they would spill
     const auto apply = [&](int r, [[maybe_unused]] const Pack<V>& from) {
         const uint32_t e = element(r);
         const Step kept = RAGGED ? step(r) : Step{ 0, e < a.g.per_channel, 0 };

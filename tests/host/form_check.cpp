@@ -1,0 +1,47 @@
+// Which shapes take the one-launch training passes (pixienn_amd/csrc/resident.h), on the host: every form that is chosen holds
+// its slice, and the lines lie where they are said to.
+#include "../../pixienn_amd/csrc/resident.h"
+
+#include <cstdio>
+
+using namespace pxh;
+
+namespace {
+
+int failed = 0, checks = 0;
+
+void check(bool good, const char* what, int batch, int channels, int spatial)
+{
+    ++checks;
+    if (!good && ++failed < 10) std::printf("%s: %d x %d x %d\n", what, batch, channels, spatial);
+}
+
+}  // namespace
+
+int main()
+{
+    for (int channels: { 1, 5, 95, 96, 512, 513, 1024 })
+        for (int spatial: { 1, 2, 3, 5, 7, 9, 49, 63, 169, 361, 1025, 2051 })
+            for (int batch = 1; batch < 40000; batch += batch < 300 ? 1 : batch / 50) {
+                const size_t values = static_cast<size_t>(batch) * spatial;
+                if (values > 200000) break;
+                for (bool backward: { false, true })
+                    for (int activation: { PXH_LEAKY, PXH_MISH }) {
+                        const ResidentForm form = resident_form(batch, channels, spatial, false, activation, backward);
+                        check(!form.per_thread && !form.small, "vectors only where planes have them whole", batch, channels, spatial);
+                        if (!form.odd) continue;
+                        const ResidentGeom g = resident_geom(batch, channels, spatial);
+                        dispatch_odd_form(form.odd, g, [&]<int V, int R, int T>() {
+                            const size_t items = V == 1 ? values : g.vectors;
+                            check(static_cast<size_t>(R) * T >= items, "a form holds its slice", batch, channels, spatial);
+                            check(V == 1 || spatial >= 4, "a vector fits a plane", batch, channels, spatial);
+                        });
+                    }
+                const bool one = odd_slice(batch, channels, spatial, false) != 0;
+                if (spatial < 4) check(one == (values <= (channels < 96 ? 6144u : 24576u)), "planes below a vector", batch, channels, spatial);
+                // a workspace too small is refused on both sides of lines that may move: this one does not
+                check(asks_for_workspace(batch, channels, spatial, false) == (channels < 96 || values > 8192), "the workspace", batch, channels, spatial);
+            }
+    std::printf("%d checks, %d failed\n", checks, failed);
+    return failed != 0;
+}
