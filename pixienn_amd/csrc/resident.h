@@ -296,11 +296,14 @@ inline int resident_vectors(int batch, int channels, int spatial, bool vec)
 //   8 x 512 x 19^2     5.9 ->  5.7   6.4 ->  6.0   7.7 ->  6.6  10.8 ->  9.8   3 x 256    7.6 ->  6.5   8.0 ->  6.9   9.7 ->  8.0  13.0 -> 11.5
 //   8 x 96 x 45^2      9.2 ->  6.8  12.7 ->  9.0  12.5 ->  9.5  17.2 -> 13.3   4 x 1024  14.3 ->  8.7  15.8 -> 10.8  16.0 -> 12.3  20.7 -> 17.1
 //   4 x 1024 x 13^2    5.1 ->  4.9   5.3 ->  5.2   5.6 ->  5.5   9.3 ->  8.9   2 x 128    5.8 ->  5.4   5.9 ->  5.7   6.7 ->  6.3  10.2 ->  9.7
-//   1 x 1024 x 13^2    4.1 ->  4.3   4.2 ->  4.5   4.4 ->  4.3   7.7 ->  7.8   1 x 64     4.5 ->  4.4   4.5 ->  4.6   5.0 ->  4.5   8.5 ->  8.1
+//   1 x 1024 x 13^2    4.2 ->  4.0   4.3 ->  4.3   4.4 ->  4.3   7.2 ->  7.1   1 x 64     4.6 ->  4.4   4.9 ->  4.7   4.9 ->  4.3   7.7 ->  7.3
+//   1 x 1024 x 19^2    5.1 ->  4.5   5.2 ->  4.6   5.4 ->  4.5   9.0 ->  7.4   1 x 128    5.4 ->  5.0   5.5 ->  5.2   5.9 ->  4.9   9.1 ->  7.8
 // (steps x lanes of the form.)  More lanes than the slice needs are slower everywhere (64 x 1024 x 13^2, backward: 4 x 1024
 // 41.4, 8 x 512 43.0; 16 x 512 x 19^2: 3 x 1024 14.3); six steps in workgroups of 256 lanes serve a thousand channels, whose
 // workgroups then run in one round (16 x 1024 x 19^2 16.7 against 18.2 with 3 x 512), three in 512 lanes up to half as many
-// (16 x 512 x 19^2, mish: 11.3 against 12.5).
+// (16 x 512 x 19^2, mish: 11.3 against 12.5).  Up to 128 vectors a step is enough (1 x 256 x 17^2, mish, backward: 1 x 128 3.8,
+// 2 x 128 4.3), and a slice of a value per lane needs no vectors, whose addresses and shared values are then the longer part of
+// a short launch (1 x 1024 x 7^2, mish: forward 3.8 against 4.2 in vectors, + shortcut 3.8 and 4.5).
 // Planes below kOddSpatial have no vector: one value a step, in forms that hold as much as those of the others.  Three launches
 // give each plane a wave of its own.
 // us, leaky and mish, one launch and (*) several: forward, + shortcut, backward
@@ -331,6 +334,7 @@ inline uint32_t odd_slice(int batch, int channels, int spatial, bool vec)
 template<typename F>
 void dispatch_odd_form(uint32_t items, const ResidentGeom& g, F&& launch)
 {
+    if (g.per_channel <= 64) return launch.template operator()<1, 1, 64>();
     if (g.spatial < kOddSpatial) {
         if (items <= 64 * 4) return launch.template operator()<1, 4, 64>();
         if (items <= 256 * 4) return launch.template operator()<1, 4, 256>();
@@ -342,6 +346,7 @@ void dispatch_odd_form(uint32_t items, const ResidentGeom& g, F&& launch)
         return launch.template operator()<1, 24, 1024>();
     }
     if (items <= 64) return launch.template operator()<4, 1, 64>();
+    if (items <= 128) return launch.template operator()<4, 1, 128>();
     if (items <= 128 * 2) return launch.template operator()<4, 2, 128>();
     if (items <= 256 * 3) return launch.template operator()<4, 3, 256>();
     if (items <= 256 * 6 && g.channels > kOddChannels) return launch.template operator()<4, 6, 256>();

@@ -35,6 +35,8 @@ int main()
                             const size_t items = V == 1 ? values : g.vectors;
                             check(static_cast<size_t>(R) * T >= items, "a form holds its slice", batch, channels, spatial);
                             check(V == 1 || spatial >= 4, "a vector fits a plane", batch, channels, spatial);
+                            if (values <= 64) check(V == 1 && R == 1 && T == 64, "a value per lane", batch, channels, spatial);
+                            else if (V == 4 && items <= 128) check(R == 1, "a vector per lane", batch, channels, spatial);
                         });
                     }
                 const bool one = odd_slice(batch, channels, spatial, false) != 0;
