@@ -23,17 +23,29 @@ def _exact(act, x):
         return np.where(x > 40, 1.0, t + np.maximum(x, -700.0) * (1.0 - t * t) * s)
 
 
-# in units of 2^-24.  A logistic is formed from an exponential good to 1.5 units in its last place, a rounded sum and a
-# quotient good to one: 4 of its value, 5 with its complement's rounding.  swish multiplies by x and adds three terms of up
-# to 1.3 (each rounded): 6 + 2 |x| s.  mish takes tanh(softplus) from u = float(1 + exp(x)): a unit of u moves it by as much
-# again, and 1 - t^2, rounded to 2^-24, is multiplied by x.
+# in units of 2^-24.  An exponential is good to one unit in its last place, 2; a logistic s from it, with a rounded sum and a
+# quotient good to one, to 4 of its value, 5 with its complement's rounding.
+# swish adds x * s and s * (1 - x * s): 4 + 1 of |x| s and 4 + 0.5 + 1 of s below -14, where the second factor rounds to 1 and
+# nothing cancels, and half a unit of the sum: 6 (1 + |x|) s.  Above, terms of up to 1.3 (each rounded) and 4 |x| s.
+# mish takes t = tanh(softplus) from u = float(1 + exp(x)), whose rounding is half a unit in its last place, 1, and moves t by
+# no more; the quotient adds 5 of t.  1 - t^2 is then off by 2 t (1 + 5 t) + 1, times |x| s, s and the products' roundings by 7 of
+# |x| s, and the sum by one of t: 1 + 6 t + |x| s (2 t (1 + 5 t) + 8).  Below -20 t is the exponential itself, and so is s:
+# 6 (1 + |x|) s.  Above 0 the terms are of the order of 1 and |x|.
 def _bound(act, x, s):
-    unit = 2.0 ** -24
+    unit, size = 2.0 ** -24, np.abs(x)
+    tail = 6.0 * (1.0 + size) * s
     if act == "swish":
-        return unit * (6.0 + 4.0 * np.abs(x) * s)
+        return unit * np.where(x < -14.0, tail, 6.0 + 4.0 * size * s)
     if act == "mish":
-        return unit * (6.0 + 4.0 * np.minimum(np.abs(x), 20.0))
-    return unit * 5.0 * np.maximum(s, 2.0 ** -126)
+        t = np.tanh(np.log1p(np.exp(np.clip(x, -700.0, 40.0))))
+        middle = 1.0 + 6.0 * t + size * s * (2.0 * t * (1.0 + 5.0 * t) + 8.0)
+        return unit * np.where(x < -20.0, tail, np.where(x < 0.0, middle, 6.0 + 4.0 * np.minimum(size, 20.0)))
+    return unit * 5.0 * s
+
+
+# (exponentials below the smallest normal float, from -87 on, have fewer digits: a unit of the smallest subnormal for each term)
+def _fewer_digits(x):
+    return 2.0 ** -149 * 4.0 * (1.0 + np.minimum(np.abs(x), 200.0)) * (x < -87.0)
 
 
 @pytest.mark.parametrize("act", ["logistic", "swish", "mish", "softplus"])
@@ -46,8 +58,12 @@ def test_gradient_over_the_whole_range(act):
     xd = x.astype(np.float64)
     s = np.where(xd > -700, 1.0 / (1.0 + np.exp(-np.clip(xd, -700.0, 700.0))), 0.0)
     err = np.abs(got - _exact(act, xd))
-    # (exponentials below the smallest normal float have fewer digits)
-    bad = err > _bound(act, xd, s) + 2.0 ** -126 * np.maximum(1.0, np.abs(xd)) * (xd < -80)
+    bound = _bound(act, xd, s) + _fewer_digits(xd)
+    # in the tail a gradient of 0 or of the wrong sign is beyond the bound
+    if act in ("swish", "mish"):
+        tail = (xd < -20.0) & (xd > -87.0)
+        assert tail.sum() > 10000 and np.all(bound[tail] < 1e-5 * np.abs(_exact(act, xd[tail])))
+    bad = err > bound
     assert not bad.any(), (act, x[bad][:5], got[bad][:5], err[bad][:5])
 
 
