@@ -45,28 +45,16 @@ def test_training_epilogue_with_shortcut_is_the_two_calls_to_the_bit(ops, act):
         ops.bn_train_act_shortcut_forward(gx, y1, m1, v1, rm1, rv1, gscale, gbias, act, gfrom, alpha, beta,
                                           pre_activation=pre1, x_saved=xs1, x_norm=xn1)
         what = "%s %s alpha %g beta %g" % (act, (N, C, HW), alpha, beta)
-        # Scalar slices of up to 8192 values and 512 channels and more: alone, the layer runs with workgroups of half the
-        # size, which add up a channel's statistics in another order than the full workgroups the fused call keeps; there
-        # the two agree to rounding of the sums (1e-6 of the statistics), everywhere else to the bit.
-        same_order = not (HW % 4 != 0 and C >= 512 and N * HW <= 8192)
-        if same_order:
-            same = assert_bit_exact
-        else:
-            sigma = np.sqrt(host(v0).astype(np.float64))
-            fl = ((np.abs(host(m0)) + sigma) / sigma).reshape(1, C, 1, 1) * 4.0 + np.abs(frm)
-
-            def same(got, want, what):
-                assert_close(got, want, 2e-6, fl if got.ndim == 4 else 1.0, what)
-        same(host(y1), host(out0), what + " output")
+        assert_bit_exact(host(y1), host(out0), what + " output")
         for name, a, b in (("pre-activation", pre1, pre0), ("x_norm", xn1, xn0), ("mean", m1, m0),
                            ("var", v1, v0), ("rolling mean", rm1, rm0), ("rolling var", rv1, rv0)):
-            same(host(a), host(b), what + " " + name)
+            assert_bit_exact(host(a), host(b), what + " " + name)
         assert_bit_exact(host(xs1), host(xs0), what + " x_saved")
         # no extra outputs, the shortcut's source in the output tensor itself (the layer writes in place of `from`)
         y2 = gpu(frm)
         m2, v2, rm2, rv2 = gpu(np.zeros(C, F)), gpu(np.zeros(C, F)), gpu(rmean), gpu(rvar)
         ops.bn_train_act_shortcut_forward(gx, y2, m2, v2, rm2, rv2, gscale, gbias, act, y2, alpha, beta)
-        same(host(y2), host(out0), what + " output, from == y")
+        assert_bit_exact(host(y2), host(out0), what + " output, from == y")
 
 
 @pytest.mark.parametrize("act", ["leaky", "mish", "linear", "swish", "relu"])
