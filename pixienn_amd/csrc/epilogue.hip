@@ -1120,10 +1120,6 @@ constexpr size_t kGroupFewest = 1u << 19, kGroupFewestSmooth = 1u << 20, kGroupF
 //   16 x 64 x 151^2            88   -> 66.5; 97   -> 73.2, 97   -> 73.3, 124  -> 118         93.2 -> 82.9; 102  -> 91.6, 104  -> 109,  144  -> 164
 // (8 x 96 x 135 x 77 and 16 x 64 x 151^2, mish, in launches of one value per access: 51, 59, 59, 84 and 110, 117, 117, 169.)
 //
-// As many members as make kGroupFill workgroups of a whole number of channels: a few more than the machine holds run in a
-// second round (8 x 96 x 135 x 77 in 576 and in 480: 33.6 -> 26.4, 64 x 200 x 25^2 600 and 400: 34.5 -> 28.8,
-// 9 x 20 x 203 x 251 520 and 500: 37.0 -> 29.3).
-//
 // Small tensors (which the caches hold for the launches that read them twice) stay with those launches: a group's second one
 // costs them more where it has something to do.  Three or five launches -> groups, us: plain; clipped with nothing to change,
 // rescaled, and clamped throughout:
@@ -1140,8 +1136,7 @@ GroupPlan grouped_backward(int batch, int channels, int spatial, bool vec, int p
     if (per_thread && (!selects(activation) || channels < kGroupAlone)) return GroupPlan{};
     const uint32_t places = group_places(s);
     // (as few members as hold the slice where the words of more would not fit: up to three channels of a few thousand vectors)
-    const size_t whole = kGroupFill / channels * channels;
-    for (const size_t workgroups: { whole > 0 ? whole : 1, static_cast<size_t>(1) }) {
+    for (const size_t workgroups: { group_fill(channels), static_cast<size_t>(1) }) {
         const GroupPlan p = group_plan(batch, channels, spatial, vec, workgroups, places);
         if (per_thread && p.members > 1) return GroupPlan{};
         if (p.members <= 1 ||

@@ -1,4 +1,4 @@
-// split_slice (pixienn_amd/csrc/grouped.h) on the host, over slices, channel counts and places of a stream.
+// split_slice and group_plan (pixienn_amd/csrc/grouped.h) on the host, over slices, channel counts and places of a stream.
 #include "../../pixienn_amd/csrc/grouped.h"
 
 #include <cstdio>
@@ -22,7 +22,7 @@ int main()
     const uint32_t per_member = kGroupItems;
     for (uint32_t places: { 0u, 2u, 8u, 16u, 64u, 510u, 512u, 608u })
         for (size_t channels: { 1, 2, 3, 5, 7, 8, 16, 31, 64, 95, 512, 1024 })
-            for (size_t workgroups: { kGroupFill, static_cast<size_t>(1) })
+            for (size_t workgroups: { group_fill(static_cast<int>(channels)), static_cast<size_t>(1) })
                 for (size_t items = 1; items < 2000000; items += items < 20000 ? 61 : items / 7) {
                     const GroupPlan p = split_slice(items, per_member, channels, workgroups, places);
                     if (!p.members) continue;
@@ -32,16 +32,24 @@ int main()
                     check(static_cast<size_t>(p.span) * (p.members - 1) < items, "every member has items", items, channels, places);
                 }
 
-    // the splits that the shapes of tests/test_gpu_shared_slices.py are chosen for
-    const struct { size_t items, channels; uint32_t per_member, members, span; } named[] = {
-        { 4097, 95, kGroupItems, 2, 2112 }, { 6144, 64, kGroupItems, 3, 2048 }, { 17521, 30, kGroupItems, 8, 2240 },
-        { 24579, 12, kGroupItems, 12, 2112 }, { 133120, 8, kGroupItems, 64, 2112 }, { 133120, 7, kGroupItems, 0, 0 },
-        { 98304, 32, kGroupItems, 16, kGroupItems }, { 24579, 130, kGroupItems, 5, 4928 }, { 4112, 512, kGroupItems, 1, 4160 },
-        { 83160, 96, 4 * kGroupItems, 6, 13888 }, { 180000, 41, 4 * kGroupItems, 13, 13888 },
-        { 393215, 32, 4 * kGroupItems, 16, 4 * kGroupItems },
+    // workgroups of a whole number of channels, as many as the device runs at once
+    for (int channels = 1; channels < 1100; ++channels) {
+        const size_t fill = group_fill(channels);
+        check(channels > 512 ? fill == 1 : fill % channels == 0 && fill <= 512 && fill + channels > 512, "whole channels", fill, channels, 512);
+    }
+
+    // the splits that the shapes of tests/test_gpu_shared_slices.py and of tests/test_gpu_odd_planes.py are chosen for
+    const struct { int batch, channels, spatial; bool vec; uint32_t items, members, span; } named[] = {
+        { 1, 95, 16388, true, 4097, 2, 2112 }, { 4, 64, 6144, true, 6144, 3, 2048 }, { 7, 30, 10012, true, 17521, 8, 2240 },
+        { 3, 12, 32772, true, 24579, 12, 2112 }, { 1, 8, 532480, true, 133120, 64, 2112 }, { 1, 7, 532480, true, 133120, 0, 0 },
+        { 4, 32, 98304, true, 98304, 16, kGroupItems }, { 3, 130, 32772, true, 24579, 5, 4928 }, { 4, 512, 4112, true, 4112, 1, 4160 },
+        { 16, 48, 10816, true, 43264, 10, 4352 },
+        { 8, 96, 10395, false, 20792, 5, 4160 }, { 32, 41, 5625, false, 45024, 12, 3776 }, { 1, 32, 393215, false, 98304, 16, kGroupItems },
+        { 1, 90, 16385, false, 4097, 2, 2112 }, { 2, 23, 25 * 1025, false, 12814, 6, 2176 }, { 3, 70, 10243, false, 7683, 3, 2624 },
     };
     for (const auto& n: named) {
-        const GroupPlan p = split_slice(n.items, n.per_member, n.channels, kGroupFill, 512);
+        const GroupPlan p = group_plan(n.batch, n.channels, n.spatial, n.vec, group_fill(n.channels), 512);
+        check(!p.members || p.items == n.items, "vectors of a named slice", n.items, n.channels, 512);
         check(p.members == n.members && p.span == n.span, "the split of a named slice", n.items, n.channels, 512);
     }
 

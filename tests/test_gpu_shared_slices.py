@@ -16,8 +16,8 @@ pytestmark = pytest.mark.gpu
 # tests/host/split_check.cpp.
 VECTORS = [(1, 95, 16388), (4, 64, 6144), (7, 30, 10012), (3, 12, 32772), (1, 8, 532480), (1, 7, 532480), (4, 32, 98304),
            (3, 130, 32772), (4, 512, 4112)]
-# values of odd planes, past kGroupScalars: six members, thirteen, and sixteen that are full but for the last value
-SCALARS = [(8, 96, 10395), (32, 41, 5625), (1, 32, 393215)]
+# odd planes: five members, twelve, and sixteen that are full (but for the last value, which its vector shares)
+ODD = [(8, 96, 10395), (32, 41, 5625), (1, 32, 393215)]
 
 
 @pytest.fixture(scope="module")
@@ -27,7 +27,7 @@ def ops():
 
 
 @pytest.mark.parametrize("act", ["leaky", "mish"])
-@pytest.mark.parametrize("shape", VECTORS + SCALARS, ids=str)
+@pytest.mark.parametrize("shape", VECTORS + ODD, ids=str)
 def test_shared_slices_backward(ops, oracle, monkeypatch, shape, act):
     for module in (epilogue, clipped):
         monkeypatch.setattr(module, "TRAIN_SHAPES", [shape])
