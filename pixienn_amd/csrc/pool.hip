@@ -55,9 +55,11 @@ __global__ __launch_bounds__(kBlock) void maxpool_fwd_generic_kernel(const float
 
 // Windows of 2 that move by one cell over a tensor of the output's size: four outputs of the flat tensor to a lane, whose cells
 // are the five from the first output on and the five a row further, whatever rows they lie in.  One output per lane read
-// each of its cells by itself; us: 32768 planes of 13 x 13 22.5 -> 13.4, 512 level (5.0).
+// each of its cells by itself; us: 32768 planes of 13 x 13 22.5 -> 13.4, 512 of 13 x 13 2.9 -> 2.7, of 26 x 26 3.5 -> 3.1.  (A
+// launch this short is one trip to memory: the outputs whose row further would end behind the tensor, taken one after the other
+// by a scan, made it 4.5.)
 __global__ __launch_bounds__(kBlock) void maxpool_fwd_step1_kernel(const float* in, float* out, int* indexes, uint32_t total,
-                                                                   PoolGeom g, FastDiv by_w, FastDiv by_h)
+                                                                   FastDiv by_w, FastDiv by_h)
 {
     const uint32_t o = (blockIdx.x * kBlock + threadIdx.x) * 4;
     if (o >= total) return;
@@ -65,33 +67,24 @@ __global__ __launch_bounds__(kBlock) void maxpool_fwd_step1_kernel(const float* 
     by_w.divmod(o, rows, x);
     by_h.divmod(rows, plane, y);
     const uint32_t w = by_w.d, h = by_h.d;
-    if (o + w + 5 > total) {
-        // the cells of a row further end with the tensor
-        for (uint32_t q = 0; q < 4 && o + q < total; ++q) {
-            float best;
-            int best_at;
-            scan_window(in, g, plane, y, x, best, best_at);
-            out[o + q] = best;
-            indexes[o + q] = best_at;
-            if (++x == w) {
-                x = 0;
-                if (++y == h) {
-                    y = 0;
-                    ++plane;
-                }
-            }
-        }
-        return;
-    }
     float a[5], b[5];
-    const Pack<4> a4 = ld_word<false>(in + o), b4 = ld_word<false>(in + o + w);
+    if (o + w + 5 <= total) {
+        const Pack<4> a4 = ld_word<false>(in + o), b4 = ld_word<false>(in + o + w);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        a[q] = a4.v[q];
-        b[q] = b4.v[q];
+        for (int q = 0; q < 4; ++q) {
+            a[q] = a4.v[q];
+            b[q] = b4.v[q];
+        }
+        a[4] = in[o + 4];
+        b[4] = in[o + w + 4];
+    } else {
+        // the cells of a row further end with the tensor: those beyond are no output's
+#pragma unroll
+        for (int q = 0; q < 5; ++q) {
+            a[q] = in[min(o + q, total - 1)];
+            b[q] = in[min(o + q + w, total - 1)];
+        }
     }
-    a[4] = in[o + 4];
-    b[4] = in[o + w + 4];
     Pack<4> value, index;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -110,8 +103,17 @@ __global__ __launch_bounds__(kBlock) void maxpool_fwd_step1_kernel(const float* 
             ++x;
         }
     }
-    st_word<false>(out + o, value);
-    st_word<false>(reinterpret_cast<float*>(indexes) + o, index);
+    if (o + 4 <= total) {
+        st_word<false>(out + o, value);
+        st_word<false>(reinterpret_cast<float*>(indexes) + o, index);
+    } else {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            if (o + q >= total) break;
+            out[o + q] = value.v[q];
+            indexes[o + q] = __float_as_int(index.v[q]);
+        }
+    }
 }
 
 // ------------------------------------------------------------------ max-pool through LDS
@@ -256,7 +258,7 @@ __global__ __launch_bounds__(kBlock) void maxpool_fwd_slide_kernel(const float* 
     float* const best_of = cells + all_rows * st.pitch;        // [all_rows][width]
     uint8_t* const tap_of = reinterpret_cast<uint8_t*>(best_of + all_rows * width);
     const uint32_t in0 = (p0 * g.ih + y_lo) * g.iw;
-    const uint32_t values = all_rows * g.iw, vectors = values / 4;
+    const uint32_t values = all_rows * g.iw, vectors = values > kBlock ? values / 4 : 0;      // (a value to a lane where that is all)
     Pack<4> v[kLoads];
     const auto fetch = [&](uint32_t first) {
 #pragma unroll
@@ -497,7 +499,8 @@ struct PoolWindows {
 
 // K: the window of a kernel that moves by one cell over rows of at least K, or 0 for any geometry.  There a window's taps are
 // told apart by one division of the distance from its first cell.  The outputs come in by 128-bit loads that are in flight
-// while the masks are cleared.  us, 8192 planes of 19 x 19: k = 5 19.3 -> 14.2, 9 34.3 -> 22.8, 13 55.5 -> 44.0; 64 of 300 x 300,
+// while the masks are cleared, one at a time where a lane has one or two (four to some of the lanes: 512 planes of 13 x 13, 3 / 2, 3.8 -> 4.5).
+// us, 8192 planes of 19 x 19: k = 5 19.3 -> 14.2, 9 34.3 -> 22.8, 13 55.5 -> 44.0; 64 of 300 x 300,
 // k = 3, 32.8 -> 24.9; 32768 of 13 x 13, k = 2, 30.1 -> 21.3.  (Any geometry, by the loads alone: 1024 of 151 x 151, 3 / 2,
 // 53.2 -> 48.7.)
 template<int K>
@@ -509,8 +512,10 @@ __global__ __launch_bounds__(kBlock) void maxpool_bwd_tile_kernel(const float* d
 {
     extern __shared__ __align__(16) float lds[];
     constexpr int kLoads = 2;
+    constexpr uint32_t kSteps = K ? 1 : 2;      // up to as many outputs a lane are taken one at a time
     const int k = K ? K : g.kernel;
     const uint32_t along = K ? K : w.along, words = K ? (K * K + 31) / 32 : w.words;
+    const int past = g.ow - static_cast<int>(along);       // from the last of a cell's windows of a row to the first of the next
     const auto by_stride = [&](uint32_t n) { return K ? n : w.by_stride.div(n); };
     uint32_t* masks = reinterpret_cast<uint32_t*>(lds);                      // [word][tile_cells]
     float* deltas = lds + words * tile_cells;                                // [tile_outputs]
@@ -532,7 +537,7 @@ __global__ __launch_bounds__(kBlock) void maxpool_bwd_tile_kernel(const float* d
     }
     const uint32_t cells = planes * rows_in * g.iw;
     const uint32_t cell0 = (p0 * g.ih + y_lo) * g.iw, out0 = (p0 * g.oh + oy_lo) * g.ow;
-    const uint32_t outputs = planes * rows_out * g.ow, vectors = outputs / 4;
+    const uint32_t outputs = planes * rows_out * g.ow, vectors = outputs > kSteps * kBlock ? outputs / 4 : 0;
     Pack<4> d[kLoads], at[kLoads];
     const auto fetch = [&](uint32_t first) {
 #pragma unroll
@@ -599,8 +604,10 @@ __global__ __launch_bounds__(kBlock) void maxpool_bwd_tile_kernel(const float* d
             }
         }
     }
-    if (threadIdx.x < outputs - 4 * vectors) {
-        const uint32_t j = 4 * vectors + threadIdx.x;
+#pragma unroll
+    for (uint32_t step = 0; step < kSteps; ++step) {
+        const uint32_t j = 4 * vectors + step * kBlock + threadIdx.x;
+        if (j >= outputs) break;
         uint32_t plane, row, ox;
         place(j, plane, row, ox);
         take(j, plane, row, ox, delta[out0 + j], indexes[out0 + j]);
@@ -630,18 +637,17 @@ __global__ __launch_bounds__(kBlock) void maxpool_bwd_tile_kernel(const float* d
         const int lift = k * g.stride;
         const int oy = static_cast<int>(by_stride(y_lo + y - g.origin - k + g.stride + lift)) - k;
         const int ox = static_cast<int>(by_stride(x - g.origin - k + g.stride + lift)) - k;
-        const int first = (static_cast<int>(plane) * rows_out + oy - oy_lo) * g.ow + ox;
+        int first = (static_cast<int>(plane) * rows_out + oy - oy_lo) * g.ow + ox;
+        if constexpr (K == 0) asm volatile("" : "+v"(first));      // formed here, not in parts between the additions, which are a chain
         for (uint32_t word = 0; word < words; ++word)
             for (uint32_t bits = masks[word * tile_cells + cell]; bits; bits &= bits - 1) {
                 const uint32_t bit = word * 32 + __builtin_ctz(bits);
-                uint32_t wy, wx;
                 if constexpr (K > 0) {
-                    wy = bit / K;
-                    wx = bit - wy * K;
+                    const uint32_t wy = bit / K, wx = bit - wy * K;
+                    acc += deltas[first + static_cast<int>(wy) * g.ow + static_cast<int>(wx)];
                 } else {
-                    w.by_along.divmod(bit, wy, wx);
+                    acc += deltas[first + static_cast<int>(bit) + static_cast<int>(w.by_along.div(bit)) * past];
                 }
-                acc += deltas[first + static_cast<int>(wy) * g.ow + static_cast<int>(wx)];
             }
         grad[cell0 + cell] = acc;
     }
@@ -886,7 +892,11 @@ bool launch_fwd_tile(const float* in, float* out, int* indexes, uint32_t planes,
         const size_t bytes = cells * 4 + segments * 5;
         const dim3 grid((planes + t.per_tile - 1) / t.per_tile * t.strips);
         const uint32_t groups = static_cast<uint32_t>(g.ow + 3) / 4;
+        // A lane takes four outputs a step: a tile needs two for each lane before that is shorter than one output per lane.  us,
+        // k = 5 and 13, 512 planes of 13 x 13 3.4 -> 4.0 and 3.7 -> 4.6, of 19 x 19 4.1 -> 4.4 and 4.6 -> 5.3, but of 26 x 26 4.9 -> 4.5 and
+        // 5.7 -> 5.4.  (Windows: those that have a form of their own, whose runs are unrolled.)
         const SlideTile st{ slide_pitch(g.kernel, groups), groups };
+        const bool runs = t.per_tile * t.rows * static_cast<uint32_t>(g.ow) > 2 * kBlock;
         const size_t slide_bytes = t.per_tile * rows_in * (4 * st.pitch + 5 * 4 * groups);
         const auto slide = [&]<int K>() {
             hipLaunchKernelGGL((maxpool_fwd_slide_kernel<K>), grid, dim3(kBlock), slide_bytes, s, in, out, indexes, t, g, st,
@@ -894,7 +904,7 @@ bool launch_fwd_tile(const float* in, float* out, int* indexes, uint32_t planes,
                                FastDiv((t.rows + kSlideRun - 1) / kSlideRun));
             return true;
         };
-        if (g.stride == 1 && slide_bytes <= kPoolLds) {
+        if (g.stride == 1 && slide_bytes <= kPoolLds && runs) {
             if (g.kernel == 3) return slide.template operator()<3>();
             if (g.kernel == 5) return slide.template operator()<5>();
             if (g.kernel == 9) return slide.template operator()<9>();
@@ -1003,7 +1013,7 @@ int pxh_maxpool_forward(const float* in, float* out, int* indexes, int batch, in
     const PoolGeom g{ ih, iw, oh, ow, kernel, stride, -padding / 2 };
     if (kernel == 2 && stride == 1 && g.origin == 0 && oh == ih && ow == iw) {
         hipLaunchKernelGGL(maxpool_fwd_step1_kernel, dim3(grid_for(total, static_cast<size_t>(kBlock) * 4)), dim3(kBlock), 0, s,
-                           in, out, indexes, total, g, FastDiv(ow), FastDiv(oh));
+                           in, out, indexes, total, FastDiv(ow), FastDiv(oh));
         return check_launch("pxh_maxpool_forward");
     }
     if (launch_fwd_tile(in, out, indexes, planes, g, s)) return check_launch("pxh_maxpool_forward");

@@ -22,6 +22,8 @@ def ops():
 CASES = [(1, 1, 1, 1, 3, 2), (3, 1, 1, 3, 3, 2), (1, 5, 2, 2, 5, 4), (1, 3, 13, 13, 13, 12), (1, 2, 12, 12, 13, 12), (2, 1, 40, 9, 9, 8),
          (2, 1, 9, 8, 9, 8), (37, 61, 19, 19, 5, 4), (1, 1300, 13, 13, 3, 2), (2, 3, 17, 18, 5, 0), (1, 4, 30, 30, 13, 0), (2, 3, 61, 47, 3, 1),
          (1, 2, 91, 130, 9, 8), (1, 2, 300, 301, 3, 2), (1, 2, 67, 95, 5, 4), (5, 7, 14, 15, 2, 1),
+         # tiles of 256 outputs (a value to a lane) and 272, of 528 and more: one plane, and several small ones
+         (1, 3, 16, 16, 3, 2), (1, 3, 16, 17, 5, 4), (1, 3, 22, 24, 9, 8), (1, 2, 26, 23, 5, 4), (2, 2100, 13, 13, 9, 8), (1, 4100, 12, 12, 13, 12),
          (1, 1, 1, 1, 2, 1), (3, 5, 1, 2, 2, 1), (2, 3, 3, 1, 2, 1), (1, 4, 13, 13, 2, 1), (7, 11, 26, 23, 2, 1), (1, 1, 8, 8, 2, 1)]
 
 
