@@ -1,4 +1,4 @@
-"""GPU parity of the one-launch training passes in their small forms (few lanes, two to twelve steps each): the checks of
+"""GPU parity of the one-launch training passes in their small forms (few lanes, two to eight steps each) and of odd planes: the checks of
 the other geometries, with their tolerances, at the last size of each form and the first of the next, with fewer channels
 than the other one-launch forms take and with more than the launch behind a clipped backward has workgroups; then the
 accuracy of their sums against 64 bits."""
@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 # 1025, 2048, 2049 (256 channels, then 257, which leave), 4096 and 4097
 VECTORS = [(1, 3, 4), (2, 5, 256), (3, 5, 172), (16, 270, 64), (1, 97, 1028), (2, 96, 1024), (27, 97, 76), (8, 7, 512),
            (25, 7, 164), (32, 264, 256), (3, 256, 2732), (3, 257, 2732), (4, 20, 4096), (1, 20, 16388)]
-# values: 1 channel of one value a plane, 256 and 257, 1024 and 1025, 2048 and 2049, 4095 and 4097, 6143 and 6145
+# odd planes: 1 channel of one value a plane, 256 values and 257, 1024 and 1025, 2048 and 2049, 4095 and 4097, 6143 and 6145
 SCALARS = [(5, 1, 1), (256, 3, 1), (1, 270, 257), (8, 5, 127), (5, 5, 205), (2048, 4, 1), (3, 300, 683), (5, 97, 819),
            (17, 9, 241), (2, 100, 2049), (1, 9, 6143), (5, 97, 1229)]
 
