@@ -396,18 +396,19 @@ __global__ __launch_bounds__(kBlock) void bn_stats_partial_kernel(const float* x
     const float shift = x[static_cast<size_t>(c) * g.spatial];
     double s1 = 0.0, s2 = 0.0;
     for_each_item(g, c, j, [&](size_t base, int seg0, int seg1, int lane) {
-        constexpr int kLoads = kSeg / (kWave * V);
+        constexpr int kLoads = V == 1 ? kValueSteps : kSegLoads;
         Pack<V> v[kLoads];
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) {
             const int off = seg0 + (u * kWave + lane) * V;
             if (off < seg1) v[u] = ld_at<V, NT, RAGGED>(x, base + ragged_start<RAGGED>(off, g.spatial));
         }
-        if constexpr (RAGGED) {
+        if constexpr (RAGGED || V == 1) {
 #pragma unroll
             for (int u = 0; u < kLoads; ++u) {
                 const int off = seg0 + (u * kWave + lane) * V;
-                const int own = off < seg1 ? off - ragged_start<RAGGED>(off, g.spatial) : V;
+                if (off >= seg1) break;
+                const int own = off - ragged_start<RAGGED>(off, g.spatial);
 #pragma unroll
                 for (int k = 0; k < V; ++k) {
                     const float d = k >= own ? v[u].v[k] - shift : 0.0f;
@@ -513,7 +514,8 @@ __global__ __launch_bounds__(kBlock) void bwd_partial_kernel(BackwardArgs a, Red
     [[maybe_unused]] double sq = 0.0;
     [[maybe_unused]] float peak = 0.0f;
     for_each_item(g, c, j, [&](size_t base, int seg0, int seg1, int lane) {
-        constexpr int kLoads = kSeg / (kWave * V);
+        constexpr int kLoads = V == 1 ? kValueSteps : kSegLoads;
+        constexpr bool kEach = RAGGED || V == 1;
         Pack<V> d[kLoads], xv[kLoads], pv[kLoads];
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) {
@@ -527,8 +529,7 @@ __global__ __launch_bounds__(kBlock) void bwd_partial_kernel(BackwardArgs a, Red
                 }
             }
         }
-        float fa = 0.0f, fb = 0.0f;
-        [[maybe_unused]] float fq = 0.0f;
+        [[maybe_unused]] float fa = 0.0f, fb = 0.0f, fq = 0.0f;
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) {
             const int off = seg0 + (u * kWave + lane) * V;
@@ -539,7 +540,7 @@ __global__ __launch_bounds__(kBlock) void bwd_partial_kernel(BackwardArgs a, Red
                     for (int q = 0; q < V; ++q) {
                         const float dv = d[u].v[q];
                         if constexpr (MODE == kFirst) {
-                            if constexpr (RAGGED) sq += static_cast<double>(q >= off - start ? dv * dv : 0.0f);
+                            if constexpr (kEach) sq += static_cast<double>(q >= off - start ? dv * dv : 0.0f);
                             else fq += dv * dv;
                             peak = fmaxf(peak, fabsf(dv));
                         } else {
@@ -556,7 +557,7 @@ __global__ __launch_bounds__(kBlock) void bwd_partial_kernel(BackwardArgs a, Red
                 }
 #pragma unroll
                 for (int q = 0; q < V; ++q) {
-                    if constexpr (RAGGED) {
+                    if constexpr (kEach) {
                         const float t = d[u].v[q];
                         sa += static_cast<double>(q >= off - start ? t : 0.0f);
                         if constexpr (BN) sb += static_cast<double>(q >= off - start ? t * (xv[u].v[q] - k.mean) : 0.0f);
@@ -573,9 +574,11 @@ __global__ __launch_bounds__(kBlock) void bwd_partial_kernel(BackwardArgs a, Red
                 }
             }
         }
-        sa += static_cast<double>(fa);
-        sb += static_cast<double>(fb);
-        if constexpr (MODE == kFirst) sq += static_cast<double>(fq);
+        if constexpr (!kEach) {
+            sa += static_cast<double>(fa);
+            sb += static_cast<double>(fb);
+            if constexpr (MODE == kFirst) sq += static_cast<double>(fq);
+        }
     });
     const double ta = block_sum(sa, slots[0]);
     const double tb = block_sum(sb, slots[1]);
@@ -1161,7 +1164,7 @@ int launch_stats_partial(const float* x, const ReduceGeom& g, double2* partial, 
     if (g.spatial % 4 == 0 && aligned16(x)) {
         if (nt) hipLaunchKernelGGL((bn_stats_partial_kernel<4, true>), grid, dim3(kBlock), 0, stream, x, g, partial, shifts);
         else hipLaunchKernelGGL((bn_stats_partial_kernel<4, false>), grid, dim3(kBlock), 0, stream, x, g, partial, shifts);
-    } else if (g.spatial >= kOddSpatial) {
+    } else if (sums_in_vectors(g.spatial)) {
         hipLaunchKernelGGL((bn_stats_partial_kernel<4, false, true>), grid, dim3(kBlock), 0, stream, x, g, partial, shifts);
     } else {
         hipLaunchKernelGGL((bn_stats_partial_kernel<1, false>), grid, dim3(kBlock), 0, stream, x, g, partial, shifts);
@@ -1550,7 +1553,7 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
         } else if (vec) {
             hipLaunchKernelGGL((bwd_partial_kernel<ACT, true, false, 4, false, MODE>), grid, dim3(kBlock), 0, s, b, g,
                                partial, clip);
-        } else if (spatial >= kOddSpatial) {
+        } else if (sums_in_vectors(spatial, activation)) {
             hipLaunchKernelGGL((bwd_partial_kernel<ACT, true, false, 4, false, MODE, true>), grid, dim3(kBlock), 0, s, b, g,
                                partial, clip);
         } else {
@@ -1673,7 +1676,7 @@ static int bias_backward(const char* who, float* delta, const float* pre_activat
         if (vec) {
             hipLaunchKernelGGL((bwd_partial_kernel<ACT, false, WRITE, 4, false, MODE>), grid, dim3(kBlock), 0, s, b, g,
                                partial, clip);
-        } else if (spatial >= kOddSpatial) {
+        } else if (sums_in_vectors(spatial, activation)) {
             hipLaunchKernelGGL((bwd_partial_kernel<ACT, false, WRITE, 4, false, MODE, true>), grid, dim3(kBlock), 0, s, b, g,
                                partial, clip);
         } else {

@@ -357,6 +357,22 @@ void dispatch_odd_form(uint32_t items, const ResidentGeom& g, F&& launch)
     return launch.template operator()<4, 6, 1024>();
 }
 
+// Whether the sums over odd planes in several launches, which give each segment of a plane a wave, take them in vectors.  Up to
+// a value per lane those only leave lanes idle, each with four times the arithmetic; in the backward of an activation with an
+// exponential, up to two, whose arithmetic is worth more than the loads.  There a lane takes a value a step, in no more steps than
+// that.  In vectors -> so, us, forward, bias-only backward, backward, clipped with nothing to change:
+//   6000 x 64 x 5, mish     113 -> 49     132 -> 55     160 -> 75      205 -> 99
+//   3000 x 16 x 3^2, leaky  22.8 -> 12.6  14.3 -> 10.9  22.1 -> 17.6   30.6 -> 25.2
+//   3000 x 16 x 7 x 9, mish 27.5 -> 19.3  26.8 -> 16.9  42.9 -> 32.1   53.1 -> 38.6
+//   3000 x 16 x 7 x 11, mish              26.7 -> 21.7  43.1 -> 35.2   53.7 -> 42.8
+//   1500 x 32 x 11^2, mish                25.5 -> 22.0  44.2 -> 37.7   55.0 -> 45.4
+// From 65 to 128 values the others are level, but for the bias-only backward (3000 x 16 x 7 x 11, leaky: 20.4 so, 19.1 in vectors).
+constexpr int kValueSteps = 2;
+inline bool sums_in_vectors(int spatial, int activation = PXH_LINEAR)
+{
+    return spatial > (selects(activation) ? 1 : kValueSteps) * kWave;
+}
+
 // Whether a plain call of a shape asks for a workspace: unless it takes a one-launch form that never depended on measured
 // limits.  Those of the others may move, also between activations, and a workspace that is too small for a shape is refused
 // on either side of them (as is growth in a capture).

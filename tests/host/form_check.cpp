@@ -44,6 +44,13 @@ int main()
                 // a workspace too small is refused on both sides of lines that may move: this one does not
                 check(asks_for_workspace(batch, channels, spatial, false) == (channels < 96 || values > 8192), "the workspace", batch, channels, spatial);
             }
+    // sums in several launches: a value a step where a lane has one (two before an exponential), and never more steps than there are
+    for (int spatial = 1; spatial < 5000; ++spatial)
+        for (int activation: { PXH_LINEAR, PXH_LEAKY, PXH_MISH, PXH_SWISH }) {
+            const bool vectors = sums_in_vectors(spatial, activation);
+            check(vectors == (spatial > (activation == PXH_LINEAR || activation == PXH_LEAKY ? 64 : 128)), "sums", 0, 0, spatial);
+            check(vectors ? spatial >= 4 : spatial <= kValueSteps * kWave, "steps of the sums", 0, 0, spatial);
+        }
     std::printf("%d checks, %d failed\n", checks, failed);
     return failed != 0;
 }

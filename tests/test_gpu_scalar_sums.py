@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 
 # one value a step: up to 64, 1024, 2048, 6144, 8192, 16384 and 24576 values; then vectors in one launch, in several, and in groups
 SHAPES = [(50, 97, 1), (300, 5, 3), (513, 97, 2), (1023, 70, 2), (2048, 96, 3), (2731, 96, 3), (8000, 96, 3),
-          (64, 256, 169), (46, 256, 361), (200, 256, 63), (3, 7, 2051), (40, 3, 5003), (68, 3, 257), (2, 23, 25625)]
+          (64, 256, 169), (46, 256, 361), (200, 256, 63), (3, 7, 2051), (40, 3, 5003), (68, 3, 257), (2, 23, 25625),
+          (3000, 3, 5), (260, 3, 63), (250, 3, 65), (130, 3, 129)]
 
 
 def check(got, want, terms, what):
