@@ -1102,7 +1102,6 @@ ClippedRegions clipped_regions(void* ws, int batch, int channels, int spatial)
 }
 
 constexpr int kGroupAlone = 512;
-constexpr size_t kGroupFewest = 1u << 19, kGroupFewestSmooth = 1u << 20, kGroupFewestOddSmooth = 7u << 20;
 
 // The groups of a backward (members 0: none).  A plain call and a clipped one take the same form, so that they agree to
 // the bit where nothing is rescaled or clamped, and what they exchange has to fit the workspaces they ask for.
@@ -1112,30 +1111,9 @@ constexpr size_t kGroupFewest = 1u << 19, kGroupFewestSmooth = 1u << 20, kGroupF
 // (16 x 128 x 76^2: 37 us where groups would take 33, mish 66 and 47).  A group of one member exchanges nothing, and from
 // kGroupAlone channels on, two to a compute unit, it is ahead (16 x 512 x 38^2: 29 -> 27 us; 16 x 384 x 38^2 22.3, 22.6), except
 // where an exponential has to be computed (37 -> 41).
-//
-// Odd planes take groups by the same line where the gradient is a select.  An exponential moves the line up: below it a call
-// that clamps throughout loses more than the others gain.  Three or five launches -> groups, us: plain; clipped with nothing
-// to change, rescaled, and clamped throughout (the launches with one value per access)
-//   2 x 16 x 151^2       leaky 13.5 -> 11.9; 18.6 -> 16.4, 18.6 -> 16.4, 22.3 -> 24.5
-//   4 x 32 x 207^2             28.4 -> 23.4; 35.8 -> 28.1, 35.8 -> 28.0, 43.8 -> 46.0   mish 33.9 -> 33.2; 41.5 -> 39.0, 41.7 -> 40.2, 54.5 -> 69.7
-//   64 x 24 x 75 x 45          28.4 -> 23.4; 35.8 -> 29.0, 35.7 -> 28.8, 43.5 -> 46.4        33.6 -> 31.8; 41.7 -> 39.1, 41.7 -> 40.4, 54.5 -> 69.2
-//   8 x 96 x 135 x 77          41   -> 26.4; 48   -> 31.2, 48   -> 31.1, 61   -> 52.5        46.4 -> 37.6; 52.6 -> 43.5, 52.8 -> 45.8, 72.3 -> 78.7
-//   16 x 64 x 151^2            88   -> 66.5; 97   -> 73.2, 97   -> 73.3, 124  -> 118         93.2 -> 82.9; 102  -> 91.6, 104  -> 109,  144  -> 164
-// (8 x 96 x 135 x 77 and 16 x 64 x 151^2, mish, in launches of one value per access: 51, 59, 59, 84 and 110, 117, 117, 169.)
-//
-// Small tensors (which the caches hold for the launches that read them twice) stay with those launches: a group's second one
-// costs them more where it has something to do.  Three or five launches -> groups, us: plain; clipped with nothing to change,
-// rescaled, and clamped throughout:
-//   2 x 16 x 104^2  leaky 12.0 -> 11.4; 17.6 -> 15.3, 17.6 -> 19.3, 20.1 -> 22.9   mish 16.1 -> 18.0; 21.4 -> 22.1, 21.5 -> 26.2, 27.2 -> 36.2
-//   2 x 16 x 160^2        13.5 -> 12.1; 18.8 -> 16.0, 18.8 -> 20.1, 21.7 -> 24.3        18.2 -> 18.8; 23.3 -> 23.1, 23.3 -> 27.3, 29.1 -> 37.7
-//   1 x 32 x 208^2        16.1 -> 12.9; 21.5 -> 16.8, 21.5 -> 21.2, 24.4 -> 25.7        22.0 -> 20.1; 27.2 -> 23.9, 27.3 -> 28.6, 33.8 -> 39.9
-//   4 x 32 x 208^2        28.2 -> 23.8; 34.9 -> 28.1, 35.0 -> 36.7, 42.8 -> 45.0        39.7 -> 34.9; 46.7 -> 40.0, 46.8 -> 48.6, 63.6 -> 69.2
-// From there on the usual call gains a tenth to a quarter; one that clamps gains from 16 x 64 x 152^2 on (121 -> 107).
 GroupPlan grouped_backward(int batch, int channels, int spatial, bool vec, int per_thread, int activation, hipStream_t s)
 {
-    const size_t total = static_cast<size_t>(batch) * channels * spatial;
-    if (total < (selects(activation) ? kGroupFewest : kGroupFewestSmooth)) return GroupPlan{};
-    if (!vec && (spatial < kOddSpatial || (!selects(activation) && total < kGroupFewestOddSmooth))) return GroupPlan{};
+    if (!enough_for_groups(static_cast<size_t>(batch) * channels * spatial, spatial, vec, selects(activation))) return GroupPlan{};
     if (per_thread && (!selects(activation) || channels < kGroupAlone)) return GroupPlan{};
     const uint32_t places = group_places(s);
     // (as few members as hold the slice where the words of more would not fit: up to three channels of a few thousand vectors)

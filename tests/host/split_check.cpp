@@ -45,13 +45,23 @@ int main()
         { 4, 32, 98304, true, 98304, 16, kGroupItems }, { 3, 130, 32772, true, 24579, 5, 4928 }, { 4, 512, 4112, true, 4112, 1, 4160 },
         { 16, 48, 10816, true, 43264, 10, 4352 },
         { 8, 96, 10395, false, 20792, 5, 4160 }, { 32, 41, 5625, false, 45024, 12, 3776 }, { 1, 32, 393215, false, 98304, 16, kGroupItems },
-        { 1, 90, 16385, false, 4097, 2, 2112 }, { 2, 23, 25 * 1025, false, 12814, 6, 2176 }, { 3, 70, 10243, false, 7683, 3, 2624 },
+        { 500, 60, 45, false, 6000, 2, 3008 }, { 700, 23, 77, false, 14000, 6, 2368 }, { 2, 23, 160001, false, 80002, 22, 3648 },
     };
     for (const auto& n: named) {
         const GroupPlan p = group_plan(n.batch, n.channels, n.spatial, n.vec, group_fill(n.channels), 512);
         check(!p.members || p.items == n.items, "vectors of a named slice", n.items, n.channels, 512);
         check(p.members == n.members && p.span == n.span, "the split of a named slice", n.items, n.channels, 512);
     }
+
+    // tensors that take groups: aligned, and odd planes where the gradient is a select
+    const struct { size_t total; int spatial; bool vec, light, groups; } sizes[] = {
+        { 1u << 19, 4, true, true, true }, { (1u << 19) - 1, 4, true, true, false }, { 1u << 20, 4, true, false, true },
+        { (1u << 20) - 1, 4, true, false, false }, { 7u << 20, 257, false, true, true }, { (7u << 20) - 1, 257, false, true, false },
+        { 1u << 29, 257, false, false, false }, { 1u << 20, 255, false, true, true }, { (1u << 20) - 1, 255, false, true, false },
+        { 1u << 20, 256, false, true, false }, { 1u << 29, 13, false, false, false }, { 1u << 29, 3, false, true, false },
+    };
+    for (const auto& n: sizes)
+        check(enough_for_groups(n.total, n.spatial, n.vec, n.light) == n.groups, "a tensor large enough", n.total, n.spatial, 0);
 
     uint32_t mask[4] = {};
     check(units_of_mask(mask, 4, 256) == 256, "no mask", 0, 0, 0);

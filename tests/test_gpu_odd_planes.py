@@ -43,15 +43,15 @@ def test_odd_planes(ops, oracle, monkeypatch, shape, act):
 
 
 # three launches: a segment of 1024 values that ends one, two and three values behind its last whole vector, and one that
-# holds a plane's last value alone; then groups: two members, the last vector of a plane in another share than the one in
-# front of it, channels that leave workgroups over, and a gradient with an exponential
+# holds a plane's last value alone; then slices of several members, and groups: two members, the last vector of a plane in another
+# share than the one in front of it, channels that leave workgroups over, small planes and large ones
 # (the pass behind the sums finishes the channels from planes of 256 values on, and up to 256 partial sums a channel: both
 # sides, aligned and odd)
 SPLIT = [(1, 5, 1025), (3, 7, 2051), (2, 9, 1022), (40, 3, 5003), (68, 3, 255), (68, 3, 257), (65, 4, 256), (1030, 2, 260), (1, 1, 4 * 1024 * 257),
          (1, 9, 16388), (3, 4, 5468),
          # one value a step, up to 64 values of a plane and 128 before an exponential, and vectors
          (3000, 2, 5), (260, 2, 63), (250, 2, 65), (130, 2, 127), (130, 2, 129)]
-GROUPS = [(1, 90, 16385), (2, 23, 25 * 1025), (3, 70, 10243), (8, 96, 10395)]
+GROUPS = [(1, 90, 16385), (2, 23, 25 * 1025), (3, 70, 10243), (8, 96, 10395), (500, 60, 45), (700, 23, 77), (2, 23, 160001)]
 
 
 @pytest.mark.parametrize("act", ["leaky", "mish"])

@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 # tests/host/split_check.cpp.
 VECTORS = [(1, 95, 16388), (4, 64, 6144), (7, 30, 10012), (3, 12, 32772), (1, 8, 532480), (1, 7, 532480), (4, 32, 98304),
            (3, 130, 32772), (4, 512, 4112)]
-# odd planes: five members, twelve, and sixteen that are full (but for the last value, which its vector shares)
+# odd planes (groups where the gradient is a select): five members, twelve, and sixteen that are full (but for the last value, which its vector shares)
 ODD = [(8, 96, 10395), (32, 41, 5625), (1, 32, 393215)]
 
 
