@@ -871,10 +871,13 @@ struct WaveItems {
     __device__ __forceinline__ int held(int u) const { return offset(u) - ragged_start<RAGGED>(offset(u), g.spatial); }
 };
 
-template<bool RAGGED>
+// Odd planes: past the caches, but for what is written beside the output.  us, all past the caches, all cached, and so: the forward
+// alone 19.0, 20.3, 19.1, with the pre-activation kept 29.0, 25.2, 24.8, and with a pass behind it that reads the output 32.0, 31.6,
+// 32.2 (8 x 60 x 133^2, leaky); 14.0, 15.9, 14.0, then 17.0, 17.3, and 23.3, 25.6 (6 x 72 x 135 x 77, mish; its backward 33.8, 34.4).
+template<bool RAGGED, bool NT>
 __device__ __forceinline__ void st_item(float* p, size_t at, const Pack<4>& v, int held)
 {
-    if constexpr (RAGGED) st_own(p + at, v, held);
+    if constexpr (RAGGED) st_own<NT>(p + at, v, held);
     else st<4, false>(p, at, v);
 }
 
@@ -934,10 +937,10 @@ __global__ __launch_bounds__(kBlock) void bn_finish_apply_kernel(EpilogueArgs a,
             }
             const size_t at = item.at(u);
             const int held = item.held(u);
-            if (a.x_saved) st_item<RAGGED>(a.x_saved, at, x[u], held);
-            if (a.x_norm) st_item<RAGGED>(a.x_norm, at, no, held);
-            if (a.pre) st_item<RAGGED>(a.pre, at, po, held);
-            st_item<RAGGED>(a.y, at, yo, held);
+            if (a.x_saved) st_item<RAGGED, false>(a.x_saved, at, x[u], held);
+            if (a.x_norm) st_item<RAGGED, false>(a.x_norm, at, no, held);
+            if (a.pre) st_item<RAGGED, false>(a.pre, at, po, held);
+            st_item<RAGGED, true>(a.y, at, yo, held);
         }
         item.next();
         fetch();
@@ -999,7 +1002,7 @@ __global__ __launch_bounds__(kBlock) void bn_finish_dx_kernel(BackwardArgs a, Re
             Pack<4> out;
 #pragma unroll
             for (int q = 0; q < 4; ++q) out.v[q] = dx_value(d[u].v[q], x[u].v[q], k);
-            st_item<RAGGED>(a.delta, item.at(u), out, item.held(u));
+            st_item<RAGGED, true>(a.delta, item.at(u), out, item.held(u));
         }
         item.next();
         fetch();

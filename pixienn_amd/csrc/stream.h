@@ -117,14 +117,18 @@ __device__ __forceinline__ void st_word(float* p, const Pack<4>& v)
 }
 
 // All but the first `held` of them.
+template<bool NT = true>
 __device__ __forceinline__ void st_own(float* p, const Pack<4>& v, int held)
 {
     if (held == 0) {
-        st_word(p, v);
+        st_word<NT>(p, v);
     } else {
 #pragma unroll
-        for (int q = 1; q < 4; ++q)
-            if (q >= held) __builtin_nontemporal_store(v.v[q], p + q);
+        for (int q = 1; q < 4; ++q) {
+            if (q < held) continue;
+            if constexpr (NT) __builtin_nontemporal_store(v.v[q], p + q);
+            else p[q] = v.v[q];
+        }
     }
 }
 
