@@ -819,10 +819,13 @@ __global__ __launch_bounds__(kBlock) void bn_dx_scalar_kernel(DxArgs a)
 //   9 x 20 x 203 x 251  26.4 -> 22.3   31.9 -> 26.7   48.6 -> 51.3   27.2 -> 23.7   32.6 -> 27.6   58.6 -> 61.3
 //   4 x 16 x 416^2      29.0 -> 27.4   35.9 -> 33.1   56.0 -> 60.2   29.3 -> 29.7   36.3 -> 37.9   66.0 -> 69.8
 //   8 x 16 x 416^2      47.0 -> 45.8   60.2 -> 69.2   104  -> 123    47.1 -> 49.6   61.6 -> 77.8   122  -> 136
-// (6 x 72 x 135 x 77, mish, without the pre-activation: 31.5 -> 28.4.)
+// (6 x 72 x 135 x 77, mish, without the pre-activation: 31.5 -> 28.4.)  The forward's line lies lower where an exponential is
+// followed by another chain, the planes are aligned and no shortcut is on top: 16 x 48 x 104^2, mish, 23.7 -> 25.0, softplus 24.0 -> 26.0,
+// 4 x 16 x 392^2 26.2 -> 27.3 and 26.1 -> 29.2, but 8 x 80 x 104^2 20.9 -> 19.3 and 21.4 -> 21.2, logistic 22.7 -> 19.4 and 25.2 -> 22.9; with a
+// shortcut 28.3 -> 26.2, and odd planes (8 x 60 x 133^2, mish) 24.5 -> 22.1, with one 28.5 -> 26.7.
 // ------------------------------------------------------------------------------------------
 constexpr int kFusedPartials = 4 * kWave;      // of a channel: a lane of the first wave takes four
-constexpr uint32_t kFusedForward = 10u << 20, kFusedBackward = 6u << 20;      // values of a tensor
+constexpr uint32_t kFusedForward = 10u << 20, kFusedForwardChain = 7u << 20, kFusedBackward = 6u << 20;      // values of a tensor
 constexpr int kFusedSpatial = 4 * kWave;       // a wave's step; planes below leave most of its lanes without a vector
 
 __device__ __forceinline__ double2 channel_sums(const double2* partial, uint32_t c, int blocks)
@@ -1168,9 +1171,9 @@ int launch_stats(const float* x, float* mean, float* var, float* rolling_mean, f
 }
 
 // Whether the pass behind the partial sums finishes the channels itself.
-bool finishes_inside(const ReduceGeom& g, uint32_t total, bool backward)
+bool finishes_inside(const ReduceGeom& g, uint32_t total, uint32_t most)
 {
-    return total <= (backward ? kFusedBackward : kFusedForward) && g.blocks <= kFusedPartials && g.spatial >= kFusedSpatial;
+    return total <= most && g.blocks <= kFusedPartials && g.spatial >= kFusedSpatial;
 }
 
 // The linear shortcut taken into a forward pass (from == nullptr: none).
@@ -1215,7 +1218,8 @@ int bn_train_forward(const char* who, const float* x, float* y, float* pre_activ
     a.x = x; a.y = y; a.pre = pre_activation; a.x_saved = x_saved; a.x_norm = x_norm;
     a.residual = res.from; a.res_alpha = res.alpha; a.res_beta = res.beta;
     const ReduceGeom g = make_geom(batch, channels, spatial);
-    if (finishes_inside(g, a.total, false)) {
+    const bool chain = vec && !res.from && (activation == PXH_MISH || activation == PXH_SOFTPLUS);
+    if (finishes_inside(g, a.total, chain ? kFusedForwardChain : kFusedForward)) {
         // (the first value of a channel, which its sums are relative to, is kept: y may be x)
         float* const shifts = static_cast<float*>(coef_region(ws, batch, channels, spatial));
         double2* const partial = static_cast<double2*>(ws);
@@ -1564,7 +1568,7 @@ static int bn_backward(const char* who, float* delta, const float* x, const floa
     if (!known) return fail_invalid("%s: unknown activation %d", who, activation);
     rc = check_launch("bn_backward_partial");
     if (rc) return rc;
-    if (!cs.on && finishes_inside(g, total, true)) {
+    if (!cs.on && finishes_inside(g, total, kFusedBackward)) {
         const BackwardFinish f{ partial, scale_updates, bias_updates, mean_delta, var_delta, batch * spatial };
         dispatch_activation(activation, [&]<int ACT>() {
             if (vec) hipLaunchKernelGGL((bn_finish_dx_kernel<ACT, false>), grid, dim3(kBlock), 0, s, b, g, f);

@@ -16,8 +16,9 @@ from util import F, assert_bit_exact, assert_close, gpu, host
 pytestmark = pytest.mark.gpu
 
 FACTORS = [(1.0, 1.0), (0.75, -1.5)]
-# a 128-bit slice of 7000 vectors: the half-size workgroups with sixteen vectors per lane
-EXTRA_SHAPES = [(4, 96, 7000)]
+# a 128-bit slice of 7000 vectors: the half-size workgroups with sixteen vectors per lane; then one whose channels are finished inside
+# the pass behind the sums with a shortcut on top, and in a launch of their own without one
+EXTRA_SHAPES = [(4, 96, 7000), (8, 95, 10400)]
 
 
 @pytest.fixture(scope="module")
