@@ -176,6 +176,8 @@ __device__ __forceinline__ void resident_bwd_channel(const ResidentBwdArgs& a, c
                     }
                     continue;
                 }
+                // (a step that the slice does not reach has nothing to compute, in any lane: mish, 2 x 583 x 25 x 28 9.7 -> 7.9 us)
+                if (r > 0 && static_cast<uint32_t>(r * T) >= a.g.per_channel / V) continue;
                 const bool valid = element(r) < a.g.per_channel;
                 float va = 0.0f, vb = 0.0f, vq = 0.0f;
 #pragma unroll
