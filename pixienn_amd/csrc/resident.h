@@ -304,6 +304,11 @@ inline int resident_vectors(int batch, int channels, int spatial, bool vec)
 // (16 x 512 x 19^2, mish: 11.3 against 12.5).  Up to 128 vectors a step is enough (1 x 256 x 17^2, mish, backward: 1 x 128 3.8,
 // 2 x 128 4.3), and a slice of a value per lane needs no vectors, whose addresses and shared values are then the longer part of
 // a short launch (1 x 1024 x 7^2, mish: forward 3.8 against 4.2 in vectors, + shortcut 3.8 and 4.5).
+// A step that few lanes or none of a workgroup need is computed all the same.  With many channels: 20 x 1024 x 7^2 (260 vectors), leaky and
+// mish, backward, 2 x 256 7.4 and 9.1, 3 x 256 8.1 and 10.5; 64 x 1024 x 7^2 (832) 4 x 256 15.1 and 17.1, 6 x 256 15.4 and 19.8.  With few, where
+// an exponential is, twice the lanes are ahead: 2 x 512 x 19^2, mish, forward 1 x 256 4.8, 2 x 128 5.2, backward 4.9 and 6.2;
+// 6 x 512 x 13^2 1 x 512 6.6, 3 x 256 7.3; 40 x 300 x 9^2 2 x 512 9.2, 3 x 512 10.5.  (Leaky, 6 x 512 x 13^2: 5.5 and 5.2; with a thousand
+// channels 4 x 1024 x 13^2, leaky, 1 x 256 5.9, 2 x 128 5.6.)
 // Planes below kOddSpatial have no vector: one value a step, in forms that hold as much as those of the others.  Three launches
 // give each plane a wave of its own.
 // us, leaky and mish, one launch and (*) several: forward, + shortcut, backward
@@ -330,8 +335,13 @@ inline uint32_t odd_slice(int batch, int channels, int spatial, bool vec)
     return items <= most ? static_cast<uint32_t>(items) : 0;
 }
 
-// Calls launch.operator()<V, R, T>() with the form for `items`: values per step, steps per lane, lanes.
-template<typename F>
+// Vectors of a slice up to which a lane takes one, with few channels: an exponential is worth more than waves, and its gradient
+// twice as much.
+template<int ACT, bool BACKWARD>
+constexpr int kOddOneStep = selects(ACT) ? 128 : BACKWARD ? 512 : 256;
+
+// Calls launch.operator()<V, R, T>() with the form for `items`: values per step, steps per lane, lanes.  ONE: kOddOneStep.
+template<int ONE, typename F>
 void dispatch_odd_form(uint32_t items, const ResidentGeom& g, F&& launch)
 {
     if (g.per_channel <= 64) return launch.template operator()<1, 1, 64>();
@@ -345,11 +355,20 @@ void dispatch_odd_form(uint32_t items, const ResidentGeom& g, F&& launch)
         if (items <= 1024 * 16) return launch.template operator()<1, 16, 1024>();
         return launch.template operator()<1, 24, 1024>();
     }
+    const bool many = g.channels > kOddChannels;
     if (items <= 64) return launch.template operator()<4, 1, 64>();
     if (items <= 128) return launch.template operator()<4, 1, 128>();
+    if constexpr (ONE >= 256)
+        if (items <= 256 && !many) return launch.template operator()<4, 1, 256>();
+    if constexpr (ONE >= 512) {
+        if (items > 256 && items <= 512 && !many) return launch.template operator()<4, 1, 512>();
+        if (items > 256 * 3 && items <= 512 * 2 && !many) return launch.template operator()<4, 2, 512>();
+    }
     if (items <= 128 * 2) return launch.template operator()<4, 2, 128>();
+    if (items <= 256 * 2 && many) return launch.template operator()<4, 2, 256>();
     if (items <= 256 * 3) return launch.template operator()<4, 3, 256>();
-    if (items <= 256 * 6 && g.channels > kOddChannels) return launch.template operator()<4, 6, 256>();
+    if (items <= 256 * 4 && many) return launch.template operator()<4, 4, 256>();
+    if (items <= 256 * 6 && many) return launch.template operator()<4, 6, 256>();
     if (items <= 512 * 3) return launch.template operator()<4, 3, 512>();
     if (items <= 512 * 4) return launch.template operator()<4, 4, 512>();
     if (items <= 512 * 6) return launch.template operator()<4, 6, 512>();

@@ -388,7 +388,7 @@ int launch_resident_backward(const char* who, const ResidentBwdArgs& r, bool cli
         const bool walks = MODE == kRedo && !large && r.g.channels > kRedoWorkgroups;
         const dim3 grid(walks ? kRedoWorkgroups : r.g.channels);
         if (form.odd) {
-            dispatch_odd_form(form.odd, r.g, [&]<int V, int R, int T>() {
+            dispatch_odd_form<kOddOneStep<ACT, true>>(form.odd, r.g, [&]<int V, int R, int T>() {
                 hipLaunchKernelGGL((bn_resident_bwd_kernel<ACT, V, R, 0, MODE, T, V == 4>), grid, dim3(T), 0, s, r);
             });
         } else if (form.small) {

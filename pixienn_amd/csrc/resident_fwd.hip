@@ -216,7 +216,7 @@ int launch_resident_forward(const char* who, const ResidentFwdArgs& r, const Res
     const auto launch = [&]<int ACT, bool RES>() {
         constexpr int kT = kResidentThreads;
         if (form.odd) {
-            dispatch_odd_form(form.odd, r.g, [&]<int V, int R, int T>() {
+            dispatch_odd_form<kOddOneStep<ACT, false>>(form.odd, r.g, [&]<int V, int R, int T>() {
                 hipLaunchKernelGGL((bn_resident_fwd_kernel<ACT, V, R, 0, T, RES, V == 4>), grid, dim3(T), 0, s, r);
             });
             return;

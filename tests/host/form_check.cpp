@@ -31,13 +31,25 @@ int main()
                         check(!form.per_thread && !form.small, "vectors only where planes have them whole", batch, channels, spatial);
                         if (!form.odd) continue;
                         const ResidentGeom g = resident_geom(batch, channels, spatial);
-                        dispatch_odd_form(form.odd, g, [&]<int V, int R, int T>() {
+                        const auto holds = [&]<int V, int R, int T>() {
                             const size_t items = V == 1 ? values : g.vectors;
                             check(static_cast<size_t>(R) * T >= items, "a form holds its slice", batch, channels, spatial);
                             check(V == 1 || spatial >= 4, "a vector fits a plane", batch, channels, spatial);
                             if (values <= 64) check(V == 1 && R == 1 && T == 64, "a value per lane", batch, channels, spatial);
                             else if (V == 4 && items <= 128) check(R == 1, "a vector per lane", batch, channels, spatial);
-                        });
+                            // vectors of up to 256 lanes: no lane has a step that none of the slice's is in
+                            if (V == 4 && T <= 256 && (T < 256 || channels > kOddChannels))
+                                check(static_cast<size_t>(R - (R == 6 ? 2 : 1)) * T < items, "no empty steps", batch, channels, spatial);
+                        };
+                        const auto one_step = [&](uint32_t most) {
+                            return [&, most]<int V, int R, int T>() {
+                                if (V == 4 && g.vectors <= most && channels <= kOddChannels) check(R == 1, "a vector per lane", batch, channels, spatial);
+                                holds.template operator()<V, R, T>();
+                            };
+                        };
+                        if (selects(activation)) dispatch_odd_form<kOddOneStep<PXH_LEAKY, true>>(form.odd, g, one_step(128));
+                        else if (backward) dispatch_odd_form<kOddOneStep<PXH_MISH, true>>(form.odd, g, one_step(512));
+                        else dispatch_odd_form<kOddOneStep<PXH_MISH, false>>(form.odd, g, one_step(256));
                     }
                 const bool one = odd_slice(batch, channels, spatial, false) != 0;
                 if (spatial < 4) check(one == (values <= (channels < 96 ? 6144u : 24576u)), "planes below a vector", batch, channels, spatial);

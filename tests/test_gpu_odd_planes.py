@@ -15,12 +15,14 @@ pytestmark = pytest.mark.gpu
 # 64 values of a slice (one to a lane) and 65; vectors of a slice: 1, 64 and 65, 128 and 130, 256 and 259, 768 and 771, 1536 (up to 512 channels and beyond) and 1539, 2049, 3072 and
 # 3075, 4096 and 4100 (few channels, which leave, and many), 6144 and 6148, 300 channels that are walked; then values of
 # planes below four, the last of each form and the first of the next: 256, 1024, 2048, 4096, 6144 (few channels, which leave, and
-# many), 8192, 16384, 24576
+# many), 8192, 16384, 24576; then more than 512 channels: 256 vectors and 260, 512 and 516, 1024 and 1028, and fewer: 512 and 514, 1024
+# and 1028
 SHAPES = [(1, 3, 4), (1, 5, 5), (7, 97, 9), (64, 97, 1), (13, 97, 5), (64, 97, 7), (65, 97, 7), (32, 97, 7), (13, 97, 17), (128, 96, 6), (37, 96, 25), (256, 97, 9), (257, 96, 9), (512, 96, 10),
           (384, 520, 13), (513, 96, 9), (683, 96, 11), (1024, 96, 9), (1025, 300, 11), (1024, 5, 14), (1025, 5, 15), (1025, 96, 15),
           (1536, 96, 15), (1537, 96, 14), (128, 97, 2), (129, 97, 2),
           (512, 5, 2), (513, 97, 2), (2048, 96, 1), (683, 97, 3), (2048, 97, 2), (2049, 97, 2), (2048, 5, 3), (3073, 5, 2), (3073, 96, 2),
-          (4096, 96, 2), (2731, 96, 3), (8192, 96, 2), (5462, 96, 3), (8192, 96, 3), (8193, 96, 3)]
+          (4096, 96, 2), (2731, 96, 3), (8192, 96, 2), (5462, 96, 3), (8192, 96, 3), (8193, 96, 3),
+          (64, 520, 13), (65, 520, 13), (128, 520, 13), (129, 520, 13), (256, 520, 13), (257, 520, 13), (256, 97, 7), (257, 97, 7), (256, 97, 13), (257, 97, 13)]
 
 
 @pytest.fixture(scope="module")
