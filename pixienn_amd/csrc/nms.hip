@@ -16,6 +16,7 @@
 #include "common.h"
 #include "pixienn_hip_test.h"
 
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -767,6 +768,30 @@ __device__ __forceinline__ bool find_block(const ImageArgs& a, uint32_t at, Plac
     return at < blocks;
 }
 
+// The two launches below take blocks by quarters.  Those are few where a list is long and nearly empty, and a workgroup for each that
+// the list could have takes a place for a trip to memory: there are kTurnWorkgroups at most, which take the quarters in turns, every
+// other turn in the opposite order, since a quarter costs more the further back its block lies in its image.  (A workgroup to a
+// quarter, no records in a list for 40000 17.2 us, so 12.7, 3 records 19.5 and 17.2; 28160 of 64 images 72.9 and 75.5.)
+constexpr uint32_t kQuarters = 4, kTurnWorkgroups = 1024;
+
+// Calls body(block, its number, quarter) for the quarters of a workgroup; `all`: those that the list could have.  (With no records
+// there are none: the group launch writes that down too.  How many there are and the first one are on their way at once: of the
+// steps of these launches, which are short, a trip to memory is the longest.)
+template<typename Body>
+__device__ __forceinline__ void in_turns(const ImageArgs& a, uint32_t all, Body&& body)
+{
+    uint32_t at = blockIdx.x;
+    const uint32_t blocks = *a.block_count;
+    PlaceBlock b = a.blocks[at / kQuarters];
+    all = min(all, blocks * kQuarters);
+    for (uint32_t turn = 0; at < all;) {
+        body(b, at / kQuarters, at % kQuarters);
+        ++turn;
+        at = turn * gridDim.x + (turn & 1 ? gridDim.x - 1 - blockIdx.x : blockIdx.x);
+        if (at < all) b = a.blocks[at / kQuarters];
+    }
+}
+
 // One workgroup per 64 records, a lane per record in each of its 16 waves, the waves side by side over
 // the image's keys.  Records of equal key keep their input order; a record's own key does not count as one (going over its
 // 64 keys again for it, a trip to memory each, was half the launch: 7000 records of 16 images 14.9 -> 7.1 us).
@@ -814,15 +839,15 @@ __global__ __launch_bounds__(kWide) void nms_place_kernel(ImageArgs a)
     a.cls[place] = static_cast<uint32_t>(min(max(d.class_index, 0), a.classes - 1));
 }
 
-// kConflictParts workgroups per block of 64 places, 16 places each: a wave holds them four times over, and its quarters and
+// A quarter of a block of 64 places to a workgroup, 16 places: a wave holds them four times over, and its quarters and
 // the 16 waves share out the places in front of them (and the block's own) evenly, from LDS; what they find is put together
 // in the words it belongs to, and a lane per word and place stores them.  A pair is some 90 instructions, the whole overlap
 // test for nearly every step of a wave, so what bounds the launch is how evenly the pairs lie on the compute units: 64
 // places to a workgroup and a wave to a word, 7000 records of 16 images took 26 us, with a word's places shared out over
 // the waves 20, now 8.0.
-constexpr uint32_t kConflictPlaces = 16, kConflictParts = 64 / kConflictPlaces;
+constexpr uint32_t kConflictPlaces = kWave / kQuarters;
 
-__global__ __launch_bounds__(kWide) void nms_conflicts_kernel(ImageArgs a)
+__global__ __launch_bounds__(kWide) void nms_conflicts_kernel(ImageArgs a, uint32_t all)
 {
     __shared__ float4 boxes[kLargeImage];
     __shared__ uint32_t classes[kLargeImage];
@@ -830,73 +855,77 @@ __global__ __launch_bounds__(kWide) void nms_conflicts_kernel(ImageArgs a)
     __shared__ uint64_t beyond[2][kConflictPlaces];
     __shared__ uint32_t slots[2][kConflictPlaces];
     const uint32_t t = threadIdx.x;
-    const uint32_t block = blockIdx.x / kConflictParts, part = blockIdx.x % kConflictParts;
-    PlaceBlock b;
-    if (!find_block(a, block, b)) return;
-    if (b.image_end - b.image_begin > kLargeImage) {
-        if (part == 0 && t < kSettledWords) a.settled[block * kSettledStride + t] = 0;
-        return;
-    }
-    const uint32_t first = b.first + part * kConflictPlaces;
-    if (first >= b.image_end) return;
-    // places of the image from here on: this workgroup's are from `first_place` to `length`
-    const uint32_t first_place = first - b.image_begin;
-    const uint32_t length = min(first + kConflictPlaces, b.image_end) - b.image_begin;
-    if (t < length) {
-        boxes[t] = a.box[b.image_begin + t];
-        classes[t] = a.cls[b.image_begin + t];
-    }
-    if (t < 2 * kMaskWords * kConflictPlaces) (&found[0][0][0])[t] = 0;
-    if (t < 2 * kConflictPlaces) {
-        (&beyond[0][0])[t] = 0;
-        (&slots[0][0])[t] = 0;
-    }
-    __syncthreads();
-    constexpr uint32_t kTeams = kWide / kConflictPlaces;
-    const uint32_t column = t % kConflictPlaces;
-    const uint32_t place = first_place + column;
-    const bool live = place < length;
-    const uint32_t share = (length + kTeams - 1) / kTeams;       // 16 at most
-    const uint32_t q_first = t / kConflictPlaces * share, q_last = min(q_first + share, live ? place : 0u);
-    const float4 box = boxes[live ? place : first_place];
-    const uint32_t cls = classes[live ? place : first_place];
-    uint32_t hits[2] = { 0, 0 };       // bit j: place q_first + j
-    for (uint32_t q = q_first; q < q_last; ++q) {
-        const bool same = classes[q] == cls;
-        if (overlaps_above(box, boxes[q], same ? a.threshold : kDuplicateOverlap)) hits[same ? 1 : 0] |= 1u << (q - q_first);
-    }
-    // a share begins anywhere in a word and may end in the next
-    const uint32_t word = q_first >> 6, shift = q_first & 63;
-#pragma unroll
-    for (int pass = 0; pass < 2; ++pass) {
-        if (!hits[pass]) continue;
-        const uint64_t low = static_cast<uint64_t>(hits[pass]) << shift;
-        const uint64_t high = shift ? static_cast<uint64_t>(hits[pass]) >> (64 - shift) : 0ull;
-        if (low) atomicOr(&found[pass][word][column], static_cast<unsigned long long>(low));
-        if (high) atomicOr(&found[pass][word + 1][column], static_cast<unsigned long long>(high));
-    }
-    __syncthreads();
-    const uint32_t most = a.mask_slots;
-    if (t < kMaskWords * kConflictPlaces && live) {
-        const uint32_t mine = t / kConflictPlaces;       // the word; `column` and `place` are those of above
+    // one part of a block; all lanes end it together
+    const auto look = [&](const PlaceBlock& b, uint32_t block, uint32_t part) {
+        if (b.image_end - b.image_begin > kLargeImage) {
+            if (part == 0 && t < kSettledWords) a.settled[block * kSettledStride + t] = 0;
+            return;
+        }
+        const uint32_t first = b.first + part * kConflictPlaces;
+        if (first >= b.image_end) return;
+        // places of the image from here on: this workgroup's are from `first_place` to `length`
+        const uint32_t first_place = first - b.image_begin;
+        const uint32_t length = min(first + kConflictPlaces, b.image_end) - b.image_begin;
+        if (t < length) {
+            boxes[t] = a.box[b.image_begin + t];
+            classes[t] = a.cls[b.image_begin + t];
+        }
+        if (t < 2 * kMaskWords * kConflictPlaces) (&found[0][0][0])[t] = 0;
+        if (t < 2 * kConflictPlaces) {
+            (&beyond[0][0])[t] = 0;
+            (&slots[0][0])[t] = 0;
+        }
+        __syncthreads();
+        constexpr uint32_t kTeams = kWide / kConflictPlaces;
+        const uint32_t column = t % kConflictPlaces;
+        const uint32_t place = first_place + column;
+        const bool live = place < length;
+        const uint32_t share = (length + kTeams - 1) / kTeams;       // 16 at most
+        const uint32_t q_first = t / kConflictPlaces * share, q_last = min(q_first + share, live ? place : 0u);
+        const float4 box = boxes[live ? place : first_place];
+        const uint32_t cls = classes[live ? place : first_place];
+        uint32_t hits[2] = { 0, 0 };       // bit j: place q_first + j
+        for (uint32_t q = q_first; q < q_last; ++q) {
+            const bool same = classes[q] == cls;
+            if (overlaps_above(box, boxes[q], same ? a.threshold : kDuplicateOverlap)) hits[same ? 1 : 0] |= 1u << (q - q_first);
+        }
+        // a share begins anywhere in a word and may end in the next
+        const uint32_t word = q_first >> 6, shift = q_first & 63;
 #pragma unroll
         for (int pass = 0; pass < 2; ++pass) {
-            const uint64_t mask = found[pass][mine][column];
-            if (!mask) continue;
-            const uint32_t slot = atomicAdd(&slots[pass][column], 1u);
-            if (slot < most) {
-                const size_t at = static_cast<size_t>(slot) * a.capacity + b.image_begin + place;
-                a.masks[pass][at] = mask;
-                a.ids[pass][at] = static_cast<uint8_t>(mine);
-            } else {
-                atomicOr(reinterpret_cast<unsigned long long*>(&beyond[pass][column]), 1ull << mine);
+            if (!hits[pass]) continue;
+            const uint64_t low = static_cast<uint64_t>(hits[pass]) << shift;
+            const uint64_t high = shift ? static_cast<uint64_t>(hits[pass]) >> (64 - shift) : 0ull;
+            if (low) atomicOr(&found[pass][word][column], static_cast<unsigned long long>(low));
+            if (high) atomicOr(&found[pass][word + 1][column], static_cast<unsigned long long>(high));
+        }
+        __syncthreads();
+        const uint32_t most = a.mask_slots;
+        if (t < kMaskWords * kConflictPlaces && live) {
+            const uint32_t mine = t / kConflictPlaces;       // the word; `column` and `place` are those of above
+#pragma unroll
+            for (int pass = 0; pass < 2; ++pass) {
+                const uint64_t mask = found[pass][mine][column];
+                if (!mask) continue;
+                const uint32_t slot = atomicAdd(&slots[pass][column], 1u);
+                if (slot < most) {
+                    const size_t at = static_cast<size_t>(slot) * a.capacity + b.image_begin + place;
+                    a.masks[pass][at] = mask;
+                    a.ids[pass][at] = static_cast<uint8_t>(mine);
+                } else {
+                    atomicOr(reinterpret_cast<unsigned long long*>(&beyond[pass][column]), 1ull << mine);
+                }
             }
         }
-    }
-    __syncthreads();
-    if (t >= kConflictPlaces || !live) return;
-    for (int pass = 0; pass < 2; ++pass) a.beyond[pass][b.image_begin + place] = beyond[pass][column];
-    a.slots[b.image_begin + place] = min(slots[0][column], most) | min(slots[1][column], most) << 8;
+        __syncthreads();
+        if (t >= kConflictPlaces || !live) return;
+        for (int pass = 0; pass < 2; ++pass) a.beyond[pass][b.image_begin + place] = beyond[pass][column];
+        a.slots[b.image_begin + place] = min(slots[0][column], most) | min(slots[1][column], most) << 8;
+    };
+    in_turns(a, all, [&](const PlaceBlock& b, uint32_t block, uint32_t part) {
+        __syncthreads();       // (a part reuses the workgroup's LDS)
+        look(b, block, part);
+    });
 }
 
 __device__ __forceinline__ uint64_t load_bits(const uint64_t* set, uint32_t word)
@@ -1174,6 +1203,10 @@ __global__ __launch_bounds__(kWide) void nms_settle_kernel(ImageArgs a)
     const uint32_t begin = a.image_begin[blockIdx.x];
     const uint32_t places = a.image_begin[blockIdx.x + 1] - begin;
     if (places > kLargeImage) return;
+    if (places == 0) {
+        if (t == 0) a.kept_images[blockIdx.x] = 0;
+        return;
+    }
     const uint32_t slots = t < places ? a.slots[begin + t] : 0;
     if (t < kMaskWords) gone[t] = 0;
     Standing s{};
@@ -1209,15 +1242,15 @@ __global__ __launch_bounds__(kWide) void nms_settle_kernel(ImageArgs a)
     if (t == 0) a.kept_images[blockIdx.x] = total;
 }
 
-// One wave per survivor, kMergeParts workgroups per block of 64: how many of each other image's survivors come before it.  A power of two of lanes share an image
+// One wave per survivor, a quarter of a block of 64 to a workgroup: how many of each other image's survivors come before it.  A power of two of lanes share an image
 // (batches of up to 64; else images take turns): they look at as many places that split what is left evenly, and the part
 // between the last that comes before and the first that does not is what is left of it.  The looks of a step are on their way at
 // once, so that a step costs one trip to memory: with four lanes four steps for 440 survivors, where halving takes nine
 // (7000 records of 16 images, the launch, with four waves to a wave's survivors: 13.7 -> 5.9 us).
-constexpr uint32_t kMergeParts = kWave / (kWide / kWave);
+static_assert(kQuarters * (kWide / kWave) == kWave, "a wave to a survivor");
 
 __global__ __launch_bounds__(kWide) void nms_merge_images_kernel(ImageArgs a, pxh_detection* kept, int* kept_count, uint32_t lanes,
-                                                                 FastDiv by_parts)
+                                                                 FastDiv by_parts, uint32_t all)
 {
     const uint32_t lane = threadIdx.x & (kWave - 1);
     const uint32_t wave = threadIdx.x / kWave;
@@ -1234,48 +1267,50 @@ __global__ __launch_bounds__(kWide) void nms_merge_images_kernel(ImageArgs a, px
     // the first images' tables on their way beside the block
     const uint32_t nearest = min(lane / lanes, images - 1);
     const uint32_t near_begin = a.image_begin[nearest], near_kept = a.kept_images[nearest];
-    PlaceBlock b;
-    if (!find_block(a, blockIdx.x / kMergeParts, b)) return;
-    const uint32_t at = b.first + blockIdx.x % kMergeParts * (kWide / kWave) + wave;
-    if (at >= min(b.first + kWave, b.image_begin + a.kept_images[b.image])) return;
-    const uint64_t key = a.kept_key[at];
-    const uint32_t source = a.kept_source[at];
-    constexpr uint32_t kRecordWords = sizeof(pxh_detection) / 4;
-    const uint32_t record = reinterpret_cast<const uint32_t*>(a.records + source)[lane % kRecordWords];
-    uint32_t before = 0;
-    for (uint32_t i0 = 0; i0 < images; i0 += per_round) {
-        const uint32_t i = i0 + lane / lanes;
-        uint32_t lo = 0, hi = 0;
-        if (i < images) {
-            lo = i0 ? a.image_begin[i] : near_begin;
-            hi = lo + (i0 ? a.kept_images[i] : near_kept);
-        }
-        const uint32_t first = lo;
-        if (i == b.image) lo = hi = at;       // the survivors of its own image: those in front of it
-        while (__ballot(lo < hi)) {
-            // lane `part` looks at place lo + length * (part + 1) / (lanes + 1): below hi, and in order
-            const uint32_t length = hi - lo;
-            const auto look = [&](uint32_t nth) { return lo + by_parts.div(length * nth); };       // length is kImageCapacity at most
-            const uint32_t place = look(part + 1);
-            bool less = false;
-            if (length) {
-                const uint64_t k = a.kept_key[place];
-                less = k < key || (k == key && a.kept_source[place] < source);
+    const auto place = [&](const PlaceBlock& b, uint32_t, uint32_t nth) {
+        const uint32_t at = b.first + nth * (kWide / kWave) + wave;
+        const uint32_t end = min(b.first + kWave, b.image_begin + a.kept_images[b.image]);
+        if (at >= end) return;
+        const uint64_t key = a.kept_key[at];
+        const uint32_t source = a.kept_source[at];
+        constexpr uint32_t kRecordWords = sizeof(pxh_detection) / 4;
+        const uint32_t record = reinterpret_cast<const uint32_t*>(a.records + source)[lane % kRecordWords];
+        uint32_t before = 0;
+        for (uint32_t i0 = 0; i0 < images; i0 += per_round) {
+            const uint32_t i = i0 + lane / lanes;
+            uint32_t lo = 0, hi = 0;
+            if (i < images) {
+                lo = i0 ? a.image_begin[i] : near_begin;
+                hi = lo + (i0 ? a.kept_images[i] : near_kept);
             }
-            // places that come before are the first ones: as many lanes as say so
-            const uint32_t count = static_cast<uint32_t>(__popcll(__ballot(less) & team));
-            if (length) {
-                const uint32_t from = count == 0 ? lo : look(count) + 1;
-                const uint32_t to = count == lanes ? hi : look(count + 1);
-                lo = from;
-                hi = to;
+            const uint32_t first = lo;
+            if (i == b.image) lo = hi = at;       // the survivors of its own image: those in front of it
+            while (__ballot(lo < hi)) {
+                // lane `part` looks at place lo + length * (part + 1) / (lanes + 1): below hi, and in order
+                const uint32_t length = hi - lo;
+                const auto look = [&](uint32_t step) { return lo + by_parts.div(length * step); };       // length is kImageCapacity at most
+                const uint32_t middle = look(part + 1);
+                bool less = false;
+                if (length) {
+                    const uint64_t k = a.kept_key[middle];
+                    less = k < key || (k == key && a.kept_source[middle] < source);
+                }
+                // places that come before are the first ones: as many lanes as say so
+                const uint32_t count = static_cast<uint32_t>(__popcll(__ballot(less) & team));
+                if (length) {
+                    const uint32_t from = count == 0 ? lo : look(count) + 1;
+                    const uint32_t to = count == lanes ? hi : look(count + 1);
+                    lo = from;
+                    hi = to;
+                }
             }
+            if (part == 0 && i < images) before += lo - first;
         }
-        if (part == 0 && i < images) before += lo - first;
-    }
 #pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) before += __shfl_xor(before, off, kWave);
-    if (lane < kRecordWords) reinterpret_cast<uint32_t*>(kept + before)[lane] = record;
+        for (int off = kWave / 2; off > 0; off >>= 1) before += __shfl_xor(before, off, kWave);
+        if (lane < kRecordWords) reinterpret_cast<uint32_t*>(kept + before)[lane] = record;
+    };
+    in_turns(a, all, place);
 }
 
 size_t align256(size_t b) { return (b + 255) & ~static_cast<size_t>(255); }
@@ -1441,14 +1476,15 @@ int pxh_nms(const pxh_detection* records, const int* count, int capacity, int ba
         hipLaunchKernelGGL(nms_count_images_kernel, per_tile, wide, 0, s, a);
         hipLaunchKernelGGL(nms_group_images_kernel, per_tile, wide, 0, s, a);
         hipLaunchKernelGGL(nms_place_kernel, per_block, wide, 0, s, a);
-        hipLaunchKernelGGL(nms_conflicts_kernel, dim3(per_block.x * kConflictParts), wide, 0, s, a);
+        const uint32_t quarters = per_block.x * kQuarters;
+        const dim3 in_turns(std::min(quarters, kTurnWorkgroups));
+        hipLaunchKernelGGL(nms_conflicts_kernel, in_turns, wide, 0, s, a, quarters);
         const unsigned helpers = static_cast<uint32_t>(capacity) > kLargeImage ? kSettleWorkgroups : 0;
         hipLaunchKernelGGL(nms_settle_kernel, dim3(batch + helpers), wide, 0, s, a);
         // as many lanes to an image as leave one for each, sixteen at most: further ones save no step worth a division
         uint32_t lanes = 1;
         while (lanes < 16 && 2 * lanes * static_cast<uint32_t>(batch) <= static_cast<uint32_t>(kWave)) lanes *= 2;
-        hipLaunchKernelGGL(nms_merge_images_kernel, dim3(per_block.x * kMergeParts), wide, 0, s, a, kept, kept_count, lanes,
-                           FastDiv(lanes + 1));
+        hipLaunchKernelGGL(nms_merge_images_kernel, in_turns, wide, 0, s, a, kept, kept_count, lanes, FastDiv(lanes + 1), quarters);
         return check_launch("pxh_nms");
     }
     int rc = resolve_workspace(workspace, workspace_bytes, carve(nullptr, capacity).bytes, &ws, as_stream(stream));
