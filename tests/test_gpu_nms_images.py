@@ -66,3 +66,10 @@ def test_equal_keys_keep_input_order(ops, oracle, sizes):
 def test_no_records(ops, oracle):
     rec = of_sizes(oracle, 3, [4], 3, 2)[:0]
     assert len(run(ops, rec, 9, 3, 0.45, 3000)) == 0
+
+
+@pytest.mark.parametrize("sizes", [[1 + 7 * i % 90 for i in range(300)], [500 - i for i in range(40)]], ids=["many", "long"])
+def test_more_quarters_of_blocks_than_workgroups(ops, oracle, sizes):
+    rec = of_sizes(oracle, 21, sizes, 4, 8)
+    assert 4 * sum(-(-n // 64) for n in sizes) > 1024
+    same(run(ops, rec, len(sizes), 4, 0.45, len(rec) + 9000), oracle.nms(rec, 0.45), len(sizes))
