@@ -1218,7 +1218,7 @@ int bn_train_forward(const char* who, const float* x, float* y, float* pre_activ
     a.x = x; a.y = y; a.pre = pre_activation; a.x_saved = x_saved; a.x_norm = x_norm;
     a.residual = res.from; a.res_alpha = res.alpha; a.res_beta = res.beta;
     const ReduceGeom g = make_geom(batch, channels, spatial);
-    const bool chain = vec && !res.from && (activation == PXH_MISH || activation == PXH_SOFTPLUS);
+    const bool chain = vec && !res.from && chains_exponential(activation);
     if (finishes_inside(g, a.total, chain ? kFusedForwardChain : kFusedForward)) {
         // (the first value of a channel, which its sums are relative to, is kept: y may be x)
         float* const shifts = static_cast<float*>(coef_region(ws, batch, channels, spatial));

@@ -222,6 +222,12 @@ struct ResidentBwdArgs {
 // the large form (128-bit vectors only) 16 vectors in registers + 8 in LDS (128 KB of the CU's 160)
 constexpr int kResidentLargeRegs = 16, kResidentLargeLds = 8;
 constexpr size_t kResidentLargeLdsBytes = static_cast<size_t>(kResidentLargeLds) * kResidentThreads * 16;
+// What a forward takes u = 1 + exp(x) through.
+constexpr bool chains_exponential(int activation)
+{
+    return activation == PXH_MISH || activation == PXH_SOFTPLUS;
+}
+
 constexpr bool selects(int activation)
 {
     return activation == PXH_LEAKY || activation == PXH_RELU || activation == PXH_LINEAR;
@@ -321,17 +327,24 @@ inline int resident_vectors(int batch, int channels, int spatial, bool vec)
 constexpr int kOddSpatial = 4;
 constexpr uint32_t kOddVectors = 6144;
 constexpr uint32_t kOddVectorsFew = 4096;         // with fewer than kResidentChannels channels (as kSmallVectors)
+// ... where an exponential is followed by another chain: workgroups of 1024 lanes, with fewer of them than compute units, are longer
+// than several launches, us, mish, forward, backward, clipped with nothing to change, rescaled, clamped throughout: 90 x 16 x 13^2 10.1 -> 8.9,
+// 14.6 -> 11.9, 18.7 -> 17.6, 26.0 -> 17.5, 32.0 -> 20.2, 8 x 64 x 45^2 10.8 -> 10.1, 16.4 -> 16.1, 20.7 -> 24.3, 27.8 -> 24.0, 34.8 -> 30.1.  Not
+// logistic (8 x 64 x 45^2: 7.8 and 8.4, 11.0 and 11.5, 15.1 and 21.0), nor 60 x 64 x 13^2 (2640 vectors: 8.3 and 10.3, 12.6 and 15.2).
+constexpr uint32_t kOddVectorsFewChain = 3072;
 constexpr uint32_t kOddValues = 4 * kOddVectors, kOddValuesFew = 6144;
 constexpr int kOddChannels = 512;
 
 // The vectors (values in planes below kOddSpatial) of a channel's slice where such a shape takes a one-launch form, else 0.
-inline uint32_t odd_slice(int batch, int channels, int spatial, bool vec)
+inline uint32_t odd_slice(int batch, int channels, int spatial, bool vec, int activation, bool backward)
 {
     if (vec) return 0;
     const bool few = channels < kResidentChannels;
     const bool values = spatial < kOddSpatial;
     const size_t items = static_cast<size_t>(batch) * (values ? spatial : (spatial + 3) / 4);
-    const uint32_t most = values ? (few ? kOddValuesFew : kOddValues) : few ? kOddVectorsFew : kOddVectors;
+    // (the forward of planes of up to a wave's width stays: several launches give each a wave)
+    const bool chain = chains_exponential(activation) && (backward || spatial > kWave);
+    const uint32_t most = values ? (few ? kOddValuesFew : kOddValues) : few ? (chain ? kOddVectorsFewChain : kOddVectorsFew) : kOddVectors;
     return items <= most ? static_cast<uint32_t>(items) : 0;
 }
 
@@ -423,7 +436,7 @@ inline ResidentForm resident_form(int batch, int channels, int spatial, bool vec
 {
     return ResidentForm{ resident_vectors(batch, channels, spatial, vec),
                          small_slice(batch, channels, spatial, vec, activation, backward),
-                         odd_slice(batch, channels, spatial, vec) };
+                         odd_slice(batch, channels, spatial, vec, activation, backward) };
 }
 
 int launch_resident_forward(const char* who, const ResidentFwdArgs& r, const ResidentForm& form, int activation, hipStream_t s);

@@ -51,7 +51,14 @@ int main()
                         else if (backward) dispatch_odd_form<kOddOneStep<PXH_MISH, true>>(form.odd, g, one_step(512));
                         else dispatch_odd_form<kOddOneStep<PXH_MISH, false>>(form.odd, g, one_step(256));
                     }
-                const bool one = odd_slice(batch, channels, spatial, false) != 0;
+                const bool one = odd_slice(batch, channels, spatial, false, PXH_LEAKY, false) != 0;
+                const size_t vectors = static_cast<size_t>(batch) * ((spatial + 3) / 4);
+                for (bool backward: { false, true }) {
+                    const size_t most = channels >= 96 ? 6144 : backward || spatial > 64 ? 3072 : 4096;
+                    if (spatial >= 4) check((odd_slice(batch, channels, spatial, false, PXH_MISH, backward) != 0) == (vectors <= most), "a chain", batch, channels, spatial);
+                    if (spatial >= 4) check((odd_slice(batch, channels, spatial, false, PXH_LOGISTIC, backward) != 0) == one, "no chain", batch, channels, spatial);
+                }
+                if (spatial >= 4) check(one == (vectors <= (channels < 96 ? 4096u : 6144u)), "light", batch, channels, spatial);
                 if (spatial < 4) check(one == (values <= (channels < 96 ? 6144u : 24576u)), "planes below a vector", batch, channels, spatial);
                 // a workspace too small is refused on both sides of lines that may move: this one does not
                 check(asks_for_workspace(batch, channels, spatial, false) == (channels < 96 || values > 8192), "the workspace", batch, channels, spatial);
