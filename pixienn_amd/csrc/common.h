@@ -118,8 +118,8 @@ __device__ __forceinline__ float softplus_apply(float x)
     return logf(exp_before_one_plus(x) + 1.0f);
 }
 
-// num / den by the hardware's reciprocal (1 ulp) and one correction of the quotient by its remainder: within an ulp of the
-// quotient, mostly its rounded value, in five instructions where the compiler's division takes a dozen.  For den in
+// num / den by the hardware's reciprocal (1 ulp) and one correction of the quotient by its remainder, formed exactly by a fused
+// multiply-add (Markstein's method): within an ulp of the quotient, mostly its rounded value, in five instructions where the compiler's division takes a dozen.  For den in
 // [1, 2^126): no scaling.
 __device__ __forceinline__ float quotient(float num, float den)
 {

@@ -811,7 +811,7 @@ __global__ __launch_bounds__(kBlock) void bn_dx_scalar_kernel(DxArgs a)
 // first items are on their way, and the channel's first workgroup writes what is left of it.  A launch that does only that
 // is 4 us, whatever the size: a chain of trips to memory and double-precision roots.  Past a size the flat pass is ahead by
 // more, whose lanes take one vector each and past the caches.  Three launches -> two, us, leaky and mish: forward,
-// + shortcut, backward with the pre-activation kept (one without takes groups in most of these)
+// + shortcut, backward with the pre-activation kept (one without takes groups where planes are aligned)
 //   2 x 16 x 160^2       9.7 ->  7.8    9.9 ->  7.8   14.4 ->  9.7   10.2 ->  8.7   10.4 ->  8.6   18.9 -> 12.2
 //   4 x 64 x 104^2      13.9 -> 10.7   14.5 -> 11.1   23.2 -> 18.0   14.3 -> 12.2   14.7 -> 12.7   29.0 -> 22.6
 //   6 x 72 x 135 x 77   17.4 -> 13.1   19.8 -> 13.8   32.6 -> 28.0   17.6 -> 14.3   20.1 -> 15.5   40.0 -> 33.7
