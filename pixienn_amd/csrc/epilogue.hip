@@ -1119,7 +1119,7 @@ constexpr int kGroupAlone = 512;
 // where an exponential has to be computed (37 -> 41).
 GroupPlan grouped_backward(int batch, int channels, int spatial, bool vec, int per_thread, int activation, hipStream_t s)
 {
-    if (!enough_for_groups(static_cast<size_t>(batch) * channels * spatial, spatial, vec, selects(activation))) return GroupPlan{};
+    if (!enough_for_groups(static_cast<size_t>(batch) * channels * spatial, spatial, vec, activation)) return GroupPlan{};
     if (per_thread && (!selects(activation) || channels < kGroupAlone)) return GroupPlan{};
     const uint32_t places = group_places(s);
     // (as few members as hold the slice where the words of more would not fit: up to three channels of a few thousand vectors)

@@ -148,7 +148,7 @@ inline size_t group_fill(int channels)
     return whole > 0 ? whole : 1;
 }
 
-// Whether a tensor is large enough for groups; `light`: the gradient is a select.
+// Whether a tensor is large enough for groups.
 //
 // Small tensors (which the caches hold for the launches that read them twice) stay with those launches: a group's second one
 // costs them more where it has something to do.  Three or five launches -> groups, us: plain; clipped with nothing to change,
@@ -159,25 +159,29 @@ inline size_t group_fill(int channels)
 //   4 x 32 x 208^2        28.2 -> 23.8; 34.9 -> 28.1, 35.0 -> 36.7, 42.8 -> 45.0        39.7 -> 34.9; 46.7 -> 40.0, 46.8 -> 48.6, 63.6 -> 69.2
 // From there on the usual call gains a tenth to a quarter; one that clamps gains from 16 x 64 x 152^2 on (121 -> 107).
 //
-// Odd planes, whose several launches leave less to gain, only where the gradient is a select: before an exponential the calls
-// that find nothing to change gain a twentieth and those that rescale or clamp lose a fifth.  Planes of 256 values and more from
-// 7 M values on, below which two launches that finish the channels serve a plain call better and a clipped one loses wherever
-// something changes; smaller ones, of which the launches give each a wave, from 1 M on.
+// Odd planes, whose several launches leave less to gain: planes of 256 values and more from 7 M values on, below which two launches
+// that finish the channels serve a plain call better and a clipped one loses wherever something changes; smaller ones, of which the
+// launches give each a wave, from 1 M on where the gradient is a select.  Not mish, whose gradient wants more registers than a
+// lane of these has: there the calls that find nothing to change gain a twentieth, and those that rescale or clamp lose a fifth.
 //   2 x 16 x 151^2      leaky  9.6 -> 11.9; 17.9 -> 16.0, 17.9 -> 20.3, 20.1 -> 24.1
 //   6 x 72 x 135 x 77         20.7 -> 23.1; 35.0 -> 27.9, 35.4 -> 35.8, 41.8 -> 43.9
 //   8 x 96 x 135 x 77         36.1 -> 26.4; 43.7 -> 31.7, 44.0 -> 43.7, 56.8 -> 52.4   mish 47.4 -> 46.8; 55.5 -> 53.4, 56.5 -> 65.8, 78.9 -> 97.8
 //   16 x 64 x 151^2           88.5 -> 66.0; 95.4 -> 72.4, 95.4 -> 105,  123  -> 119         95.8 -> 92.3; 105 -> 103, 106 -> 136, 158 -> 185
 //   16 x 90 x 151^2           123  -> 85.5; 130  -> 89.6, 129  -> 134,  169  -> 149         133  -> 113;  144 -> 131, 144 -> 178, 202 -> 235
+//   8 x 96 x 135 x 77, logistic 40.5 -> 30.7; 48.5 -> 35.4, 48.4 -> 47.2, 64.7 -> 58.6       tanh 41.9 -> 31.2; 49.7 -> 37.6, 49.9 -> 49.6, 67.0 -> 66.8
+//   16 x 64 x 151^2, logistic   89.7 -> 69.7; 103 -> 76.3,  103  -> 109,  137  -> 127
 //   200 x 16 x 13^2           12.4 -> 12.3; 18.3 -> 16.3, 18.6 -> 20.1, 21.1 -> 24.0
 //   400 x 16 x 13^2           16.6 -> 14.0; 23.7 -> 18.0, 24.1 -> 22.3, 27.5 -> 26.2
 //   3000 x 40 x 5^2           36.4 -> 25.6; 46.5 -> 30.1, 47.3 -> 37.4, 61.7 -> 47.5
 constexpr size_t kGroupFewest = 1u << 19, kGroupFewestSmooth = 1u << 20, kGroupFewestOdd = 7u << 20, kGroupFewestOddSmall = 1u << 20;
 constexpr int kGroupOddSmall = 256;
 
-inline bool enough_for_groups(size_t total, int spatial, bool vec, bool light)
+inline bool enough_for_groups(size_t total, int spatial, bool vec, int activation)
 {
+    const bool light = selects(activation);
     if (vec) return total >= (light ? kGroupFewest : kGroupFewestSmooth);
-    return light && spatial >= kOddSpatial && total >= (spatial < kGroupOddSmall ? kGroupFewestOddSmall : kGroupFewestOdd);
+    if (spatial < kOddSpatial || activation == PXH_MISH) return false;
+    return total >= (light && spatial < kGroupOddSmall ? kGroupFewestOddSmall : kGroupFewestOdd);
 }
 
 constexpr uint32_t kLooks = 1u << 22;

@@ -53,15 +53,16 @@ int main()
         check(p.members == n.members && p.span == n.span, "the split of a named slice", n.items, n.channels, 512);
     }
 
-    // tensors that take groups: aligned, and odd planes where the gradient is a select
-    const struct { size_t total; int spatial; bool vec, light, groups; } sizes[] = {
-        { 1u << 19, 4, true, true, true }, { (1u << 19) - 1, 4, true, true, false }, { 1u << 20, 4, true, false, true },
-        { (1u << 20) - 1, 4, true, false, false }, { 7u << 20, 257, false, true, true }, { (7u << 20) - 1, 257, false, true, false },
-        { 1u << 29, 257, false, false, false }, { 1u << 20, 255, false, true, true }, { (1u << 20) - 1, 255, false, true, false },
-        { 1u << 20, 256, false, true, false }, { 1u << 29, 13, false, false, false }, { 1u << 29, 3, false, true, false },
+    // tensors that take groups: aligned, and odd planes
+    const struct { size_t total; int spatial; bool vec; int activation; bool groups; } sizes[] = {
+        { 1u << 19, 4, true, PXH_LEAKY, true }, { (1u << 19) - 1, 4, true, PXH_LEAKY, false }, { 1u << 20, 4, true, PXH_MISH, true },
+        { (1u << 20) - 1, 4, true, PXH_MISH, false }, { 7u << 20, 257, false, PXH_LEAKY, true }, { (7u << 20) - 1, 257, false, PXH_LEAKY, false },
+        { 7u << 20, 257, false, PXH_LOGISTIC, true }, { (7u << 20) - 1, 13, false, PXH_SWISH, false }, { 7u << 20, 13, false, PXH_TANH, true },
+        { 1u << 29, 257, false, PXH_MISH, false }, { 1u << 20, 255, false, PXH_RELU, true }, { (1u << 20) - 1, 255, false, PXH_RELU, false },
+        { 1u << 20, 256, false, PXH_LINEAR, false }, { 1u << 29, 3, false, PXH_LEAKY, false }, { 1u << 29, 3, false, PXH_LOGISTIC, false },
     };
     for (const auto& n: sizes)
-        check(enough_for_groups(n.total, n.spatial, n.vec, n.light) == n.groups, "a tensor large enough", n.total, n.spatial, 0);
+        check(enough_for_groups(n.total, n.spatial, n.vec, n.activation) == n.groups, "a tensor large enough", n.total, n.spatial, 0);
 
     uint32_t mask[4] = {};
     check(units_of_mask(mask, 4, 256) == 256, "no mask", 0, 0, 0);

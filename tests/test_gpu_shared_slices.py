@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 # tests/host/split_check.cpp.
 VECTORS = [(1, 95, 16388), (4, 64, 6144), (7, 30, 10012), (3, 12, 32772), (1, 8, 532480), (1, 7, 532480), (4, 32, 98304),
            (3, 130, 32772), (4, 512, 4112)]
-# odd planes (groups where the gradient is a select): five members, twelve, and sixteen that are full (but for the last value, which its vector shares)
+# odd planes (groups but for mish): five members, twelve, and sixteen that are full (but for the last value, which its vector shares)
 ODD = [(8, 96, 10395), (32, 41, 5625), (1, 32, 393215)]
 
 
@@ -33,6 +33,12 @@ def test_shared_slices_backward(ops, oracle, monkeypatch, shape, act):
         monkeypatch.setattr(module, "TRAIN_SHAPES", [shape])
     epilogue.test_bn_backward_matches_oracle(ops, oracle, act, False)
     clipped.test_bn_backward_clipped_matches_rescale_clip_then_backward(ops, oracle, act, False)
+
+
+@pytest.mark.parametrize("act", ["logistic", "softplus"])
+@pytest.mark.parametrize("shape", ODD, ids=str)
+def test_shared_slices_of_odd_planes_before_an_exponential(ops, oracle, monkeypatch, shape, act):
+    test_shared_slices_backward(ops, oracle, monkeypatch, shape, act)
 
 
 class Layer:
