@@ -819,10 +819,11 @@ __global__ __launch_bounds__(kBlock) void bn_dx_scalar_kernel(DxArgs a)
 //   9 x 20 x 203 x 251  26.4 -> 22.3   31.9 -> 26.7   48.6 -> 51.3   27.2 -> 23.7   32.6 -> 27.6   58.6 -> 61.3
 //   4 x 16 x 416^2      29.0 -> 27.4   35.9 -> 33.1   56.0 -> 60.2   29.3 -> 29.7   36.3 -> 37.9   66.0 -> 69.8
 //   8 x 16 x 416^2      47.0 -> 45.8   60.2 -> 69.2   104  -> 123    47.1 -> 49.6   61.6 -> 77.8   122  -> 136
-// (6 x 72 x 135 x 77, mish, without the pre-activation: 31.5 -> 28.4.)  The forward's line lies lower where an exponential is
-// followed by another chain, the planes are aligned and no shortcut is on top: 16 x 48 x 104^2, mish, 23.7 -> 25.0, softplus 24.0 -> 26.0,
-// 4 x 16 x 392^2 26.2 -> 27.3 and 26.1 -> 29.2, but 8 x 80 x 104^2 20.9 -> 19.3 and 21.4 -> 21.2, logistic 22.7 -> 19.4 and 25.2 -> 22.9; with a
-// shortcut 28.3 -> 26.2, and odd planes (8 x 60 x 133^2, mish) 24.5 -> 22.1, with one 28.5 -> 26.7.
+// (6 x 72 x 135 x 77, mish, without the pre-activation: 31.5 -> 28.4.)  The forward's line lies lower where the
+// exponential is followed by a logarithm, and for mish on aligned planes with no shortcut on top: softplus 8 x 80 x 104^2 21.4 -> 21.2, but
+// 16 x 48 x 104^2 24.0 -> 26.0, 4 x 16 x 392^2 26.1 -> 29.2, 38 x 69 x 47 x 85 28.5 -> 35.8, with a shortcut 33.9 -> 39.4; mish 8 x 80 x 104^2
+// 20.9 -> 19.3, 16 x 48 x 104^2 23.7 -> 25.0, 4 x 16 x 392^2 26.2 -> 27.3, with a shortcut 28.3 -> 26.2 and 31.2 -> 29.6, odd planes
+// (8 x 60 x 133^2) 24.5 -> 22.1, with one 28.5 -> 26.7; logistic 22.7 -> 19.4 and 25.2 -> 22.9.
 // ------------------------------------------------------------------------------------------
 constexpr int kFusedPartials = 4 * kWave;      // of a channel: a lane of the first wave takes four
 constexpr uint32_t kFusedForward = 10u << 20, kFusedForwardChain = 7u << 20, kFusedBackward = 6u << 20;      // values of a tensor
@@ -1218,7 +1219,7 @@ int bn_train_forward(const char* who, const float* x, float* y, float* pre_activ
     a.x = x; a.y = y; a.pre = pre_activation; a.x_saved = x_saved; a.x_norm = x_norm;
     a.residual = res.from; a.res_alpha = res.alpha; a.res_beta = res.beta;
     const ReduceGeom g = make_geom(batch, channels, spatial);
-    const bool chain = vec && !res.from && chains_exponential(activation);
+    const bool chain = activation == PXH_SOFTPLUS || (activation == PXH_MISH && vec && !res.from);
     if (finishes_inside(g, a.total, chain ? kFusedForwardChain : kFusedForward)) {
         // (the first value of a channel, which its sums are relative to, is kept: y may be x)
         float* const shifts = static_cast<float*>(coef_region(ws, batch, channels, spatial));
